@@ -231,8 +231,14 @@ static int pick_family(const cuasr_amd_srgemm_desc *d, long long batch = 1) {
   const long long direct_groups = (long long)((c.m + tile_m - 1) / tile_m) * ((c.n + tile_n - 1) / tile_n) * d->split_k_slices * batch;
   const long long rounds = (direct_groups + slots - 1) / slots;
   // >= 7/8 of its rounds (fp64: 95 % -- its staged tile is within 10 % of the direct one, so a last round that
-  // is 11 % empty, 5120^2, already costs more than the direct tile gains: 28.3 against 29.5 TOPS)
-  const bool fills = f64 ? direct_groups * 100 >= rounds * slots * 95 : direct_groups * 8 >= rounds * slots * 7;
+  // is 11 % empty, 5120^2, already costs more than the direct tile gains: 28.3 against 29.5 TOPS) ...
+  const bool rounds_filled = f64 ? direct_groups * 100 >= rounds * slots * 95 : direct_groups * 8 >= rounds * slots * 7;
+  // ... with outputs that exist: its tiles may not cover more than 1.15 times what the staged family's 64 x 64 tiles
+  // cover, which is about what its rate is worth (1024 products of 64^3: 58.6 us on mostly empty tiles of 256 x 128,
+  // 18.6 on the staged ones; 2048 products of 100^3 in double, whose 128 x 128 tiles cover no more: 262 against 302)
+  const double covered = (double)direct_groups * tile_m * tile_n;
+  const double covered64 = 4096.0 * ((c.m + 63) / 64) * ((c.n + 63) / 64) * d->split_k_slices * (double)batch;
+  const bool fills = rounds_filled && covered <= 1.15 * covered64;
   const bool have_valu = find_valu(d->dtype, d->add_op, d->mult_op) != nullptr;
   // or-and: the staged tile turns its panels into masks on their way to LDS and spends one
   // `acc | (a & b)` per term; the direct tile cannot (its panels never pass through registers)

@@ -232,6 +232,23 @@ template <typename T, typename TI = T> __device__ __forceinline__ void select_ba
   }
 }
 
+// The same without writing to the problem record
+struct Operands {
+  const void *A, *B, *C;
+  void *D;
+};
+template <typename T> __device__ __forceinline__ Operands batch_operands(const Problem &p) {
+  Operands o{p.A, p.B, p.C, p.D};
+  if (p.batch > 1) {
+    const long long z = blockIdx.z;
+    o.A = reinterpret_cast<const T *>(p.A) + z * p.batch_a;
+    o.B = reinterpret_cast<const T *>(p.B) + z * p.batch_b;
+    if (p.C) o.C = reinterpret_cast<const T *>(p.C) + z * p.batch_c;
+    o.D = reinterpret_cast<T *>(p.D) + z * p.batch_d;
+  }
+  return o;
+}
+
 // Epilogue scalars resolved on the device (alpha/beta may live in device memory).
 template <typename T> struct EpilogueScalars {
   T alpha, beta, ident;

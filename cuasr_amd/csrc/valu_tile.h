@@ -374,22 +374,31 @@ struct ValuTile {
   // as they stand (no mask to turn back, no zero whose sign depends on the rest of the range).
   static constexpr bool SUB_SLICES = has_native_fold<T, ADD>::value && !MASKED && !ZERO_SIGN;
 
-  static __device__ __forceinline__ void run(const Problem &p, Smem &sm) {
+  // (asked for before the product: at its end the compiler wants the problem record's scalars in memory it can address,
+  // and every lane of every wave then starts by storing 64 bytes of them -- 16 MB for a batch of 1000 products of 32^3)
+  static __device__ __forceinline__ EpilogueScalars<T> scalars(const Problem &p) {
+    if (!p.workspace) return resolve_scalars<T>(p, MUL);
+    const T ident = scalar_as<T>(p.add_identity);
+    return EpilogueScalars<T>{ident, ident, ident, false};
+  }
+
+  static __device__ __forceinline__ void run(const Problem &p, const Operands &o, Smem &sm) {
     int m0, n0, kb, ke;
     tile_and_range(p, m0, n0, kb, ke);
+    const EpilogueScalars<T> e = scalars(p);
     S acc[TM][TN];
-    accumulate(p, sm, m0, n0, kb, ke, (ke - kb + BK - 1) / BK, acc);
-    finish(p, acc, m0, n0, kb, ke);
+    accumulate(p, o, sm, m0, n0, kb, ke, (ke - kb + BK - 1) / BK, acc);
+    finish(p, o, e, acc, m0, n0, kb, ke);
   }
 
   // acc = identity, then the terms of k in [kb, ke).  The 256 threads that share `sm` pass
   // 1 + `sync_tiles` barriers (sync_tiles >= the number of k-tiles of the range, so that groups of
   // one workgroup whose ranges differ in length stay in step).
-  static __device__ __forceinline__ void accumulate(const Problem &p, Smem &sm, int m0, int n0, int kb, int ke, int sync_tiles,
-                                                    S (&acc)[TM][TN]) {
+  static __device__ __forceinline__ void accumulate(const Problem &p, const Operands &o, Smem &sm, int m0, int n0, int kb, int ke,
+                                                    int sync_tiles, S (&acc)[TM][TN]) {
     const int tid = threadIdx.x & 255, tx = tid & 15, ty = tid >> 4;
-    const T *A = reinterpret_cast<const T *>(p.A);
-    const T *B = reinterpret_cast<const T *>(p.B);
+    const T *A = reinterpret_cast<const T *>(o.A);
+    const T *B = reinterpret_cast<const T *>(o.B);
     const T ident = scalar_as<T>(p.add_identity);
     const bool a_xc = p.sa_m == 1, b_xc = p.sb_n == 1;
 
@@ -470,49 +479,68 @@ struct ValuTile {
 
   // ---- epilogue: D = add(mult(alpha, acc), mult(beta, C)), or raw partials; [kb, ke) is the
   // k range the accumulators cover (ZERO_SIGN looks into it)
-  // (row_step, row_first: only the rows i = row_first, row_first + row_step, ... of the thread's outputs)
-  static __device__ __forceinline__ void finish(const Problem &p, S (&acc)[TM][TN], int m0, int n0, int kb, int ke,
-                                                int row_step = 1, int row_first = 0) {
+  // (acc[q] is row i = row_first + q row_step of the thread's outputs)
+  template <int NR>
+  static __device__ __forceinline__ void finish(const Problem &p, const Operands &o, const EpilogueScalars<T> &e, S (&acc)[NR][TN],
+                                                int m0, int n0, int kb, int ke, int row_step = 1, int row_first = 0) {
     const int tid = threadIdx.x & 255, tx = tid & 15, ty = tid >> 4;
-    const T *A = reinterpret_cast<const T *>(p.A);
-    const T *B = reinterpret_cast<const T *>(p.B);
-    const T ident = scalar_as<T>(p.add_identity);
-    T *out;
-    long long ld_out;
+    const T *A = reinterpret_cast<const T *>(o.A);
+    const T *B = reinterpret_cast<const T *>(o.B);
+    T *out = reinterpret_cast<T *>(o.D);
+    long long ld_out = p.ldd;
     const bool partial = p.workspace != nullptr;
-    EpilogueScalars<T> e;
     if (partial) {
       out = reinterpret_cast<T *>(p.workspace) + (long long)(p.k_sub > 1 ? blockIdx.y / p.k_sub : blockIdx.y) * p.m * p.n;
       ld_out = p.n;
-      e.alpha = e.beta = e.ident = ident;
-      e.source_needed = false;
-    } else {
-      out = reinterpret_cast<T *>(p.D);
-      ld_out = p.ldd;
-      e = resolve_scalars<T>(p, MUL);
     }
+    auto row_of = [&](int q) {
+      const int i = row_first + q * row_step;
+      return m0 + ty * VW + (i / VW) * 16 * VW + (i % VW);
+    };
     if constexpr (SUB_SLICES) {
       if (partial && p.k_sub > 1) {
         // one of several workgroups on this slice's tile: fold into the partial tile, which the host has filled
         // with the additive identity
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int row = m0 + ty * VW + (i / VW) * 16 * VW + (i % VW);
-          if (row >= p.m || i % row_step != row_first) continue;
+        for (int q = 0; q < NR; ++q) {
+          const int row = row_of(q);
+          if (row >= p.m) continue;
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
             const int col = n0 + tx * VW + (j / VW) * 16 * VW + (j % VW);
-            if (col < p.n) native_fold<ADD>(out + (long long)row * ld_out + col, acc[i][j]);
+            if (col < p.n) native_fold<ADD>(out + (long long)row * ld_out + col, acc[q][j]);
           }
         }
         return;
       }
     }
-    const T *C = reinterpret_cast<const T *>(p.C);
+    const T *C = reinterpret_cast<const T *>(o.C);
+    // All of the thread's source elements are requested together, at clamped indices (the main loop's fragments are
+    // dead, so there are registers for them): D may be C, so the compiler keeps every load behind the store before it,
+    // and a round trip to memory per row made a short product's epilogue as long as the product.
+    T src[NR][TN];
+    if (e.source_needed) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int row = m0 + ty * VW + (i / VW) * 16 * VW + (i % VW);
-      if (row >= p.m || i % row_step != row_first) continue;
+      for (int q = 0; q < NR; ++q) {
+        const T *row = C + (long long)min(row_of(q), p.m - 1) * p.ldc;
+#pragma unroll
+        for (int g = 0; g < GN; ++g) {
+          const int col = n0 + tx * VW + g * 16 * VW;
+          if (VEC && (!CAREFUL || col + VW <= p.n)) {
+            const gvec_t t = *reinterpret_cast<const gvec_t *>(row + (CAREFUL ? col : min(col, p.n - VW)));
+#pragma unroll
+            for (int c = 0; c < VW; ++c) src[q][g * VW + c] = t[c];
+          } else {
+#pragma unroll
+            for (int c = 0; c < VW; ++c) src[q][g * VW + c] = row[min(col + c, p.n - 1)];
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      const int row = row_of(q);
+      if (row >= p.m) continue;
 #pragma unroll
       for (int g = 0; g < GN; ++g) {
         const int col = n0 + tx * VW + g * 16 * VW;
@@ -521,9 +549,9 @@ struct ValuTile {
 #pragma unroll
         for (int c = 0; c < VW; ++c) {
           if constexpr (MASKED) {
-            v[c] = acc[i][g * VW + c] ? T(1) : T(0);
+            v[c] = acc[q][g * VW + c] ? T(1) : T(0);
           } else {
-            v[c] = acc[i][g * VW + c];
+            v[c] = acc[q][g * VW + c];
             if constexpr (ZERO_SIGN) {
               if (v[c] == T(0) && ke > kb)
                 v[c] = last_zero_product(A + (long long)row * p.sa_m + (long long)kb * p.sa_k, p.sa_k,
@@ -536,17 +564,8 @@ struct ValuTile {
 #pragma unroll
           for (int c = 0; c < VW; ++c) v[c] = Op<MUL>::apply(e.alpha, v[c]);
           if (e.source_needed) {
-            T src[VW];
-            if (VEC && (!CAREFUL || col + VW <= p.n)) {
-              const gvec_t t = *reinterpret_cast<const gvec_t *>(C + (long long)row * p.ldc + col);
 #pragma unroll
-              for (int c = 0; c < VW; ++c) src[c] = t[c];
-            } else {
-#pragma unroll
-              for (int c = 0; c < VW; ++c) src[c] = C[(long long)row * p.ldc + min(col + c, p.n - 1)];
-            }
-#pragma unroll
-            for (int c = 0; c < VW; ++c) v[c] = fold_epilogue<ADD, MUL>(v[c], Op<MUL>::apply(e.beta, src[c]));
+            for (int c = 0; c < VW; ++c) v[c] = fold_epilogue<ADD, MUL>(v[c], Op<MUL>::apply(e.beta, src[q][g * VW + c]));
           }
         }
         if (VEC && (!CAREFUL || col + VW <= p.n)) {
@@ -560,17 +579,15 @@ struct ValuTile {
             if (col + c < p.n) out[(long long)row * ld_out + col + c] = v[c];
         }
       }
-      __builtin_amdgcn_sched_barrier(0);  // one row of C in flight at a time
     }
   }
 };
 
 template <typename T, int ADD, int MUL, int TM, int TN, int BK, bool VEC, bool CAREFUL = false>
-__global__ __launch_bounds__(256) WAVES_ATTR void valu_srgemm_kernel(Problem p) {
+__global__ __launch_bounds__(256) WAVES_ATTR void valu_srgemm_kernel(const Problem p) {
   using Tile = ValuTile<T, ADD, MUL, TM, TN, BK, VEC, CAREFUL>;
   __shared__ typename Tile::Smem sm;
-  select_batch<T>(p);
-  Tile::run(p, sm);
+  Tile::run(p, batch_operands<T>(p), sm);
 }
 
 // The same tile with the k range shared out inside the workgroup, for launches that would
@@ -584,59 +601,48 @@ __global__ __launch_bounds__(256) WAVES_ATTR void valu_srgemm_kernel(Problem p) 
 template <typename T, int ADD> struct order_free : std::integral_constant<bool, !(ADD == kPlus && is_fp<T>::value)> {};
 
 template <typename T, int ADD, int MUL, int TM, int TN, int BK, bool VEC, bool CAREFUL, int G>
-__global__ __launch_bounds__(256 * G) void valu_ksplit_kernel(Problem p) {
+__global__ __launch_bounds__(256 * G) void valu_ksplit_kernel(const Problem p) {
   using Tile = ValuTile<T, ADD, MUL, TM, TN, BK, VEC, CAREFUL>;
   using S = typename Tile::S;
   static_assert(order_free<T, ADD>::value, "a floating-point sum depends on the grouping of its terms");
-  static_assert(G * sizeof(typename Tile::Smem) >= (G - 1) * sizeof(S) * TM * TN * 256 && TM % G == 0, "the groups' accumulators must fit the panel space");
-  __shared__ typename Tile::Smem sm[G];
-  select_batch<T>(p);
+  static_assert(TM % G == 0, "whole rows of the threads' outputs per group");
+  __shared__ union {
+    typename Tile::Smem panels[G];
+    S acc[G][TM * TN * 256];
+  } sm;
+  const Operands o = batch_operands<T>(p);
   const int g = threadIdx.x >> 8, tid = threadIdx.x & 255;
   int m0, n0, kb, ke;
   Tile::tile_and_range(p, m0, n0, kb, ke);
+  const EpilogueScalars<T> e = Tile::scalars(p);
   const int tiles = max((ke - kb + BK - 1) / BK, 0), per = (tiles + G - 1) / G;
   const int gkb = min(ke, kb + g * per * BK), gke = min(ke, gkb + per * BK);
   S acc[TM][TN];
-  Tile::accumulate(p, sm[g], m0, n0, gkb, gke, per, acc);  // ends with a barrier: every group is done with its panels
-  // The panels are dead now.  Group d takes the rows i = d, d + G, ... of the threads' outputs: every group leaves
-  // its accumulators of the other groups' rows in the panel space, and each group then folds its rows over the
-  // groups in ascending k order (acc = add(acc, partial), as the split-K reduction does) and runs their epilogue --
-  // one G-th of the fold, of the reads of C and of the stores each.
-  // Where group h's row i (of group i % G != h) lies: rows in the order of i, without h's own
-  constexpr int ROWS_OUT = TM - TM / G, AREA = ROWS_OUT * TN * 256;
-  auto slot = [](int h, int i) { return (i / G) * (G - 1) + (i % G < h ? i % G : i % G - 1); };
-  S *area = reinterpret_cast<S *>(&sm[0]);
+  Tile::accumulate(p, o, sm.panels[g], m0, n0, gkb, gke, per, acc);  // ends with a barrier: every group is done with its panels
+  // The panels are dead now: their space takes every group's accumulators.  Group d then takes the rows i = d, d + G,
+  // ... of the threads' outputs, folds them over the groups in ascending k order (acc = add(acc, partial), as the
+  // split-K reduction does) and runs their epilogue -- one G-th of the fold, of the reads of C and of the stores each.
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    if (i % G == g) continue;
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) area[g * AREA + (slot(g, i) * TN + j) * 256 + tid] = acc[i][j];
-  }
+    for (int j = 0; j < TN; ++j) sm.acc[g][(i * TN + j) * 256 + tid] = acc[i][j];
   __syncthreads();
+  S part[TM / G][TN];
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    if (i % G != g) continue;
+  for (int q = 0; q < TM / G; ++q)
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      S v = acc[i][j];  // (overwritten unless g == 0)
+      const int at = ((g + q * G) * TN + j) * 256 + tid;
+      S v = sm.acc[0][at];
 #pragma unroll
-      for (int h = 0; h < G; ++h) {
-        if (h == i % G) {  // this row's own group: from its registers
-          if (h > 0) {
-            if constexpr (Tile::MASKED) v |= acc[i][j];
-            else v = Op<ADD>::apply(v, acc[i][j]);
-          }
-        } else {
-          const S w = area[h * AREA + (slot(h, i) * TN + j) * 256 + tid];
-          if (h == 0) v = w;
-          else if constexpr (Tile::MASKED) v |= w;
-          else v = Op<ADD>::apply(v, w);
-        }
+      for (int h = 1; h < G; ++h) {
+        const S w = sm.acc[h][at];
+        if constexpr (Tile::MASKED) v |= w;
+        else v = Op<ADD>::apply(v, w);
       }
-      acc[i][j] = v;
+      part[q][j] = v;
     }
-  }
-  Tile::finish(p, acc, m0, n0, kb, ke, G, g);
+  Tile::finish(p, o, e, part, m0, n0, kb, ke, G, g);
 }
 
 // Extents along every contiguous direction are multiples of the vector width: no vector straddles
@@ -672,6 +678,10 @@ static void launch_ksplit(const Problem &p, dim3 grid, hipStream_t s) {
     launch_kernel((valu_ksplit_kernel<T, ADD, MUL, TM, TN, BK, true, true, G>), grid, dim3(256 * G), 0, s, p);
 }
 
+}  // namespace cuasr_amd
+#include "small_tile.h"
+namespace cuasr_amd {
+
 #ifndef CUASR_AMD_KSPLIT2_MAX
 #define CUASR_AMD_KSPLIT2_MAX 1024
 #endif
@@ -685,10 +695,11 @@ static hipError_t launch_valu(const Problem &p, hipStream_t s) {
   dim3 grid((unsigned)tiles, slice_groups(p), p.batch);
   if constexpr (KSPLIT && order_free<T, ADD>::value) {
     // 256 compute units: up to 256 workgroups get four groups (1024 threads, four waves per SIMD),
-    // up to 512 two; each group wants a few k-tiles of its own to be worth the fold at the end
+    // up to 1024 two; each group wants a k-tile or more of its own to be worth the fold at the end (900 x 900 x 200
+    // in k-tiles of 16: 10.5 us against 17.8 in one group)
     const long long groups = tiles * grid.y * grid.z;
     const long long k_range = p.workspace ? p.k_per_slice / (p.k_sub > 1 ? p.k_sub : 1) : p.k;
-    if (vector_possible<T>(p) && k_range >= 8LL * BK) {
+    if (vector_possible<T>(p) && k_range >= 128) {
       if (groups <= 256) {
         launch_ksplit<T, ADD, MUL, TM, TN, BK, 4>(p, grid, s);
         return take_launch_status();
@@ -723,19 +734,27 @@ static hipError_t launch_valu(const Problem &p, hipStream_t s) {
 template <typename T, int ADD, int MUL, int TM, int TN, int BK, int TM_SMALL, int TN_SMALL, int BK_SMALL = BK>
 static hipError_t launch_valu_sized(const Problem &p, hipStream_t s) {
   constexpr int BM = 16 * TM, BN = 16 * TN;
+  if constexpr (order_free<T, ADD>::value) {
+    if (small_preferred<T, ADD>(p)) return launch_small<T, ADD, MUL>(p, s);
+  }
   const long long groups = (long long)((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN) * slice_groups(p) * p.batch;
   const long long rounds = (groups + 1023) / 1024;
+  // ... and those tiles do not reach much further past the edges than the quarter-size ones: a batch of 1000 products of
+  // 64 x 64 filled 1000 full-size tiles to a quarter (37.8 us; 18.2 on the quarter-size ones)
+  constexpr int SM = 16 * TM_SMALL, SN = 16 * TN_SMALL;
+  const long long groups_small = (long long)((p.m + SM - 1) / SM) * ((p.n + SN - 1) / SN) * slice_groups(p) * p.batch;
+  const bool covers_more = groups * BM * BN * 16 > groups_small * SM * SN * 17;
   if constexpr (order_free<T, ADD>::value) {
     // 192 .. 256 full-size workgroups (2048^2: exactly 256) are one per compute unit for most of the
     // chip: two groups per workgroup give every SIMD its two waves, and the full-size tile then runs
     // at the rate it has on large problems, which the quarter-size tile does not reach
     const long long k_range = p.workspace ? p.k_per_slice / (p.k_sub > 1 ? p.k_sub : 1) : p.k;
-    if (groups >= 192 && groups <= 256 && k_range >= 8LL * BK && vector_possible<T>(p) && p.m > 0 && p.n > 0) {
+    if (groups >= 192 && groups <= 256 && !covers_more && k_range >= 8LL * BK && vector_possible<T>(p) && p.m > 0 && p.n > 0) {
       launch_ksplit<T, ADD, MUL, TM, TN, BK, 2>(p, dim3((unsigned)(groups / slice_groups(p) / p.batch), slice_groups(p), p.batch), s);
       return take_launch_status();
     }
   }
-  if (groups * 100 < rounds * 1024 * (long long)(CUASR_AMD_FULL_TILE_FILL_PERCENT))
+  if (covers_more || groups * 100 < rounds * 1024 * (long long)(CUASR_AMD_FULL_TILE_FILL_PERCENT))
     return launch_valu<T, ADD, MUL, TM_SMALL, TN_SMALL, BK_SMALL, true>(p, s);
   return launch_valu<T, ADD, MUL, TM, TN, BK>(p, s);
 }
