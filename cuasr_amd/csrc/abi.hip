@@ -29,8 +29,6 @@ bool direct_can_run(const Problem &);
 bool direct64_can_run(const Problem &);
 bool mfma_f32_can_run(const Problem &);
 bool mfma_f64_can_run(const Problem &);
-bool mfma_direct_f32_can_run(const Problem &);
-bool mfma_direct_f64_can_run(const Problem &);
 
 launch_fn find_or_and_on_masks(int dtype);
 
@@ -204,8 +202,8 @@ enum Family { kNaive = 1, kValu = 2, kMfma = 3, kDirect = 4, kStreamK = 5 };
 static int pick_family(const cuasr_amd_srgemm_desc *d, long long batch = 1) {
   if (d->kernel != CUASR_AMD_KERNEL_AUTO) return d->kernel;
   // plus-times is the one semiring a matrix instruction computes as is
-  // (its tile is 128 x 128: below 128 tiles half the compute units and more stand idle, and the
-  // vector-ALU tiles, which are smaller, are faster -- 1024^3: 31 against 22 TFLOP/s)
+  // (its tile is 128 x 128: below 128 tiles half the compute units and more stand idle; float and double then run on
+  // the matrix cores in smaller blocks, under the name of the family those outputs belong to -- family_fn)
   // (binary16: the matrix-core kernel accumulates in float and is not bit-identical to the binary16 sums of the
   // vector-ALU tile and the oracle, so it runs only when the descriptor asks for it)
   if (d->add_op == kPlus && d->mult_op == kMultiplies && d->dtype != CUASR_AMD_F16 && mfma_usable(d)) {
@@ -337,7 +335,13 @@ static launch_fn family_fn(int family, const cuasr_amd_srgemm_desc *d) {
   switch (family) {
     case kMfma: return find_mfma(d->dtype, d->add_op, d->mult_op);
     case kDirect: return find_direct(d->dtype, d->add_op, d->mult_op);
-    case kValu: return find_valu(d->dtype, d->add_op, d->mult_op);
+    case kValu:
+      // AUTO's plus-times in float and double below 128 tiles of 128 x 128: the matrix cores in blocks of 32 x 32
+      // (1024^3: 25 - 28 us against 81 on the vector ALU; sums in the matrix instruction's order, as in larger products)
+      if (d->kernel == CUASR_AMD_KERNEL_AUTO && d->add_op == kPlus && d->mult_op == kMultiplies &&
+          (d->dtype == CUASR_AMD_F32 || d->dtype == CUASR_AMD_F64))
+        return find_mfma(d->dtype, d->add_op, d->mult_op);
+      return find_valu(d->dtype, d->add_op, d->mult_op);
     default: return find_naive(d->dtype);
   }
 }
@@ -365,13 +369,8 @@ static int batched_family(const cuasr_amd_srgemm_desc *desc, int batch, int64_t 
   }
   bool in_grid = (family == kValu || family == kDirect) && batch > 1;
   if (family == kMfma && batch > 1 && desc->add_op == kPlus && desc->mult_op == kMultiplies) {
-    // the hand-scheduled matrix-core tiles take a batch in the grid too; the compiled ones (ragged k, unaligned
-    // products) do not: ask with the first launch's problem
-    Problem probe = canonical(desc);
-    probe.batch = batch < 65535 ? batch : 65535;
-    probe.batch_a = col ? stride_b : stride_a;
-    probe.batch_b = col ? stride_a : stride_b;
-    in_grid = (desc->dtype == CUASR_AMD_I8 || desc->dtype == CUASR_AMD_F16) ? true : desc->dtype == CUASR_AMD_F64 ? mfma_direct_f64_can_run(probe) : mfma_direct_f32_can_run(probe);
+    // the matrix-core launchers take the batch as it is: in the grid wherever that is the faster way
+    in_grid = true;
   }
   *in_grid_out = in_grid;
   return family;

@@ -85,6 +85,21 @@ static inline bool can_run(const Problem &p) {
   return true;
 }
 
+// the products of a batch one after the other, for kernels that take one per launch
+template <typename T> static inline hipError_t launch_each(Problem p, hipStream_t s, hipError_t (*one)(const Problem &, hipStream_t)) {
+  const int batch = p.batch;
+  p.batch = 1;
+  hipError_t e = hipSuccess;
+  for (int i = 0; i < batch && e == hipSuccess; ++i) {
+    e = one(p, s);
+    p.A = static_cast<const T *>(p.A) + p.batch_a;
+    p.B = static_cast<const T *>(p.B) + p.batch_b;
+    if (p.C) p.C = static_cast<const T *>(p.C) + p.batch_c;
+    p.D = static_cast<T *>(p.D) + p.batch_d;
+  }
+  return e;
+}
+
 // what the element-aligned form of the compiled plus-times kernel asks for: one contiguous direction per operand
 static inline bool loose_can_run(const Problem &p) {
   return (p.sa_m == 1 || p.sa_k == 1) && (p.sb_n == 1 || p.sb_k == 1);

@@ -25,6 +25,9 @@
 
 namespace cuasr_amd {
 
+hipError_t mfma_small_f32(const Problem &, hipStream_t);       // mfma_small.hip
+bool mfma_small_preferred_f32(const Problem &, bool direct);
+
 bool mfma_direct_f32_can_run(const Problem &);                // mfma_direct_f32.hip
 hipError_t mfma_direct_f32_launch(const Problem &, bool wide, hipStream_t);
 
@@ -364,11 +367,13 @@ static hipError_t launch(const Problem &p, hipStream_t s) {
   // tile, 5120^3: 133 against 117, 6144^3: 150 against 136); where both fill theirs (4096^3: 149.1 and 149.8) the
   // wide one, which moves a quarter less data per flop.
   const long long batch = p.batch > 1 ? p.batch : 1;
-  if (!loose && mfma_direct_f32_can_run(p)) {
+  const bool direct = !loose && mfma_direct_f32_can_run(p);
+  if (mfma_small_preferred_f32(p, direct)) return mfma_small_f32(p, s);
+  if (direct) {
     auto fill = [](long long groups) { return (double)groups / (256.0 * (double)((groups + 255) / 256)); };
     return mfma_direct_f32_launch(p, fill(wide * slices * batch) >= 0.995 * fill(tiles * slices * batch), s);
   }
-  if (batch > 1) return hipErrorNotSupported;  // the compiled kernels take one product per launch
+  if (batch > 1) return mfma_panel::launch_each<float>(p, s, launch);  // the compiled kernels take one product per launch
   // the 128 x 256 tile when its workgroups fill >= 7/8 of whole rounds of 512 (two per compute unit)
   const long long rounds = (wide * slices + 511) / 512;
   const bool wide_tile = wide * slices * 8 >= rounds * 512 * 7;

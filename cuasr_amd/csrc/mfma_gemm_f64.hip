@@ -17,9 +17,12 @@
 // column l % 16 in register r = 0..3 of lane l.  LDS panels are k-major,
 // [k][LD] doubles: a fragment read is 16 consecutive doubles of 4 consecutive
 // rows, one ds_read_b64 per lane.
-#include "semiring.h"
+#include "mfma_common.h"
 
 namespace cuasr_amd {
+
+hipError_t mfma_small_f64(const Problem &, hipStream_t);       // mfma_small.hip
+bool mfma_small_preferred_f64(const Problem &, bool direct);
 
 bool mfma_direct_f64_can_run(const Problem &);                // mfma_direct_f64.hip
 hipError_t mfma_direct_f64_launch(const Problem &, hipStream_t);
@@ -298,8 +301,10 @@ static hipError_t launch(const Problem &p, hipStream_t s) {
   if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
   // whole k-tiles, loadable straight into LDS: the hand-scheduled form of the same tile (faster at every size
   // measured, also where a round of workgroups is mostly empty: 2048^3 71.9 against 54.8 TFLOP/s)
-  if (!loose && mfma_direct_f64_can_run(p)) return mfma_direct_f64_launch(p, s);
-  if (p.batch > 1) return hipErrorNotSupported;  // the compiled kernel takes one product per launch
+  const bool direct = !loose && mfma_direct_f64_can_run(p);
+  if (mfma_small_preferred_f64(p, direct)) return mfma_small_f64(p, s);
+  if (direct) return mfma_direct_f64_launch(p, s);
+  if (p.batch > 1) return mfma_panel::launch_each<double>(p, s, launch);  // the compiled kernel takes one product per launch
   dim3 grid((unsigned)tiles, p.workspace ? p.slices : 1);
   if (loose) launch_kernel(gemm_mfma_f64_kernel<true>, grid, dim3(256), 0, s, p);
   else launch_kernel(gemm_mfma_f64_kernel<false>, grid, dim3(256), 0, s, p);

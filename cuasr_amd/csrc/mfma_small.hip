@@ -1,0 +1,293 @@
+// plus-times for float and double on the matrix cores, for outputs (and batches of outputs) whose 128 x 128 tiles
+// would leave compute units idle, and for double operands the vector loads of the larger tiles cannot fetch:
+//     D = alpha * (A . B) + beta * C      with v_mfma_f32_32x32x2_f32 / v_mfma_f64_16x16x4_f64
+//
+// A wave owns a 32 x 32 block of the output (or 2 x 2 of them) and a share of k; KG waves of a workgroup share a block's k, wave g on the
+// chunks g, g + KG, ... (16 floats or 8 doubles of k each), and WM x WN blocks make the workgroup's tile.  The
+// instruction takes one value of k per 32 (double: 16) lanes and leaves open which, as long as A and B agree, so every
+// lane fetches what it multiplies straight from memory -- 16 bytes of k of its row where k is contiguous, one element
+// per k of its column where it is not -- and there is no LDS, no barrier and nothing to align in the main loop: row
+// indices are clamped lane by lane, and only the last chunk of a k range that is not whole chunks looks at its end
+// (k past it is multiplied as zero).  The next chunk is requested before a chunk's eight matrix instructions (512
+// cycles; 2 x 2 blocks: 2048) are issued.  The KG partial sums meet in LDS, each wave finishing a KG-th of the block's
+// rows.  512^3 41.5 -> 6.7 us (float), 55.4 -> 9.6 (double); 1024^3 80.6 -> 25 - 28 and 110 -> 43; 64 x 4096 x 4096 308 ->
+// 34 and 421 -> 48 (the vector-ALU tiles before it); 2048 products of 100^3, each a launch of its own before, 25 ms -> 0.16.
+// Bound: operands from L2 (1024^3 moves 134 MB in 64 x 64 tiles, at 5.5 TB/s).
+#include "mfma_common.h"
+
+namespace cuasr_amd {
+namespace mfma_small {
+
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef float v4f_loose __attribute__((ext_vector_type(4), aligned(4)));
+typedef double v2d_loose __attribute__((ext_vector_type(2), aligned(8)));
+
+// What the two element types do differently.  A lane's operands of a chunk: 8 floats of one row of 32, or 2 doubles of
+// each of two rows 16 apart; element i of them is k = k_of(lane, i) of the chunk.
+template <typename T> struct Form;
+template <> struct Form<float> {
+  static constexpr int KC = 16, ROWS = 1, PER = 8;   // k per chunk, rows per lane, k per lane and row
+  typedef v16f block_t[1];
+  static __device__ __forceinline__ int row_of(int lane, int) { return lane & 31; }
+  static __device__ __forceinline__ int k_of(int lane, int i) { return (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3); }
+  static __device__ __forceinline__ void load_k(float (&r)[PER], const float *at) {   // at: k = k_of(lane, 0)
+    const v4f_loose lo = *reinterpret_cast<const v4f_loose *>(at), hi = *reinterpret_cast<const v4f_loose *>(at + 8);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      r[e] = lo[e];
+      r[4 + e] = hi[e];
+    }
+  }
+  static __device__ __forceinline__ void multiply(block_t &acc, const float (&a)[ROWS][PER], const float (&b)[ROWS][PER], int i) {
+    acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[0][i], b[0][i], acc[0], 0, 0, 0);
+  }
+  // accumulator e (0..15) of a lane: its place in the block
+  static __device__ __forceinline__ float &at(block_t &acc, int e) { return reinterpret_cast<float *>(&acc[0])[e]; }
+  static __device__ __forceinline__ int out_row(int lane, int e) { return 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3); }
+  static __device__ __forceinline__ int out_col(int lane, int) { return lane & 31; }
+};
+template <> struct Form<double> {
+  static constexpr int KC = 8, ROWS = 2, PER = 2;
+  typedef v4d block_t[4];
+  static __device__ __forceinline__ int row_of(int lane, int r) { return 16 * r + (lane & 15); }
+  static __device__ __forceinline__ int k_of(int lane, int i) { return (lane >> 4) * 2 + i; }
+  static __device__ __forceinline__ void load_k(double (&r)[PER], const double *at) {
+    const v2d_loose v = *reinterpret_cast<const v2d_loose *>(at);
+    r[0] = v[0];
+    r[1] = v[1];
+  }
+  static __device__ __forceinline__ void multiply(block_t &acc, const double (&a)[ROWS][PER], const double (&b)[ROWS][PER], int i) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) acc[x * 2 + y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[x][i], b[y][i], acc[x * 2 + y], 0, 0, 0);
+  }
+  static __device__ __forceinline__ double &at(block_t &acc, int e) { return reinterpret_cast<double *>(&acc[e >> 2])[e & 3]; }
+  static __device__ __forceinline__ int out_row(int lane, int e) { return 16 * (e >> 3) + (lane >> 4) + 4 * (e & 3); }
+  static __device__ __forceinline__ int out_col(int lane, int e) { return 16 * ((e >> 2) & 1) + (lane & 15); }
+};
+
+// RB: 32 x 32 blocks per wave along either direction
+template <typename T, int RB, int WM, int WN, int KG>
+__global__ __launch_bounds__(64 * WM * WN * KG) void mfma_small_kernel(const Problem p) {
+  using F = Form<T>;
+  constexpr int WT = 32 * RB, BM = WT * WM, BN = WT * WN, OUTS = 16 / KG;
+  __shared__ T fold_area[KG > 1 ? KG : 1][WM * WN][KG > 1 ? 16 : 1][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kg = wave / (WM * WN), block = wave % (WM * WN), wm = block / WN, wn = block % WN;
+  const int tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN;
+  int bm, bn;
+  mfma_panel::tile_coords(blockIdx.x, tiles_m, tiles_n, bm, bn);
+  const int m0 = bm * BM + wm * WT, n0 = bn * BN + wn * WT;
+  const Operands o = batch_operands<T>(p);
+  int kb = 0, ke = p.k;
+  if (p.workspace) {
+    kb = blockIdx.y * p.k_per_slice;
+    ke = min(p.k, kb + p.k_per_slice);
+  }
+  const bool a_kc = p.sa_k == 1, b_kc = p.sb_k == 1;
+
+  typename F::block_t acc[RB][RB];
+#pragma unroll
+  for (int x = 0; x < RB; ++x)
+#pragma unroll
+    for (int y = 0; y < RB; ++y)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) F::at(acc[x][y], e) = kg == 0 ? scalar_as<T>(p.add_identity) : T(0);   // 0 for plus
+
+  // a lane's rows (columns of B), at its first k of the wave's first chunk
+  constexpr int NR = RB * F::ROWS;
+  const T *pa[NR], *pb[NR];
+  const int k0 = kb + kg * F::KC;
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const int x = r / F::ROWS * 32 + F::row_of(lane, r % F::ROWS);
+    pa[r] = reinterpret_cast<const T *>(o.A) + (long long)min(m0 + x, p.m - 1) * p.sa_m + (long long)(k0 + F::k_of(lane, 0)) * p.sa_k;
+    pb[r] = reinterpret_cast<const T *>(o.B) + (long long)min(n0 + x, p.n - 1) * p.sb_n + (long long)(k0 + F::k_of(lane, 0)) * p.sb_k;
+  }
+  const long long step_a = (long long)KG * F::KC * p.sa_k, step_b = (long long)KG * F::KC * p.sb_k;
+  struct Chunk { T a[RB][F::ROWS][F::PER], b[RB][F::ROWS][F::PER]; };
+  auto load = [&](T (&r)[RB][F::ROWS][F::PER], const T *(&at)[NR], long long s_k, bool kc) {
+#pragma unroll
+    for (int x = 0; x < NR; ++x) {
+      T (&to)[F::PER] = r[x / F::ROWS][x % F::ROWS];
+      if (kc) {
+        F::load_k(to, at[x]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < F::PER; ++i) to[i] = at[x][(long long)(F::k_of(0, i)) * s_k];
+      }
+    }
+  };
+  auto fetch = [&](Chunk &c) {
+    load(c.a, pa, p.sa_k, a_kc);
+    load(c.b, pb, p.sb_k, b_kc);
+#pragma unroll
+    for (int x = 0; x < NR; ++x) {
+      pa[x] += step_a;
+      pb[x] += step_b;
+    }
+  };
+  auto multiply = [&](const Chunk &c) {
+#pragma unroll
+    for (int i = 0; i < F::PER; ++i)
+#pragma unroll
+      for (int x = 0; x < RB; ++x)
+#pragma unroll
+        for (int y = 0; y < RB; ++y) F::multiply(acc[x][y], c.a[x], c.b[y], i);
+  };
+  const int whole = max(ke - kb, 0) / F::KC;                  // whole chunks of the range
+  int chunks = whole > kg ? (whole - kg + KG - 1) / KG : 0;   // ... of which this wave's
+  Chunk c0, c1;
+  if (chunks > 0) fetch(c0);
+  for (; chunks >= 2; chunks -= 2) {
+    fetch(c1);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(c0);
+    if (chunks > 2) fetch(c0);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(c1);
+  }
+  if (chunks == 1) multiply(c0);
+  if (whole % KG == kg && kb + whole * F::KC < ke) {
+    // the rest of the k range, less than a chunk: what is past its end counts as zero in both operands
+    const int left = ke - (kb + whole * F::KC);
+#pragma unroll
+    for (int x = 0; x < NR; ++x)
+#pragma unroll
+      for (int i = 0; i < F::PER; ++i) {
+        const int kk = F::k_of(lane, i), back = min(kk, left - 1) - F::k_of(lane, 0);   // (pointers stand at k_of(lane, 0))
+        const T va = pa[x][back * p.sa_k], vb = pb[x][back * p.sb_k];
+        c0.a[x / F::ROWS][x % F::ROWS][i] = kk < left ? va : T(0);
+        c0.b[x / F::ROWS][x % F::ROWS][i] = kk < left ? vb : T(0);
+      }
+    multiply(c0);
+  }
+
+  // ---- epilogue: this wave finishes accumulators kg * OUTS ... of every lane of each of its blocks
+  T *out = reinterpret_cast<T *>(o.D);
+  long long ld_out = p.ldd;
+  const bool partial = p.workspace != nullptr;
+  EpilogueScalars<T> e{T(1), T(0), T(0), false};
+  if (partial) {
+    out = reinterpret_cast<T *>(p.workspace) + (long long)blockIdx.y * p.m * p.n;
+    ld_out = p.n;
+  } else {
+    e = resolve_scalars<T>(p, kMultiplies);
+  }
+  const T *C = reinterpret_cast<const T *>(o.C);
+#pragma unroll
+  for (int x = 0; x < RB; ++x)
+#pragma unroll
+    for (int y = 0; y < RB; ++y) {
+      const int r0 = m0 + 32 * x, q0 = n0 + 32 * y;
+      T src[OUTS], res[OUTS];
+      if (e.source_needed) {
+#pragma unroll
+        for (int q = 0; q < OUTS; ++q) {
+          const int row = min(r0 + F::out_row(lane, kg * OUTS + q), p.m - 1), col = min(q0 + F::out_col(lane, kg * OUTS + q), p.n - 1);
+          src[q] = C[(long long)row * p.ldc + col];
+        }
+      }
+      if constexpr (KG > 1) {
+        if (x + y > 0) __syncthreads();   // (the block before has been read)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) fold_area[kg][block][i][lane] = F::at(acc[x][y], i);
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < OUTS; ++q) {
+          T v = fold_area[0][block][kg * OUTS + q][lane];
+#pragma unroll
+          for (int g = 1; g < KG; ++g) v += fold_area[g][block][kg * OUTS + q][lane];
+          res[q] = v;
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < OUTS; ++q) res[q] = F::at(acc[x][y], q);
+      }
+#pragma unroll
+      for (int q = 0; q < OUTS; ++q) {
+        const int row = r0 + F::out_row(lane, kg * OUTS + q), col = q0 + F::out_col(lane, kg * OUTS + q);
+        if (row >= p.m || col >= p.n) continue;
+        T v = res[q];
+        if (!partial) {
+          v = e.alpha * v;
+          if (e.source_needed) v = v + e.beta * src[q];
+        }
+        out[(long long)row * ld_out + col] = v;
+      }
+    }
+}
+
+template <typename T, int RB, int WM, int WN, int KG> static hipError_t launch_as(const Problem &p, hipStream_t s) {
+  constexpr int BM = 32 * RB * WM, BN = 32 * RB * WN;
+  const long long tiles = (long long)((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN);
+  if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
+  launch_kernel((mfma_small_kernel<T, RB, WM, WN, KG>), dim3((unsigned)tiles, p.workspace ? p.slices : 1, p.batch), dim3(64 * WM * WN * KG), 0, s, p);
+  return take_launch_status();
+}
+
+static long long launches_of(const Problem &p) { return (p.workspace ? p.slices : 1) * (long long)(p.batch > 1 ? p.batch : 1); }
+static long long tiles_of(const Problem &p, int tile) { return (long long)((p.m + tile - 1) / tile) * ((p.n + tile - 1) / tile) * launches_of(p); }
+
+// Which form.  Waves of 64 x 64 (four or, for double, eight of them sharing k) fetch half as much per operation, and
+// carry most of the work where their tiles fill the chip's 256 compute units and k is long (1024^3: float 25 - 28 us
+// against 34 - 39 in single blocks, double 43 - 44 against 47 - 62; 512 x 512 x 8192 in 8 slices: 63 against 71 and 91
+// against 122; but 1200^3, 361 tiles for two rounds of 256: 65 against 60).  Four single-block waves side by side on a
+// 64 x 64 tile, nothing to fold, win where there are many tiles and k is short (1024 products of 64^3: 15.7 us against
+// 19.7 with k shared, 500 of 112 x 64 x 112: 22 against 24).  Everything else is one block per workgroup with k shared
+// by as many waves as leave each a few chunks (512^3: 6.7 us; 256 x 256 x 2048: 17; 64 x 4096 x 4096: 34, and 46 with
+// four waves).
+enum Shape { kBlock4, kBlock8, kBlock16, kSideBySide, kWide };
+template <typename T> static Shape shape_for(const Problem &p) {
+  const long long t32 = tiles_of(p, 32), t64 = tiles_of(p, 64);
+  const long long k_range = p.workspace ? p.k_per_slice : p.k, chunks = (k_range + Form<T>::KC - 1) / Form<T>::KC;
+  const bool covers_more = t64 * 3 > t32;   // (64 x 64 tiles reach a third further past the edges, or more)
+  if (!covers_more && k_range >= 512 && t64 >= 192 && (sizeof(T) == 8 || t64 > 1024 || t64 * 4 >= (t64 + 255) / 256 * 256 * 3)) return kWide;
+  if (!covers_more && t32 >= (sizeof(T) == 8 ? 2048 : 1024) && chunks <= 16) return kSideBySide;
+  if (t32 <= 256 && chunks >= 128) return kBlock16;
+  return t32 <= 512 && chunks >= 16 ? kBlock8 : kBlock4;
+}
+
+template <typename T> static hipError_t launch(const Problem &p, hipStream_t s) {
+  if (p.m == 0 || p.n == 0) return hipSuccess;
+  switch (shape_for<T>(p)) {
+    case kWide: return launch_as<T, 2, 1, 1, sizeof(T)>(p, s);
+    case kSideBySide: return launch_as<T, 1, 2, 2, 1>(p, s);
+    case kBlock16: return launch_as<T, 1, 1, 1, 16>(p, s);
+    case kBlock8: return launch_as<T, 1, 1, 1, 8>(p, s);
+    default: return launch_as<T, 1, 1, 1, 4>(p, s);
+  }
+}
+
+// Against the 128 x 128 tiles.  The hand-scheduled ones take whole rounds of 256 compute units, each about 16 us and
+// 0.053 us per k (double 0.109) -- 1536^3, 144 tiles, 101 (187) us; 2048^3, 256 tiles, 132 (243) us; 2000 products of 128 x
+// 128 x 32 138 (144) us.  The compiled ones (ragged k, operands off 16 bytes) take 20 us and 0.125 (0.23) us per k
+// with one tile per compute unit, 30 (40) us and 0.165 (0.29) with two -- 2001 x 1999 x 2000 275 (476) us, 3001 x 3003 x
+// 3001 935 (1518) us, 4095 x 4093 x 64 106 (139) --, and every product of a batch is a launch of its own.  The blocks here run at the rates below whatever the extents (203 (305)
+// and 675 (1003) us for those two): L2, not the matrix cores, feeds them.
+template <typename T> static bool preferred(const Problem &p, bool direct) {
+  if (p.m == 0 || p.n == 0) return false;
+  constexpr bool f64 = sizeof(T) == 8;
+  const double k = p.workspace ? p.k_per_slice : p.k;
+  const Shape shape = shape_for<T>(p);
+  const long long t64 = tiles_of(p, 64);
+  const double fill64 = (double)t64 / (256.0 * (double)((t64 + 255) / 256));
+  const double rate = shape == kWide ? (f64 ? 55e6 : 85e6) * fill64 : shape == kSideBySide ? 48e6 : f64 ? 40e6 : 58e6;   // operations per us
+  const double here = 4.0 + 2.0 * 1024.0 * (double)tiles_of(p, 32) * k / rate;
+  const long long batch = p.batch > 1 && !direct ? p.batch : 1, tiles = tiles_of(p, 128) / batch, rest = tiles % 512;
+  const double one_per_unit = 20.0 + (f64 ? 0.23 : 0.125) * k, two_per_unit = (f64 ? 40.0 : 30.0) + (f64 ? 0.29 : 0.165) * k;
+  const double there = direct ? 4.0 + (double)((tiles + 255) / 256) * (16.0 + (f64 ? 0.109 : 0.053) * k)
+                              : (double)batch * (4.0 + (double)(tiles / 512) * two_per_unit + (rest > 256 ? two_per_unit : rest > 0 ? one_per_unit : 0.0));
+  return here < there;
+}
+
+}  // namespace mfma_small
+
+hipError_t mfma_small_f32(const Problem &p, hipStream_t s) { return mfma_small::launch<float>(p, s); }
+hipError_t mfma_small_f64(const Problem &p, hipStream_t s) { return mfma_small::launch<double>(p, s); }
+// direct: the 128 x 128 tile would be the hand-scheduled one
+bool mfma_small_preferred_f32(const Problem &p, bool direct) { return mfma_small::preferred<float>(p, direct); }
+bool mfma_small_preferred_f64(const Problem &p, bool direct) { return mfma_small::preferred<double>(p, direct); }
+
+}  // namespace cuasr_amd

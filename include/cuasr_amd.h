@@ -179,11 +179,11 @@ int cuasr_amd_srgemm(const cuasr_amd_srgemm_desc *desc, void *stream);
  * products; the outputs must lie at least one matrix apart, strides must not be
  * negative (CUASR_AMD_ERROR_INVALID_PROBLEM otherwise).  The kernel family is
  * chosen once, for the whole batch (what fills the chip is the batch, not one
- * product); on the vector-ALU tiles, and on the matrix-core tiles for products
- * whose k is a multiple of 16 and whose operands (batch strides included) are
- * 16-byte aligned, the product index is part of the grid, so a batch of many
- * small products is a single launch; the other matrix-core kernels and the
- * naive kernel run the products one after the other on the stream.  Each
+ * product); on the vector-ALU tiles and the matrix-core kernels the product
+ * index is part of the grid, so a batch of many small products is a single
+ * launch (large plus-times products that the hand-scheduled matrix-core tiles
+ * cannot fetch -- ragged k, operands or strides off 16 bytes -- and the
+ * naive kernel run one after the other on the stream).  Each
  * product's result is that of a single cuasr_amd_srgemm on its operands. */
 int cuasr_amd_srgemm_batched(const cuasr_amd_srgemm_desc *desc, int batch, int64_t stride_a,
                              int64_t stride_b, int64_t stride_c, int64_t stride_d, void *stream);
@@ -316,7 +316,9 @@ int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64_t ld, int3
                                   int64_t ldp, void *workspace, int panels, void *stream);
 
 /* Name of the kernel family AUTO would choose for this descriptor
- * ("naive", "valu", "valu_direct", "valu_streamk", "mfma"; "valu_direct+valu" when a block of the output runs on
+ * ("naive", "valu", "valu_direct", "valu_streamk", "mfma"; "valu" also names what AUTO runs for float and double
+ * plus-times below 128 tiles of 128 x 128, which is the matrix cores in smaller blocks -- sums to rounding, while a
+ * forced CUASR_AMD_KERNEL_VALU sums in ascending k; "valu_direct+valu" when a block of the output runs on
  * the direct-to-LDS tile and the strips around it on the staged one), or NULL if the descriptor
  * is invalid. */
 const char *cuasr_amd_selected_kernel(const cuasr_amd_srgemm_desc *desc);

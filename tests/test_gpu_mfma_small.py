@@ -1,0 +1,56 @@
+"""Float and double plus-times on the matrix cores in blocks of 32 x 32 (small outputs, batches, ragged doubles): every
+form the dispatch can take, block edges, k remainders, layouts, partial tiles and batches.  Operands are small integers,
+so every product and partial sum is exact and the order of a sum cannot show."""
+import numpy as np
+import pytest
+
+from helpers import to_device, to_host
+
+pytestmark = pytest.mark.gpu
+
+NPD = {"f32": np.float32, "f64": np.float64}
+# one block and its edges, k of one, of a chunk (16 floats, 8 doubles) and its neighbours; four, eight and sixteen waves on
+# a block; waves of 64 x 64 (k >= 512, 192 .. 256 tiles); tiles that stay on the 128 x 128 kernels, compiled and not
+SHAPES = [(1, 1, 1), (32, 32, 16), (33, 31, 7), (31, 65, 17), (100, 60, 24), (70, 40, 2100), (300, 700, 130), (1000, 900, 515),
+          (1024, 1024, 512), (2001, 1999, 300), (4096, 4095, 37)]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f64"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_block_sizes_and_edges(oracle, lib, dtype, shape):
+    import torch
+    import cuasr_amd
+    from cuasr_amd import inputs
+    m, n, k = shape
+    for i, order in enumerate(("FFF", "CCC", "CFC", "FCF") if m * n < 500000 else ("CFF", "FCC")):
+        A, B, C = [inputs.integers(50 + i + (j << 40), r, c, -4, 4, NPD[dtype], o) for j, (r, c, o) in enumerate(zip((m, k, m), (k, n, n), order))]
+        for alpha, beta in ((1.0, 0.0), (2.0, -1.0)):
+            want = oracle.srgemm("plus", "multiplies", A, B, C, alpha, beta, 0.0)
+            dD = to_device(np.zeros_like(C))
+            cuasr_amd.srgemm("plus", "multiplies", to_device(A), to_device(B), to_device(C), dD, alpha, beta, 0.0, 1.0)
+            torch.cuda.synchronize()
+            assert np.array_equal(to_host(dD, dtype), want), (shape, dtype, order, alpha)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f64"])
+def test_slices_and_batches(oracle, lib, dtype):
+    import torch
+    import cuasr_amd
+    from cuasr_amd import inputs
+    for m, n, k, slices in ((70, 41, 530, 3), (512, 500, 4096, 8)):
+        A, B, C = [inputs.integers(5 + (j << 40), r, c, -4, 4, NPD[dtype], o) for j, (r, c, o) in enumerate(zip((m, k, m), (k, n, n), "CFC"))]
+        want = oracle.srgemm("plus", "multiplies", A, B, C, 2.0, -1.0, 0.0)
+        work = torch.empty(cuasr_amd.splitk_workspace_bytes(m, n, slices, dtype) // 4, dtype=torch.int32, device="cuda")
+        for fn in (cuasr_amd.srgemm_splitk, cuasr_amd.srgemm_splitk_serial):
+            dC = to_device(C)
+            fn("plus", "multiplies", to_device(A), to_device(B), dC, dC, slices, work, 2.0, -1.0, 0.0, 1.0)   # D is C
+            torch.cuda.synchronize()
+            assert np.array_equal(to_host(dC, dtype), want), (m, n, k, fn.__name__)
+    # in the grid: few blocks, many tiles with a short k, strides off 16 bytes; one after the other: products that fill the chip
+    for b, m, n, k in ((37, 33, 20, 41), (700, 64, 60, 33), (2, 2001, 1999, 300)):
+        A, B, C = [inputs.integers(9 + (j << 40), b * r, c, -4, 4, NPD[dtype], "C").reshape(b, r, c) for j, (r, c) in enumerate(((m, k), (k, n), (m, n)))]
+        dD = torch.zeros(b, m, n, dtype=torch.from_numpy(C).dtype, device="cuda")
+        cuasr_amd.srgemm_batched("plus", "multiplies", *(torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (A, B, C)), dD, 1.0, 1.0, 0.0, 1.0)
+        torch.cuda.synchronize()
+        want = np.matmul(A.astype(np.float64), B.astype(np.float64)) + C
+        assert np.array_equal(dD.cpu().numpy(), want), (b, m, n, k)
