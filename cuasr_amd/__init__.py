@@ -119,6 +119,21 @@ def load():
     return _lib
 
 
+_launch_fns = None
+
+
+def _launchers():
+    """cuasr_amd_srgemm, _batched and _splitk as functions that take the descriptor as bytes or by reference."""
+    global _launch_fns
+    if _launch_fns is None:
+        lib = load()
+        ptr, i64 = ctypes.c_void_p, ctypes.c_int64
+        kinds = (("cuasr_amd_srgemm", (ptr, ptr)), ("cuasr_amd_srgemm_batched", (ptr, ctypes.c_int, i64, i64, i64, i64, ptr)),
+                 ("cuasr_amd_srgemm_splitk", (ptr, ptr, ptr)))
+        _launch_fns = [ctypes.CFUNCTYPE(ctypes.c_int, *args)((name, lib)) for name, args in kinds]
+    return _launch_fns
+
+
 # --------------------------------------------------------------------------
 # Semiring constants, as the reference functors define them
 # (include/cuasr/functional.h:28-36, :41-42, :84-85, :127-128, :167-168,
@@ -175,6 +190,31 @@ def _set_scalar(s, value, dtype):
         s.u32 = int(value) & 0xFFFFFFFF
 
 
+def _strided(ptr, rows, cols, s0, s1):
+    """(pointer, leading dimension, layout, rows, cols) of a matrix given by its strides."""
+    if s0 == 1 and (cols <= 1 or s1 >= rows):
+        return ptr, s1 if cols > 1 else max(rows, 1), COLUMN_MAJOR, rows, cols
+    if s1 == 1 and (rows <= 1 or s0 >= cols):
+        return ptr, s0 if rows > 1 else max(cols, 1), ROW_MAJOR, rows, cols
+    raise ValueError("matrix must have unit stride along rows or columns")
+
+
+def _operand(t):
+    """The same of a MatRef or a 2-D torch tensor."""
+    if isinstance(t, MatRef):
+        return t.ptr, t.ld, t.layout, t.rows, t.cols
+    rows, cols = t.shape
+    s0, s1 = t.stride()
+    return _strided(t.data_ptr(), rows, cols, s0, s1)
+
+
+def _slice_operand(t):
+    """The same of the first matrix of a 3-D torch tensor."""
+    _, rows, cols = t.shape
+    _, s0, s1 = t.stride()
+    return _strided(t.data_ptr(), rows, cols, s0, s1)
+
+
 class MatRef:
     """A matrix in device memory: pointer, leading dimension (elements), layout."""
 
@@ -184,44 +224,49 @@ class MatRef:
     @staticmethod
     def of(t):
         """From a 2-D torch tensor whose rows or columns are contiguous."""
-        if isinstance(t, MatRef):
-            return t
-        rows, cols = t.shape
-        s0, s1 = t.stride()
-        if s0 == 1 and (cols <= 1 or s1 >= rows):
-            return MatRef(t.data_ptr(), s1 if cols > 1 else max(rows, 1), COLUMN_MAJOR, rows, cols)
-        if s1 == 1 and (rows <= 1 or s0 >= cols):
-            return MatRef(t.data_ptr(), s0 if rows > 1 else max(cols, 1), ROW_MAJOR, rows, cols)
-        raise ValueError("matrix must have unit stride along rows or columns")
+        return t if isinstance(t, MatRef) else MatRef(*_operand(t))
+
+
+_dtype_names = None
 
 
 def _torch_dtype_name(t):
-    import torch
-    return {torch.float32: "f32", torch.float64: "f64", torch.int32: "i32",
-            getattr(torch, "uint32", None): "u32", torch.float16: "f16"}[t.dtype]
+    global _dtype_names
+    if _dtype_names is None:
+        import torch
+        _dtype_names = {torch.float32: "f32", torch.float64: "f64", torch.int32: "i32",
+                        getattr(torch, "uint32", None): "u32", torch.float16: "f16"}
+    return _dtype_names[t.dtype]
 
 
-def make_desc(add_op, mult_op, dtype, A, B, C, D, alpha, beta, add_identity, mult_identity,
-              split_k_slices=1, kernel="auto", alpha_ptr=None, beta_ptr=None):
-    a, b, d = MatRef.of(A), MatRef.of(B), MatRef.of(D)
-    c = MatRef.of(C) if C is not None else MatRef(0, d.ld, d.layout, d.rows, d.cols)
+def _problem(a, b, c, d):
+    """Layouts, extents and the four (pointer, leading dimension) pairs, in the descriptor's order, of operands given as
+    _operand gives them (c may be None)."""
+    ap, lda, la, am, ak = a
+    bp, ldb, lb, bk, bn = b
+    dp, ldd, ld, m, n = d
+    if c is None:
+        cp, ldc = 0, ldd
+    else:
+        cp, ldc, lc, crows, ccols = c
+        if cp and lc != ld:
+            # only a contiguous vector can be read in either layout
+            if min(m, n) > 1 or ldc != (1 if (lc == COLUMN_MAJOR) == (crows == 1) else max(crows, ccols)):
+                raise ValueError("C and D must share a layout")
+            ldc = max(ccols, 1) if ld == ROW_MAJOR and crows == 1 else max(crows, 1) if ld == COLUMN_MAJOR and ccols == 1 else 1
+    if ak != bk or am != m or bn != n:
+        raise ValueError("shape mismatch")
+    return la, lb, ld, m, n, ak, ap, lda, bp, ldb, cp, ldc, dp, ldd
+
+
+def _fill_desc(add_op, mult_op, dtype, problem, alpha, beta, add_identity, mult_identity, split_k_slices=1, kernel="auto",
+               alpha_ptr=None, beta_ptr=None):
     desc = SrgemmDesc()
     desc.add_op, desc.mult_op, desc.dtype = OPS[add_op], OPS[mult_op], DTYPES[dtype]
-    desc.layout_a, desc.layout_b, desc.layout_c = a.layout, b.layout, d.layout
-    if c.ptr and c.layout != d.layout:
-        # only a contiguous vector can be read in either layout
-        if min(d.rows, d.cols) > 1 or c.ld != (1 if (c.layout == COLUMN_MAJOR) == (c.rows == 1) else max(c.rows, c.cols)):
-            raise ValueError("C and D must share a layout")
-        c = MatRef(c.ptr, max(c.cols, 1) if d.layout == ROW_MAJOR and c.rows == 1 else
-                   max(c.rows, 1) if d.layout == COLUMN_MAJOR and c.cols == 1 else 1, d.layout, c.rows, c.cols)
-    if a.cols != b.rows or (a.rows, b.cols) != (d.rows, d.cols):
-        raise ValueError("shape mismatch")
-    desc.m, desc.n, desc.k = d.rows, d.cols, a.cols
+    (desc.layout_a, desc.layout_b, desc.layout_c, desc.m, desc.n, desc.k, ap, desc.lda, bp, desc.ldb, cp, desc.ldc,
+     dp, desc.ldd) = problem
+    desc.A, desc.B, desc.C, desc.D = ap or None, bp or None, cp or None, dp or None
     desc.split_k_slices = split_k_slices
-    desc.A, desc.lda = a.ptr or None, a.ld
-    desc.B, desc.ldb = b.ptr or None, b.ld
-    desc.C, desc.ldc = c.ptr or None, c.ld
-    desc.D, desc.ldd = d.ptr or None, d.ld
     _set_scalar(desc.alpha, alpha, dtype)
     _set_scalar(desc.beta, beta, dtype)
     _set_scalar(desc.add_identity, add_identity, dtype)
@@ -233,11 +278,43 @@ def make_desc(add_op, mult_op, dtype, A, B, C, D, alpha, beta, add_identity, mul
     return desc
 
 
+def make_desc(add_op, mult_op, dtype, A, B, C, D, alpha, beta, add_identity, mult_identity,
+              split_k_slices=1, kernel="auto", alpha_ptr=None, beta_ptr=None):
+    problem = _problem(_operand(A), _operand(B), _operand(C) if C is not None else None, _operand(D))
+    return _fill_desc(add_op, mult_op, dtype, problem, alpha, beta, add_identity, mult_identity, split_k_slices, kernel,
+                      alpha_ptr, beta_ptr)
+
+
+# The descriptor as one packed record, for the calls that launch: filling a ctypes structure field by field took longer
+# than the kernel of a small product runs (min-plus 256^3, 6.0 us: 9.5 us a call in a loop of calls, 5.9 now).  Scalars the record's format does not take as they are -- a float
+# beyond the range of binary32, a float where an integer belongs, binary16 -- go through the structure.
+_RECORDS = {dt: struct.Struct("@10iPqPqPqPq" + 4 * scalar + "PPii")
+            for dt, scalar in (("f32", "f4x"), ("f64", "d"), ("i32", "i4x"), ("i8", "i4x"))}
+assert all(r.size == ctypes.sizeof(SrgemmDesc) for r in _RECORDS.values())
+
+
+def _packed(add_op, mult_op, dtype, problem, alpha, beta, add_identity, mult_identity, split_k_slices=1, kernel="auto",
+            alpha_ptr=None, beta_ptr=None):
+    """Bytes (or a SrgemmDesc passed by reference) for the launching entry points."""
+    record = _RECORDS.get(dtype)
+    if record is not None:
+        la, lb, lc, m, n, k, *pointers = problem
+        try:
+            return record.pack(OPS[add_op], OPS[mult_op], DTYPES[dtype], la, lb, lc, m, n, k, split_k_slices, *pointers,
+                               alpha, beta, add_identity, mult_identity, alpha_ptr or 0, beta_ptr or 0, KERNELS[kernel], 0)
+        except (struct.error, OverflowError, TypeError):
+            pass
+    return ctypes.byref(_fill_desc(add_op, mult_op, dtype, problem, alpha, beta, add_identity, mult_identity, split_k_slices,
+                                   kernel, alpha_ptr, beta_ptr))
+
+
 def _stream_handle(stream):
-    if stream is None:
-        import torch
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return ctypes.c_void_p(int(getattr(stream, "cuda_stream", stream)))
+    if stream is not None:
+        return int(getattr(stream, "cuda_stream", stream))
+    import torch
+    if torch.cuda.is_initialized():   # what current_stream().cuda_stream says, without making a Stream object
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def srgemm(add_op, mult_op, A, B, C, D, alpha=None, beta=None, add_identity=None,
@@ -254,9 +331,9 @@ def srgemm(add_op, mult_op, A, B, C, D, alpha=None, beta=None, add_identity=None
     beta = op_annihilator(mult_op, dtype, infinities) if beta is None else beta
     add_identity = op_identity(add_op, dtype, infinities) if add_identity is None else add_identity
     mult_identity = op_identity(mult_op, dtype, infinities) if mult_identity is None else mult_identity
-    desc = make_desc(add_op, mult_op, dtype, A, B, C, D, alpha, beta, add_identity, mult_identity,
-                     1, kernel, alpha_ptr, beta_ptr)
-    st = load().cuasr_amd_srgemm(ctypes.byref(desc), _stream_handle(stream))
+    problem = _problem(_operand(A), _operand(B), _operand(C) if C is not None else None, _operand(D))
+    st = _launchers()[0](_packed(add_op, mult_op, dtype, problem, alpha, beta, add_identity, mult_identity, 1, kernel, alpha_ptr,
+                                 beta_ptr), _stream_handle(stream))
     if st != SUCCESS:
         raise CuasrError(st, "cuasr_amd_srgemm")
     return D
@@ -270,9 +347,9 @@ def srgemm_batched(add_op, mult_op, A, B, C, D, alpha, beta, add_identity, mult_
     batch = D.shape[0]
     if batch == 0:
         return D
-    desc = make_desc(add_op, mult_op, dtype, A[0], B[0], C[0], D[0], alpha, beta, add_identity, mult_identity, 1, kernel)
-    st = load().cuasr_amd_srgemm_batched(ctypes.byref(desc), batch, A.stride(0), B.stride(0), C.stride(0), D.stride(0),
-                                         _stream_handle(stream))
+    problem = _problem(_slice_operand(A), _slice_operand(B), _slice_operand(C), _slice_operand(D))
+    st = _launchers()[1](_packed(add_op, mult_op, dtype, problem, alpha, beta, add_identity, mult_identity, 1, kernel), batch,
+                         A.stride(0), B.stride(0), C.stride(0), D.stride(0), _stream_handle(stream))
     if st != SUCCESS:
         raise CuasrError(st, "cuasr_amd_srgemm_batched")
     return D
@@ -295,10 +372,10 @@ def srgemm_splitk(add_op, mult_op, A, B, C, D, slices, workspace, alpha=None, be
     beta = op_annihilator(mult_op, dtype, infinities) if beta is None else beta
     add_identity = op_identity(add_op, dtype, infinities) if add_identity is None else add_identity
     mult_identity = op_identity(mult_op, dtype, infinities) if mult_identity is None else mult_identity
-    desc = make_desc(add_op, mult_op, dtype, A, B, C, D, alpha, beta, add_identity, mult_identity,
-                     slices, kernel, alpha_ptr, beta_ptr)
+    problem = _problem(_operand(A), _operand(B), _operand(C) if C is not None else None, _operand(D))
     ws = workspace.data_ptr() if hasattr(workspace, "data_ptr") else workspace
-    st = load().cuasr_amd_srgemm_splitk(ctypes.byref(desc), ctypes.c_void_p(ws or None), _stream_handle(stream))
+    st = _launchers()[2](_packed(add_op, mult_op, dtype, problem, alpha, beta, add_identity, mult_identity, slices, kernel, alpha_ptr,
+                                 beta_ptr), ws or None, _stream_handle(stream))
     if st != SUCCESS:
         raise CuasrError(st, "cuasr_amd_srgemm_splitk")
     return D
