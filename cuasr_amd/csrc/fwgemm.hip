@@ -114,6 +114,10 @@ __global__ void __launch_bounds__(256) fwgemm_naive_kernel(FwArgs g) {
 template <typename T> struct vec4_of;
 template <> struct vec4_of<float> { typedef float type __attribute__((ext_vector_type(4))); };
 template <> struct vec4_of<double> { typedef double type __attribute__((ext_vector_type(4))); };
+// four elements at element alignment: the same load instruction, and a matrix whose leading dimension is odd takes it too
+template <typename T> struct uvec4_of;
+template <> struct uvec4_of<float> { typedef float type __attribute__((ext_vector_type(4), aligned(4))); };
+template <> struct uvec4_of<double> { typedef double type __attribute__((ext_vector_type(4), aligned(8))); };
 
 // One thread per output row and four columns, for products too small for the tile kernel but on the
 // critical path (the block row and the block column of a blocked Floyd-Warshall step): a workgroup of 256
@@ -250,6 +254,7 @@ template <typename T, int THREADS, int CHUNK, bool HAS_AT, int ROW_BITS, int COL
 __device__ __forceinline__ void lookup_queue(const FwArgs &g, const uint32_t *q_code, const T *q_want, int count, int tid,
                                              int m0, int n0) {
   typedef typename vec4_of<T>::type V4;
+  typedef typename uvec4_of<T>::type U4;
   constexpr int G = CHUNK / 4, GROUPS = THREADS / G;
   constexpr int UN = sizeof(T) == 4 ? 8 : 4;
   static_assert(G == 4 || G == 8, "lanes per element");
@@ -257,7 +262,7 @@ __device__ __forceinline__ void lookup_queue(const FwArgs &g, const uint32_t *q_
   T *dist = static_cast<T *>(g.dist);
   const int sub = tid % G;
   for (int e0 = tid / G; e0 < count; e0 += UN * GROUPS) {
-    int r[UN], c[UN], k0[UN];
+    int r[UN], c[UN], k0[UN], chunk0[UN];
     T want[UN];
     V4 pa[UN], pb[UN];
     bool live[UN];
@@ -269,10 +274,13 @@ __device__ __forceinline__ void lookup_queue(const FwArgs &g, const uint32_t *q_
       want[u] = q_want[live[u] ? e : e0];
       r[u] = m0 + int(code & ((1u << ROW_BITS) - 1));
       c[u] = n0 + int((code >> ROW_BITS) & ((1u << COL_BITS) - 1));
-      k0[u] = int(code >> (ROW_BITS + COL_BITS)) * CHUNK + 4 * sub;
-      pb[u] = *reinterpret_cast<const V4 *>(B + k0[u] + int64_t(c[u]) * g.ldb);
+      // (in a ragged last chunk the lanes past its end look at the last four k once more: two lanes that find the same
+      // k store the same two values, and no k before the chunk has a product as low as the chunk's minimum)
+      chunk0[u] = int(code >> (ROW_BITS + COL_BITS)) * CHUNK;
+      k0[u] = min(chunk0[u] + 4 * sub, g.k - 4);
+      pb[u] = *reinterpret_cast<const U4 *>(B + k0[u] + int64_t(c[u]) * g.ldb);
       if constexpr (HAS_AT) {
-        pa[u] = *reinterpret_cast<const V4 *>(At + k0[u] + int64_t(r[u]) * g.ldat);
+        pa[u] = *reinterpret_cast<const U4 *>(At + k0[u] + int64_t(r[u]) * g.ldat);
       } else {
 #pragma unroll
         for (int x = 0; x < 4; ++x) pa[u][x] = A[r[u] + int64_t(k0[u] + x) * g.lda];
@@ -289,7 +297,7 @@ __device__ __forceinline__ void lookup_queue(const FwArgs &g, const uint32_t *q_
         first = hit ? x : first;
         value = pick(hit, prod, value);
       }
-      const int key = first < 4 ? 4 * sub + first : CHUNK;  // where in the chunk my first hit is
+      const int key = first < 4 ? k0[u] - chunk0[u] + first : CHUNK;  // where in the chunk my first hit is
       const int best = group_min<G>(key);
       if (live[u] && first < 4 && key == best) {
         dist[r[u] + int64_t(c[u]) * g.ldc] = value;
@@ -301,12 +309,18 @@ __device__ __forceinline__ void lookup_queue(const FwArgs &g, const uint32_t *q_
 
 // 256 threads as 16 x 16; each owns TM x TN outputs in groups of four rows /
 // columns that lie 64 apart, so a workgroup covers (16 TM) x (16 TN).
-// GUARD = false: whole tiles, 16-byte aligned columns of A and B (vector loads).
-// GUARD = true : any extents and alignment; out-of-range operands read as
-//                +infinity, whose products never improve anything.
+// GUARD = false: at least one tile in either direction and four k; any alignment.  A tile at a far edge starts
+//                earlier instead of reaching past the matrix, and leaves alone what the tile before it stores; a ragged
+//                last chunk of k is fetched element by element.
+// GUARD = true : any extents; every operand's element fetched by itself behind a test of its indices, those out
+//                of range read as +infinity, whose products never improve anything.
+// (Bounds tests on every fetch and one lookup per lane made this kernel's launch 197 us at n = 2000 where n = 2048 takes
+// 84.  With the edge tiles moved, whole blocked Floyd-Warshall jobs of n = 1533 / 2000 / 3000: 2833 / 3636 / 11053 us
+// -> 1298 / 1703 / 3888; double, n = 2000: 3685 -> 2453.)
 template <typename T, int TM, int TN, int SN, int BK, bool GUARD, bool HAS_AT>
 __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int block_x, const int block_y) {
   typedef typename vec4_of<T>::type V4;
+  typedef typename uvec4_of<T>::type U4;
   constexpr int BM = 16 * TM, BN = 16 * TN, PAD = 4;
   constexpr int NA = BM * BK / 4 / 256, NB = BN * BK / 4 / 256;
   static_assert(TM % 4 == 0 && TN % SN == 0 && SN % 4 == 0 && BK % 4 == 0 && BK % 2 == 0 && NA >= 1 && NB >= 1, "tile shape");
@@ -317,9 +331,10 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
   const T *B = static_cast<const T *>(g.B);
   const int tid = threadIdx.x & 255;
   const int tx = tid & 15, ty = tid >> 4;
-  const int m0 = block_x * BM, n0 = block_y * BN;
+  const int first_m = block_x * BM, first_n = block_y * BN;   // the first row and column this workgroup stores
+  const int m0 = GUARD ? first_m : min(first_m, g.m - BM), n0 = GUARD ? first_n : min(first_n, g.n - BN);
   // (the host only passes ranges whose ends fall on tile boundaries or beyond the matrix)
-  if ((m0 < g.skip_r1 && m0 + BM > g.skip_r0) || (n0 < g.skip_c1 && n0 + BN > g.skip_c0)) return;
+  if ((first_m < g.skip_r1 && first_m + BM > g.skip_r0) || (first_n < g.skip_c1 && first_n + BN > g.skip_c0)) return;
   const T inf = std::numeric_limits<T>::infinity();
 
   auto row_of = [&](int i) { return m0 + (i >> 2) * 64 + tx * 4 + (i & 3); };
@@ -327,11 +342,14 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
 
   V4 ra[NA], rb[NB];
   auto fetch = [&](int k0) {
+    const bool whole = !GUARD && k0 + BK <= g.k;
+    int tid_t = tid;   // (the ragged chunk's addresses are worked out on the spot, not kept through the main loop)
+    if (!GUARD && !whole) asm volatile("" : "+v"(tid_t));
 #pragma unroll
     for (int p = 0; p < NA; ++p) {
-      const int v = tid + p * 256, r = (v % (BM / 4)) * 4, kk = v / (BM / 4);
-      if constexpr (!GUARD) {
-        ra[p] = *reinterpret_cast<const V4 *>(A + (m0 + r) + int64_t(k0 + kk) * g.lda);
+      const int v = tid_t + p * 256, r = (v % (BM / 4)) * 4, kk = v / (BM / 4);
+      if (whole) {
+        ra[p] = *reinterpret_cast<const U4 *>(A + (m0 + r) + int64_t(k0 + kk) * g.lda);
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -340,9 +358,9 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
     }
 #pragma unroll
     for (int p = 0; p < NB; ++p) {
-      const int v = tid + p * 256, kk = (v % (BK / 4)) * 4, c = v / (BK / 4);
-      if constexpr (!GUARD) {
-        rb[p] = *reinterpret_cast<const V4 *>(B + (k0 + kk) + int64_t(n0 + c) * g.ldb);
+      const int v = tid_t + p * 256, kk = (v % (BK / 4)) * 4, c = v / (BK / 4);
+      if (whole) {
+        rb[p] = *reinterpret_cast<const U4 *>(B + (k0 + kk) + int64_t(n0 + c) * g.ldb);
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -386,21 +404,23 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
     for (int i = 0; i < TM; ++i) {
       const int r = row_of(i), c = col_of(j);
       chunk[i][j] = -1;
-      if constexpr (!GUARD) acc[i][j] = static_cast<const T *>(g.dist)[r + int64_t(c) * g.ldc];
-      else acc[i][j] = (r < g.m && c < g.n) ? static_cast<const T *>(g.dist)[r + int64_t(c) * g.ldc] : -inf;
+      if constexpr (GUARD) acc[i][j] = (r < g.m && c < g.n) ? static_cast<const T *>(g.dist)[r + int64_t(c) * g.ldc] : -inf;
     }
   if constexpr (!GUARD) {
-    // a lane's rows come in runs of four: one 16-byte load per run when dist allows it
-    const size_t vb = 4 * sizeof(T);
-    if (reinterpret_cast<uintptr_t>(g.dist) % vb == 0 && g.ldc % 4 == 0) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; i += 4) {
+        const V4 v = *reinterpret_cast<const U4 *>(static_cast<const T *>(g.dist) + row_of(i) + int64_t(col_of(j)) * g.ldc);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) acc[i + x][j] = v[x];
+      }
+    if (m0 < first_m || n0 < first_n) {  // another tile's elements: nothing is lower than -infinity
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int i = 0; i < TM; i += 4) {
-          const V4 v = *reinterpret_cast<const V4 *>(static_cast<const T *>(g.dist) + row_of(i) + int64_t(col_of(j)) * g.ldc);
-#pragma unroll
-          for (int x = 0; x < 4; ++x) acc[i + x][j] = v[x];
-        }
+        for (int i = 0; i < TM; ++i)
+          if (row_of(i) < first_m || col_of(j) < first_n) acc[i][j] = -inf;
     }
   }
 
@@ -466,7 +486,7 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
   int tx2 = tx, ty2 = ty;
   asm volatile("" : "+v"(tx2), "+v"(ty2));
   if constexpr (!GUARD) {
-    // Whole, aligned tiles.  Improved elements are few in most launches and scattered over the
+    // Improved elements are few in most launches and scattered over the
     // lanes, so they are first collected in a queue in LDS (the panels are no longer needed) and the
     // queue is then worked off by all 256 threads (lookup_queue): no lane waits for an element that did
     // not improve.  The queue takes as many whole columns j of the lanes' outputs as fit (one column
@@ -1280,19 +1300,15 @@ template <typename T, int TM, int TN, int SN, int BK>
 hipError_t launch_tile(const FwArgs &g, hipStream_t stream) {
   constexpr int BM = 16 * TM, BN = 16 * TN;
   // (the unguarded form queues improved elements with their chunk of BK k-values in 18 bits)
-  const bool whole = g.m % BM == 0 && g.n % BN == 0 && g.k % BK == 0 && g.k < (1 << 22);
-  const size_t vec = 4 * sizeof(T);
-  const bool aligned = reinterpret_cast<uintptr_t>(g.A) % vec == 0 && reinterpret_cast<uintptr_t>(g.B) % vec == 0 &&
-                       g.lda % 4 == 0 && g.ldb % 4 == 0;
+  const bool whole = g.m >= BM && g.n >= BN && g.k >= 4 && g.k < (1 << 22);
   if (g.ahead_bb > 0 && (FW_BLOCK % BM || FW_BLOCK % BN)) return hipErrorInvalidValue;
   dim3 grid((g.m + BM - 1) / BM, (g.n + BN - 1) / BN + (g.ahead_bb > 0 ? 1 : 0));
   if (g.At) {
-    const bool at_aligned = reinterpret_cast<uintptr_t>(g.At) % vec == 0 && g.ldat % 4 == 0;
-    if (whole && aligned && at_aligned)
+    if (whole)
       launch_kernel((fwgemm_tile_kernel<T, TM, TN, SN, BK, false, true>), grid, dim3(256), 0, stream, g);
     else
       launch_kernel((fwgemm_tile_kernel<T, TM, TN, SN, BK, true, true>), grid, dim3(256), 0, stream, g);
-  } else if (whole && aligned) {
+  } else if (whole) {
     launch_kernel((fwgemm_tile_kernel<T, TM, TN, SN, BK, false, false>), grid, dim3(256), 0, stream, g);
   } else {
     launch_kernel((fwgemm_tile_kernel<T, TM, TN, SN, BK, true, false>), grid, dim3(256), 0, stream, g);

@@ -61,6 +61,16 @@ def test_ragged_extents_and_leading_dimensions(oracle, dtype, kernel):
     run_case(oracle, 128, 128, 32, dtype, True, kernel, pad=(4, 4, 8, 12))
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("m,n,k", [(128, 128, 4), (129, 255, 5), (191, 128, 18), (255, 385, 31), (257, 129, 35), (128, 129, 3)])
+def test_edge_tiles_start_earlier(oracle, dtype, m, n, k):
+    """One tile and a little more in either direction, chunks of k with one to fifteen left over, every alignment of the
+    columns: an element near the far edge is computed by two tiles and stored by one."""
+    for pad in ((0, 0, 0, 0), (1, 3, 2, 1)):
+        run_case(oracle, m, n, k, dtype, True, "valu", pad)
+        run_case(oracle, m, n, k, dtype, False, "valu", pad, seed=9)
+
+
 def test_first_of_many_equal_products(oracle):
     """Every product equal: the first k wins where it improves, nothing moves where it does not."""
     m = n = 128
