@@ -250,13 +250,12 @@ template <int G> __device__ __forceinline__ int group_min(int v) {
   if constexpr (G == 8) v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, true));  // each eight mirrored
   return v;
 }
-template <typename T, int THREADS, int CHUNK, bool HAS_AT, int ROW_BITS, int COL_BITS>
+template <typename T, int THREADS, int CHUNK, bool HAS_AT, int ROW_BITS, int COL_BITS, int UN>
 __device__ __forceinline__ void lookup_queue(const FwArgs &g, const uint32_t *q_code, const T *q_want, int count, int tid,
                                              int m0, int n0) {
   typedef typename vec4_of<T>::type V4;
   typedef typename uvec4_of<T>::type U4;
   constexpr int G = CHUNK / 4, GROUPS = THREADS / G;
-  constexpr int UN = sizeof(T) == 4 ? 8 : 4;
   static_assert(G == 4 || G == 8, "lanes per element");
   const T *A = static_cast<const T *>(g.A), *B = static_cast<const T *>(g.B), *At = static_cast<const T *>(g.At);
   T *dist = static_cast<T *>(g.dist);
@@ -307,8 +306,8 @@ __device__ __forceinline__ void lookup_queue(const FwArgs &g, const uint32_t *q_
   }
 }
 
-// 256 threads as 16 x 16; each owns TM x TN outputs in groups of four rows /
-// columns that lie 64 apart, so a workgroup covers (16 TM) x (16 TN).
+// NT threads as 16 x TY; each owns TM x TN outputs in groups of four rows / columns that
+// lie 64 / 4 TY apart, so a workgroup covers (16 TM) x (TY TN).
 // GUARD = false: at least one tile in either direction and four k; any alignment.  A tile at a far edge starts
 //                earlier instead of reaching past the matrix, and leaves alone what the tile before it stores; a ragged
 //                last chunk of k is fetched element by element.
@@ -317,19 +316,23 @@ __device__ __forceinline__ void lookup_queue(const FwArgs &g, const uint32_t *q_
 // (Bounds tests on every fetch and one lookup per lane made this kernel's launch 197 us at n = 2000 where n = 2048 takes
 // 84.  With the edge tiles moved, whole blocked Floyd-Warshall jobs of n = 1533 / 2000 / 3000: 2833 / 3636 / 11053 us
 // -> 1298 / 1703 / 3888; double, n = 2000: 3685 -> 2453.)
-template <typename T, int TM, int TN, int SN, int BK, bool GUARD, bool HAS_AT>
-__device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int block_x, const int block_y) {
+template <typename T, int NT, int TM, int TN, int BK> struct FwTileLds {
+  static constexpr int TY = NT / 16, BM = 16 * TM, BN = TY * TN, PAD = 4;
+  alignas(16) T as[2][BK][BM + PAD], bs[2][BK][BN + PAD];
+  int wave_count[NT / 64][TN];
+};
+template <typename T, int NT, int TM, int TN, int WPE, int BK, bool GUARD, bool HAS_AT>
+__device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int block_x, const int block_y, FwTileLds<T, NT, TM, TN, BK> &sm) {
   typedef typename vec4_of<T>::type V4;
   typedef typename uvec4_of<T>::type U4;
-  constexpr int BM = 16 * TM, BN = 16 * TN, PAD = 4;
-  constexpr int NA = BM * BK / 4 / 256, NB = BN * BK / 4 / 256;
-  static_assert(TM % 4 == 0 && TN % SN == 0 && SN % 4 == 0 && BK % 4 == 0 && BK % 2 == 0 && NA >= 1 && NB >= 1, "tile shape");
-  __shared__ __attribute__((aligned(16))) T as[2][BK][BM + PAD];
-  __shared__ __attribute__((aligned(16))) T bs[2][BK][BN + PAD];
-
+  constexpr int TY = NT / 16, BM = 16 * TM, BN = TY * TN;
+  constexpr int NA = BM * BK / 4 / NT, NB = BN * BK / 4 / NT;
+  static_assert(TM % 4 == 0 && TN % 4 == 0 && BK % 4 == 0 && NA >= 1 && NB >= 1, "tile shape");
+  auto &as = sm.as;
+  auto &bs = sm.bs;
   const T *A = static_cast<const T *>(g.A);
   const T *B = static_cast<const T *>(g.B);
-  const int tid = threadIdx.x & 255;
+  const int tid = threadIdx.x;
   const int tx = tid & 15, ty = tid >> 4;
   const int first_m = block_x * BM, first_n = block_y * BN;   // the first row and column this workgroup stores
   const int m0 = GUARD ? first_m : min(first_m, g.m - BM), n0 = GUARD ? first_n : min(first_n, g.n - BN);
@@ -338,7 +341,7 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
   const T inf = std::numeric_limits<T>::infinity();
 
   auto row_of = [&](int i) { return m0 + (i >> 2) * 64 + tx * 4 + (i & 3); };
-  auto col_of = [&](int j) { return n0 + (j >> 2) * 64 + ty * 4 + (j & 3); };
+  auto col_of = [&](int j) { return n0 + (j >> 2) * (4 * TY) + ty * 4 + (j & 3); };
 
   V4 ra[NA], rb[NB];
   auto fetch = [&](int k0) {
@@ -347,7 +350,7 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
     if (!GUARD && !whole) asm volatile("" : "+v"(tid_t));
 #pragma unroll
     for (int p = 0; p < NA; ++p) {
-      const int v = tid_t + p * 256, r = (v % (BM / 4)) * 4, kk = v / (BM / 4);
+      const int v = tid_t + p * NT, r = (v % (BM / 4)) * 4, kk = v / (BM / 4);
       if (whole) {
         ra[p] = *reinterpret_cast<const U4 *>(A + (m0 + r) + int64_t(k0 + kk) * g.lda);
       } else {
@@ -358,7 +361,7 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
     }
 #pragma unroll
     for (int p = 0; p < NB; ++p) {
-      const int v = tid_t + p * 256, kk = (v % (BK / 4)) * 4, c = v / (BK / 4);
+      const int v = tid_t + p * NT, kk = (v % (BK / 4)) * 4, c = v / (BK / 4);
       if (whole) {
         rb[p] = *reinterpret_cast<const U4 *>(B + (k0 + kk) + int64_t(n0 + c) * g.ldb);
       } else {
@@ -371,39 +374,67 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
   auto stage = [&](int buf) {
 #pragma unroll
     for (int p = 0; p < NA; ++p) {
-      const int v = tid + p * 256, r = (v % (BM / 4)) * 4, kk = v / (BM / 4);
+      const int v = tid + p * NT, r = (v % (BM / 4)) * 4, kk = v / (BM / 4);
       *reinterpret_cast<V4 *>(&as[buf][kk][r]) = ra[p];
     }
 #pragma unroll
     for (int p = 0; p < NB; ++p) {
-      const int v = tid + p * 256, kk = (v % (BK / 4)) * 4, c = v / (BK / 4);
+      const int v = tid + p * NT, kk = (v % (BK / 4)) * 4, c = v / (BK / 4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) bs[buf][kk + e][c] = rb[p][e];
     }
   };
 
+  // U k-values per step: 4-byte elements take two products in a 3-input minimum
+  constexpr int U = sizeof(T) == 4 ? 2 : 1;
+  // fragment sets: with two waves per SIMD the next step's is read while this one is computed on; four hide the
+  // reads behind each other, and have no registers for it
+  constexpr int NF = WPE <= 2 ? 2 : 1;
   struct Frag {
-    T a[2][4], b[2][SN];
+    T a[U][TM], b[U][TN];
   };
-  auto load_frag = [&](Frag &f, int buf, int kk, int qi, int qj) {
+  auto load_frag = [&](Frag &f, int buf, int kk) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      *reinterpret_cast<V4 *>(&f.a[u][0]) = *reinterpret_cast<const V4 *>(&as[buf][kk + u][qi * 64 + tx * 4]);
+    for (int u = 0; u < U; ++u) {
 #pragma unroll
-      for (int q = 0; q < SN / 4; ++q)
-        *reinterpret_cast<V4 *>(&f.b[u][q * 4]) =
-            *reinterpret_cast<const V4 *>(&bs[buf][kk + u][(qj * (SN / 4) + q) * 64 + ty * 4]);
+      for (int q = 0; q < TM / 4; ++q) {
+        const V4 v = *reinterpret_cast<const V4 *>(&as[buf][kk + u][q * 64 + tx * 4]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f.a[u][q * 4 + e] = v[e];
+      }
+#pragma unroll
+      for (int q = 0; q < TN / 4; ++q) {
+        const V4 v = *reinterpret_cast<const V4 *>(&bs[buf][kk + u][q * (4 * TY) + ty * 4]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f.b[u][q * 4 + e] = v[e];
+      }
     }
   };
 
-  T acc[TM][TN];
-  int32_t chunk[TM][TN];
+  T acc[TM][TN], seen[TM][TN];   // running minima, now and at the end of the chunk before
+  // the chunk of each element's last strict improvement, -1 for none: 16 bits each, two to a register, where
+  // registers are short
+  constexpr bool PACK = WPE > 2;
+  uint32_t packed[TM][TN / 2];
+  int32_t wide[TM][TN];
+  auto chunk_of = [&](int i, int j) { return PACK ? int32_t(int16_t(packed[i][j / 2] >> (16 * (j & 1)))) : wide[i][j]; };
+  auto improved_in = [&](int i, int j) { return PACK ? (packed[i][j / 2] >> (16 * (j & 1)) & 0xffffu) != 0xffffu : wide[i][j] >= 0; };
+  auto record = [&](int i, int j, bool lower, int t) {
+    if constexpr (PACK) {
+      uint32_t &w = packed[i][j / 2];
+      const uint32_t with = j & 1 ? (w & 0xffffu) | uint32_t(t) << 16 : (w & 0xffff0000u) | uint32_t(t);
+      w = lower ? with : w;
+    } else {
+      wide[i][j] = lower ? t : wide[i][j];
+    }
+  };
 #pragma unroll
   for (int j = 0; j < TN; ++j)
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int r = row_of(i), c = col_of(j);
-      chunk[i][j] = -1;
+      if constexpr (PACK) packed[i][j / 2] = 0xffffffffu;
+      else wide[i][j] = -1;
       if constexpr (GUARD) acc[i][j] = (r < g.m && c < g.n) ? static_cast<const T *>(g.dist)[r + int64_t(c) * g.ldc] : -inf;
     }
   if constexpr (!GUARD) {
@@ -433,47 +464,44 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
   for (int t = 0; t < tiles; ++t) {
     const int cur = t & 1;
     if (t + 1 < tiles) fetch((t + 1) * BK);
-    // one block of 4 x SN outputs at a time, so that only its chunk minima are live
+    // The minima run on through the chunk; an element that is lower after it than before it improved in it.  (Each
+    // operand fragment serves a thread's whole 8 x 4 outputs: with blocks of 4 x 4, each with chunk minima of its own, the
+    // loop was bound by LDS reads.)
 #pragma unroll
-    for (int qi = 0; qi < TM / 4; ++qi)
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int qj = 0; qj < TN / SN; ++qj) {
-        T best[4][SN];
-        // two k-values per step (a 3-input minimum per pair of products); the next
-        // step's fragments are read from LDS while this one is computed, and the
-        // scheduling barriers keep the reads of later steps from being hoisted
-        // (a whole tile's fragments do not fit in registers)
-        Frag f[2];
-        load_frag(f[0], cur, 0, qi, qj);
+      for (int i = 0; i < TM; ++i) seen[i][j] = acc[i][j];
+    Frag f[NF];
+    if constexpr (NF == 2) load_frag(f[0], cur, 0);
 #pragma unroll
-        for (int kp = 0; kp < BK / 2; ++kp) {
-          if (kp + 1 < BK / 2) load_frag(f[(kp + 1) & 1], cur, 2 * (kp + 1), qi, qj);
-          __builtin_amdgcn_sched_barrier(0);
-          const Frag &x = f[kp & 1];
+    for (int s = 0; s < BK / U; ++s) {
+      if constexpr (NF == 1) load_frag(f[0], cur, U * s);
+      else if (s + 1 < BK / U) load_frag(f[(s + 1) % NF], cur, U * (s + 1));
+      __builtin_amdgcn_sched_barrier(0);
+      const Frag &x = f[s % NF];
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int h = 0; h < TM; h += 4) {  // (the sums of four outputs, then their minima: no minimum waits for its own sums)
+          T sum[U][4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int u = 0; u < U; ++u) sum[u][i] = x.a[u][h + i] + x.b[u][j];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-#pragma unroll
-            for (int j = 0; j < SN; ++j) {
-              const T p0 = x.a[0][i] + x.b[0][j], p1 = x.a[1][i] + x.b[1][j];
-              best[i][j] = kp == 0 ? hw_min<T>(p0, p1) : hw_min<T>(hw_min<T>(best[i][j], p0), p1);
-              // ties the arithmetic to this place in the instruction order: without it
-              // instruction selection emits it next to its only use, after every read
-              asm volatile("" : "+v"(best[i][j]));
-            }
-            __builtin_amdgcn_sched_barrier(0);
+            // (as instructions: from the builtin the compiler first "quiets" what comes round the loop)
+            if constexpr (U == 2) asm("v_min3_f32 %0, %0, %1, %2" : "+v"(acc[h + i][j]) : "v"(sum[0][i]), "v"(sum[U - 1][i]));
+            else asm("v_min_f64 %0, %0, %1" : "+v"(acc[h + i][j]) : "v"(sum[0][i]));
           }
+          if constexpr (WPE > 2) __builtin_amdgcn_sched_barrier(0);
         }
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-          for (int j = 0; j < SN; ++j) {
-            T &running = acc[qi * 4 + i][qj * SN + j];
-            int32_t &where = chunk[qi * 4 + i][qj * SN + j];
-            const bool lower = best[i][j] < running;
-            running = lower ? best[i][j] : running;
-            where = lower ? t : where;
-          }
-      }
+      for (int i = 0; i < TM; ++i) record(i, j, acc[i][j] < seen[i][j], t);
     if (t + 1 < tiles) stage(cur ^ 1);
     __syncthreads();
   }
@@ -488,17 +516,17 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
   if constexpr (!GUARD) {
     // Improved elements are few in most launches and scattered over the
     // lanes, so they are first collected in a queue in LDS (the panels are no longer needed) and the
-    // queue is then worked off by all 256 threads (lookup_queue): no lane waits for an element that did
+    // queue is then worked off by all threads (lookup_queue): no lane waits for an element that did
     // not improve.  The queue takes as many whole columns j of the lanes' outputs as fit (one column
-    // always does: at most 256 x TM elements), so a tile with few improved elements -- the usual case --
+    // always does: at most NT x TM elements), so a tile with few improved elements -- the usual case --
     // is done in one round of queueing, barrier and lookups, not one per column.
-    constexpr int CAP = (sizeof(as) / sizeof(int) < sizeof(bs) / sizeof(T) ? sizeof(as) / sizeof(int) : sizeof(bs) / sizeof(T)) / 256 * 256;
-    static_assert(CAP >= 256 * TM && BM <= 128 && BN <= 128, "a column of the lanes' outputs must fit in the panels");
+    constexpr int CAP = (sizeof(as) / sizeof(int) < sizeof(bs) / sizeof(T) ? sizeof(as) / sizeof(int) : sizeof(bs) / sizeof(T)) / NT * NT;
+    static_assert(CAP >= NT * TM && BM <= 128 && BN <= 128, "a column of the lanes' outputs must fit in the panels");
     // Where an element goes in the queue follows from counts alone, without a shared counter (whose every use is a
     // round trip to LDS that the next one waits for): column by column, inside a column wave by wave, inside a wave
     // row i by row i, inside a row lane by lane.  Each wave counts its improved elements per column first.
-    __shared__ int wave_count[4][TN];
-    uint32_t *q_code = reinterpret_cast<uint32_t *>(&as[0][0][0]);  // row | column << 7 | chunk << 14 (the host sees to k < 2^22)
+    auto &wave_count = sm.wave_count;
+    uint32_t *q_code = reinterpret_cast<uint32_t *>(&as[0][0][0]);  // row | column << 7 | chunk << 14 (the host sees to k < 2^19)
     T *q_want = reinterpret_cast<T *>(&bs[0][0][0]);                // the minimum found
     const int wave = tid >> 6;
     __syncthreads();  // everybody is done with the panels
@@ -506,7 +534,7 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
     for (int j = 0; j < TN; ++j) {
       int n_improved = 0;  // in this column, over the wave
 #pragma unroll
-      for (int i = 0; i < TM; ++i) n_improved += __builtin_popcountll(__builtin_amdgcn_ballot_w64(chunk[i][j] >= 0));
+      for (int i = 0; i < TM; ++i) n_improved += __builtin_popcountll(__builtin_amdgcn_ballot_w64(improved_in(i, j)));
       if ((tid & 63) == 0) wave_count[wave][j] = n_improved;
     }
     __syncthreads();
@@ -515,7 +543,7 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
     for (int j = 0; j < TN; ++j) {
       before_me[j] = col_count[j] = 0;
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
+      for (int w = 0; w < NT / 64; ++w) {
         const int n = __builtin_amdgcn_readfirstlane(wave_count[w][j]);
         before_me[j] += w < wave ? n : 0;
         col_count[j] += n;
@@ -538,11 +566,11 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
           int slot0 = base + before_me[j];  // of my wave's next row of this column
 #pragma unroll
           for (int i = 0; i < TM; ++i) {
-            const unsigned long long improved = __builtin_amdgcn_ballot_w64(chunk[i][j] >= 0);
-            if (chunk[i][j] >= 0) {
+            const unsigned long long improved = __builtin_amdgcn_ballot_w64(improved_in(i, j));
+            if (improved_in(i, j)) {
               const int slot = slot0 + __builtin_amdgcn_mbcnt_hi(uint32_t(improved >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(improved), 0u));
-              q_code[slot] = uint32_t((i >> 2) * 64 + tx2 * 4 + (i & 3)) | uint32_t((j >> 2) * 64 + ty2 * 4 + (j & 3)) << 7 |
-                             uint32_t(chunk[i][j]) << 14;
+              q_code[slot] = uint32_t((i >> 2) * 64 + tx2 * 4 + (i & 3)) | uint32_t((j >> 2) * (4 * TY) + ty2 * 4 + (j & 3)) << 7 |
+                             uint32_t(chunk_of(i, j)) << 14;
               q_want[slot] = acc[i][j];
             }
             slot0 += __builtin_popcountll(improved);
@@ -550,7 +578,7 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
           base += col_count[j];
         }
         __syncthreads();
-        lookup_queue<T, 256, BK, HAS_AT, 7, 7>(g, q_code, q_want, total, tid, m0, n0);
+        lookup_queue<T, NT, BK, HAS_AT, 7, 7, (sizeof(T) == 8 || WPE > 2) ? 4 : 8>(g, q_code, q_want, total, tid, m0, n0);
         __syncthreads();  // the queue is free again
       }
       j0 = j1;
@@ -559,12 +587,12 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
   }
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int c = n0 + (j >> 2) * 64 + ty2 * 4 + (j & 3);
+    const int c = n0 + (j >> 2) * (4 * TY) + ty2 * 4 + (j & 3);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int r = m0 + (i >> 2) * 64 + tx2 * 4 + (i & 3);
-      const int ch = chunk[i][j];
-      if (ch < 0) continue;
+      if (!improved_in(i, j)) continue;
+      const int ch = chunk_of(i, j);
       if constexpr (GUARD) {
         if (r >= g.m || c >= g.n) continue;
       }
@@ -604,79 +632,104 @@ constexpr int FW_BLOCK = 128;  // vertices per block step of the blocked Floyd-W
 // critical path: nothing that follows reads a diagonal block's predecessors, and the product is spread over 64
 // workgroups of a later launch.
 //
-// What stays on the critical path is fw_close_dist: the 128 dependent steps for the distances alone, an addition
-// and a minimum per element and step (half the instructions of a step that also selects predecessors, and none
-// that reads a comparison mask), by one workgroup of 256 threads with an 8 x 8 patch per thread.  Every row and
-// column that a step publishes to LDS for the next one also goes to hist (row k and column k as step k reads them),
-// and the block as it was found goes there too.
+// What stays on the critical path is fw_close_dist: the 128 dependent steps for the distances alone, by one workgroup.
+// They are taken in strips of sixteen.  The steps of a strip read nothing but its sixteen rows and its sixteen columns,
+// so those are brought up to date first, each row and column as far as the step that reads it:
+//   - every element of the strip's columns is lowered by the strip's earlier steps, row by row independently of the other
+//     rows but for the 16 x 16 block on the diagonal; a lane takes one row of the matrix (a lane of the other half of the
+//     waves one column), and beside it one row of the diagonal block, of which every group of sixteen lanes holds a copy:
+//     what step k needs of the diagonal block's row k is then one lane's value handed round inside sixteen lanes, an
+//     operand of the addition, and the sixteen steps need no barrier and nothing from LDS;
+//   - the rows and columns as their steps read them go to LDS and to hist;
+//   - every element of the block is lowered by all sixteen steps at once, a min-plus product with a 3-input minimum per
+//     two steps -- the same sums and the same minima as step by step, so the distances are the same to the bit.
+// Two barriers per sixteen steps.  (One barrier per two steps, rows and columns published through LDS, took 68 us (4-byte
+// elements) and 110 us (8-byte) alone on the chip.)
 //
 // The hardware minimum prefers -0 to +0 where the strict comparison keeps whichever came first.  Sums and minima
 // of data free of -0 never produce one, so the block is searched for a -0 when it is loaded, and a block with
 // one is closed by fw_close_dist_exact instead: the same steps with a comparison and a select, the block in place.
 //
 // hist: FW_BLOCK x FW_BLOCK elements each of  col[k * FW_BLOCK + i] = d[i][k] before step k,
-// row[k * FW_BLOCK + j] = d[k][j] before step k,  init[(8 * (i % 8) + j % 8) * 256 + i / 8 + 16 * (j / 8)] = d[i][j] before
-// the closure.
+// row[k * FW_BLOCK + j] = d[k][j] before step k,  init[i + j * FW_BLOCK] = d[i][j] before the closure.
+constexpr int FW_STRIP = 16;
+// columns and rows of a strip as its first step finds them, and as their own steps read them
+template <typename T> struct FwCloseLds {
+  T cols[FW_STRIP][FW_BLOCK], rows[FW_STRIP][FW_BLOCK], step_cols[FW_STRIP][FW_BLOCK], step_rows[FW_STRIP][FW_BLOCK];
+};
+
+// a thread's patch of the block: PM x PN elements, rows PM ti .., columns PN tj ..
+template <int NT> struct FwPatch {
+  static constexpr int PM = NT == 256 ? 8 : 4, PN = FW_BLOCK * FW_BLOCK / NT / PM, TI = FW_BLOCK / PM;
+  static_assert(PN % 4 == 0 && FW_BLOCK % PM == 0 && TI * (FW_BLOCK / PN) == NT && FW_STRIP % PN == 0, "patch");
+};
+
+// v of lane K of each group of sixteen lanes
+template <int K, typename T> __device__ __forceinline__ T row_lane(T v) {
+  if constexpr (sizeof(T) == 4) {
+    const int b = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(b, b, 0x150 + K, 0xf, 0xf, true));
+  } else {
+    const long long b = __builtin_bit_cast(long long, v);
+    const int lo = int(b), hi = int(b >> 32);
+    const unsigned l = (unsigned)__builtin_amdgcn_update_dpp(lo, lo, 0x150 + K, 0xf, 0xf, true);
+    const unsigned h = (unsigned)__builtin_amdgcn_update_dpp(hi, hi, 0x150 + K, 0xf, 0xf, true);
+    return __builtin_bit_cast(T, (long long)((unsigned long long)h << 32 | l));
+  }
+}
+
 // (returns false, with nothing done, when the block holds a -0)
-// (A function of its own, not inlined: as part of a kernel that also holds the other form and a product's tile, the
-// compiler's register allocation moves parts of the patch to scratch memory inside the step loop, where any wait for
-// memory also waits for the stores to hist.  Alone, either form fits the registers.)
-template <typename T>
-__device__ __attribute__((noinline)) bool fw_close_dist_fast(T *d_anywhere, int64_t ld, int bb, T *hist_anywhere,
-                                                           __attribute__((address_space(3))) T *colbuf,
-                                                           __attribute__((address_space(3))) T *rowbuf) {
+template <typename T, int NT>
+__device__ __forceinline__ bool fw_close_dist_fast(T *d, int64_t ld, int bb, T *hist, FwCloseLds<T> &sm) {
   typedef typename vec4_of<T>::type V4;
-  typedef __attribute__((address_space(3))) T LT;
-  typedef __attribute__((address_space(3))) V4 LV4;
-  // (both are device memory, which a function that is not a kernel has to be told: a store to "memory of some
-  // kind" counts as an LDS access as well, and the waits for LDS before each barrier would wait for it)
-  typedef __attribute__((address_space(1))) T GT;
-  typedef __attribute__((address_space(1))) V4 GV4;
-  GT *const d = (GT *)d_anywhere, *const hist = (GT *)hist_anywhere;
-  // colbuf, rowbuf: lines of FW_BLOCK elements in LDS for columns k (and k + 1) as the steps read them, and for
-  // the rows: two sets of one line for 8-byte elements (lines 0 and 2), four sets of two lines for 4-byte elements
-  const int tid = threadIdx.x & 255, ti = tid & 15, tj = tid >> 4;  // rows 8 ti .. 8 ti + 7, columns 8 tj .. 8 tj + 7
+  typedef typename uvec4_of<T>::type U4;
+  constexpr int PM = FwPatch<NT>::PM, PN = FwPatch<NT>::PN, TI = FwPatch<NT>::TI;
+  const int tid = threadIdx.x, ti = tid % TI, tj = tid / TI;
   const T inf = std::numeric_limits<T>::infinity();
-  GT *hist_col = hist, *hist_row = hist + FW_BLOCK * FW_BLOCK, *init = hist + 2 * FW_BLOCK * FW_BLOCK;
-  T cur[8][8];  // [row in patch][column in patch]
-  // loads from clamped addresses, then a select (a branch per element would keep 64 lane masks alive); a column's
-  // addresses differ by the clamped row, so that the 64 loads in flight do not need 64 addresses in registers
-  int ic[8];
+  T *hist_col = hist, *hist_row = hist + FW_BLOCK * FW_BLOCK, *init = hist + 2 * FW_BLOCK * FW_BLOCK;
+  T cur[PN][PM];  // [column in patch][row in patch]
+  if (bb == FW_BLOCK) {
 #pragma unroll
-  for (int a = 0; a < 8; ++a) ic[a] = min(8 * ti + a, bb - 1);
+    for (int b = 0; b < PN; ++b)
 #pragma unroll
-  for (int b = 0; b < 8; ++b) {
-    const int j = 8 * tj + b;
-    const GT *column = d + int64_t(min(j, bb - 1)) * ld;
+      for (int a = 0; a < PM; a += 4) {
+        const V4 v = *reinterpret_cast<const U4 *>(d + PM * ti + a + int64_t(PN * tj + b) * ld);
 #pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      const T v = column[ic[a]];
-      cur[a][b] = (8 * ti + a < bb && j < bb) ? v : inf;
-    }
+        for (int e = 0; e < 4; ++e) cur[b][a + e] = v[e];
+      }
+  } else {
+    // loads from clamped addresses, then a select (a branch per element would keep all the lane masks alive)
+#pragma unroll
+    for (int b = 0; b < PN; ++b)
+#pragma unroll
+      for (int a = 0; a < PM; ++a) {
+        const T v = d[min(PM * ti + a, bb - 1) + int64_t(min(PN * tj + b, bb - 1)) * ld];
+        cur[b][a] = (PM * ti + a < bb && PN * tj + b < bb) ? v : inf;
+      }
   }
-  {
-    // a block with a -0 is left to the other form (a function of its own too: as part of this one the registers
-    // it needs would be taken from this one's loop)
-    bool negative_zero = false;
+  bool negative_zero = false;
 #pragma unroll
-    for (int b = 0; b < 8; ++b)
+  for (int b = 0; b < PN; ++b)
 #pragma unroll
-      for (int a = 0; a < 8; ++a) negative_zero |= cur[a][b] == T(0) && __builtin_signbit(cur[a][b]);
-    if (__syncthreads_or(negative_zero)) return false;
-  }
-  // (element by element, a thread's elements 256 apart: written four at a time, the patch's registers would have
-  // to be adjacent in fours, and the compiler moves parts of the patch to scratch memory over that in the loop below)
+    for (int a = 0; a < PM; ++a) negative_zero |= cur[b][a] == T(0) && __builtin_signbit(cur[b][a]);
+  if (__syncthreads_or(negative_zero)) return false;
+  auto put4 = [](T *to, const T *from) {
+    V4 v;
 #pragma unroll
-  for (int b = 0; b < 8; ++b)
+    for (int e = 0; e < 4; ++e) v[e] = from[e];
+    *reinterpret_cast<V4 *>(to) = v;
+  };
 #pragma unroll
-    for (int a = 0; a < 8; ++a) init[(8 * a + b) * 256 + tid] = cur[a][b];
+  for (int b = 0; b < PN; ++b)
+#pragma unroll
+    for (int a = 0; a < PM; a += 4) put4(&init[PM * ti + a + (PN * tj + b) * FW_BLOCK], &cur[b][a]);
   // (the minimum as an instruction: from the builtin the compiler first "quiets" an operand whose origin it
   // does not know, such as anything that comes round the loop, an instruction more per element)
   auto relax = [](T &x, const T cand) {
     if constexpr (sizeof(T) == 4) asm("v_min_f32 %0, %0, %1" : "+v"(x) : "v"(cand));
     else asm("v_min_f64 %0, %0, %1" : "+v"(x) : "v"(cand));
   };
-  // two steps' candidates at once, in the steps' order
+  // two steps' candidates at once
   auto relax2 = [&](T &x, const T first, const T second) {
     if constexpr (sizeof(T) == 4) {
       asm("v_min3_f32 %0, %0, %1, %2" : "+v"(x) : "v"(first), "v"(second));
@@ -685,310 +738,153 @@ __device__ __attribute__((noinline)) bool fw_close_dist_fast(T *d_anywhere, int6
       relax(x, second);
     }
   };
-  // Rows and columns go to LDS two elements per instruction, each from a register of its own: as 16-byte stores the
-  // compiler wants every row of the patch AND every column of it in four adjacent registers, cannot have both, and
-  // moves parts of the patch to scratch memory in the attempt.  colbuf / rowbuf: [2 * buffer + which of the pair]
-  auto lds = [](const LT *q) { return (unsigned)(size_t)q; };
-  auto write2 = [](unsigned addr, const T x, const T y, auto at) {
-    constexpr int AT = decltype(at)::value;  // in elements
-    if constexpr (sizeof(T) == 4) asm volatile("ds_write2_b32 %0, %1, %2 offset0:%3 offset1:%4" ::"v"(addr), "v"(x), "v"(y), "n"(AT), "n"(AT + 1) : "memory");
-    else asm volatile("ds_write2_b64 %0, %1, %2 offset0:%3 offset1:%4" ::"v"(addr), "v"(x), "v"(y), "n"(AT), "n"(AT + 1) : "memory");
+  auto get4 = [](T *x, const T *from) {
+    const V4 v = *reinterpret_cast<const V4 *>(from);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = v[e];
   };
-  // row S of the patch to row_at, column S to col_at (S is a compile-time constant, the step loop being unrolled
-  // by eight: indexed by a run-time value the patch would live in scratch memory)
-  auto put_row = [&](unsigned row_at, auto sc, auto at) {
-    constexpr int S = decltype(sc)::value, AT = decltype(at)::value;
-    write2(row_at, cur[S][0], cur[S][1], std::integral_constant<int, AT + 0>{});
-    write2(row_at, cur[S][2], cur[S][3], std::integral_constant<int, AT + 2>{});
-    write2(row_at, cur[S][4], cur[S][5], std::integral_constant<int, AT + 4>{});
-    write2(row_at, cur[S][6], cur[S][7], std::integral_constant<int, AT + 6>{});
-  };
-  auto put_col = [&](unsigned col_at, auto sc, auto at) {
-    constexpr int S = decltype(sc)::value, AT = decltype(at)::value;
-    write2(col_at, cur[0][S], cur[1][S], std::integral_constant<int, AT + 0>{});
-    write2(col_at, cur[2][S], cur[3][S], std::integral_constant<int, AT + 2>{});
-    write2(col_at, cur[4][S], cur[5][S], std::integral_constant<int, AT + 4>{});
-    write2(col_at, cur[6][S], cur[7][S], std::integral_constant<int, AT + 6>{});
-  };
-  auto get8 = [&](T (&x)[8], const LT *from) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const V4 v = *reinterpret_cast<const LV4 *>(from + 4 * h);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) x[4 * h + e] = v[e];
-    }
-  };
-  auto put8 = [&](GT *to, const T (&x)[8]) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      V4 v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = x[4 * h + e];
-      *reinterpret_cast<GV4 *>(to + 4 * h) = v;
-    }
-  };
-
-  if constexpr (sizeof(T) == 8) {
-    // ---- 8-byte elements: one step per barrier, in one part.  The patch takes half the register file, and a
-    // second set of rows and columns on its way beside the one in use pushes parts of the patch into scratch
-    // memory.  (The product beside this closure takes twice as long anyway.)
-    const unsigned row_lds[2] = {lds(rowbuf + (0) * FW_BLOCK + 8 * tj), lds(rowbuf + (2) * FW_BLOCK + 8 * tj)};
-    const unsigned col_lds[2] = {lds(colbuf + (0) * FW_BLOCK + 8 * ti), lds(colbuf + (2) * FW_BLOCK + 8 * ti)};
-    T ci[8], rj[8];  // column k at my rows, row k at my columns, for the step in hand
-    auto publish = [&](int kn, auto bufc, auto sc) {
-      constexpr int BUF = decltype(bufc)::value;
-      if ((kn >> 3) == ti) put_row(row_lds[BUF], sc, std::integral_constant<int, 0>{});  // my patch holds row kn
-      if ((kn >> 3) == tj) put_col(col_lds[BUF], sc, std::integral_constant<int, 0>{});  // my patch holds column kn
-      // (the barrier that follows is the compiler's, which does not know of the instructions above)
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    };
-    // what step kn reads goes to hist from the registers of the threads of the first patch row / column, which
-    // together have read all of it
-    auto fetch = [&](int buf, int kn) {
-      get8(ci, colbuf + (2 * buf) * FW_BLOCK + 8 * ti);
-      get8(rj, rowbuf + (2 * buf) * FW_BLOCK + 8 * tj);
-      if (kn >= FW_BLOCK) return;
-      if (tj == 0) put8(&hist_col[kn * FW_BLOCK + 8 * ti], ci);
-      if (ti == 0) put8(&hist_row[kn * FW_BLOCK + 8 * tj], rj);
-    };
-    auto step = [&](int k, auto uc) {
-      constexpr int U = decltype(uc)::value;  // k & 7
-#pragma unroll
-      for (int a = 0; a < 8; ++a)
-#pragma unroll
-        for (int b = 0; b < 8; ++b) relax(cur[a][b], ci[a] + rj[b]);
-      __builtin_amdgcn_sched_barrier(0);
-      // into the other pair of buffers: nobody reads it before the barrier, and nobody is still reading it
-      // from the step before (everybody has passed that step's barrier, and used what it read before that)
-      publish(k + 1, std::integral_constant<int, (U & 1) ^ 1>{}, std::integral_constant<int, (U + 1) & 7>{});
-      __syncthreads();
-      fetch((U & 1) ^ 1, k + 1);
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    publish(0, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
-    __syncthreads();
-    fetch(0, 0);
-    // steps beyond bb (up to the next multiple of eight) read rows and columns of the padding, which hold
-    // +infinity and improve nothing
+  // steps beyond bb (up to the next multiple of sixteen) read rows and columns of the padding, which hold
+  // +infinity and improve nothing
 #pragma unroll 1
-    for (int k8 = 0; k8 < bb; k8 += 8) {
-      step(k8 + 0, std::integral_constant<int, 0>{});
-      step(k8 + 1, std::integral_constant<int, 1>{});
-      step(k8 + 2, std::integral_constant<int, 2>{});
-      step(k8 + 3, std::integral_constant<int, 3>{});
-      step(k8 + 4, std::integral_constant<int, 4>{});
-      step(k8 + 5, std::integral_constant<int, 5>{});
-      step(k8 + 6, std::integral_constant<int, 6>{});
-      step(k8 + 7, std::integral_constant<int, 7>{});
+  for (int k0 = 0; k0 < bb; k0 += FW_STRIP) {
+    // the strip's columns and rows, as they are before its first step
+    if (unsigned(PN * tj - k0) < FW_STRIP) {
+#pragma unroll
+      for (int b = 0; b < PN; ++b)
+#pragma unroll
+        for (int a = 0; a < PM; a += 4) put4(&sm.cols[PN * tj - k0 + b][PM * ti + a], &cur[b][a]);
     }
-  } else {
-    // ---- 4-byte elements: two steps per barrier, in two parts.
-    //
-    // Steps k and k + 1 (k even) together.  Before them the owners publish columns k and k + 1 and rows k and k + 1
-    // as they are before step k.  What step k + 1 reads is column k + 1 and row k + 1 AFTER step k, and every thread
-    // can work that out for its own rows and columns from what has been published:
-    //   d[i][k+1] after step k = min(d[i][k+1], d[i][k] + d[k][k+1]),  d[k+1][j] after step k = min(d[k+1][j], d[k+1][k] + d[k][j])
-    // (the sums and comparisons that step k itself makes for those elements, made again).  An element then takes
-    // both steps' candidates in one 3-input minimum: three instructions per element and two steps instead of four,
-    // and one round of publish / barrier / read-back per two steps.
-    //
-    // The steps depend on each other, and what lies between two pairs of them (publishing, the barrier, reading
-    // back) would add its full latency to every pair.  So a pair is done in two parts:
-    //   A. the patch's rows and columns (k + 2) & 7 and (k + 3) & 7 -- every thread's, since which thread owns
-    //      rows / columns k + 2 and k + 3 is only known at run time -- then the owners publish them, then the barrier;
-    //   B. the reads for the next pair are issued, and the other 36 elements are done while they are on their way.
-    //
-    // The published lines are what hist gets (for these element types hist holds, for odd k, column k and row k as
-    // they are before step k - 1: fw_parents_block makes the same correction), copied from LDS by half the threads
-    // a barrier after they were published.  There are four sets of lines in LDS, used in turn: a set is written again
-    // three barriers after it was read for the last time.  (Nothing in this loop may wait for memory: stores
-    // to hist are on their way all the time, and a wait for any load would wait for them.)
-    const unsigned row_lds[4] = {lds(rowbuf + (0) * FW_BLOCK + 8 * tj), lds(rowbuf + (2) * FW_BLOCK + 8 * tj), lds(rowbuf + (4) * FW_BLOCK + 8 * tj), lds(rowbuf + (6) * FW_BLOCK + 8 * tj)};
-    const unsigned col_lds[4] = {lds(colbuf + (0) * FW_BLOCK + 8 * ti), lds(colbuf + (2) * FW_BLOCK + 8 * ti), lds(colbuf + (4) * FW_BLOCK + 8 * ti), lds(colbuf + (6) * FW_BLOCK + 8 * ti)};
-    // (the lines' addresses in vector registers of the thread's own: as values that are the same for all
-    // threads the compiler fetches them again for every pair, and waits for that with the reads above)
-    unsigned row_at_0 = lds(rowbuf), col_at_0 = lds(colbuf);
-    asm volatile("" : "+v"(row_at_0), "+v"(col_at_0));
+    if (unsigned(PM * ti - k0) < FW_STRIP) {
+#pragma unroll
+      for (int a = 0; a < PM; ++a)
+#pragma unroll
+        for (int b = 0; b < PN; b += 4) {
+          const T v[4] = {cur[b][a], cur[b + 1][a], cur[b + 2][a], cur[b + 3][a]};
+          put4(&sm.rows[PM * ti - k0 + a][PN * tj + b], v);
+        }
+    }
+    __syncthreads();
+    // waves 0 and 1: a row of the strip's columns per lane; waves 2 and 3: a column of its rows (the diagonal block
+    // transposed with them; an addition's operands change places and its result stays)
+    if (tid < 2 * FW_BLOCK) {
+      T(*const lines)[FW_BLOCK] = tid < FW_BLOCK ? sm.cols : sm.rows;
+      T(*const step_lines)[FW_BLOCK] = tid < FW_BLOCK ? sm.step_cols : sm.step_rows;
+      T *const kept = (tid < FW_BLOCK ? hist_col : hist_row) + k0 * FW_BLOCK;
+      const int at = tid & (FW_BLOCK - 1);
+      T x[FW_STRIP], diag[FW_STRIP];
+#pragma unroll
+      for (int q = 0; q < FW_STRIP; ++q) {
+        x[q] = lines[q][at];
+        diag[q] = lines[q][k0 + (tid & 15)];
+      }
+      static_for<FW_STRIP - 1>([&](auto kc) {
+        constexpr int K = decltype(kc)::value;
+        // (lines before K have been read by their steps: this strip needs them no more.  All sums of a step, then all
+        // minima: one behind the other each would wait for the one before it)
+        T sum_x[FW_STRIP], sum_diag[FW_STRIP];
+#pragma unroll
+        for (int q = K + 1; q < FW_STRIP; ++q) {
+          const T step = row_lane<K>(diag[q]);
+          sum_x[q] = x[K] + step;
+          sum_diag[q] = diag[K] + step;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = K + 1; q < FW_STRIP; ++q) relax(diag[q], sum_diag[q]);
+#pragma unroll
+        for (int q = K + 1; q < FW_STRIP; ++q) relax(x[q], sum_x[q]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+#pragma unroll
+      for (int q = 0; q < FW_STRIP; ++q) {
+        step_lines[q][at] = x[q];
+        kept[q * FW_BLOCK + at] = x[q];
+      }
+    }
+    __syncthreads();
     struct Lines {
-      T c0[8], c1[8], r0[8], r1[8];  // columns k, k + 1 at my rows, rows k, k + 1 at my columns, before step k
-      T at_01, at_10;                // d[k][k + 1], d[k + 1][k]
+      T c[2][PM], r[2][PN];
     };
-    auto publish = [&](int kn, auto setc, auto sc) {
-      constexpr int SET = decltype(setc)::value, S = decltype(sc)::value;
-      if ((kn >> 3) == ti) {  // my patch holds rows kn and kn + 1
-        put_row(row_lds[SET], std::integral_constant<int, S>{}, std::integral_constant<int, 0>{});
-        put_row(row_lds[SET], std::integral_constant<int, S + 1>{}, std::integral_constant<int, FW_BLOCK>{});
-      }
-      if ((kn >> 3) == tj) {  // my patch holds columns kn and kn + 1
-        put_col(col_lds[SET], std::integral_constant<int, S>{}, std::integral_constant<int, 0>{});
-        put_col(col_lds[SET], std::integral_constant<int, S + 1>{}, std::integral_constant<int, FW_BLOCK>{});
-      }
-      // (the barrier that follows is the compiler's, which does not know of the instructions above)
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    };
-    auto fetch = [&](Lines &l, int set, int kn) {
-      get8(l.c0, colbuf + (2 * set) * FW_BLOCK + 8 * ti);
-      get8(l.c1, colbuf + (2 * set + 1) * FW_BLOCK + 8 * ti);
-      get8(l.r0, rowbuf + (2 * set) * FW_BLOCK + 8 * tj);
-      get8(l.r1, rowbuf + (2 * set + 1) * FW_BLOCK + 8 * tj);
-      const unsigned at = unsigned(((2 * set) * FW_BLOCK + ((kn + 1) & (FW_BLOCK - 1))) * sizeof(T));
-      l.at_01 = *(const LT *)(size_t)(row_at_0 + at);
-      l.at_10 = *(const LT *)(size_t)(col_at_0 + at);
-    };
-    // the four lines of a set (steps kn and kn + 1) from LDS to hist: 16 bytes per thread of the first two waves
-    const int line = tid >> 5, piece = 4 * (tid & 31);
-    GT *const hist_line = (line < 2 ? hist_col : hist_row) + (line & 1) * FW_BLOCK + piece;
-    auto keep = [&](int set, int kn) {
-      if (tid < 128 && kn < FW_BLOCK)
-        *reinterpret_cast<GV4 *>(hist_line + kn * FW_BLOCK) =
-            *(const LV4 *)(size_t)((line < 2 ? col_at_0 : row_at_0) + unsigned(((2 * set + (line & 1)) * FW_BLOCK + piece) * sizeof(T)));
-    };
-    Lines cur_l;
-    auto pair = [&](int k, auto uc) {
-      constexpr int U = decltype(uc)::value;  // k & 7: 0, 2, 4, 6
-      constexpr int N = (U + 2) & 7;          // the rows and columns N, N + 1 of the patch are what steps k + 2, k + 3 may need
-      constexpr int O[6] = {N > 0 ? 0 : 2, N > 0 ? 1 : 3, N > 2 ? 2 : 4, N > 2 ? 3 : 5, N > 4 ? 4 : 6, N > 4 ? 5 : 7};
-      constexpr int SET = U >> 1;
-      Lines &l = cur_l;
-      // column k + 1 and row k + 1 after step k
+    constexpr int NL = PM * PN * sizeof(T) > 256 ? 1 : 2;   // (a patch of 64 doubles leaves no registers for a second set)
+    Lines lines[NL];
+    auto read = [&](Lines &l, int kk) {
 #pragma unroll
-      for (int x = 0; x < 8; ++x) {
-        relax(l.c1[x], l.c0[x] + l.at_01);
-        relax(l.r1[x], l.at_10 + l.r0[x]);
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int a = 0; a < PM; a += 4) get4(&l.c[u][a], &sm.step_cols[kk + u][PM * ti + a]);
+#pragma unroll
+        for (int b = 0; b < PN; b += 4) get4(&l.r[u][b], &sm.step_rows[kk + u][PN * tj + b]);
       }
-      auto both = [&](auto ac, auto bc) {
-        constexpr int A = decltype(ac)::value, B = decltype(bc)::value;
-        relax2(cur[A][B], l.c0[A] + l.r0[B], l.c1[A] + l.r1[B]);
-      };
-      // A.
-      static_for<8>([&](auto bc) {
-        both(std::integral_constant<int, N>{}, bc);
-        both(std::integral_constant<int, N + 1>{}, bc);
-      });
-      static_for<6>([&](auto ic) {
-        both(std::integral_constant<int, O[decltype(ic)::value]>{}, std::integral_constant<int, N>{});
-        both(std::integral_constant<int, O[decltype(ic)::value]>{}, std::integral_constant<int, N + 1>{});
-      });
-      __builtin_amdgcn_sched_barrier(0);
-      publish(k + 2, std::integral_constant<int, (SET + 1) & 3>{}, std::integral_constant<int, N>{});
-      __syncthreads();
-      Lines next;
-      fetch(next, (SET + 1) & 3, k + 2);
-      __builtin_amdgcn_sched_barrier(0);
-      // B.
-      static_for<6>([&](auto ic) {
-        static_for<6>([&](auto jc) {
-          both(std::integral_constant<int, O[decltype(ic)::value]>{}, std::integral_constant<int, O[decltype(jc)::value]>{});
-        });
-      });
-      __builtin_amdgcn_sched_barrier(0);
-      keep((SET + 1) & 3, k + 2);
-      cur_l = next;
     };
-    publish(0, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
-    __syncthreads();
-    fetch(cur_l, 0, 0);
-    keep(0, 0);
-    // steps beyond bb (up to the next multiple of eight) read rows and columns of the padding, which hold
-    // +infinity and improve nothing
-#pragma unroll 1
-    for (int k8 = 0; k8 < bb; k8 += 8) {
-      pair(k8 + 0, std::integral_constant<int, 0>{});
-      pair(k8 + 2, std::integral_constant<int, 2>{});
-      pair(k8 + 4, std::integral_constant<int, 4>{});
-      pair(k8 + 6, std::integral_constant<int, 6>{});
+    if constexpr (NL == 2) read(lines[0], 0);
+#pragma unroll
+    for (int kk = 0; kk < FW_STRIP; kk += 2) {
+      if constexpr (NL == 1) read(lines[0], kk);
+      else if (kk + 2 < FW_STRIP) read(lines[((kk >> 1) + 1) % NL], kk + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      const Lines &l = lines[(kk >> 1) % NL];
+#pragma unroll
+      for (int b = 0; b < PN; ++b) {
+        T s0[PM], s1[PM];
+#pragma unroll
+        for (int a = 0; a < PM; ++a) {
+          s0[a] = l.c[0][a] + l.r[0][b];
+          s1[a] = l.c[1][a] + l.r[1][b];
+        }
+#pragma unroll
+        for (int a = 0; a < PM; ++a) relax2(cur[b][a], s0[a], s1[a]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
+    // (no barrier: what the next strip writes before its first one has been read by everybody before this strip's second)
   }
 #pragma unroll
-  for (int b = 0; b < 8; ++b)
+  for (int b = 0; b < PN; ++b)
 #pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      const int i = 8 * ti + a, j = 8 * tj + b;
-      T v = cur[a][b];
-      asm volatile("" : "+v"(v));  // (a value of its own: see the stores of init above)
-      if (i < bb && j < bb) d[i + int64_t(j) * ld] = v;
+    for (int a = 0; a < PM; ++a) {
+      const int i = PM * ti + a, j = PN * tj + b;
+      if (i < bb && j < bb) d[i + int64_t(j) * ld] = cur[b][a];
     }
   return true;
 }
 
-// The same closure for a block that holds a -0: comparison and select, one step per barrier, and the block's rows and
-// columns handed from step to step through the block itself in device memory (every thread stores what it lowered,
-// and reads column k and row k from there), with the step loop rolled.  Two to three times slower than the form
-// above, a fraction of its code, and nothing of it in scratch memory -- a form like the one above with comparisons
-// keeps 64 comparison masks and as many candidates alive and spills hundreds of registers, which every workgroup
-// of the kernel pays for in scratch space, whether it ever sees a -0 or not.
-template <typename T>
+// The same closure for a block that holds a -0: comparison and select, two barriers per step, the block itself in device
+// memory (every thread keeps to its own elements) and column k and row k read from hist.  Several times slower than the
+// form above and little code, out of the way of the other's registers.
+template <typename T, int NT>
 __device__ __attribute__((noinline)) void fw_close_dist_exact(T *d_anywhere, int64_t ld, int bb, T *hist_anywhere) {
   typedef __attribute__((address_space(1))) T GT;
   GT *const d = (GT *)d_anywhere, *const hist = (GT *)hist_anywhere;
   GT *hist_col = hist, *hist_row = hist + FW_BLOCK * FW_BLOCK, *init = hist + 2 * FW_BLOCK * FW_BLOCK;
-  const int tid = threadIdx.x & 255, ti = tid & 15, tj = tid >> 4;  // rows 8 ti .. 8 ti + 7, columns 8 tj .. 8 tj + 7
+  // a thread's elements: row i, columns j0, j0 + NT / FW_BLOCK, ...
+  const int tid = threadIdx.x, i = tid & (FW_BLOCK - 1), j0 = tid / FW_BLOCK;
   const T inf = std::numeric_limits<T>::infinity();
-  // (rows and columns of the padding are computed on the block's last row / column and never stored)
-  int ic[8];
-#pragma unroll
-  for (int a = 0; a < 8; ++a) ic[a] = min(8 * ti + a, bb - 1);
-  T cur[8][8];
-#pragma unroll
-  for (int b = 0; b < 8; ++b) {
-    const GT *column = d + int64_t(min(8 * tj + b, bb - 1)) * ld;
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      cur[a][b] = (8 * ti + a < bb && 8 * tj + b < bb) ? column[ic[a]] : inf;
-      init[(8 * a + b) * 256 + tid] = cur[a][b];
-    }
-  }
-  // what hist holds for 4-byte elements (fw_parents_block): for odd k column k and row k as before step k - 1
-  constexpr int PAIRED = sizeof(T) == 4 ? 1 : 0;
+  for (int j = j0; j < FW_BLOCK; j += NT / FW_BLOCK) init[i + j * FW_BLOCK] = i < bb && j < bb ? T(d[i + int64_t(j) * ld]) : inf;
 #pragma unroll 1
   for (int k = 0; k < bb; ++k) {
     __syncthreads();  // what step k - 1 lowered is in the block
-    T ci[8], rj[8];
-#pragma unroll
-    for (int a = 0; a < 8; ++a) ci[a] = d[ic[a] + int64_t(k) * ld];
-#pragma unroll
-    for (int b = 0; b < 8; ++b) rj[b] = d[k + int64_t(min(8 * tj + b, bb - 1)) * ld];
-    if (!PAIRED || !(k & 1)) {
-      const int lines = PAIRED ? 2 : 1;
-      for (int q = 0; q < lines; ++q) {
-        const int kq = min(k + q, bb - 1);
-        if (tj == 0)
-#pragma unroll
-          for (int a = 0; a < 8; ++a) hist_col[(k + q) * FW_BLOCK + 8 * ti + a] = 8 * ti + a < bb ? (q ? T(d[ic[a] + int64_t(kq) * ld]) : ci[a]) : inf;
-        if (ti == 0)
-#pragma unroll
-          for (int b = 0; b < 8; ++b)
-            hist_row[(k + q) * FW_BLOCK + 8 * tj + b] = 8 * tj + b < bb ? (q ? T(d[kq + int64_t(min(8 * tj + b, bb - 1)) * ld]) : rj[b]) : inf;
-      }
+    if (j0 == 0) {
+      hist_col[k * FW_BLOCK + i] = i < bb ? T(d[i + int64_t(k) * ld]) : inf;
+      hist_row[k * FW_BLOCK + i] = i < bb ? T(d[k + int64_t(i) * ld]) : inf;
     }
-    __syncthreads();  // everybody has read column k and row k (and k + 1) before anybody stores
-#pragma unroll
-    for (int b = 0; b < 8; ++b)
-#pragma unroll
-      for (int a = 0; a < 8; ++a) {
-        const T cand = ci[a] + rj[b];
-        if (cand < cur[a][b]) {
-          cur[a][b] = cand;
-          if (8 * ti + a < bb && 8 * tj + b < bb) d[8 * ti + a + int64_t(8 * tj + b) * ld] = cand;
-        }
-      }
+    __syncthreads();  // column k and row k are in hist before anybody lowers anything
+    const T ci = hist_col[k * FW_BLOCK + i];
+#pragma unroll 4
+    for (int j = j0; j < bb; j += NT / FW_BLOCK) {
+      const T cand = ci + hist_row[k * FW_BLOCK + j];
+      if (i < bb && cand < d[i + int64_t(j) * ld]) d[i + int64_t(j) * ld] = cand;
+    }
   }
 }
 
-template <typename T>
-__device__ __forceinline__ void fw_close_dist(T *d, int64_t ld, int bb, T *hist) {
-  typedef __attribute__((address_space(3))) T LT;
-  constexpr int LINES = sizeof(T) == 4 ? 8 : 4;
-  __shared__ __attribute__((aligned(32))) T colbuf[LINES * FW_BLOCK], rowbuf[LINES * FW_BLOCK];
-  if (!fw_close_dist_fast<T>(d, ld, bb, hist, (LT *)colbuf, (LT *)rowbuf)) fw_close_dist_exact<T>(d, ld, bb, hist);
+template <typename T, int NT>
+__device__ __forceinline__ void fw_close_dist(T *d, int64_t ld, int bb, T *hist, FwCloseLds<T> &sm) {
+  if (!fw_close_dist_fast<T, NT>(d, ld, bb, hist, sm)) fw_close_dist_exact<T, NT>(d, ld, bb, hist);
 }
 
 // The predecessors of a diagonal block whose distances fw_close_dist has closed: workgroup b of 64 (256 threads)
 // takes rows 64 (b & 1) .. + 63 and columns 4 (b >> 1) .. + 3, one element per thread, and runs the literal scan
 // over the recorded columns and rows.  Only predecessors are written: the distances are those already there.
-// For 4-byte elements hist holds, for odd k, column k and row k as they are before step k - 1; step k - 1's
-// update of them is made here as fw_close_dist makes it (with the comparison: it never differs from the minimum
-// on a block without -0, and a block with one was closed with the comparison).
 template <typename T>
 __device__ __forceinline__ void fw_parents_block(const T *hist, int32_t *parent, int64_t ldp, int bb, int k_base, int b) {
   const int row = (b & 1) * 64 + (threadIdx.x & 63);
@@ -996,54 +892,25 @@ __device__ __forceinline__ void fw_parents_block(const T *hist, int32_t *parent,
   if (row >= bb || col >= bb) return;
   const T *hist_row = hist + FW_BLOCK * FW_BLOCK;
   const T *hc = hist + row, *hr = hist_row + col;
-  T curr = hist[2 * FW_BLOCK * FW_BLOCK + (8 * (row & 7) + (col & 7)) * 256 + (row >> 3) + 16 * (col >> 3)];
+  T curr = hist[2 * FW_BLOCK * FW_BLOCK + row + col * FW_BLOCK];
   int32_t p = -1;
   auto scan = [&](const T prod, int k) {
     const bool lower = prod < curr;
     curr = pick(lower, prod, curr);
     p = lower ? k : p;
   };
-  if constexpr (sizeof(T) == 4) {
-    auto steps = [&](const T c0, T c1, const T r0, T r1, const T at_01, const T at_10, int k) {
-      scan(c0 + r0, k);
-      const T via_c = c0 + at_01, via_r = at_10 + r0;
-      c1 = pick(via_c < c1, via_c, c1);
-      r1 = pick(via_r < r1, via_r, r1);
-      if (k + 1 < bb) scan(c1 + r1, k + 1);
-    };
-    int k = 0;
-    for (; k + 16 <= bb; k += 16) {  // sixteen k at a time, their operands requested together
-      T cv[16], rv[16], at_01[8], at_10[8];
+  int k = 0;
+  for (; k + 16 <= bb; k += 16) {  // sixteen k at a time, their operands requested together
+    T cv[16], rv[16];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        cv[u] = hc[(k + u) * FW_BLOCK];
-        rv[u] = hr[(k + u) * FW_BLOCK];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        at_01[u] = hist_row[(k + 2 * u) * FW_BLOCK + k + 2 * u + 1];
-        at_10[u] = hist[(k + 2 * u) * FW_BLOCK + k + 2 * u + 1];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) steps(cv[2 * u], cv[2 * u + 1], rv[2 * u], rv[2 * u + 1], at_01[u], at_10[u], k + 2 * u);
+    for (int u = 0; u < 16; ++u) {
+      cv[u] = hc[(k + u) * FW_BLOCK];
+      rv[u] = hr[(k + u) * FW_BLOCK];
     }
-    for (; k < bb; k += 2)
-      steps(hc[k * FW_BLOCK], hc[(k + 1) * FW_BLOCK], hr[k * FW_BLOCK], hr[(k + 1) * FW_BLOCK], hist_row[k * FW_BLOCK + k + 1],
-            hist[k * FW_BLOCK + k + 1], k);
-  } else {
-    int k = 0;
-    for (; k + 16 <= bb; k += 16) {  // sixteen k at a time, their operands requested together
-      T cv[16], rv[16];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        cv[u] = hc[(k + u) * FW_BLOCK];
-        rv[u] = hr[(k + u) * FW_BLOCK];
-      }
-#pragma unroll
-      for (int u = 0; u < 16; ++u) scan(cv[u] + rv[u], k + u);
-    }
-    for (; k < bb; ++k) scan(hc[k * FW_BLOCK] + hr[k * FW_BLOCK], k);
+    for (int u = 0; u < 16; ++u) scan(cv[u] + rv[u], k + u);
   }
+  for (; k < bb; ++k) scan(hc[k * FW_BLOCK] + hr[k * FW_BLOCK], k);
   if (p >= 0) parent[row + int64_t(col) * ldp] = k_base + p;
 }
 
@@ -1055,14 +922,14 @@ constexpr int FW_PARENT_BLOCKS = (FW_BLOCK / 64) * (FW_BLOCK / 4);
 
 // two independent products in one launch (the block row and the block column of a blocked
 // Floyd-Warshall step, each too small to fill the chip): after the first FW_PARENT_BLOCKS workgroups, which
-// with hist set find the predecessors of the diagonal block at k_base (closed by fw_close_dist in the launch
-// before) and otherwise have nothing to do, the next blocks0 workgroups work on g0, the others on g1
+// find the predecessors of the diagonal block at k_base (closed by fw_close_dist in a launch before), the next
+// blocks0 workgroups work on g0, the others on g1
 template <typename T>
 __global__ void __launch_bounds__(256) fwgemm_pair_kernel(FwArgs g0, FwArgs g1, int blocks0, const T *hist, int32_t *hist_parent,
                                                           int64_t ldp, int hist_bb, int k_base) {
   int b = blockIdx.x;
   if (b < FW_PARENT_BLOCKS) {
-    if (hist) fw_parents_block<T>(hist, hist_parent, ldp, hist_bb, k_base, b);
+    fw_parents_block<T>(hist, hist_parent, ldp, hist_bb, k_base, b);
     return;
   }
   b -= FW_PARENT_BLOCKS;
@@ -1081,10 +948,15 @@ __global__ void __launch_bounds__(256) fwgemm_pair_kernel(FwArgs g0, FwArgs g1, 
 // 128 dependent steps take about as long as the whole product and nothing else of the next block step can
 // start before them; here they cost one of the launch's 512 places.  Only where a tile is a whole
 // diagonal block (4-byte elements; the host asks for nothing else).
-template <typename T, int TM, int TN, int SN, int BK, bool GUARD, bool HAS_AT>
-__global__ void __launch_bounds__(256, 2) fwgemm_tile_kernel(FwArgs g) {
-  constexpr int BM = 16 * TM, BN = 16 * TN;
+template <typename T, int NT, int TM, int TN, int WPE, int BK, bool GUARD, bool HAS_AT>
+__global__ void __launch_bounds__(NT, WPE) fwgemm_tile_kernel(FwArgs g) {
+  typedef FwTileLds<T, NT, TM, TN, BK> TileLds;
+  constexpr int BM = TileLds::BM, BN = TileLds::BN;
   constexpr bool CAN_CLOSE = FW_BLOCK % BM == 0 && FW_BLOCK % BN == 0;
+  __shared__ union {
+    TileLds tile;
+    FwCloseLds<T> close;
+  } sm;
   int bx = blockIdx.x, by = blockIdx.y;
   if constexpr (CAN_CLOSE) {
     if (g.ahead_bb > 0) {
@@ -1094,11 +966,13 @@ __global__ void __launch_bounds__(256, 2) fwgemm_tile_kernel(FwArgs g) {
         // its place for most of the launch, so it goes to the die that has the least to do: with a number of
         // tile columns that is a multiple of eight, the tiles of the skipped rows -- which return at once --
         // all have numbers that are bx modulo eight.  (On any other die the last tile waits for the
-        // closure's place and the launch ends 15 us later.)
-        const int closer = (gridDim.x % 8 == 0 && g.skip_r1 > g.skip_r0) ? (g.skip_r0 / BM) % 8 : 0;
+        // closure's place and the launch ends 15 us later.)  And it takes the number in its row that those tiles have in
+        // theirs: a die deals its workgroups to its shader engines in turn, so the places left empty are those.  (With the
+        // number modulo eight, at 16 x 16 tiles of one workgroup per compute unit, every second step took 68 us, not 44.)
+        const int closer = g.skip_r1 > g.skip_r0 ? g.skip_r0 / BM : 0;
         if (bx == closer)
-          fw_close_dist<T>(static_cast<T *>(g.dist) + g.ahead0 + int64_t(g.ahead0) * g.ldc, g.ldc, g.ahead_bb,
-                           static_cast<T *>(g.hist));
+          fw_close_dist<T, NT>(static_cast<T *>(g.dist) + g.ahead0 + int64_t(g.ahead0) * g.ldc, g.ldc, g.ahead_bb,
+                               static_cast<T *>(g.hist), sm.close);
         return;
       }
       by -= 1;
@@ -1106,7 +980,7 @@ __global__ void __launch_bounds__(256, 2) fwgemm_tile_kernel(FwArgs g) {
       if (r0 >= 0 && r0 < FW_BLOCK && c0 >= 0 && c0 < FW_BLOCK) return;
     }
   }
-  fwgemm_tile_body<T, TM, TN, SN, BK, GUARD, HAS_AT>(g, bx, by);
+  fwgemm_tile_body<T, NT, TM, TN, WPE, BK, GUARD, HAS_AT>(g, bx, by, sm.tile);
 }
 
 // ---- the predecessor-tracking product on the hand-scheduled direct-to-LDS tile (direct_tile.h, direct_asm.h)
@@ -1276,7 +1150,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
         base += row_count[I];
       });
       __syncthreads();
-      lookup_queue<float, 512, FWD_CHUNK, true, 7, 8>(g, q_code, q_want, total, tid, m0, n0);
+      lookup_queue<float, 512, FWD_CHUNK, true, 7, 8, 8>(g, q_code, q_want, total, tid, m0, n0);
       __syncthreads();  // the queue is free again
     }
     i0 = i1;
@@ -1296,22 +1170,20 @@ bool fwgemm_direct_ok(const FwArgs &g) {
   return int64_t(g.m / 128) * (g.n / 256) <= 0x7fffffff;
 }
 
-template <typename T, int TM, int TN, int SN, int BK>
+template <typename T, int NT, int TM, int TN, int WPE, int BK>
 hipError_t launch_tile(const FwArgs &g, hipStream_t stream) {
-  constexpr int BM = 16 * TM, BN = 16 * TN;
-  // (the unguarded form queues improved elements with their chunk of BK k-values in 18 bits)
-  const bool whole = g.m >= BM && g.n >= BN && g.k >= 4 && g.k < (1 << 22);
+  constexpr int BM = 16 * TM, BN = NT / 16 * TN;
+  // (chunks of BK k-values are numbered in 15 bits)
+  const bool whole = g.m >= BM && g.n >= BN && g.k >= 4 && g.k < (1 << 19);
   if (g.ahead_bb > 0 && (FW_BLOCK % BM || FW_BLOCK % BN)) return hipErrorInvalidValue;
   dim3 grid((g.m + BM - 1) / BM, (g.n + BN - 1) / BN + (g.ahead_bb > 0 ? 1 : 0));
+  // (GUARD form: fetches element by element, with registers to spare)
   if (g.At) {
-    if (whole)
-      launch_kernel((fwgemm_tile_kernel<T, TM, TN, SN, BK, false, true>), grid, dim3(256), 0, stream, g);
-    else
-      launch_kernel((fwgemm_tile_kernel<T, TM, TN, SN, BK, true, true>), grid, dim3(256), 0, stream, g);
-  } else if (whole) {
-    launch_kernel((fwgemm_tile_kernel<T, TM, TN, SN, BK, false, false>), grid, dim3(256), 0, stream, g);
+    if (whole) launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, WPE, BK, false, true>), grid, dim3(NT), 0, stream, g);
+    else launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, 2, BK, true, true>), grid, dim3(NT), 0, stream, g);
   } else {
-    launch_kernel((fwgemm_tile_kernel<T, TM, TN, SN, BK, true, false>), grid, dim3(256), 0, stream, g);
+    if (whole) launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, WPE, BK, false, false>), grid, dim3(NT), 0, stream, g);
+    else launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, 2, BK, true, false>), grid, dim3(NT), 0, stream, g);
   }
   return take_launch_status();
 }
@@ -1375,86 +1247,12 @@ __global__ void __launch_bounds__(256) snapshot_pair_kernel(const T *src0, T *w0
     if (c0 + 4 * u < cols) w[r + int64_t(c0 + 4 * u) * ldw] = v[u];
 }
 
-// Floyd-Warshall inside one diagonal block of at most FW_BLOCK x FW_BLOCK: k ascending,
-// d[i][j] > d[i][k] + d[k][j] => d[i][j] = the sum, parent = k_base + k.  One workgroup of 1024
-// threads holds the block in registers, a 4 x 4 patch per thread.  Step k needs column k and row k
-// only, and they do not change during step k (the block's diagonal is not negative): every step
-// reads them from two 128-element LDS buffers and publishes column k + 1 and row k + 1 into the
-// other pair, so one barrier per step is enough and a thread reads two vectors per 16 updates.
+// A diagonal block's distances closed by a launch of its own: a job's first block, and every block of a job too small for
+// the tile kernel.  Its predecessors follow with those of the other blocks.
 template <typename T>
-__global__ void __launch_bounds__(1024) fw_diagonal_kernel(T *d, int64_t ld, int32_t *parent, int64_t ldp, int bb, int k_base) {
-  typedef typename vec4_of<T>::type V4;
-  __shared__ __attribute__((aligned(32))) T colbuf[2][FW_BLOCK];  // d[i][k] for the step that reads this buffer
-  __shared__ __attribute__((aligned(32))) T rowbuf[2][FW_BLOCK];  // d[k][j]
-  const int ti = threadIdx.x & 31, tj = threadIdx.x >> 5;  // rows 4 ti .. 4 ti + 3, columns 4 tj .. 4 tj + 3
-  const T inf = std::numeric_limits<T>::infinity();
-  T cur[4][4];  // [row in patch][column in patch]
-  int32_t par[4][4];
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int i = 4 * ti + a, j = 4 * tj + b;
-      cur[a][b] = (i < bb && j < bb) ? d[i + int64_t(j) * ld] : inf;
-      par[a][b] = -1;
-    }
-  // S = kn & 3, the row / column of the patch that is published, is a compile-time constant
-  // (the step loop is unrolled by four): indexed by a run-time value the patch would be
-  // moved to scratch memory, and every step would wait for memory
-  auto publish = [&](int kn, int buf, auto sc) {
-    constexpr int S = decltype(sc)::value;
-    if ((kn >> 2) == ti) {  // my patch holds row kn
-      V4 v;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) v[b] = cur[S][b];
-      *reinterpret_cast<V4 *>(&rowbuf[buf][4 * tj]) = v;
-    }
-    if ((kn >> 2) == tj) {  // my patch holds column kn
-      V4 v;
-#pragma unroll
-      for (int a = 0; a < 4; ++a) v[a] = cur[a][S];
-      *reinterpret_cast<V4 *>(&colbuf[buf][4 * ti]) = v;
-    }
-  };
-  auto step = [&](int k, auto uc) {
-    constexpr int U = decltype(uc)::value;  // k & 3
-    const int buf = U & 1;
-    const V4 ci = *reinterpret_cast<const V4 *>(&colbuf[buf][4 * ti]);
-    const V4 rj = *reinterpret_cast<const V4 *>(&rowbuf[buf][4 * tj]);
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const T cand = ci[a] + rj[b];
-        const bool lower = cand < cur[a][b];
-        cur[a][b] = pick(lower, cand, cur[a][b]);
-        par[a][b] = lower ? k_base + k : par[a][b];
-      }
-    // the other pair of buffers: nobody reads it before the barrier, and nobody is still
-    // reading it from the step before (everybody has passed that step's barrier)
-    publish(k + 1, buf ^ 1, std::integral_constant<int, (U + 1) & 3>{});
-    __syncthreads();
-  };
-  publish(0, 0, std::integral_constant<int, 0>{});
-  __syncthreads();
-  // steps beyond bb (up to the next multiple of four) read rows and columns of the padding,
-  // which hold +infinity and improve nothing
-  for (int k4 = 0; k4 < bb; k4 += 4) {
-    step(k4 + 0, std::integral_constant<int, 0>{});
-    step(k4 + 1, std::integral_constant<int, 1>{});
-    step(k4 + 2, std::integral_constant<int, 2>{});
-    step(k4 + 3, std::integral_constant<int, 3>{});
-  }
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int i = 4 * ti + a, j = 4 * tj + b;
-      if (i < bb && j < bb && par[a][b] >= 0) {
-        d[i + int64_t(j) * ld] = cur[a][b];
-        parent[i + int64_t(j) * ldp] = par[a][b];
-      }
-    }
+__global__ void __launch_bounds__(512) fw_close_kernel(T *d, int64_t ld, int bb, T *hist) {
+  __shared__ FwCloseLds<T> sm;
+  fw_close_dist<T, 512>(d, ld, bb, hist, sm);
 }
 
 template <typename T> hipError_t launch_naive(const FwArgs &g, hipStream_t stream) {
@@ -1495,13 +1293,12 @@ struct FwExtra {
   void *hist = nullptr;
   bool *closed_ahead = nullptr;
 };
-// one-thread-per-element kernel or tiles: a launch of a few workgroups is better spread over one thread per
-// element, and so is one of few tiles (the tile kernel's workgroups would each run alone on a compute
-// unit): measured on square problems, the two kernels meet at about 100 tiles (1024^3: 193 against 270 us,
-// 1280^3: 356 against 334, 1408^3: 466 against 366)
-bool takes_naive_kernel(int m, int n, int kernel) {
+// One-thread-per-element kernel or tiles: a launch of few tiles leaves most of the chip idle.  Measured on square problems
+// (one thread per element / tiles): f32 896^3 135 / 140 us, 1024^3 187 / 169, 1152^3 270 / 181; f64 768^3 208 / 241, 896^3
+// 346 / 281.
+bool takes_naive_kernel(int dtype, int m, int n, int kernel) {
   const int64_t tiles = ((int64_t(m) + 127) / 128) * ((int64_t(n) + 127) / 128);
-  const bool tiny = int64_t(m) * n < 64 * 64 || tiles < 96;
+  const bool tiny = int64_t(m) * n < 64 * 64 || tiles < (dtype == CUASR_AMD_F32 ? 64 : 48);
   return kernel == CUASR_AMD_KERNEL_NAIVE || (kernel == CUASR_AMD_KERNEL_AUTO && tiny);
 }
 int fwgemm_run(int dtype, int m, int n, int k, const void *A, int64_t lda, const void *B, int64_t ldb, void *dist,
@@ -1511,7 +1308,7 @@ int fwgemm_run(int dtype, int m, int n, int k, const void *A, int64_t lda, const
   FwArgs g{m, n, k, A, lda, B, ldb, dist, ldc, parent, ldp, x.At, x.ldat, x.k_base,
            x.skip_r0, x.skip_r1, x.skip_c0, x.skip_c1, nullptr, 0, 0, 0, nullptr};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool naive = takes_naive_kernel(m, n, kernel);
+  const bool naive = takes_naive_kernel(dtype, m, n, kernel);
   if (!naive && x.ahead_bb > 0 && x.hist) {
     g.ahead0 = x.ahead0;
     g.ahead_bb = x.ahead_bb;
@@ -1523,8 +1320,19 @@ int fwgemm_run(int dtype, int m, int n, int k, const void *A, int64_t lda, const
     launch_kernel(fwgemm_direct_kernel, dim3((unsigned)(int64_t(g.m / 128) * (g.n / 256))), dim3(512), 0, s, g);
     return take_launch_status() == hipSuccess ? CUASR_AMD_SUCCESS : CUASR_AMD_ERROR_INTERNAL;
   }
-  if (dtype == CUASR_AMD_F32) e = naive ? launch_naive<float>(g, s) : launch_tile<float, 8, 8, 4, 16>(g, s);
-  else e = naive ? launch_naive<double>(g, s) : launch_tile<double, 4, 8, 4, 16>(g, s);
+  // 4-byte elements: while every tile (and the closure of a diagonal block) has a compute unit to itself, the form with two
+  // waves per SIMD and registers for a second set of fragments and twice the lookups in flight; with more tiles two of
+  // four waves share one (n = 2000, 225 tiles and a closure: 1287 against 1409 us a job; n = 3000, 529 tiles: 3621
+  // against 3446).  8-byte elements have registers for two waves only.
+  const int64_t tm = (int64_t(g.m) + 127) / 128, tn = (int64_t(g.n) + 127) / 128;
+  const int64_t skip_m = g.skip_r1 > g.skip_r0 ? 1 : 0, skip_n = g.skip_c1 > g.skip_c0 ? 1 : 0;
+  const bool one_each = (tm - skip_m) * (tn - skip_n) <= 256;
+  if (dtype == CUASR_AMD_F32) {
+    e = naive ? launch_naive<float>(g, s) : one_each ? launch_tile<float, 512, 8, 4, 2, 16>(g, s) : launch_tile<float, 512, 8, 4, 4, 16>(g, s);
+  }
+  else {
+    e = naive ? launch_naive<double>(g, s) : one_each ? launch_tile<double, 512, 8, 4, 2, 16>(g, s) : launch_tile<double, 256, 4, 8, 2, 16>(g, s);
+  }
   return e == hipSuccess ? CUASR_AMD_SUCCESS : CUASR_AMD_ERROR_INTERNAL;
 }
 }  // namespace
@@ -1602,20 +1410,21 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
   char *C = R + es * FW_BLOCK * size_t(nn);             // block column, n x FW_BLOCK,  leading dimension nn
   char *Ct = C + es * FW_BLOCK * size_t(nn);            // updated block column with k contiguous, leading dimension FW_BLOCK
   char *H = Ct + es * FW_BLOCK * size_t(nn);            // columns, rows and first state of the diagonal block being closed
-  // this step's diagonal block had its distances closed during the step before, beside that step's big product;
-  // its predecessors are still to be found from what that closure recorded in H
+  // With tiles a step's launch also closes the next block, after a launch that updates it; without, a closure alone on
+  // the chip takes half a step.  f32, n = 1000 (64 tiles): 635 us a job with tiles, 595 without; from 81 tiles on the
+  // tiles win (f64 from 49: n = 1001 984 against 1130).
+  const bool naive = takes_naive_kernel(dtype, n, n, CUASR_AMD_KERNEL_AUTO) || (!f64 && n <= 1024);
+  // this step's diagonal block had its distances closed during the step before, beside that step's big product
+  // (its predecessors are always still to be found, from what the closure recorded in H)
   bool closed = false;
   for (int k0 = 0; k0 < n; k0 += FW_BLOCK) {
     const int bb = n - k0 < FW_BLOCK ? n - k0 : FW_BLOCK;
     char *Dkk = D + es * (size_t(k0) + size_t(k0) * size_t(ld));
     int32_t *Pkk = parent + size_t(k0) + size_t(k0) * size_t(ldp);
     // 1. the diagonal block, closed by one workgroup
-    const bool parents_due = closed;
     if (!closed) {
-      if (f64)
-        launch_kernel(fw_diagonal_kernel<double>, dim3(1), dim3(1024), 0, s, reinterpret_cast<double *>(Dkk), ld, Pkk, ldp, bb, k0);
-      else
-        launch_kernel(fw_diagonal_kernel<float>, dim3(1), dim3(1024), 0, s, reinterpret_cast<float *>(Dkk), ld, Pkk, ldp, bb, k0);
+      if (f64) launch_kernel(fw_close_kernel<double>, dim3(1), dim3(512), 0, s, reinterpret_cast<double *>(Dkk), ld, bb, reinterpret_cast<double *>(H));
+      else launch_kernel(fw_close_kernel<float>, dim3(1), dim3(512), 0, s, reinterpret_cast<float *>(Dkk), ld, bb, reinterpret_cast<float *>(H));
       if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
     }
     // 2. snapshots of block row and block column (the products below read these, so that no
@@ -1654,17 +1463,15 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
       const dim3 grid(FW_PARENT_BLOCKS + blocks0 + blocks1);
       if (f64)
         launch_kernel(fwgemm_pair_kernel<double>, grid, dim3(256), 0, s, g0, g1, blocks0,
-                      reinterpret_cast<const double *>(parents_due ? H : nullptr), Pkk, ldp, bb, k0);
+                      reinterpret_cast<const double *>(H), Pkk, ldp, bb, k0);
       else
         launch_kernel(fwgemm_pair_kernel<float>, grid, dim3(256), 0, s, g0, g1, blocks0,
-                      reinterpret_cast<const float *>(parents_due ? H : nullptr), Pkk, ldp, bb, k0);
+                      reinterpret_cast<const float *>(H), Pkk, ldp, bb, k0);
       if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
     } else {
-      if (parents_due) {
-        if (f64) launch_kernel(fw_parents_kernel<double>, dim3(FW_PARENT_BLOCKS), dim3(256), 0, s, reinterpret_cast<const double *>(H), Pkk, ldp, bb, k0);
-        else launch_kernel(fw_parents_kernel<float>, dim3(FW_PARENT_BLOCKS), dim3(256), 0, s, reinterpret_cast<const float *>(H), Pkk, ldp, bb, k0);
-        if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
-      }
+      if (f64) launch_kernel(fw_parents_kernel<double>, dim3(FW_PARENT_BLOCKS), dim3(256), 0, s, reinterpret_cast<const double *>(H), Pkk, ldp, bb, k0);
+      else launch_kernel(fw_parents_kernel<float>, dim3(FW_PARENT_BLOCKS), dim3(256), 0, s, reinterpret_cast<const float *>(H), Pkk, ldp, bb, k0);
+      if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
       FwExtra xr = x, xc = x;
       xr.skip_c0 = xc.skip_r0 = k0;
       xr.skip_c1 = xc.skip_r1 = k0 + bb;
@@ -1692,7 +1499,7 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
     x.ldat = FW_BLOCK;
     x.skip_r0 = x.skip_c0 = k0;
     x.skip_r1 = x.skip_c1 = k0 + bb;
-    if (x.ahead_bb > 0 && !takes_naive_kernel(n, n, CUASR_AMD_KERNEL_AUTO)) {
+    if (x.ahead_bb > 0 && !naive) {
       // this step's update of that block, by a launch of its own (64 workgroups, a few microseconds): the
       // closure can then start with the big product instead of after one of its tiles
       const int a0 = x.ahead0, abb = x.ahead_bb;
@@ -1705,7 +1512,7 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
     } else {
       x.ahead_bb = 0;
     }
-    r = fwgemm_run(dtype, n, n, bb, Dcol, ld, Drow, ld, dist, ld, parent, ldp, x, CUASR_AMD_KERNEL_AUTO, stream);
+    r = fwgemm_run(dtype, n, n, bb, Dcol, ld, Drow, ld, dist, ld, parent, ldp, x, naive ? CUASR_AMD_KERNEL_NAIVE : CUASR_AMD_KERNEL_AUTO, stream);
     if (r != CUASR_AMD_SUCCESS) return r;
   }
   return CUASR_AMD_SUCCESS;

@@ -71,6 +71,32 @@ def test_edge_tiles_start_earlier(oracle, dtype, m, n, k):
         run_case(oracle, m, n, k, dtype, False, "valu", pad, seed=9)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_more_tiles_than_compute_units(oracle, dtype):
+    """From 257 tiles of 128 x 128 on the tile kernel takes the form that shares a compute unit between two workgroups."""
+    for m, n, k in [(2048, 2048, 32), (2049, 2177, 37)]:
+        run_case(oracle, m, n, k, dtype, True, "auto")
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [112, 113, 127, 129, 1281 + 16, 2080])
+def test_apsp_blocked_strips_of_a_diagonal_block(oracle, n, dtype):
+    """Diagonal blocks with a last strip of one to sixteen rows, weights whose sums round (so an addition made in another
+    order shows), alone (small n) and beside the product's tiles (from 1281 on; 2080: two workgroups per compute unit)."""
+    import torch
+    rng = np.random.default_rng(31 * n)
+    W = np.where(rng.random((n, n)) < max(0.01, 6.0 / n), rng.random((n, n)) * 9 + 0.5, np.inf).astype(dtype)
+    np.fill_diagonal(W, 0)
+    dD = to_device(np.asfortranarray(W))
+    dP = torch.full((n, n), -1, dtype=torch.int32, device="cuda").t()
+    ws = torch.empty(cuasr_amd.apsp_blocked_workspace_bytes(n, "f32" if dtype == np.float32 else "f64"), dtype=torch.uint8, device="cuda")
+    cuasr_amd.apsp_blocked(dD, dP, ws)
+    want_d, want_p = np.asfortranarray(W), np.full((n, n), -1, np.int32, order="F")
+    oracle.apsp_blocked(want_d, want_p, 128)
+    assert_same_bits(np.ascontiguousarray(dD.cpu().numpy()), np.ascontiguousarray(want_d), "dist")
+    assert np.array_equal(dP.cpu().numpy(), want_p)
+
+
 def test_first_of_many_equal_products(oracle):
     """Every product equal: the first k wins where it improves, nothing moves where it does not."""
     m = n = 128
