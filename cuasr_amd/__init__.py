@@ -210,7 +210,9 @@ def _operand(t):
 
 def _slice_operand(t):
     """The same of the first matrix of a 3-D torch tensor."""
-    _, rows, cols = t.shape
+    batch, rows, cols = t.shape
+    if batch == 0:
+        raise IndexError("a batch of operands must not be empty")
     _, s0, s1 = t.stride()
     return _strided(t.data_ptr(), rows, cols, s0, s1)
 
@@ -286,8 +288,9 @@ def make_desc(add_op, mult_op, dtype, A, B, C, D, alpha, beta, add_identity, mul
 
 
 # The descriptor as one packed record, for the calls that launch: filling a ctypes structure field by field took longer
-# than the kernel of a small product runs (min-plus 256^3, 6.0 us: 9.5 us a call in a loop of calls, 5.9 now).  Scalars the record's format does not take as they are -- a float
-# beyond the range of binary32, a float where an integer belongs, binary16 -- go through the structure.
+# than the kernel of a small product runs (min-plus 256^3, 6.0 us: 9.5 us a call in a loop of calls, 5.9 now).  Scalars
+# the record's format does not take as they are -- a float beyond the range of binary32, a float where an integer
+# belongs, binary16 -- go through the structure.
 _RECORDS = {dt: struct.Struct("@10iPqPqPqPq" + 4 * scalar + "PPii")
             for dt, scalar in (("f32", "f4x"), ("f64", "d"), ("i32", "i4x"), ("i8", "i4x"))}
 assert all(r.size == ctypes.sizeof(SrgemmDesc) for r in _RECORDS.values())

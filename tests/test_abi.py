@@ -324,3 +324,12 @@ def test_reference_call_sites_compile():
     hipcc cross-compiles it here; tests/test_gpu_cpp_api.py runs it on the GPU."""
     import build_cpp
     assert os.path.exists(build_cpp.build("test_reference_call_sites"))
+
+
+@pytest.mark.parametrize("empty", [0, 1, 2])
+def test_batched_operand_without_products_is_refused(lib, empty):
+    """An output batch with an operand that holds no product at all; refused before anything is launched."""
+    torch = pytest.importorskip("torch")
+    ops = [torch.zeros(0 if i == empty else 3, 4, 4) for i in range(3)]
+    with pytest.raises(IndexError):
+        cuasr_amd.srgemm_batched("minimum", "plus", *ops, torch.zeros(3, 4, 4), 0.0, 0.0, float("inf"), 0.0, stream=0)
