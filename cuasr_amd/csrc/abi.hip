@@ -119,7 +119,17 @@ static bool streamk_usable(const cuasr_amd_srgemm_desc *d) {
 // 70 % or more of the compute units get one tile each and none gets two: the plain direct tile then beats both the
 // shared tiles, whose folds cost more than the idle units (2560^3 min-plus: 60 - 66 against 54 - 57 TOPS), and the
 // staged tile (2816^3: 71 against 60)
-static bool one_tile_each(long long tiles) { return tiles <= 256 && tiles * 10 >= 256 * 7; }
+// Bit operations on words: from 7/8 of the compute units on (xor-and 3000 x 2500 x 2000, 240 tiles: 377 - 434 us by
+// layout against 487 - 538 on the shared tiles and 493 - 512 on the staged one; 3000 x 2500 x 300: 67 - 77 against 81 - 84
+// on the staged one; but 2048^3, 128 tiles: 367 - 416 against 216 - 224 on the shared ones), where the tiles cover about
+// what the staged family's cover.
+static bool one_tile_each(const cuasr_amd_srgemm_desc *d, const Problem &c) {
+  const long long tiles = (long long)((c.m + 255) / 256) * ((c.n + 127) / 128);
+  if (tiles > 256) return false;
+  if (d->mult_op == kPlus) return tiles * 10 >= 256 * 7;
+  if (!is_bitwise(d->add_op) || !is_bitwise(d->mult_op) || tiles * 8 < 256 * 7) return false;
+  return tiles * 256 * 128 * 100 <= 4096LL * 115 * ((c.m + 63) / 64) * ((c.n + 63) / 64);
+}
 
 static bool streamk_preferred(const cuasr_amd_srgemm_desc *d, long long batch) {
   if (batch != 1 || d->split_k_slices != 1 || !streamk_usable(d)) return false;
@@ -130,7 +140,7 @@ static bool streamk_preferred(const cuasr_amd_srgemm_desc *d, long long batch) {
   const long long tiles = (long long)((c.m + 255) / 256) * ((c.n + 127) / 128), ktiles = (c.k + 15) / 16;
   const long long rounds = (tiles + 511) / 512;
   if (tiles * 10 >= rounds * 512 * 9) return false;   // >= 90 % of the places filled: nothing to gain
-  if (d->mult_op == kPlus && one_tile_each(tiles)) return false;   // (the plain tile, one per compute unit: pick_family)
+  if (one_tile_each(d, c)) return false;   // (the plain tile, one per compute unit: pick_family)
   return tiles >= 64 && tiles * ktiles >= 512 * 48;
 }
 
@@ -253,11 +263,10 @@ static int pick_family(const cuasr_amd_srgemm_desc *d, long long batch = 1) {
   const bool slow_direct = (d->dtype == CUASR_AMD_I32 || d->dtype == CUASR_AMD_U32) && d->add_op == kPlus &&
                            d->mult_op == kMultiplies && !kc2;
   if (streamk_preferred(d, batch)) return kStreamK;
-  // min-plus / max-plus, which would otherwise share their tiles out (measured for those only: generalised to every
-  // pair and type, the rule lost as often as it won; xor-and on words at 2560^3: 63 against 66 TOPS on the staged tile)
-  if (batch == 1 && d->split_k_slices == 1 && streamk_usable(d) && d->mult_op == kPlus &&
-      one_tile_each((long long)((c.m + 255) / 256) * ((c.n + 127) / 128)))
-    return kDirect;
+  // min-plus / max-plus and, nearer to a full round, bit operations, which would otherwise share their tiles out
+  // (generalised to every pair, type and share of the round, the rule lost as often as it won; xor-and on words at
+  // 2560^3, 200 tiles: 63 against 66 TOPS on the staged tile)
+  if (batch == 1 && d->split_k_slices == 1 && streamk_usable(d) && one_tile_each(d, c)) return kDirect;
   if (direct_usable(d) && ((fills && !((both_kc || masked || slow_direct) && have_valu)) || !have_valu)) return kDirect;
   if (have_valu) return kValu;
   if (mfma_usable(d)) return kMfma;

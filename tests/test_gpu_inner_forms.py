@@ -193,3 +193,29 @@ def test_or_and_split_k(oracle, lib, dtype):
             assert_same_bits(got, want, f"split-K or-and {dtype} S={slices} beta={beta}")
             got = launch("logical_or", "logical_and", dtype, A, B, C, 1, beta, 0, 1, "valu", splitk=slices, serial=True)
             assert_same_bits(got, want, f"serial split-K or-and {dtype} S={slices} beta={beta}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,direct", [((3580, 2044, 4), True), ((3332, 1924, 36), True), ((4096, 2048, 332), True),
+                                          ((3332, 1920, 332), False), ((4100, 2048, 64), False), ((57300, 132, 16), False)])
+def test_bit_operations_with_a_direct_tile_per_compute_unit(oracle, lib, shape, direct):
+    """xor-and on words around the rule for 224 .. 256 direct tiles of 256 x 128: both ends of its range (14 x 16 and
+    16 x 16 tiles, ragged and whole), one tile column less, one tile row more, and tiles that are mostly empty."""
+    import ctypes
+    import numpy as np
+    import torch
+    import cuasr_amd
+    from cuasr_amd import inputs
+    from helpers import assert_same_bits, to_device, to_host
+    m, n, k = shape
+    ones = 0xFFFFFFFF
+    for order in ("CCC", "FCC", "CFC"):
+        A, B, C = (inputs.words32(5 + i, r, c, o) for i, (r, c, o) in enumerate(zip((m, k, m), (k, n, n), order)))
+        want = oracle.srgemm("bit_xor", "bit_and", A, B, C, ones, ones, 0)
+        dA, dB, dC, dD = (to_device(x) for x in (A, B, C, np.zeros_like(C)))
+        if order != "CFC":   # (both operands k-contiguous: tiles of 128 x 128 and another rule)
+            d = cuasr_amd.make_desc("bit_xor", "bit_and", "u32", dA, dB, dC, dD, ones, ones, 0, ones)
+            assert (lib.cuasr_amd_selected_kernel(ctypes.byref(d)) == b"valu_direct") == direct, (shape, order)
+        cuasr_amd.srgemm("bit_xor", "bit_and", dA, dB, dC, dD, ones, ones, 0, ones, dtype="u32")
+        torch.cuda.synchronize()
+        assert_same_bits(to_host(dD, "u32"), want, f"{shape} {order}")
