@@ -354,7 +354,9 @@ struct DirectTile {
     const int tid = threadIdx.x, tx = tid % TX, ty = tid / TX, lane = tid & 63, wave = tid >> 6;
     const T *A = reinterpret_cast<const T *>(p.A);
     const T *B = reinterpret_cast<const T *>(p.B);
-    const T ident = scalar_as<T>(p.add_identity);
+    // (of the ranges of k that are folded together only the first starts from the caller's identity where the add is an
+    // exclusive or, in which a value that is not zero may count only once)
+    const T ident = ADD == kBitXor && mode != kEpilogue && kb > 0 ? T(0) : scalar_as<T>(p.add_identity);
 
     // each wave moves 2 x 1 KiB of the A panel and 2 x 1 KiB of the B panel per k-tile
     const char *base_a = reinterpret_cast<const char *>(A + (long long)m0 * p.sa_m + (long long)kb * p.sa_k);

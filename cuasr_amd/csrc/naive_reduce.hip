@@ -221,7 +221,8 @@ template <typename T, bool SERIAL> static hipError_t launch_reduce(const Problem
 }
 
 // ------------------------------------------------------------ source term for the stream-K tiles
-// D <- mult(beta, C) where the source is needed, else the additive identity, on the output tiles (bm x bn) from
+// D <- mult(beta, C) where the source is needed, else the additive identity (exclusive or: zero, the caller's identity
+// coming with the first range of k), on the output tiles (bm x bn) from
 // `first` on in the stream-K tile order: what the workgroups that share those tiles fold their ranges of k into
 // (the epilogue's add then has nothing left to do).  One workgroup per tile.  D may be C.
 template <typename T> __global__ __launch_bounds__(256) void prepare_fold_kernel(Problem p, int bm, int bn, long long first) {
@@ -233,7 +234,7 @@ template <typename T> __global__ __launch_bounds__(256) void prepare_fold_kernel
   for (int idx = threadIdx.x; idx < bm * bn; idx += 256) {
     const int row = m0 + idx / bn, col = n0 + idx % bn;
     if (row < p.m && col < p.n) {
-      T v = e.ident;
+      T v = p.add_op == kBitXor ? T(0) : e.ident;
       if (e.source_needed) v = apply_op<T>(p.mult_op, e.beta, reinterpret_cast<const T *>(p.C)[(long long)row * p.ldc + col]);
       reinterpret_cast<T *>(p.D)[(long long)row * p.ldd + col] = v;
     }

@@ -164,10 +164,11 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int NB, int W> s
     request_source(0, 0);   // it arrives under the product
 
     S acc[RM][RN];
+    const S init = Ops::start(p, wave == 0 && p.k_sub <= 1);
 #pragma unroll
     for (int i = 0; i < RM; ++i)
 #pragma unroll
-      for (int j = 0; j < RN; ++j) acc[i][j] = Ops::staged(ident);
+      for (int j = 0; j < RN; ++j) acc[i][j] = init;
     Panels &pn = sm.p[wave];
     T ra[BM * KC / 64], rb[BN * KC / 64];
     int k0 = kb + wave * KC;

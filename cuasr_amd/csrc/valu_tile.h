@@ -382,30 +382,38 @@ struct ValuTile {
     return EpilogueScalars<T>{ident, ident, ident, false};
   }
 
+  // What an accumulator starts from: the caller's identity.  Where several accumulators of one output meet, a copy of
+  // a value that is not the add's own identity may count only once in a sum or an exclusive or (the other adds take
+  // it any number of times), so all but the first start from zero there.
+  static __device__ __forceinline__ S start(const Problem &p, bool first) {
+    const T ident = scalar_as<T>(p.add_identity);
+    if constexpr (ADD == kPlus || ADD == kBitXor) return first ? staged(ident) : S(0);
+    else return staged(ident);
+  }
+
   static __device__ __forceinline__ void run(const Problem &p, const Operands &o, Smem &sm) {
     int m0, n0, kb, ke;
     tile_and_range(p, m0, n0, kb, ke);
     const EpilogueScalars<T> e = scalars(p);
     S acc[TM][TN];
-    accumulate(p, o, sm, m0, n0, kb, ke, (ke - kb + BK - 1) / BK, acc);
+    accumulate(p, o, sm, m0, n0, kb, ke, (ke - kb + BK - 1) / BK, start(p, p.k_sub <= 1), acc);   // (parts of a slice: it is in the workspace)
     finish(p, o, e, acc, m0, n0, kb, ke);
   }
 
-  // acc = identity, then the terms of k in [kb, ke).  The 256 threads that share `sm` pass
+  // acc = init, then the terms of k in [kb, ke).  The 256 threads that share `sm` pass
   // 1 + `sync_tiles` barriers (sync_tiles >= the number of k-tiles of the range, so that groups of
   // one workgroup whose ranges differ in length stay in step).
   static __device__ __forceinline__ void accumulate(const Problem &p, const Operands &o, Smem &sm, int m0, int n0, int kb, int ke,
-                                                    int sync_tiles, S (&acc)[TM][TN]) {
+                                                    int sync_tiles, S init, S (&acc)[TM][TN]) {
     const int tid = threadIdx.x & 255, tx = tid & 15, ty = tid >> 4;
     const T *A = reinterpret_cast<const T *>(o.A);
     const T *B = reinterpret_cast<const T *>(o.B);
-    const T ident = scalar_as<T>(p.add_identity);
     const bool a_xc = p.sa_m == 1, b_xc = p.sb_n == 1;
 
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = staged(ident);
+      for (int j = 0; j < TN; ++j) acc[i][j] = init;
 
     const int ntiles = max((ke - kb + BK - 1) / BK, 0);
     T ra[A_ELEMS], rb[B_ELEMS];
@@ -618,7 +626,7 @@ __global__ __launch_bounds__(256 * G) void valu_ksplit_kernel(const Problem p) {
   const int tiles = max((ke - kb + BK - 1) / BK, 0), per = (tiles + G - 1) / G;
   const int gkb = min(ke, kb + g * per * BK), gke = min(ke, gkb + per * BK);
   S acc[TM][TN];
-  Tile::accumulate(p, o, sm.panels[g], m0, n0, gkb, gke, per, acc);  // ends with a barrier: every group is done with its panels
+  Tile::accumulate(p, o, sm.panels[g], m0, n0, gkb, gke, per, Tile::start(p, g == 0 && p.k_sub <= 1), acc);  // ends with a barrier: every group is done with its panels
   // The panels are dead now: their space takes every group's accumulators.  Group d then takes the rows i = d, d + G,
   // ... of the threads' outputs, folds them over the groups in ascending k order (acc = add(acc, partial), as the
   // split-K reduction does) and runs their epilogue -- one G-th of the fold, of the reads of C and of the stores each.
