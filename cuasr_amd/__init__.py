@@ -290,7 +290,8 @@ def make_desc(add_op, mult_op, dtype, A, B, C, D, alpha, beta, add_identity, mul
 # The descriptor as one packed record, for the calls that launch: filling a ctypes structure field by field took longer
 # than the kernel of a small product runs (min-plus 256^3, 6.0 us: 9.5 us a call in a loop of calls, 5.9 now).  Scalars
 # the record's format does not take as they are -- a float beyond the range of binary32, a float where an integer
-# belongs, binary16 -- go through the structure.
+# belongs, binary16 -- go through the structure.  So do addresses that are not plain ints: the record would
+# take the VALUE of an integer tensor for an address where the structure refuses the tensor.
 _RECORDS = {dt: struct.Struct("@10iPqPqPqPq" + 4 * scalar + "PPii")
             for dt, scalar in (("f32", "f4x"), ("f64", "d"), ("i32", "i4x"), ("i8", "i4x"))}
 assert all(r.size == ctypes.sizeof(SrgemmDesc) for r in _RECORDS.values())
@@ -300,7 +301,7 @@ def _packed(add_op, mult_op, dtype, problem, alpha, beta, add_identity, mult_ide
             alpha_ptr=None, beta_ptr=None):
     """Bytes (or a SrgemmDesc passed by reference) for the launching entry points."""
     record = _RECORDS.get(dtype)
-    if record is not None:
+    if record is not None and (alpha_ptr is None or type(alpha_ptr) is int) and (beta_ptr is None or type(beta_ptr) is int):
         la, lb, lc, m, n, k, *pointers = problem
         try:
             return record.pack(OPS[add_op], OPS[mult_op], DTYPES[dtype], la, lb, lc, m, n, k, split_k_slices, *pointers,
@@ -378,7 +379,7 @@ def srgemm_splitk(add_op, mult_op, A, B, C, D, slices, workspace, alpha=None, be
     problem = _problem(_operand(A), _operand(B), _operand(C) if C is not None else None, _operand(D))
     ws = workspace.data_ptr() if hasattr(workspace, "data_ptr") else workspace
     st = _launchers()[2](_packed(add_op, mult_op, dtype, problem, alpha, beta, add_identity, mult_identity, slices, kernel, alpha_ptr,
-                                 beta_ptr), ws or None, _stream_handle(stream))
+                                 beta_ptr), ctypes.c_void_p(ws or None), _stream_handle(stream))
     if st != SUCCESS:
         raise CuasrError(st, "cuasr_amd_srgemm_splitk")
     return D

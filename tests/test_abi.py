@@ -333,3 +333,16 @@ def test_batched_operand_without_products_is_refused(lib, empty):
     ops = [torch.zeros(0 if i == empty else 3, 4, 4) for i in range(3)]
     with pytest.raises(IndexError):
         cuasr_amd.srgemm_batched("minimum", "plus", *ops, torch.zeros(3, 4, 4), 0.0, 0.0, float("inf"), 0.0, stream=0)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f64", "i32"])
+@pytest.mark.parametrize("field", ["alpha_ptr", "beta_ptr"])
+def test_an_integer_tensor_is_no_address(dtype, field):
+    """A one-element integer tensor where an address belongs: refused, not read as the number it holds."""
+    torch = pytest.importorskip("torch")
+    ops = [(0x10000, 4, ROW_MAJOR, 4, 4)] * 4
+    args = ("minimum", "plus", dtype, cuasr_amd._problem(*ops), 0, 0, 0, 0)
+    assert isinstance(cuasr_amd._packed(*args), bytes)
+    assert isinstance(cuasr_amd._packed(*args, **{field: 0x20000}), bytes)
+    with pytest.raises(TypeError):
+        cuasr_amd._packed(*args, **{field: torch.tensor([0x20000], dtype=torch.int64)})
