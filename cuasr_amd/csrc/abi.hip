@@ -29,6 +29,8 @@ bool direct_can_run(const Problem &);
 bool direct64_can_run(const Problem &);
 bool mfma_f32_can_run(const Problem &);
 bool mfma_f64_can_run(const Problem &);
+bool mfma_gemm_f32_batch_in_grid(const Problem &);
+bool mfma_gemm_f64_batch_in_grid(const Problem &);
 
 launch_fn find_or_and_on_masks(int dtype);
 
@@ -355,22 +357,30 @@ static launch_fn family_fn(int family, const cuasr_amd_srgemm_desc *d) {
   }
 }
 
+// The problem of a strided batch's first launch.  A column-major output runs as the transposed problem: the roles of A
+// and B swap, and so do their strides.
+static Problem batch_problem(const cuasr_amd_srgemm_desc *desc, int batch, int64_t stride_a, int64_t stride_b, int64_t stride_c,
+                             int64_t stride_d) {
+  const bool col = desc->layout_c == CUASR_AMD_COLUMN_MAJOR;
+  Problem p = canonical(desc);
+  p.batch = batch < 65535 ? batch : 65535;
+  p.batch_a = col ? stride_b : stride_a;
+  p.batch_b = col ? stride_a : stride_b;
+  p.batch_c = stride_c;
+  p.batch_d = stride_d;
+  return p;
+}
+
 // Which family a strided batch runs on, and whether the product index goes into the grid (one launch for
 // the whole batch) or the batch becomes a sequence of launches.  -1: the descriptor names the direct-to-LDS
 // tile and the batch strides do not keep its 16-byte alignment.
 static int batched_family(const cuasr_amd_srgemm_desc *desc, int batch, int64_t stride_a, int64_t stride_b, int64_t stride_c,
                           int64_t stride_d, bool *in_grid_out) {
-  const bool col = desc->layout_c == CUASR_AMD_COLUMN_MAJOR;
   int family = pick_family(desc, batch);
   if (family == kDirect && batch > 1) {
     // the direct-to-LDS tiles fetch 16-byte vectors: a batch stride that is no multiple of 16 bytes leaves the
     // later products misaligned; the staged tile takes any element alignment, with the batch still in the grid
-    Problem probe = canonical(desc);
-    probe.batch = batch < 65535 ? batch : 65535;
-    probe.batch_a = col ? stride_b : stride_a;
-    probe.batch_b = col ? stride_a : stride_b;
-    probe.batch_c = stride_c;
-    probe.batch_d = stride_d;
+    const Problem probe = batch_problem(desc, batch, stride_a, stride_b, stride_c, stride_d);
     if (!(desc->dtype == CUASR_AMD_F64 ? direct64_can_run(probe) : direct_can_run(probe))) {
       if (desc->kernel == CUASR_AMD_KERNEL_VALU_DIRECT) return -1;  // asked for by name
       family = find_valu(desc->dtype, desc->add_op, desc->mult_op) ? kValu : kNaive;
@@ -378,8 +388,7 @@ static int batched_family(const cuasr_amd_srgemm_desc *desc, int batch, int64_t 
   }
   bool in_grid = (family == kValu || family == kDirect) && batch > 1;
   if (family == kMfma && batch > 1 && desc->add_op == kPlus && desc->mult_op == kMultiplies) {
-    // the matrix-core launchers take the batch as it is: in the grid wherever that is the faster way
-    in_grid = true;
+    in_grid = true;   // (the matrix-core launchers take the batch as it is, and split it themselves where they must)
   }
   *in_grid_out = in_grid;
   return family;
@@ -428,7 +437,14 @@ const char *cuasr_amd_selected_kernel_batched(const cuasr_amd_srgemm_desc *desc,
   if (!desc || batch < 1 || stride_a < 0 || stride_b < 0 || stride_c < 0 || stride_d < 0) return nullptr;
   if (validate(desc, false) != CUASR_AMD_SUCCESS) return nullptr;
   bool in_grid = false;
-  switch (batched_family(desc, batch, stride_a, stride_b, stride_c, stride_d, &in_grid)) {
+  const int family = batched_family(desc, batch, stride_a, stride_b, stride_c, stride_d, &in_grid);
+  if (in_grid && desc->add_op == kPlus && desc->mult_op == kMultiplies && (desc->dtype == CUASR_AMD_F32 || desc->dtype == CUASR_AMD_F64) &&
+      family_fn(family, desc) == find_mfma(desc->dtype, desc->add_op, desc->mult_op)) {
+    // the matrix-core launcher takes the batch, and splits it where the compiled tiles have to do it: ask with its first launch's problem
+    const Problem probe = batch_problem(desc, batch, stride_a, stride_b, stride_c, stride_d);
+    in_grid = desc->dtype == CUASR_AMD_F64 ? mfma_gemm_f64_batch_in_grid(probe) : mfma_gemm_f32_batch_in_grid(probe);
+  }
+  switch (family) {
     case kMfma: return in_grid ? "mfma" : "mfma, a launch per product";
     case kDirect: return in_grid ? "valu_direct" : "valu_direct, a launch per product";
     case kValu: return in_grid ? "valu" : "valu, a launch per product";
@@ -469,10 +485,10 @@ int cuasr_amd_srgemm(const cuasr_amd_srgemm_desc *desc, void *stream) {
   return fn(p, s) == hipSuccess ? CUASR_AMD_SUCCESS : CUASR_AMD_ERROR_INTERNAL;
 }
 
-// A strided batch.  The tile kernels -- the vector-ALU ones and the hand-scheduled matrix-core ones -- take the
-// product index from the grid (blockIdx.z), so a batch of small products is one launch that fills the chip; the
-// compiled matrix-core kernels (ragged k, unaligned products) and the naive kernel, and batches beyond the
-// grid's 65535, are sequences of launches.
+// A strided batch.  The tile kernels -- the vector-ALU ones, the hand-scheduled matrix-core ones and the matrix-core
+// blocks of mfma_small.hip -- take the product index from the grid (blockIdx.z), so a batch of small products is one
+// launch that fills the chip; the compiled matrix-core tiles (products with ragged k or unaligned operands too large for
+// the blocks) and the naive kernel, and batches beyond the grid's 65535, are sequences of launches.
 int cuasr_amd_srgemm_batched(const cuasr_amd_srgemm_desc *desc, int batch, int64_t stride_a, int64_t stride_b,
                              int64_t stride_c, int64_t stride_d, void *stream) {
   if (!desc || batch < 0 || stride_a < 0 || stride_b < 0 || stride_c < 0 || stride_d < 0)
@@ -491,12 +507,7 @@ int cuasr_amd_srgemm_batched(const cuasr_amd_srgemm_desc *desc, int batch, int64
   if (in_grid) {
     const launch_fn fn = family_fn(family, desc);
     if (!fn) return CUASR_AMD_ERROR_NOT_SUPPORTED;
-    Problem p = canonical(desc);
-    // a column-major output runs as the transposed problem: the roles of A and B swap, and so do their strides
-    p.batch_a = col ? stride_b : stride_a;
-    p.batch_b = col ? stride_a : stride_b;
-    p.batch_c = stride_c;
-    p.batch_d = stride_d;
+    Problem p = batch_problem(desc, batch, stride_a, stride_b, stride_c, stride_d);
     hipStream_t s = static_cast<hipStream_t>(stream);
     for (int first = 0; first < batch; first += 65535) {
       p.batch = batch - first < 65535 ? batch - first : 65535;

@@ -390,6 +390,12 @@ static hipError_t launch(const Problem &p, hipStream_t s) {
 
 }  // namespace gemm_mfma
 
+// a batch is one launch, but on the compiled tiles
+bool mfma_gemm_f32_batch_in_grid(const Problem &p) {
+  const bool direct = mfma_panel::can_run(p) && mfma_direct_f32_can_run(p);
+  return direct || mfma_small_preferred_f32(p, direct);
+}
+
 // plus-times runs on the matrix cores whatever the operands' extents and alignment
 bool mfma_gemm_f32_can_run(const Problem &p) { return mfma_panel::loose_can_run(p); }
 

@@ -313,6 +313,12 @@ static hipError_t launch(const Problem &p, hipStream_t s) {
 
 }  // namespace gemm_mfma_f64
 
+// a batch is one launch, but on the compiled tiles
+bool mfma_gemm_f64_batch_in_grid(const Problem &p) {
+  const bool direct = gemm_mfma_f64::can_run(p) && mfma_direct_f64_can_run(p);
+  return direct || mfma_small_preferred_f64(p, direct);
+}
+
 launch_fn find_mfma_f64(int add_op, int mult_op) {
   if (add_op == kPlus && mult_op == kMultiplies) return gemm_mfma_f64::launch;
   return nullptr;

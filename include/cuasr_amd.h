@@ -181,10 +181,13 @@ int cuasr_amd_srgemm(const cuasr_amd_srgemm_desc *desc, void *stream);
  * chosen once, for the whole batch (what fills the chip is the batch, not one
  * product); on the vector-ALU tiles and the matrix-core kernels the product
  * index is part of the grid, so a batch of many small products is a single
- * launch (large plus-times products that the hand-scheduled matrix-core tiles
- * cannot fetch -- ragged k, operands or strides off 16 bytes -- and the
+ * launch (the largest plus-times products that the hand-scheduled matrix-core
+ * tiles cannot fetch -- ragged k, operands or strides off 16 bytes -- and the
  * naive kernel run one after the other on the stream).  Each
- * product's result is that of a single cuasr_amd_srgemm on its operands. */
+ * product's result is that of a single cuasr_amd_srgemm on its operands; for
+ * plus-times on float and double under AUTO that holds to rounding only, since
+ * how a sum is shared out depends on the extents and on the batch
+ * (CUASR_AMD_KERNEL_VALU sums in ascending k in either call). */
 int cuasr_amd_srgemm_batched(const cuasr_amd_srgemm_desc *desc, int batch, int64_t stride_a,
                              int64_t stride_b, int64_t stride_c, int64_t stride_d, void *stream);
 

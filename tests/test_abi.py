@@ -346,3 +346,16 @@ def test_an_integer_tensor_is_no_address(dtype, field):
     assert isinstance(cuasr_amd._packed(*args, **{field: 0x20000}), bytes)
     with pytest.raises(TypeError):
         cuasr_amd._packed(*args, **{field: torch.tensor([0x20000], dtype=torch.int64)})
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f64"])
+def test_batched_plus_times_says_where_it_is_a_launch_per_product(lib, dtype):
+    """Large products that the hand-scheduled matrix-core tiles cannot fetch (here: a stride off 16 bytes) run one after the
+    other; those they can fetch, and small ones of any extent, are one launch."""
+    sel = lambda m, n, k, batch, odd=0: lib.cuasr_amd_selected_kernel_batched(
+        ctypes.byref(desc(m=m, n=n, k=k, dtype=dtype, add="plus", mult="multiplies")), batch, m * k + odd, k * n, m * n, m * n)
+    assert sel(4096, 4096, 4096, 2, odd=1) == b"mfma, a launch per product"
+    assert sel(4096, 4096, 4096, 2) == b"mfma"
+    assert sel(2001, 1999, 300, 2) == b"mfma"
+    assert sel(100, 100, 100, 2000) == b"mfma"
+    assert sel(64, 64, 64, 20) == b"valu"
