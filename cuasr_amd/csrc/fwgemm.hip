@@ -647,8 +647,10 @@ constexpr int FW_BLOCK = 128;  // vertices per block step of the blocked Floyd-W
 // elements) and 110 us (8-byte) alone on the chip.)
 //
 // The hardware minimum prefers -0 to +0 where the strict comparison keeps whichever came first.  Sums and minima
-// of data free of -0 never produce one, so the block is searched for a -0 when it is loaded, and a block with
-// one is closed by fw_close_dist_exact instead: the same steps with a comparison and a select, the block in place.
+// of data free of -0 never produce one, so the block is searched for a -0 when it is loaded, and in a block with
+// one every element is lowered by a comparison and a select, in the same strips (EXACT).  A job whose every diagonal
+// block holds a -0, n = 1000 / 2000 / 4096: 855 / 1478 / 4180 us in float, 1181 / 2360 / 7893 in double.  (A step at a time with the
+// block in device memory: 5458 / 10790 / 22905 and 5901 / 12842 / 46159.)
 //
 // hist: FW_BLOCK x FW_BLOCK elements each of  col[k * FW_BLOCK + i] = d[i][k] before step k,
 // row[k * FW_BLOCK + j] = d[k][j] before step k,  init[i + j * FW_BLOCK] = d[i][j] before the closure.
@@ -678,56 +680,30 @@ template <int K, typename T> __device__ __forceinline__ T row_lane(T v) {
   }
 }
 
-// (returns false, with nothing done, when the block holds a -0)
-template <typename T, int NT>
-__device__ __forceinline__ bool fw_close_dist_fast(T *d, int64_t ld, int bb, T *hist, FwCloseLds<T> &sm) {
+// The strips.  EXACT: lowered by comparison and select, for a block that holds a -0.
+template <typename T, int NT, bool EXACT>
+__device__ __forceinline__ void fw_close_strips(T (&cur)[FwPatch<NT>::PN][FwPatch<NT>::PM], int bb, T *hist, FwCloseLds<T> &sm) {
   typedef typename vec4_of<T>::type V4;
-  typedef typename uvec4_of<T>::type U4;
   constexpr int PM = FwPatch<NT>::PM, PN = FwPatch<NT>::PN, TI = FwPatch<NT>::TI;
   const int tid = threadIdx.x, ti = tid % TI, tj = tid / TI;
-  const T inf = std::numeric_limits<T>::infinity();
-  T *hist_col = hist, *hist_row = hist + FW_BLOCK * FW_BLOCK, *init = hist + 2 * FW_BLOCK * FW_BLOCK;
-  T cur[PN][PM];  // [column in patch][row in patch]
-  if (bb == FW_BLOCK) {
-#pragma unroll
-    for (int b = 0; b < PN; ++b)
-#pragma unroll
-      for (int a = 0; a < PM; a += 4) {
-        const V4 v = *reinterpret_cast<const U4 *>(d + PM * ti + a + int64_t(PN * tj + b) * ld);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) cur[b][a + e] = v[e];
-      }
-  } else {
-    // loads from clamped addresses, then a select (a branch per element would keep all the lane masks alive)
-#pragma unroll
-    for (int b = 0; b < PN; ++b)
-#pragma unroll
-      for (int a = 0; a < PM; ++a) {
-        const T v = d[min(PM * ti + a, bb - 1) + int64_t(min(PN * tj + b, bb - 1)) * ld];
-        cur[b][a] = (PM * ti + a < bb && PN * tj + b < bb) ? v : inf;
-      }
-  }
-  bool negative_zero = false;
-#pragma unroll
-  for (int b = 0; b < PN; ++b)
-#pragma unroll
-    for (int a = 0; a < PM; ++a) negative_zero |= cur[b][a] == T(0) && __builtin_signbit(cur[b][a]);
-  if (__syncthreads_or(negative_zero)) return false;
+  T *hist_col = hist, *hist_row = hist + FW_BLOCK * FW_BLOCK;
   auto put4 = [](T *to, const T *from) {
     V4 v;
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = from[e];
     *reinterpret_cast<V4 *>(to) = v;
   };
-#pragma unroll
-  for (int b = 0; b < PN; ++b)
-#pragma unroll
-    for (int a = 0; a < PM; a += 4) put4(&init[PM * ti + a + (PN * tj + b) * FW_BLOCK], &cur[b][a]);
   // (the minimum as an instruction: from the builtin the compiler first "quiets" an operand whose origin it
   // does not know, such as anything that comes round the loop, an instruction more per element)
   auto relax = [](T &x, const T cand) {
-    if constexpr (sizeof(T) == 4) asm("v_min_f32 %0, %0, %1" : "+v"(x) : "v"(cand));
-    else asm("v_min_f64 %0, %0, %1" : "+v"(x) : "v"(cand));
+    if constexpr (EXACT) {
+      const bool lower = cand < x;
+      x = pick(lower, cand, x);
+    } else if constexpr (sizeof(T) == 4) {
+      asm("v_min_f32 %0, %0, %1" : "+v"(x) : "v"(cand));
+    } else {
+      asm("v_min_f64 %0, %0, %1" : "+v"(x) : "v"(cand));
+    }
   };
   // two steps' candidates at once
   auto relax2 = [&](T &x, const T first, const T second) {
@@ -781,19 +757,29 @@ __device__ __forceinline__ bool fw_close_dist_fast(T *d, int64_t ld, int bb, T *
         constexpr int K = decltype(kc)::value;
         // (lines before K have been read by their steps: this strip needs them no more.  All sums of a step, then all
         // minima: one behind the other each would wait for the one before it)
-        T sum_x[FW_STRIP], sum_diag[FW_STRIP];
+        if constexpr (EXACT) {
 #pragma unroll
-        for (int q = K + 1; q < FW_STRIP; ++q) {
-          const T step = row_lane<K>(diag[q]);
-          sum_x[q] = x[K] + step;
-          sum_diag[q] = diag[K] + step;
+          for (int q = K + 1; q < FW_STRIP; ++q) {
+            const T step = row_lane<K>(diag[q]);
+            relax(x[q], x[K] + step);
+            relax(diag[q], diag[K] + step);
+            if (q % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+          }
+        } else {
+          T sum_x[FW_STRIP], sum_diag[FW_STRIP];
+#pragma unroll
+          for (int q = K + 1; q < FW_STRIP; ++q) {
+            const T step = row_lane<K>(diag[q]);
+            sum_x[q] = x[K] + step;
+            sum_diag[q] = diag[K] + step;
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int q = K + 1; q < FW_STRIP; ++q) relax(diag[q], sum_diag[q]);
+#pragma unroll
+          for (int q = K + 1; q < FW_STRIP; ++q) relax(x[q], sum_x[q]);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int q = K + 1; q < FW_STRIP; ++q) relax(diag[q], sum_diag[q]);
-#pragma unroll
-        for (int q = K + 1; q < FW_STRIP; ++q) relax(x[q], sum_x[q]);
-        __builtin_amdgcn_sched_barrier(0);
       });
 #pragma unroll
       for (int q = 0; q < FW_STRIP; ++q) {
@@ -802,42 +788,94 @@ __device__ __forceinline__ bool fw_close_dist_fast(T *d, int64_t ld, int bb, T *
       }
     }
     __syncthreads();
-    struct Lines {
-      T c[2][PM], r[2][PN];
-    };
-    constexpr int NL = PM * PN * sizeof(T) > 256 ? 1 : 2;   // (a patch of 64 doubles leaves no registers for a second set)
-    Lines lines[NL];
-    auto read = [&](Lines &l, int kk) {
+    if constexpr (EXACT) {
+      // a step at a time and a column at a time: as above the sums and comparison masks under way take more registers
+      // than the patch leaves
+#pragma unroll 1
+      for (int kk = 0; kk < FW_STRIP; ++kk) {
+        T c[PM], r[PN];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+        for (int a = 0; a < PM; a += 4) get4(&c[a], &sm.step_cols[kk][PM * ti + a]);
 #pragma unroll
-        for (int a = 0; a < PM; a += 4) get4(&l.c[u][a], &sm.step_cols[kk + u][PM * ti + a]);
+        for (int b = 0; b < PN; b += 4) get4(&r[b], &sm.step_rows[kk][PN * tj + b]);
 #pragma unroll
-        for (int b = 0; b < PN; b += 4) get4(&l.r[u][b], &sm.step_rows[kk + u][PN * tj + b]);
-      }
-    };
-    if constexpr (NL == 2) read(lines[0], 0);
+        for (int b = 0; b < PN; ++b) {
 #pragma unroll
-    for (int kk = 0; kk < FW_STRIP; kk += 2) {
-      if constexpr (NL == 1) read(lines[0], kk);
-      else if (kk + 2 < FW_STRIP) read(lines[((kk >> 1) + 1) % NL], kk + 2);
-      __builtin_amdgcn_sched_barrier(0);
-      const Lines &l = lines[(kk >> 1) % NL];
-#pragma unroll
-      for (int b = 0; b < PN; ++b) {
-        T s0[PM], s1[PM];
-#pragma unroll
-        for (int a = 0; a < PM; ++a) {
-          s0[a] = l.c[0][a] + l.r[0][b];
-          s1[a] = l.c[1][a] + l.r[1][b];
+          for (int a = 0; a < PM; ++a) relax(cur[b][a], c[a] + r[b]);
+          __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int a = 0; a < PM; ++a) relax2(cur[b][a], s0[a], s1[a]);
       }
-      __builtin_amdgcn_sched_barrier(0);
+    } else {
+      struct Lines {
+        T c[2][PM], r[2][PN];
+      };
+      constexpr int NL = PM * PN * sizeof(T) > 256 ? 1 : 2;   // (a patch of 64 doubles leaves no registers for a second set)
+      Lines lines[NL];
+      auto read = [&](Lines &l, int kk) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+          for (int a = 0; a < PM; a += 4) get4(&l.c[u][a], &sm.step_cols[kk + u][PM * ti + a]);
+#pragma unroll
+          for (int b = 0; b < PN; b += 4) get4(&l.r[u][b], &sm.step_rows[kk + u][PN * tj + b]);
+        }
+      };
+      if constexpr (NL == 2) read(lines[0], 0);
+#pragma unroll
+      for (int kk = 0; kk < FW_STRIP; kk += 2) {
+        if constexpr (NL == 1) read(lines[0], kk);
+        else if (kk + 2 < FW_STRIP) read(lines[((kk >> 1) + 1) % NL], kk + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        const Lines &l = lines[(kk >> 1) % NL];
+#pragma unroll
+        for (int b = 0; b < PN; ++b) {
+          T s0[PM], s1[PM];
+#pragma unroll
+          for (int a = 0; a < PM; ++a) {
+            s0[a] = l.c[0][a] + l.r[0][b];
+            s1[a] = l.c[1][a] + l.r[1][b];
+          }
+#pragma unroll
+          for (int a = 0; a < PM; ++a) relax2(cur[b][a], s0[a], s1[a]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     // (no barrier: what the next strip writes before its first one has been read by everybody before this strip's second)
   }
+}
+
+template <typename T, int NT>
+__device__ __forceinline__ void fw_load_patch(T (&cur)[FwPatch<NT>::PN][FwPatch<NT>::PM], const T *d, int64_t ld, int bb) {
+  typedef typename vec4_of<T>::type V4;
+  typedef typename uvec4_of<T>::type U4;
+  constexpr int PM = FwPatch<NT>::PM, PN = FwPatch<NT>::PN, TI = FwPatch<NT>::TI;
+  const int ti = threadIdx.x % TI, tj = threadIdx.x / TI;
+  const T inf = std::numeric_limits<T>::infinity();
+  if (bb == FW_BLOCK) {
+#pragma unroll
+    for (int b = 0; b < PN; ++b)
+#pragma unroll
+      for (int a = 0; a < PM; a += 4) {
+        const V4 v = *reinterpret_cast<const U4 *>(d + PM * ti + a + int64_t(PN * tj + b) * ld);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) cur[b][a + e] = v[e];
+      }
+  } else {
+    // loads from clamped addresses, then a select (a branch per element would keep all the lane masks alive)
+#pragma unroll
+    for (int b = 0; b < PN; ++b)
+#pragma unroll
+      for (int a = 0; a < PM; ++a) {
+        const T v = d[min(PM * ti + a, bb - 1) + int64_t(min(PN * tj + b, bb - 1)) * ld];
+        cur[b][a] = (PM * ti + a < bb && PN * tj + b < bb) ? v : inf;
+      }
+  }
+}
+template <typename T, int NT>
+__device__ __forceinline__ void fw_store_patch(const T (&cur)[FwPatch<NT>::PN][FwPatch<NT>::PM], T *d, int64_t ld, int bb) {
+  constexpr int PM = FwPatch<NT>::PM, PN = FwPatch<NT>::PN, TI = FwPatch<NT>::TI;
+  const int ti = threadIdx.x % TI, tj = threadIdx.x / TI;
 #pragma unroll
   for (int b = 0; b < PN; ++b)
 #pragma unroll
@@ -845,41 +883,54 @@ __device__ __forceinline__ bool fw_close_dist_fast(T *d, int64_t ld, int bb, T *
       const int i = PM * ti + a, j = PN * tj + b;
       if (i < bb && j < bb) d[i + int64_t(j) * ld] = cur[b][a];
     }
-  return true;
 }
 
-// The same closure for a block that holds a -0: comparison and select, two barriers per step, the block itself in device
-// memory (every thread keeps to its own elements) and column k and row k read from hist.  Several times slower than the
-// form above and little code, out of the way of the other's registers.
+// A block that holds a -0, by a function of its own that fetches the block again: for patches that leave no registers (as
+// part of its caller it takes them from the caller's loop: double, n = 2500, without a -0: 3250 us a job instead of 3056).
 template <typename T, int NT>
-__device__ __attribute__((noinline)) void fw_close_dist_exact(T *d_anywhere, int64_t ld, int bb, T *hist_anywhere) {
-  typedef __attribute__((address_space(1))) T GT;
-  GT *const d = (GT *)d_anywhere, *const hist = (GT *)hist_anywhere;
-  GT *hist_col = hist, *hist_row = hist + FW_BLOCK * FW_BLOCK, *init = hist + 2 * FW_BLOCK * FW_BLOCK;
-  // a thread's elements: row i, columns j0, j0 + NT / FW_BLOCK, ...
-  const int tid = threadIdx.x, i = tid & (FW_BLOCK - 1), j0 = tid / FW_BLOCK;
-  const T inf = std::numeric_limits<T>::infinity();
-  for (int j = j0; j < FW_BLOCK; j += NT / FW_BLOCK) init[i + j * FW_BLOCK] = i < bb && j < bb ? T(d[i + int64_t(j) * ld]) : inf;
-#pragma unroll 1
-  for (int k = 0; k < bb; ++k) {
-    __syncthreads();  // what step k - 1 lowered is in the block
-    if (j0 == 0) {
-      hist_col[k * FW_BLOCK + i] = i < bb ? T(d[i + int64_t(k) * ld]) : inf;
-      hist_row[k * FW_BLOCK + i] = i < bb ? T(d[k + int64_t(i) * ld]) : inf;
-    }
-    __syncthreads();  // column k and row k are in hist before anybody lowers anything
-    const T ci = hist_col[k * FW_BLOCK + i];
-#pragma unroll 4
-    for (int j = j0; j < bb; j += NT / FW_BLOCK) {
-      const T cand = ci + hist_row[k * FW_BLOCK + j];
-      if (i < bb && cand < d[i + int64_t(j) * ld]) d[i + int64_t(j) * ld] = cand;
-    }
-  }
+__device__ __attribute__((noinline)) void fw_close_dist_exact(__attribute__((address_space(1))) T *d, int64_t ld, int bb,
+                                                              __attribute__((address_space(1))) T *hist,
+                                                              __attribute__((address_space(3))) FwCloseLds<T> *sm) {
+  T cur[FwPatch<NT>::PN][FwPatch<NT>::PM];
+  fw_load_patch<T, NT>(cur, (const T *)d, ld, bb);
+  fw_close_strips<T, NT, true>(cur, bb, (T *)hist, *(FwCloseLds<T> *)sm);
+  fw_store_patch<T, NT>(cur, (T *)d, ld, bb);
 }
 
 template <typename T, int NT>
 __device__ __forceinline__ void fw_close_dist(T *d, int64_t ld, int bb, T *hist, FwCloseLds<T> &sm) {
-  if (!fw_close_dist_fast<T, NT>(d, ld, bb, hist, sm)) fw_close_dist_exact<T, NT>(d, ld, bb, hist);
+  typedef typename vec4_of<T>::type V4;
+  constexpr int PM = FwPatch<NT>::PM, PN = FwPatch<NT>::PN, TI = FwPatch<NT>::TI;
+  const int ti = threadIdx.x % TI, tj = threadIdx.x / TI;
+  T *init = hist + 2 * FW_BLOCK * FW_BLOCK;
+  T cur[PN][PM];  // [column in patch][row in patch]
+  fw_load_patch<T, NT>(cur, d, ld, bb);
+  bool negative_zero = false;
+#pragma unroll
+  for (int b = 0; b < PN; ++b)
+#pragma unroll
+    for (int a = 0; a < PM; ++a) negative_zero |= cur[b][a] == T(0) && __builtin_signbit(cur[b][a]);
+#pragma unroll
+  for (int b = 0; b < PN; ++b)
+#pragma unroll
+    for (int a = 0; a < PM; a += 4) {
+      V4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = cur[b][a + e];
+      *reinterpret_cast<V4 *>(&init[PM * ti + a + (PN * tj + b) * FW_BLOCK]) = v;
+    }
+  if (__syncthreads_or(negative_zero)) {
+    if constexpr (PM * PN * sizeof(T) > 256) {
+      fw_close_dist_exact<T, NT>((__attribute__((address_space(1))) T *)d, ld, bb, (__attribute__((address_space(1))) T *)hist,
+                                 (__attribute__((address_space(3))) FwCloseLds<T> *)&sm);
+      return;
+    } else {
+      fw_close_strips<T, NT, true>(cur, bb, hist, sm);
+    }
+  } else {
+    fw_close_strips<T, NT, false>(cur, bb, hist, sm);
+  }
+  fw_store_patch<T, NT>(cur, d, ld, bb);
 }
 
 // The predecessors of a diagonal block whose distances fw_close_dist has closed: workgroup b of 64 (256 threads)

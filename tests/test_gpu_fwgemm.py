@@ -79,10 +79,11 @@ def test_more_tiles_than_compute_units(oracle, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("n", [112, 113, 127, 129, 1281 + 16, 2080])
+@pytest.mark.parametrize("n", [112, 113, 127, 129, 1281 + 16, 2080, 2193])
 def test_apsp_blocked_strips_of_a_diagonal_block(oracle, n, dtype):
     """Diagonal blocks with a last strip of one to sixteen rows, weights whose sums round (so an addition made in another
-    order shows), alone (small n) and beside the product's tiles (from 1281 on; 2080: two workgroups per compute unit)."""
+    order shows), alone (small n) and beside the product's tiles (1297 and 2080: each with a compute unit to itself; 2193: 17 x 17
+    of them, two workgroups on one)."""
     import torch
     rng = np.random.default_rng(31 * n)
     W = np.where(rng.random((n, n)) < max(0.01, 6.0 / n), rng.random((n, n)) * 9 + 0.5, np.inf).astype(dtype)
@@ -247,15 +248,16 @@ def test_apsp_blocked_floyd_warshall(oracle, n, pad, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-def test_apsp_blocked_keeps_the_sign_of_a_zero(oracle, dtype):
+@pytest.mark.parametrize("n", [113, 529, 1475, 2193])   # closed alone; beside tiles with a compute unit each; two workgroups on one
+def test_apsp_blocked_keeps_the_sign_of_a_zero(oracle, n, dtype):
     """Edges of weight +0 and -0: a sum of two -0 is -0, and the strict comparison keeps whichever zero was
     there first, where a hardware minimum would prefer -0.  The diagonal blocks that hold a -0 are closed by
     comparison and select; dist (bit for bit, so with its signs) and parent equal the oracle's."""
     import torch
-    n = 1475
     rng = np.random.default_rng(4242)
-    W = np.where(rng.random((n, n)) < 0.004, rng.integers(1, 9, (n, n)), np.inf).astype(dtype)
-    zeros = rng.random((n, n)) < 0.004
+    share = max(0.004, 3.0 / n)
+    W = np.where(rng.random((n, n)) < share, rng.integers(1, 9, (n, n)), np.inf).astype(dtype)
+    zeros = rng.random((n, n)) < share
     W[zeros] = rng.choice(np.array([0.0, -0.0], dtype), int(zeros.sum()))
     # every diagonal block but the fourth has a -0 of its own
     W[128 * 3:128 * 4, 128 * 3:128 * 4][W[128 * 3:128 * 4, 128 * 3:128 * 4] == 0] = 0.0
@@ -275,7 +277,7 @@ def test_apsp_blocked_keeps_the_sign_of_a_zero(oracle, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("n,pad", [(100, 0), (384, 0), (513, 1), (700, 4), (1475, 1)])
+@pytest.mark.parametrize("n,pad", [(100, 0), (384, 0), (513, 1), (700, 4), (1475, 1), (2193, 3)])
 def test_apsp_blocked_with_tiled_panels(oracle, n, pad, dtype):
     """The way a block step updates its block row and column from n = 16257 on (two launches of the tiled
     kernel with the diagonal block skipped, then a transposing copy of the column), forced at sizes the
