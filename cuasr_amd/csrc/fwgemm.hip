@@ -177,6 +177,7 @@ template <typename T> __device__ __forceinline__ void fwgemm_rowcols_block(const
   auto compute = [&](const T (&av)[CK], T bl, int k0, int buf) {
     typedef typename vec4_of<T>::type V4;
     bstage[wave][buf][lane] = bl;
+    wave_lds_order();
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       T bv[CK];
@@ -206,6 +207,7 @@ template <typename T> __device__ __forceinline__ void fwgemm_rowcols_block(const
         par[c] = lower ? g.k_base + k0 + first : par[c];
       }
     }
+    wave_lds_order();
   };
   // the next chunk's A values are requested before this chunk is worked on: a wave has eight chunks and a
   // compute unit sixteen such waves, too few to hide a memory round trip per chunk behind each other

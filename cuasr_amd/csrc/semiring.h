@@ -232,6 +232,15 @@ template <typename T, typename TI = T> __device__ __forceinline__ void select_ba
   }
 }
 
+// Between a wave's stores to LDS and the reads of what other lanes of the same wave stored (or those reads and the stores
+// that follow them): the hardware keeps a wave's LDS accesses in order, and this keeps the compiler from changing theirs,
+// which it may where it can tell one lane's two addresses apart.  No instruction comes of it.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // The same without writing to the problem record
 struct Operands {
   const void *A, *B, *C;

@@ -181,6 +181,7 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int NB, int W> s
       const bool vec = inside && k0 + KC <= ke;
       store<BM>(ra, pn.a, a_xc, vec, lane);
       store<BN>(rb, pn.b, b_xc, vec, lane);
+      wave_lds_order();   // other lanes read what a lane has stored
       const int kn = k0 + W * KC;
       if (kn < ke) {
         const bool vn = inside && kn + KC <= ke;
@@ -208,6 +209,7 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int NB, int W> s
           compute<1>(acc, f);
         }
       }
+      wave_lds_order();   // ... before the next chunk takes its place
     }
     T *out = reinterpret_cast<T *>(ops.D);
     long long ld_out = p.ldd;
