@@ -160,7 +160,7 @@ template <typename T> __device__ __forceinline__ void fwgemm_rowcols_block(const
   // belongs to the wave (no barrier: a wave's LDS accesses complete in order) and read back as broadcasts.
   // Through scalar loads instead, every chunk and column waited for a scalar-cache miss, and every add read
   // a scalar register, which costs it a second issue slot.
-  __shared__ T bstage[4][2][NC * CK];
+  __shared__ alignas(4 * sizeof(T)) T bstage[4][2][NC * CK];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const T *blane = static_cast<const T *>(g.B) + int64_t(min(col0 + (lane >> 4), g.n - 1)) * g.ldb;
   const T *ap = static_cast<const T *>(g.A) + row;
@@ -320,7 +320,7 @@ __device__ __forceinline__ void lookup_queue(const FwArgs &g, const uint32_t *q_
 // -> 1298 / 1703 / 3888; double, n = 2000: 3685 -> 2453.)
 template <typename T, int NT, int TM, int TN, int BK> struct FwTileLds {
   static constexpr int TY = NT / 16, BM = 16 * TM, BN = TY * TN, PAD = 4;
-  alignas(16) T as[2][BK][BM + PAD], bs[2][BK][BN + PAD];
+  alignas(4 * sizeof(T)) T as[2][BK][BM + PAD], bs[2][BK][BN + PAD];   // (accessed four elements at a time)
   int wave_count[NT / 64][TN];
 };
 template <typename T, int NT, int TM, int TN, int WPE, int BK, bool GUARD, bool HAS_AT>
@@ -659,8 +659,12 @@ constexpr int FW_BLOCK = 128;  // vertices per block step of the blocked Floyd-W
 constexpr int FW_STRIP = 16;
 // columns and rows of a strip as its first step finds them, and as their own steps read them
 template <typename T> struct FwCloseLds {
-  T cols[FW_STRIP][FW_BLOCK], rows[FW_STRIP][FW_BLOCK], step_cols[FW_STRIP][FW_BLOCK], step_rows[FW_STRIP][FW_BLOCK];
+  // (accessed four elements at a time)
+  alignas(4 * sizeof(T)) T cols[FW_STRIP][FW_BLOCK], rows[FW_STRIP][FW_BLOCK], step_cols[FW_STRIP][FW_BLOCK], step_rows[FW_STRIP][FW_BLOCK];
 };
+
+static_assert(alignof(FwCloseLds<float>) >= alignof(vec4_of<float>::type) && alignof(FwCloseLds<double>) >= alignof(vec4_of<double>::type),
+              "read and written as vectors");
 
 // a thread's patch of the block: PM x PN elements, rows PM ti .., columns PN tj ..
 template <int NT> struct FwPatch {
