@@ -7,17 +7,17 @@
 // thread folds and finishes 1024 / (64 W) outputs of a row-contiguous run.
 //
 // Why: an output of 256 x 256 is 16 blocks of 64 x 64, which left 240 of 256 compute units idle; 32 x 32 blocks
-// spread it over 64 of them, with sixteen waves each whatever the length of k.
+// spread it over 64 of them, with four to sixteen waves each by the length of k (launch_small).
 #pragma once
 
 namespace cuasr_amd {
 
-// RM x RN: outputs per lane, in groups of four rows / columns that lie 32 apart; KC: k per chunk; NB: fragment sets.
-template <typename T, int ADD, int MUL, int RM, int RN, int KC, int NB, int W> struct SmallTile {
+// KC: k per chunk.
+template <typename T, int ADD, int MUL, int KC, int W> struct SmallTile {
   using Ops = ValuTile<T, ADD, MUL, 4, 4, 32, true, false>;   // its operators, masks and zero-sign lookup
   using S = typename Ops::S;
   static constexpr int VW = 16 / sizeof(T);
-  static constexpr int BM = 8 * RM, BN = 8 * RN;
+  static constexpr int R = 4, BLOCK = 8 * R;       // outputs per lane and per wave along either direction
   // rows of 36 floats (40 doubles) more than a multiple of 32: the four k-groups that neighbouring lanes of a
   // k-contiguous load write lie 16 (doubles: 32) banks apart, so the transposing stores do not collide
   static constexpr int PAD = sizeof(S) == 8 ? 8 : 4;
@@ -27,19 +27,20 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int NB, int W> s
   static constexpr int SV = 16 / sizeof(S);
   typedef S s4_t __attribute__((ext_vector_type(SV)));
 
-  struct alignas(16) Panels { S a[KC][BM + PAD], b[KC][BN + PAD]; };
+  struct alignas(16) Panels { S a[KC][BLOCK + PAD], b[KC][BLOCK + PAD]; };
   union Smem {
     Panels p[W];
     S acc[W][16 * ASTRIDE];
   };
 
-  // One operand's chunk, ROWS x KC, into registers.  VEC: the block lies inside the matrix (the caller moved its origin
+  static constexpr int PER = BLOCK * KC / 64;      // elements of a chunk per lane and operand
+  static constexpr int XV = BLOCK / VW, KV = KC / VW, DK = 64 / XV, DX = 64 / KV;   // DK of k (DX of x): what one load of the wave covers
+
+  // One operand's chunk, BLOCK x KC, into registers.  VEC: the block lies inside the matrix (the caller moved its origin
   // back where it would not) and the chunk is whole, so 16-byte loads at element alignment; otherwise element by
   // element with clamped indices (what lands past an edge is never stored, k past the end never used).
-  template <int ROWS, int PER>
   static __device__ __forceinline__ void load(T (&r)[PER], const T *base, long long s_x, long long s_k, int x_end, int k0, int k_end, bool xc,
                                               bool vec, int lane) {
-    constexpr int XV = ROWS / VW, KV = KC / VW, DK = 64 / XV, DX = 64 / KV;   // rows of k (of x) that one load of the wave covers
     if (vec) {
       const int xx = xc ? lane % XV * VW : lane / KV, kk = xc ? lane / XV : lane % KV * VW;
       const T *src = base + (long long)xx * s_x + (long long)(k0 + kk) * s_k;
@@ -57,14 +58,12 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int NB, int W> s
 #pragma unroll
       for (int p = 0; p < PER; ++p) {
         const int el = l + 64 * p;
-        const int xx = min(xc ? el % ROWS : el / KC, x_end - 1), kk = min(k0 + (xc ? el / ROWS : el % KC), k_end - 1);
+        const int xx = min(xc ? el % BLOCK : el / KC, x_end - 1), kk = min(k0 + (xc ? el / BLOCK : el % KC), k_end - 1);
         r[p] = base[(long long)xx * s_x + (long long)kk * s_k];
       }
     }
   }
-  template <int ROWS, int PER>
-  static __device__ __forceinline__ void store(const T (&r)[PER], S (*dst)[ROWS + PAD], bool xc, bool vec, int lane) {
-    constexpr int XV = ROWS / VW, KV = KC / VW, DK = 64 / XV, DX = 64 / KV;
+  static __device__ __forceinline__ void store(const T (&r)[PER], S (*dst)[BLOCK + PAD], bool xc, bool vec, int lane) {
     if (vec) {
       if (xc) {
 #pragma unroll
@@ -85,34 +84,34 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int NB, int W> s
 #pragma unroll
       for (int p = 0; p < PER; ++p) {
         const int el = lane + 64 * p;
-        dst[xc ? el / ROWS : el % KC][xc ? el % ROWS : el / KC] = Ops::staged(r[p]);
+        dst[xc ? el / BLOCK : el % KC][xc ? el % BLOCK : el / KC] = Ops::staged(r[p]);
       }
     }
   }
 
-  template <int U> struct Frag { S a[U][RM], b[U][RN]; };
+  template <int U> struct Frag { S a[U][R], b[U][R]; };
   template <int U> static __device__ __forceinline__ void fragment(Frag<U> &f, const Panels &pn, int kk, int ly, int lx) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
 #pragma unroll
-      for (int h = 0; h < RM / SV; ++h) {
-        const s4_t t = *reinterpret_cast<const s4_t *>(&pn.a[kk + u][h * SV / 4 * 32 + ly * 4 + h * SV % 4]);
+      for (int h = 0; h < R / SV; ++h) {
+        const s4_t t = *reinterpret_cast<const s4_t *>(&pn.a[kk + u][ly * R + h * SV]);
 #pragma unroll
         for (int e = 0; e < SV; ++e) f.a[u][h * SV + e] = t[e];
       }
 #pragma unroll
-      for (int h = 0; h < RN / SV; ++h) {
-        const s4_t t = *reinterpret_cast<const s4_t *>(&pn.b[kk + u][h * SV / 4 * 32 + lx * 4 + h * SV % 4]);
+      for (int h = 0; h < R / SV; ++h) {
+        const s4_t t = *reinterpret_cast<const s4_t *>(&pn.b[kk + u][lx * R + h * SV]);
 #pragma unroll
         for (int e = 0; e < SV; ++e) f.b[u][h * SV + e] = t[e];
       }
     }
   }
-  template <int U> static __device__ __forceinline__ void compute(S (&acc)[RM][RN], const Frag<U> &f) {
+  template <int U> static __device__ __forceinline__ void compute(S (&acc)[R][R], const Frag<U> &f) {
 #pragma unroll
-    for (int i = 0; i < RM; ++i) {
+    for (int i = 0; i < R; ++i) {
 #pragma unroll
-      for (int j = 0; j < RN; ++j) {
+      for (int j = 0; j < R; ++j) {
         if constexpr (U == 2 && !(Ops::MASKED || Ops::ZERO_SIGN || Ops::FUSED)) {
           const T t0 = Op<MUL>::apply(f.a[0][i], f.b[0][j]), t1 = Op<MUL>::apply(f.a[1][i], f.b[1][j]);
           acc[i][j] = fold<ADD, MUL>(t1, fold<ADD, MUL>(t0, acc[i][j]));   // one three-input minimum
@@ -121,20 +120,19 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int NB, int W> s
           for (int u = 0; u < U; ++u) acc[i][j] = Ops::term(acc[i][j], f.a[u][i], f.b[u][j]);
         }
       }
-      if constexpr (RM * RN > 16) __builtin_amdgcn_sched_barrier(0);
     }
   }
 
   static __device__ __forceinline__ void run(const Problem &p, const Operands &ops, Smem &sm) {
     constexpr int U = sizeof(S) == 8 ? 1 : 2;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lx = lane & 7, ly = lane >> 3;
-    const int tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN;
+    const int tiles_m = (p.m + BLOCK - 1) / BLOCK, tiles_n = (p.n + BLOCK - 1) / BLOCK;
     int bm, bn;
     Ops::tile_coords(blockIdx.x, tiles_m, tiles_n, bm, bn);
-    const int first_m = bm * BM, first_n = bn * BN;       // the first row and column this workgroup stores
+    const int first_m = bm * BLOCK, first_n = bn * BLOCK;       // the first row and column this workgroup stores
     // blocks at the far edges start earlier instead of reaching past the matrix: what they compute twice is not stored
-    const bool inside = p.m >= BM && p.n >= BN;
-    const int m0 = inside ? min(first_m, p.m - BM) : first_m, n0 = inside ? min(first_n, p.n - BN) : first_n;
+    const bool inside = p.m >= BLOCK && p.n >= BLOCK;
+    const int m0 = inside ? min(first_m, p.m - BLOCK) : first_m, n0 = inside ? min(first_n, p.n - BLOCK) : first_n;
     int kb = 0, ke = p.k;
     if (p.workspace) {
       const int parts = p.k_sub > 1 ? p.k_sub : 1, slice = blockIdx.y / parts, part = blockIdx.y % parts;
@@ -153,53 +151,47 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int NB, int W> s
     e.source_needed = false;
     if (!partial) e = resolve_scalars<T>(p, MUL);
     const T *C = reinterpret_cast<const T *>(ops.C);
-    const int oc = threadIdx.x & 31, orow0 = threadIdx.x >> 5;   // this thread's outputs of a 32 x 32 block: column oc, rows orow0 + 2 W o
+    const int oc = threadIdx.x & 31, orow0 = threadIdx.x >> 5;   // this thread's outputs of the block: column oc, rows orow0 + 2 W o
     T src[OUTS];
-    auto request_source = [&](int hi, int hj) {
-      if (!e.source_needed) return;
+    if (e.source_needed) {   // it arrives under the product
 #pragma unroll
       for (int o = 0; o < OUTS; ++o)
-        src[o] = C[(long long)min(m0 + hi * 32 + orow0 + 2 * W * o, p.m - 1) * p.ldc + min(n0 + hj * 32 + oc, p.n - 1)];
-    };
-    request_source(0, 0);   // it arrives under the product
+        src[o] = C[(long long)min(m0 + orow0 + 2 * W * o, p.m - 1) * p.ldc + min(n0 + oc, p.n - 1)];
+    }
 
-    S acc[RM][RN];
+    S acc[R][R];
     const S init = Ops::start(p, wave == 0 && p.k_sub <= 1);
 #pragma unroll
-    for (int i = 0; i < RM; ++i)
+    for (int i = 0; i < R; ++i)
 #pragma unroll
-      for (int j = 0; j < RN; ++j) acc[i][j] = init;
+      for (int j = 0; j < R; ++j) acc[i][j] = init;
     Panels &pn = sm.p[wave];
-    T ra[BM * KC / 64], rb[BN * KC / 64];
+    T ra[PER], rb[PER];
     int k0 = kb + wave * KC;
     if (k0 < ke) {
       const bool vec = inside && k0 + KC <= ke;
-      load<BM>(ra, A, p.sa_m, p.sa_k, p.m - m0, k0, ke, a_xc, vec, lane);
-      load<BN>(rb, B, p.sb_n, p.sb_k, p.n - n0, k0, ke, b_xc, vec, lane);
+      load(ra, A, p.sa_m, p.sa_k, p.m - m0, k0, ke, a_xc, vec, lane);
+      load(rb, B, p.sb_n, p.sb_k, p.n - n0, k0, ke, b_xc, vec, lane);
     }
     for (; k0 < ke; k0 += W * KC) {
       const bool vec = inside && k0 + KC <= ke;
-      store<BM>(ra, pn.a, a_xc, vec, lane);
-      store<BN>(rb, pn.b, b_xc, vec, lane);
+      store(ra, pn.a, a_xc, vec, lane);
+      store(rb, pn.b, b_xc, vec, lane);
       wave_lds_order();   // other lanes read what a lane has stored
       const int kn = k0 + W * KC;
       if (kn < ke) {
         const bool vn = inside && kn + KC <= ke;
-        load<BM>(ra, A, p.sa_m, p.sa_k, p.m - m0, kn, ke, a_xc, vn, lane);
-        load<BN>(rb, B, p.sb_n, p.sb_k, p.n - n0, kn, ke, b_xc, vn, lane);
+        load(ra, A, p.sa_m, p.sa_k, p.m - m0, kn, ke, a_xc, vn, lane);
+        load(rb, B, p.sb_n, p.sb_k, p.n - n0, kn, ke, b_xc, vn, lane);
       }
       if (k0 + KC <= ke) {
-        Frag<U> f[NB];
-        if constexpr (NB == 2) fragment<U>(f[0], pn, 0, ly, lx);
+        Frag<U> f[2];
+        fragment<U>(f[0], pn, 0, ly, lx);
 #pragma unroll
         for (int s = 0; s < KC / U; ++s) {
-          if constexpr (NB == 2) {
-            if (s + 1 < KC / U) fragment<U>(f[(s + 1) & 1], pn, U * (s + 1), ly, lx);
-          } else {
-            fragment<U>(f[0], pn, U * s, ly, lx);
-          }
+          if (s + 1 < KC / U) fragment<U>(f[(s + 1) & 1], pn, U * (s + 1), ly, lx);
           __builtin_amdgcn_sched_barrier(0);
-          compute<U>(acc, f[s % NB]);
+          compute<U>(acc, f[s & 1]);
         }
       } else {
 #pragma unroll 1
@@ -217,56 +209,50 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int NB, int W> s
       out = reinterpret_cast<T *>(p.workspace) + (long long)(p.k_sub > 1 ? blockIdx.y / p.k_sub : blockIdx.y) * p.m * p.n;
       ld_out = p.n;
     }
+    __syncthreads();   // the panels are dead: their space takes the accumulators
 #pragma unroll
-    for (int hi = 0; hi < RM / 4; ++hi)
+    for (int i = 0; i < R; ++i)
 #pragma unroll
-      for (int hj = 0; hj < RN / 4; ++hj) {
-        if (hi + hj > 0) request_source(hi, hj);
-        __syncthreads();   // the panels (the block before) are dead: their space takes the accumulators
+      for (int j = 0; j < R; ++j) sm.acc[wave][(i * R + j) * ASTRIDE + lane] = acc[i][j];
+    __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+    for (int o = 0; o < OUTS; ++o) {
+      const int orow = orow0 + 2 * W * o, row = m0 + orow, col = n0 + oc;
+      const int at = ((orow & 3) * 4 + (oc & 3)) * ASTRIDE + (orow >> 2) * 8 + (oc >> 2);
+      S s = sm.acc[0][at];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) sm.acc[wave][(i * 4 + j) * ASTRIDE + lane] = acc[hi * 4 + i][hj * 4 + j];
-        __syncthreads();
-#pragma unroll
-        for (int o = 0; o < OUTS; ++o) {
-          const int orow = orow0 + 2 * W * o, row = m0 + hi * 32 + orow, col = n0 + hj * 32 + oc;
-          const int at = ((orow & 3) * 4 + (oc & 3)) * ASTRIDE + (orow >> 2) * 8 + (oc >> 2);
-          S s = sm.acc[0][at];
-#pragma unroll
-          for (int w = 1; w < W; ++w) {
-            if constexpr (Ops::MASKED) s |= sm.acc[w][at];
-            else s = Op<ADD>::apply(s, sm.acc[w][at]);
-          }
-          if (row < first_m || row >= p.m || col < first_n || col >= p.n) continue;
-          T v;
-          if constexpr (Ops::MASKED) v = s ? T(1) : T(0);
-          else v = s;
-          if constexpr (Ops::ZERO_SIGN) {
-            if (v == T(0) && ke > kb)
-              v = Ops::last_zero_product(A + (long long)(row - m0) * p.sa_m + (long long)kb * p.sa_k, p.sa_k,
-                                         B + (long long)(col - n0) * p.sb_n + (long long)kb * p.sb_k, p.sb_k, ke - kb, v);
-          }
-          T *dst = out + (long long)row * ld_out + col;
-          if constexpr (Ops::SUB_SLICES) {
-            if (partial && p.k_sub > 1) {
-              native_fold<ADD>(dst, v);
-              continue;
-            }
-          }
-          if (!partial) {
-            v = Op<MUL>::apply(e.alpha, v);
-            if (e.source_needed) v = fold_epilogue<ADD, MUL>(v, Op<MUL>::apply(e.beta, src[o]));
-          }
-          *dst = v;
+      for (int w = 1; w < W; ++w) {
+        if constexpr (Ops::MASKED) s |= sm.acc[w][at];
+        else s = Op<ADD>::apply(s, sm.acc[w][at]);
+      }
+      if (row < first_m || row >= p.m || col < first_n || col >= p.n) continue;
+      T v;
+      if constexpr (Ops::MASKED) v = s ? T(1) : T(0);
+      else v = s;
+      if constexpr (Ops::ZERO_SIGN) {
+        if (v == T(0) && ke > kb)
+          v = Ops::last_zero_product(A + (long long)(row - m0) * p.sa_m + (long long)kb * p.sa_k, p.sa_k,
+                                     B + (long long)(col - n0) * p.sb_n + (long long)kb * p.sb_k, p.sb_k, ke - kb, v);
+      }
+      T *dst = out + (long long)row * ld_out + col;
+      if constexpr (Ops::SUB_SLICES) {
+        if (partial && p.k_sub > 1) {
+          native_fold<ADD>(dst, v);
+          continue;
         }
       }
+      if (!partial) {
+        v = Op<MUL>::apply(e.alpha, v);
+        if (e.source_needed) v = fold_epilogue<ADD, MUL>(v, Op<MUL>::apply(e.beta, src[o]));
+      }
+      *dst = v;
+    }
   }
 };
 
-template <typename T, int ADD, int MUL, int RM, int RN, int KC, int NB, int W, int WPE>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(WPE))) void small_srgemm_kernel(const Problem p) {
-  using Tile = SmallTile<T, ADD, MUL, RM, RN, KC, NB, W>;
+template <typename T, int ADD, int MUL, int KC, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void small_srgemm_kernel(const Problem p) {
+  using Tile = SmallTile<T, ADD, MUL, KC, W>;
   __shared__ typename Tile::Smem sm;
   Tile::run(p, batch_operands<T>(p), sm);
 }
@@ -285,11 +271,11 @@ template <typename T, int ADD> static bool small_preferred(const Problem &p) {
   const long long groups32 = (long long)((p.m + 31) / 32) * ((p.n + 31) / 32) * slice_groups(p) * p.batch;
   return sizeof(T) == 4 && groups32 * 10 <= groups64 * 25;
 }
-template <typename T, int ADD, int MUL, int RM, int RN, int KC, int NB, int W, int WPE> static hipError_t launch_small_as(const Problem &p, hipStream_t s) {
-  const long long tiles = (long long)((p.m + 8 * RM - 1) / (8 * RM)) * ((p.n + 8 * RN - 1) / (8 * RN));
+template <typename T, int ADD, int MUL, int KC, int W> static hipError_t launch_small_as(const Problem &p, hipStream_t s) {
+  const long long tiles = (long long)((p.m + 31) / 32) * ((p.n + 31) / 32);
   if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
   const dim3 grid((unsigned)tiles, slice_groups(p), p.batch);
-  launch_kernel((small_srgemm_kernel<T, ADD, MUL, RM, RN, KC, NB, W, WPE>), grid, dim3(64 * W), 0, s, p);
+  launch_kernel((small_srgemm_kernel<T, ADD, MUL, KC, W>), grid, dim3(64 * W), 0, s, p);
   return take_launch_status();
 }
 
@@ -305,9 +291,9 @@ template <typename T, int ADD, int MUL> static hipError_t launch_small(const Pro
   // 2048: 21.8 us against 24.1 with eight; 512^3, two chunks each: 10.3 against 9.6), eight want two (900 x 900 x 200,
   // 841 blocks: 16.5 us against 14.6 with four; 832^3, 676 blocks of 52 chunks: 26.8 against 29.5).
   const int w = groups <= 256 && chunks >= 64 ? 16 : (groups <= 512 && chunks >= 8) || chunks >= 32 ? 8 : 4;
-  if (w == 16) return launch_small_as<T, ADD, MUL, 4, 4, KC, 2, 16, 4>(p, s);
-  if (w == 8) return launch_small_as<T, ADD, MUL, 4, 4, KC, 2, 8, 4>(p, s);
-  return launch_small_as<T, ADD, MUL, 4, 4, KC, 2, 4, 4>(p, s);
+  if (w == 16) return launch_small_as<T, ADD, MUL, KC, 16>(p, s);
+  if (w == 8) return launch_small_as<T, ADD, MUL, KC, 8>(p, s);
+  return launch_small_as<T, ADD, MUL, KC, 4>(p, s);
 }
 
 }  // namespace cuasr_amd
