@@ -19,6 +19,7 @@
 //     sequential scan would.
 // Operands must be free of NaN and of -infinity (+infinity marks "no edge").
 #include "direct_tile.h"
+#include "launch_rules.h"
 #include "semiring.h"
 
 #include <limits>
@@ -1350,14 +1351,6 @@ struct FwExtra {
   void *hist = nullptr;
   bool *closed_ahead = nullptr;
 };
-// One-thread-per-element kernel or tiles: a launch of few tiles leaves most of the chip idle.  Measured on square problems
-// (one thread per element / tiles): f32 896^3 135 / 140 us, 1024^3 187 / 169, 1152^3 270 / 181; f64 768^3 208 / 241, 896^3
-// 346 / 281.
-bool takes_naive_kernel(int dtype, int m, int n, int kernel) {
-  const int64_t tiles = ((int64_t(m) + 127) / 128) * ((int64_t(n) + 127) / 128);
-  const bool tiny = int64_t(m) * n < 64 * 64 || tiles < (dtype == CUASR_AMD_F32 ? 64 : 48);
-  return kernel == CUASR_AMD_KERNEL_NAIVE || (kernel == CUASR_AMD_KERNEL_AUTO && tiny);
-}
 int fwgemm_run(int dtype, int m, int n, int k, const void *A, int64_t lda, const void *B, int64_t ldb, void *dist,
                int64_t ldc, int32_t *parent, int64_t ldp, const FwExtra &x, int kernel, void *stream) {
   const int st = check(dtype, m, n, k, A, lda, B, ldb, dist, ldc, parent, ldp, kernel);
@@ -1365,7 +1358,8 @@ int fwgemm_run(int dtype, int m, int n, int k, const void *A, int64_t lda, const
   FwArgs g{m, n, k, A, lda, B, ldb, dist, ldc, parent, ldp, x.At, x.ldat, x.k_base,
            x.skip_r0, x.skip_r1, x.skip_c0, x.skip_c1, nullptr, 0, 0, 0, nullptr};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool naive = takes_naive_kernel(dtype, m, n, kernel);
+  const bool naive = kernel == CUASR_AMD_KERNEL_NAIVE ||
+                     (kernel == CUASR_AMD_KERNEL_AUTO && fwgemm_one_thread_each(dtype == CUASR_AMD_F64, x.At != nullptr, m, n));
   if (!naive && x.ahead_bb > 0 && x.hist) {
     g.ahead0 = x.ahead0;
     g.ahead_bb = x.ahead_bb;
@@ -1380,15 +1374,17 @@ int fwgemm_run(int dtype, int m, int n, int k, const void *A, int64_t lda, const
   // 4-byte elements: while every tile (and the closure of a diagonal block) has a compute unit to itself, the form with two
   // waves per SIMD and registers for a second set of fragments and twice the lookups in flight; with more tiles two of
   // four waves share one (n = 2000, 225 tiles and a closure: 1287 against 1409 us a job; n = 3000, 529 tiles: 3621
-  // against 3446).  8-byte elements have registers for two waves only.
+  // against 3446).  8-byte elements have registers for two waves only; there a block step's product (rows and columns to
+  // skip, k = 128) takes the larger tile wherever it has a compute unit to itself.
   const int64_t tm = (int64_t(g.m) + 127) / 128, tn = (int64_t(g.n) + 127) / 128;
   const int64_t skip_m = g.skip_r1 > g.skip_r0 ? 1 : 0, skip_n = g.skip_c1 > g.skip_c0 ? 1 : 0;
   const bool one_each = (tm - skip_m) * (tn - skip_n) <= 256;
+  const bool half_tile = skip_m + skip_n == 0 && fwgemm_f64_half_tile(g.At != nullptr, (int64_t(g.m) + 63) / 64 * tn);
   if (dtype == CUASR_AMD_F32) {
     e = naive ? launch_naive<float>(g, s) : one_each ? launch_tile<float, 512, 8, 4, 2, 16>(g, s) : launch_tile<float, 512, 8, 4, 4, 16>(g, s);
   }
   else {
-    e = naive ? launch_naive<double>(g, s) : one_each ? launch_tile<double, 512, 8, 4, 2, 16>(g, s) : launch_tile<double, 256, 4, 8, 2, 16>(g, s);
+    e = naive ? launch_naive<double>(g, s) : one_each && !half_tile ? launch_tile<double, 512, 8, 4, 2, 16>(g, s) : launch_tile<double, 256, 4, 8, 2, 16>(g, s);
   }
   return e == hipSuccess ? CUASR_AMD_SUCCESS : CUASR_AMD_ERROR_INTERNAL;
 }
@@ -1470,7 +1466,7 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
   // With tiles a step's launch also closes the next block, after a launch that updates it; without, a closure alone on
   // the chip takes half a step.  f32, n = 1000 (64 tiles): 635 us a job with tiles, 595 without; from 81 tiles on the
   // tiles win (f64 from 49: n = 1001 984 against 1130).
-  const bool naive = takes_naive_kernel(dtype, n, n, CUASR_AMD_KERNEL_AUTO) || (!f64 && n <= 1024);
+  const bool naive = n <= (f64 ? 768 : 1024);
   // this step's diagonal block had its distances closed during the step before, beside that step's big product
   // (its predecessors are always still to be found, from what the closure recorded in H)
   bool closed = false;
@@ -1569,7 +1565,7 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
     } else {
       x.ahead_bb = 0;
     }
-    r = fwgemm_run(dtype, n, n, bb, Dcol, ld, Drow, ld, dist, ld, parent, ldp, x, naive ? CUASR_AMD_KERNEL_NAIVE : CUASR_AMD_KERNEL_AUTO, stream);
+    r = fwgemm_run(dtype, n, n, bb, Dcol, ld, Drow, ld, dist, ld, parent, ldp, x, naive ? CUASR_AMD_KERNEL_NAIVE : CUASR_AMD_KERNEL_VALU, stream);
     if (r != CUASR_AMD_SUCCESS) return r;
   }
   return CUASR_AMD_SUCCESS;

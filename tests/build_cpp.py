@@ -22,6 +22,7 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=off", 
 PROGRAMS = {
     "test_device_api": ("test_device_api.cpp", "host"),
     "host_splitk_models": ("host_splitk_models.cpp", "host-only"),
+    "host_launch_rules": ("host_launch_rules.cpp", "host-only"),
     "test_user_functor": ("test_user_functor.hip", "hip"),
     "test_reference_call_sites": ("test_reference_call_sites.hip", "hip"),
 }

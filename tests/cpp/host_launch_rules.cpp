@@ -1,0 +1,23 @@
+// Answers, for lines of sizes on standard input, what csrc/launch_rules.h chooses: host code only (g++).
+//   fwgemm <f64> <image> <m> <n>           1: one thread per element, 2: tiles of 128 x 128, 3: of 64 x 128
+#include <cstdio>
+#include <cstring>
+
+#include "../../cuasr_amd/csrc/launch_rules.h"
+
+int main() {
+  char what[16];
+  while (std::scanf("%15s", what) == 1) {
+    int answer;
+    if (!std::strcmp(what, "fwgemm")) {
+      int f64, image, m, n;
+      if (std::scanf("%d %d %d %d", &f64, &image, &m, &n) != 4) return 2;
+      const long long half_tiles = (long long)((m + 63) / 64) * ((n + 127) / 128);
+      answer = cuasr_amd::fwgemm_one_thread_each(f64, image, m, n) ? 1 : f64 && cuasr_amd::fwgemm_f64_half_tile(image, half_tiles) ? 3 : 2;
+    } else {
+      return 2;
+    }
+    std::printf("%d\n", answer);
+  }
+  return 0;
+}

@@ -466,3 +466,26 @@ def test_apsp_drivers_can_be_captured_in_a_graph(oracle):
             oracle.fwgemm(snap, snap, want_d, want_p)
         assert_same_bits(np.ascontiguousarray(d_sq.cpu().numpy()), np.ascontiguousarray(want_d), f"squaring, seed {seed}")
         assert np.array_equal(p_sq.cpu().numpy(), want_p)
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float32, 1100), (np.float32, 1160), (np.float64, 768), (np.float64, 801), (np.float64, 1450)])
+def test_squaring_on_both_sides_of_the_lines(oracle, dtype, n):
+    """One squaring where the kernel changes: one thread per element, then tiles (double: of 64 x 128, then of 128 x 128)."""
+    import torch
+    rng = np.random.default_rng(n)
+    W = np.where(rng.random((n, n)) < 0.1, rng.integers(1, 50, (n, n)), np.inf).astype(dtype)
+    np.fill_diagonal(W, 0)
+    dD = to_device(np.asfortranarray(W))
+    dP = torch.full((n, n), -1, dtype=torch.int32, device="cuda").t()
+    ws = torch.empty(cuasr_amd.apsp_workspace_bytes(n, "f32" if dtype == np.float32 else "f64"), dtype=torch.uint8, device="cuda")
+    cuasr_amd.apsp_squaring(dD, dP, ws, iterations=1)
+    want_d, want_p = np.asfortranarray(W), np.full((n, n), -1, np.int32, order="F")
+    oracle.fwgemm(np.asfortranarray(W), np.asfortranarray(W), want_d, want_p)
+    assert_same_bits(dD.cpu().numpy(), want_d, "dist")
+    assert np.array_equal(dP.cpu().numpy(), want_p)
+
+
+@pytest.mark.parametrize("dtype,m,n,k", [(np.float32, 1448, 1448, 21), (np.float32, 1449, 1453, 21), (np.float64, 905, 900, 37), (np.float64, 930, 1001, 37)])
+def test_products_on_both_sides_of_the_lines(oracle, dtype, m, n, k):
+    run_case(oracle, m, n, k, dtype, True, "auto")
+    run_case(oracle, m, n, k, dtype, False, "auto", pad=(1, 3, 2, 1))
