@@ -5,6 +5,15 @@
 
 namespace cuasr_amd {
 
+// The staged family's full-size tile with its k shared by two groups of threads, against the quarter-size tile (area_ratio
+// of which make a full one).  192 .. 256 full-size workgroups are one per compute unit for most of the chip, whatever their
+// number; the quarter-size tiles' time goes by the most that one compute unit gets.  So the full-size tile wins where
+// that is as many as make a full one: fp32 min-plus 1984^3, 256 full or 961 quarter-size tiles (four per unit), 223 against 250
+// us; 1824^3, 225 or 841, 202 against 223; but 1700^3, 196 or 729 (three per unit), 193 against 169.
+inline bool two_group_full_tile(long long full, long long quarter, int area_ratio) {
+  return full >= 192 && full <= 256 && quarter > 256LL * (area_ratio - 1);
+}
+
 // fwgemm: one thread per element, or tiles of 128 x 128.  The first takes time by outputs, the second by the tiles on the
 // fullest compute unit (one, here) and, without a k-contiguous image of A at hand, by lookups that gather 16 cache lines per
 // improved element.  us on square problems, one thread per element / tiles.  Without the image: float 1000^3 165 / 310, 1152^3

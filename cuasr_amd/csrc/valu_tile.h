@@ -19,6 +19,7 @@
 // blockIdx.x walks output tiles through an XCD-aware, row-grouped order;
 // blockIdx.y is the split-K slice.
 #pragma once
+#include "launch_rules.h"
 #include "semiring.h"
 
 #ifndef WAVES_ATTR
@@ -748,18 +749,22 @@ static hipError_t launch_valu_sized(const Problem &p, hipStream_t s) {
   const long long groups = (long long)((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN) * slice_groups(p) * p.batch;
   const long long rounds = (groups + 1023) / 1024;
   // ... and those tiles do not reach much further past the edges than the quarter-size ones: a batch of 1000 products of
-  // 64 x 64 filled 1000 full-size tiles to a quarter (37.8 us; 18.2 on the quarter-size ones)
+  // 64 x 64 filled 1000 full-size tiles to a quarter (37.8 us; 18.2 on the quarter-size ones).  An eighth more is less than
+  // their rate is worth (940 x 16384 x 500, a fifteenth more, both operands k-contiguous: 246 us, 261 on the smaller ones)
   constexpr int SM = 16 * TM_SMALL, SN = 16 * TN_SMALL;
   const long long groups_small = (long long)((p.m + SM - 1) / SM) * ((p.n + SN - 1) / SN) * slice_groups(p) * p.batch;
-  const bool covers_more = groups * BM * BN * 16 > groups_small * SM * SN * 17;
+  const bool covers_more = groups * BM * BN * 8 > groups_small * SM * SN * 9;
   if constexpr (order_free<T, ADD>::value) {
     // 192 .. 256 full-size workgroups (2048^2: exactly 256) are one per compute unit for most of the
     // chip: two groups per workgroup give every SIMD its two waves, and the full-size tile then runs
-    // at the rate it has on large problems, which the quarter-size tile does not reach
-    const long long k_range = p.workspace ? p.k_per_slice / (p.k_sub > 1 ? p.k_sub : 1) : p.k;
-    if (groups >= 192 && groups <= 256 && !covers_more && k_range >= 8LL * BK && vector_possible<T>(p) && p.m > 0 && p.n > 0) {
-      launch_ksplit<T, ADD, MUL, TM, TN, BK, 2>(p, dim3((unsigned)(groups / slice_groups(p) / p.batch), slice_groups(p), p.batch), s);
-      return take_launch_status();
+    // at the rate it has on large problems, which the quarter-size tile does not reach.  With one instruction per term it
+    // does (or-and 1984^3 203 us against 209 on the full-size tile, xor-and 1950^3 200 against 213).
+    if constexpr (ADD != kLogicalOr && ADD != kBitXor && ADD != kBitOr && ADD != kBitAnd) {
+      const long long k_range = p.workspace ? p.k_per_slice / (p.k_sub > 1 ? p.k_sub : 1) : p.k;
+      if (two_group_full_tile(groups, groups_small, BM * BN / (SM * SN)) && k_range >= 8LL * BK && vector_possible<T>(p) && p.m > 0 && p.n > 0) {
+        launch_ksplit<T, ADD, MUL, TM, TN, BK, 2>(p, dim3((unsigned)(groups / slice_groups(p) / p.batch), slice_groups(p), p.batch), s);
+        return take_launch_status();
+      }
     }
   }
   if (covers_more || groups * 100 < rounds * 1024 * (long long)(CUASR_AMD_FULL_TILE_FILL_PERCENT))

@@ -1,5 +1,6 @@
 // Answers, for lines of sizes on standard input, what csrc/launch_rules.h chooses: host code only (g++).
 //   fwgemm <f64> <image> <m> <n>           1: one thread per element, 2: tiles of 128 x 128, 3: of 64 x 128
+//   staged <m> <n> <batch> <full m> <full n>   1: the full-size tile in two groups, 0: not (quarter-size: 64 x 64)
 #include <cstdio>
 #include <cstring>
 
@@ -15,7 +16,10 @@ int main() {
       const long long half_tiles = (long long)((m + 63) / 64) * ((n + 127) / 128);
       answer = cuasr_amd::fwgemm_one_thread_each(f64, image, m, n) ? 1 : f64 && cuasr_amd::fwgemm_f64_half_tile(image, half_tiles) ? 3 : 2;
     } else {
-      return 2;
+      long long m, n, batch, bm, bn;
+      if (std::scanf("%lld %lld %lld %lld %lld", &m, &n, &batch, &bm, &bn) != 5) return 2;
+      const long long full = (m + bm - 1) / bm * ((n + bn - 1) / bn) * batch, quarter = (m + 63) / 64 * ((n + 63) / 64) * batch;
+      answer = cuasr_amd::two_group_full_tile(full, quarter, int(bm * bn / 4096));
     }
     std::printf("%d\n", answer);
   }

@@ -20,3 +20,13 @@ def test_fwgemm_takes_the_faster_kernel():
         (1, 1, 700, one), (1, 1, 768, one), (1, 1, 800, half), (1, 1, 1024, half), (1, 1, 1408, half), (1, 1, 1536, tile), (1, 1, 2048, tile)]
     got = _ask(["fwgemm %d %d %d %d" % (f64, image, n, n) for f64, image, n, _ in cases])
     assert got == [kernel for *_, kernel in cases]
+
+
+def test_staged_tiles_take_the_faster_size():
+    cases = [  # m, n, batch, full-size tile, two groups on it
+        (1700, 1700, 1, 128, 128, 0), (1728, 1728, 1, 128, 128, 0), (2048, 1536, 1, 128, 128, 0), (1750, 1750, 1, 128, 128, 1),
+        (1824, 1824, 1, 128, 128, 1), (1950, 1950, 1, 128, 128, 1), (1984, 1984, 1, 128, 128, 1), (2048, 2048, 1, 128, 128, 1),
+        (2100, 2100, 1, 128, 128, 0), (1650, 1650, 1, 128, 128, 0),                                      # 289 of them; 169
+        (64, 64, 200, 128, 128, 0), (180, 200, 64, 128, 128, 0), (100, 100, 240, 128, 128, 1)]           # a batch of small products
+    got = _ask(["staged %d %d %d %d %d" % c[:5] for c in cases])
+    assert got == [c[5] for c in cases]
