@@ -37,17 +37,27 @@ template <typename T, int ADD, int MUL, int KC, int W> struct SmallTile {
   static constexpr int XV = BLOCK / VW, KV = KC / VW, DK = 64 / XV, DX = 64 / KV;   // DK of k (DX of x): what one load of the wave covers
 
   // One operand's chunk, BLOCK x KC, into registers.  VEC: the block lies inside the matrix (the caller moved its origin
-  // back where it would not) and the chunk is whole, so 16-byte loads at element alignment; otherwise element by
-  // element with clamped indices (what lands past an edge is never stored, k past the end never used).
+  // back where it would not) and the chunk is whole, so 16-byte loads at element alignment.  A matrix narrower than a block
+  // still takes them along k, from clamped rows.  Otherwise element by element with clamped indices (what lands past an edge
+  // is never stored, k past the end never used).
   static __device__ __forceinline__ void load(T (&r)[PER], const T *base, long long s_x, long long s_k, int x_end, int k0, int k_end, bool xc,
                                               bool vec, int lane) {
-    if (vec) {
+    if (vec && (xc || x_end >= BLOCK)) {
       const int xx = xc ? lane % XV * VW : lane / KV, kk = xc ? lane / XV : lane % KV * VW;
       const T *src = base + (long long)xx * s_x + (long long)(k0 + kk) * s_k;
       const long long next = xc ? DK * s_k : DX * s_x;
 #pragma unroll
       for (int p = 0; p < PER / VW; ++p) {
         const gvec_t t = *reinterpret_cast<const gvec_t *>(src + p * next);
+#pragma unroll
+        for (int e = 0; e < VW; ++e) r[p * VW + e] = t[e];
+      }
+    } else if (vec) {
+      int l = lane;   // (as below)
+      asm volatile("" : "+v"(l));
+#pragma unroll
+      for (int p = 0; p < PER / VW; ++p) {
+        const gvec_t t = *reinterpret_cast<const gvec_t *>(base + (long long)min(l / KV + p * DX, x_end - 1) * s_x + (k0 + l % KV * VW));
 #pragma unroll
         for (int e = 0; e < VW; ++e) r[p * VW + e] = t[e];
       }
@@ -131,8 +141,7 @@ template <typename T, int ADD, int MUL, int KC, int W> struct SmallTile {
     Ops::tile_coords(blockIdx.x, tiles_m, tiles_n, bm, bn);
     const int first_m = bm * BLOCK, first_n = bn * BLOCK;       // the first row and column this workgroup stores
     // blocks at the far edges start earlier instead of reaching past the matrix: what they compute twice is not stored
-    const bool inside = p.m >= BLOCK && p.n >= BLOCK;
-    const int m0 = inside ? min(first_m, p.m - BLOCK) : first_m, n0 = inside ? min(first_n, p.n - BLOCK) : first_n;
+    const int m0 = p.m >= BLOCK ? min(first_m, p.m - BLOCK) : first_m, n0 = p.n >= BLOCK ? min(first_n, p.n - BLOCK) : first_n;
     int kb = 0, ke = p.k;
     if (p.workspace) {
       const int parts = p.k_sub > 1 ? p.k_sub : 1, slice = blockIdx.y / parts, part = blockIdx.y % parts;
@@ -165,24 +174,27 @@ template <typename T, int ADD, int MUL, int KC, int W> struct SmallTile {
     for (int i = 0; i < R; ++i)
 #pragma unroll
       for (int j = 0; j < R; ++j) acc[i][j] = init;
+    // an output narrower than a block gives up the vectors along its narrow side, and no others (or-and, 1 x 65536 x 256: 42.7
+    // us with every operand element by element, 23.5 now; 10 x 60000 x 200: 38.6 and 24.5)
+    const bool vec_a = p.m >= BLOCK || !a_xc, vec_b = p.n >= BLOCK || !b_xc;
     Panels &pn = sm.p[wave];
     T ra[PER], rb[PER];
     int k0 = kb + wave * KC;
     if (k0 < ke) {
-      const bool vec = inside && k0 + KC <= ke;
-      load(ra, A, p.sa_m, p.sa_k, p.m - m0, k0, ke, a_xc, vec, lane);
-      load(rb, B, p.sb_n, p.sb_k, p.n - n0, k0, ke, b_xc, vec, lane);
+      const bool whole = k0 + KC <= ke;
+      load(ra, A, p.sa_m, p.sa_k, p.m - m0, k0, ke, a_xc, vec_a && whole, lane);
+      load(rb, B, p.sb_n, p.sb_k, p.n - n0, k0, ke, b_xc, vec_b && whole, lane);
     }
     for (; k0 < ke; k0 += W * KC) {
-      const bool vec = inside && k0 + KC <= ke;
-      store(ra, pn.a, a_xc, vec, lane);
-      store(rb, pn.b, b_xc, vec, lane);
+      const bool whole = k0 + KC <= ke;
+      store(ra, pn.a, a_xc, vec_a && whole, lane);
+      store(rb, pn.b, b_xc, vec_b && whole, lane);
       wave_lds_order();   // other lanes read what a lane has stored
       const int kn = k0 + W * KC;
       if (kn < ke) {
-        const bool vn = inside && kn + KC <= ke;
-        load(ra, A, p.sa_m, p.sa_k, p.m - m0, kn, ke, a_xc, vn, lane);
-        load(rb, B, p.sb_n, p.sb_k, p.n - n0, kn, ke, b_xc, vn, lane);
+        const bool whole_next = kn + KC <= ke;
+        load(ra, A, p.sa_m, p.sa_k, p.m - m0, kn, ke, a_xc, vec_a && whole_next, lane);
+        load(rb, B, p.sb_n, p.sb_k, p.n - n0, kn, ke, b_xc, vec_b && whole_next, lane);
       }
       if (k0 + KC <= ke) {
         Frag<U> f[2];

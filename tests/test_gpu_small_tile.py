@@ -79,3 +79,29 @@ def test_small_outputs_in_place_in_slices_and_in_batches(oracle, lib, pair):
         for i in range(0, b, 9):
             want = oracle.srgemm(add, mult, *ops[i], one, one, ident)
             assert_same_bits(to_host(dD[i], dt), want, f"{pair} product {i} of {b}")
+
+
+@pytest.mark.parametrize("pair", PAIRS)
+@pytest.mark.parametrize("shape", [(1, 200, 300), (20, 97, 100), (500, 31, 70), (33, 2, 48), (17, 16, 129)])
+def test_outputs_narrower_than_a_block(oracle, lib, pair, shape):
+    """Vectors along k from clamped rows where an operand's rows are fewer than a block's, whole blocks on the other side;
+    rows spaced wider than they are long."""
+    import torch
+    import cuasr_amd
+    from cuasr_amd import inputs
+    add, mult, dt = pair
+    ident, one = cuasr_amd.op_identity(add, dt, True), cuasr_amd.op_identity(mult, dt, True)
+    for i, order in enumerate(("FFF", "CCC", "CFC", "FCF")):
+        A, B, C = _case(inputs, dt, *shape, order, 131 + i)
+        want = oracle.srgemm(add, mult, A, B, C, one, one, ident)
+        wide = []
+        for x in (A, B):   # the leading dimension three elements more than it has to be
+            t = to_device(x)
+            base = t if x.flags.c_contiguous else t.t()
+            room = torch.zeros(base.shape[0], base.shape[1] + 3, dtype=base.dtype, device="cuda")
+            room[:, :base.shape[1]] = base
+            wide.append(room[:, :base.shape[1]] if x.flags.c_contiguous else room[:, :base.shape[1]].t())
+        dD = to_device(np.zeros_like(C))
+        cuasr_amd.srgemm(add, mult, *wide, to_device(C), dD, one, one, ident, one, dtype=dt, kernel="valu")
+        torch.cuda.synchronize()
+        assert_same_bits(to_host(dD, dt), want, f"{pair} {shape} {order}")
