@@ -54,3 +54,33 @@ def test_slices_and_batches(oracle, lib, dtype):
         torch.cuda.synchronize()
         want = np.matmul(A.astype(np.float64), B.astype(np.float64)) + C
         assert np.array_equal(dD.cpu().numpy(), want), (b, m, n, k)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f64"])
+@pytest.mark.parametrize("shape", [(33, 31, 7), (100, 60, 24), (70, 40, 2101), (300, 700, 133), (512, 512, 512), (1024, 1000, 515)])
+def test_sums_of_numbers_that_round(lib, dtype, shape):
+    """Normal numbers against a sum in 64 bits (double: in extended precision): a sum of k products in any order is off by at
+    most k roundings of the sum of magnitudes.  The operands' rows are longer than the matrices, and what lies past k and
+    past the far rows and columns is NaN and infinity, none of which may reach a result."""
+    import torch
+    import cuasr_amd
+    m, n, k = shape
+    rng = np.random.default_rng(m * n + k)
+    npd = NPD[dtype]
+    A, B = rng.standard_normal((m, k)).astype(npd), rng.standard_normal((k, n)).astype(npd)
+    wide = np.float64 if dtype == "f32" else np.longdouble
+    want = A.astype(wide) @ B.astype(wide)
+    bound = k * np.finfo(npd).eps * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64))
+    for order in ("CC", "FF", "CF", "FC"):
+        ops = []
+        for x, o in zip((A, B), order):
+            x = x if o == "C" else x.T
+            room = np.where(rng.random((x.shape[0] + 3, x.shape[1] + 5)) < 0.5, np.nan, np.inf).astype(npd)
+            room[:x.shape[0], :x.shape[1]] = x
+            t = torch.from_numpy(room).cuda()[:x.shape[0], :x.shape[1]]
+            ops.append(t if o == "C" else t.t())
+        dD = torch.zeros(m, n, dtype=ops[0].dtype, device="cuda")
+        cuasr_amd.srgemm("plus", "multiplies", *ops, dD, dD, 1.0, 0.0, 0.0, 1.0)
+        torch.cuda.synchronize()
+        diff = np.abs(dD.cpu().numpy().astype(wide) - want).astype(np.float64)
+        assert (diff <= bound).all(), (shape, order, float((diff / bound).max()))
