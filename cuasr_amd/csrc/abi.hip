@@ -116,8 +116,6 @@ static bool streamk_usable(const cuasr_amd_srgemm_desc *d) {
   return ((d->alpha.bits ^ d->mult_identity.bits) & mask) == 0;
 }
 
-// ... and worth it: the plain tiles would leave a good part of their last round of 512 places empty, and every
-// workgroup's share of the k-tiles is long enough to carry a tile's prologue and fold
 // 70 % or more of the compute units get one tile each and none gets two: the plain direct tile then beats both the
 // shared tiles, whose folds cost more than the idle units (2560^3 min-plus: 60 - 66 against 54 - 57 TOPS), and the
 // staged tile (2816^3: 71 against 60)
@@ -133,6 +131,8 @@ static bool one_tile_each(const cuasr_amd_srgemm_desc *d, const Problem &c) {
   return tiles * 256 * 128 * 100 <= 4096LL * 115 * ((c.m + 63) / 64) * ((c.n + 63) / 64);
 }
 
+// The stream-K form is worth it: the plain tiles would leave a good part of their last round of 512 places empty, and every
+// workgroup's share of the k-tiles is long enough to carry a tile's prologue and fold
 static bool streamk_preferred(const cuasr_amd_srgemm_desc *d, long long batch) {
   if (batch != 1 || d->split_k_slices != 1 || !streamk_usable(d)) return false;
   // min-max and max-min spend two instructions per term and their staged tile is within 5 % of the direct one:
@@ -348,7 +348,7 @@ static launch_fn family_fn(int family, const cuasr_amd_srgemm_desc *d) {
     case kDirect: return find_direct(d->dtype, d->add_op, d->mult_op);
     case kValu:
       // AUTO's plus-times in float and double below 128 tiles of 128 x 128: the matrix cores in blocks of 32 x 32
-      // (1024^3: 25 - 28 us against 81 on the vector ALU; sums in the matrix instruction's order, as in larger products)
+      // (1024^3: 24 - 28 us by layout against 81 on the vector ALU; sums in the matrix instruction's order, as in larger products)
       if (d->kernel == CUASR_AMD_KERNEL_AUTO && d->add_op == kPlus && d->mult_op == kMultiplies &&
           (d->dtype == CUASR_AMD_F32 || d->dtype == CUASR_AMD_F64))
         return find_mfma(d->dtype, d->add_op, d->mult_op);

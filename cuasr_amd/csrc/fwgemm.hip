@@ -1004,8 +1004,8 @@ __global__ void __launch_bounds__(256) fwgemm_pair_kernel(FwArgs g0, FwArgs g1, 
 // whose first workgroup -- the first one the launch starts -- closes the next block step's diagonal
 // block while the workgroups of the other rows do the product's tiles, all but that block.  The block's
 // 128 dependent steps take about as long as the whole product and nothing else of the next block step can
-// start before them; here they cost one of the launch's 512 places.  Only where a tile is a whole
-// diagonal block (4-byte elements; the host asks for nothing else).
+// start before them; here they cost one of the launch's 512 places.  Only where whole tiles make up a
+// diagonal block (all shapes the host launches, of either element type).
 template <typename T, int NT, int TM, int TN, int WPE, int BK, bool GUARD, bool HAS_AT>
 __global__ void __launch_bounds__(NT, WPE) fwgemm_tile_kernel(FwArgs g) {
   typedef FwTileLds<T, NT, TM, TN, BK> TileLds;

@@ -10,9 +10,9 @@
 // indices are clamped lane by lane, and only the last chunk of a k range that is not whole chunks looks at its end
 // (k past it is multiplied as zero).  The next chunk is requested before a chunk's eight matrix instructions (512
 // cycles; 2 x 2 blocks: 2048) are issued.  The KG partial sums meet in LDS, each wave finishing a KG-th of the block's
-// rows.  512^3 41.5 -> 6.7 us (float), 55.4 -> 9.6 (double); 1024^3 80.6 -> 25 - 28 and 110 -> 43; 64 x 4096 x 4096 308 ->
+// rows.  512^3 41.5 -> 6.7 us (float), 55.4 -> 9.6 (double); 1024^3 80.6 -> 24 - 28 by layout and 110 -> 42 - 45 (operands in cache; 30.7 and up on new ones); 64 x 4096 x 4096 308 ->
 // 34 and 421 -> 48 (the vector-ALU tiles before it); 2048 products of 100^3, each a launch of its own before, 25 ms -> 0.16.
-// Bound: operands from L2 (1024^3 moves 134 MB in 64 x 64 tiles, at 5.5 TB/s).
+// Bound: most likely the operands' way from L2 (1024^3 moves 134 MB in 64 x 64 tiles, 4.4 - 5.6 TB/s); no counter has been read.
 #include "mfma_common.h"
 
 namespace cuasr_amd {
@@ -231,7 +231,7 @@ static long long launches_of(const Problem &p) { return (p.workspace ? p.slices 
 static long long tiles_of(const Problem &p, int tile) { return (long long)((p.m + tile - 1) / tile) * ((p.n + tile - 1) / tile) * launches_of(p); }
 
 // Which form.  Waves of 64 x 64 (four or, for double, eight of them sharing k) fetch half as much per operation, and
-// carry most of the work where their tiles fill the chip's 256 compute units and k is long (1024^3: float 25 - 28 us
+// carry most of the work where their tiles fill the chip's 256 compute units and k is long (1024^3: float 24 - 28 us
 // against 34 - 39 in single blocks, double 43 - 44 against 47 - 62; 512 x 512 x 8192 in 8 slices: 63 against 71 and 91
 // against 122; but 1200^3, 361 tiles for two rounds of 256: 65 against 60).  Four single-block waves side by side on a
 // 64 x 64 tile, nothing to fold, win where there are many tiles and k is short (1024 products of 64^3: 15.7 us against
