@@ -272,7 +272,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
 // The 64 x 64 staged tile with its k range shared out over 1024 threads is the better one from about 176 workgroups on
 // (min-plus f32, 60 % of the chip's compute units: 832^3, 169 of them, 30.3 against 26.8 us here; 896^3, 196, 31.5
 // against 36.5), for 8-byte elements from 128 (640^3, 100: 47.9 against 34.3 us; 768^3, 144: 56.8 against 56.1; 832^3:
-// 60.8 against 62.5).  Integer plus-times stays there at every size (its multiply-adds spill here: 512^3 30.9 against 48 us).
+// 60.8 against 62.5; this kernel's double figures are 6 - 10 % lower since, 512^3 17.6 -> 15.7).  Integer plus-times stays there at every size (its multiply-adds spill here: 512^3 30.9 against 48 us).
 template <typename T, int ADD> static bool small_preferred(const Problem &p) {
   if (ADD == kPlus || p.k < 1) return false;
   const long long groups64 = (long long)((p.m + 63) / 64) * ((p.n + 63) / 64) * slice_groups(p) * p.batch;
