@@ -1359,7 +1359,7 @@ int fwgemm_run(int dtype, int m, int n, int k, const void *A, int64_t lda, const
            x.skip_r0, x.skip_r1, x.skip_c0, x.skip_c1, nullptr, 0, 0, 0, nullptr};
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool naive = kernel == CUASR_AMD_KERNEL_NAIVE ||
-                     (kernel == CUASR_AMD_KERNEL_AUTO && fwgemm_one_thread_each(dtype == CUASR_AMD_F64, x.At != nullptr, m, n));
+                     (kernel == CUASR_AMD_KERNEL_AUTO && fwgemm_one_thread_each(dtype == CUASR_AMD_F64, x.At != nullptr, m, n, k));
   if (!naive && x.ahead_bb > 0 && x.hist) {
     g.ahead0 = x.ahead0;
     g.ahead_bb = x.ahead_bb;
@@ -1379,7 +1379,7 @@ int fwgemm_run(int dtype, int m, int n, int k, const void *A, int64_t lda, const
   const int64_t tm = (int64_t(g.m) + 127) / 128, tn = (int64_t(g.n) + 127) / 128;
   const int64_t skip_m = g.skip_r1 > g.skip_r0 ? 1 : 0, skip_n = g.skip_c1 > g.skip_c0 ? 1 : 0;
   const bool one_each = (tm - skip_m) * (tn - skip_n) <= 256;
-  const bool half_tile = skip_m + skip_n == 0 && fwgemm_f64_half_tile(g.At != nullptr, (int64_t(g.m) + 63) / 64 * tn);
+  const bool half_tile = skip_m + skip_n == 0 && fwgemm_f64_half_tile(g.At != nullptr, g.m, (int64_t(g.m) + 63) / 64 * tn);
   if (dtype == CUASR_AMD_F32) {
     e = naive ? launch_naive<float>(g, s) : one_each ? launch_tile<float, 512, 8, 4, 2, 16>(g, s) : launch_tile<float, 512, 8, 4, 4, 16>(g, s);
   }

@@ -14,20 +14,27 @@ inline bool two_group_full_tile(long long full, long long quarter, int area_rati
   return full >= 192 && full <= 256 && quarter > 256LL * (area_ratio - 1);
 }
 
-// fwgemm: one thread per element, or tiles of 128 x 128.  The first takes time by outputs, the second by the tiles on the
-// fullest compute unit (one, here) and, without a k-contiguous image of A at hand, by lookups that gather 16 cache lines per
-// improved element.  us on square problems, one thread per element / tiles.  Without the image: float 1000^3 165 / 310, 1152^3
+// fwgemm: one thread per element, or tiles of 128 x 128.  The first takes time by columns of 64 outputs, and more than its share
+// once A's columns leave the L2 (long k); the second by the tiles on the fullest compute unit (one, here) and, without a
+// k-contiguous image of A at hand, by lookups that gather 16 cache lines per improved element, whatever k.  us on square problems, one thread per element / tiles.  Without the image: float 1000^3 165 / 310, 1152^3
 // 241 / 472, 1408^3 428 / 555, 1536^3 544 / 453; double 800^3 247 / 328, 900^3 360 / 377, 1000^3 449 / 333.  With it
 // (three squarings): float 1000 526 / 638, 1100 699 / 716, 1152 758 / 701; double 700 516 / 632, 768 634 / 650, 800 776 / 669.
-inline bool fwgemm_one_thread_each(bool f64, bool k_contiguous_image, int m, int n) {
-  const int64_t tiles_worth = f64 ? (k_contiguous_image ? 37 : 50) : (k_contiguous_image ? 76 : 128);
-  return int64_t(m) * n < tiles_worth * 128 * 128;
+// Long and short k without it: float 1100 x 1100 x 4000 1215 / 966; double 200 x 3000 x 2500 1816 / 1076, 1100 x 1100 x 64 48 / 106.  One row: 1 x 100000 x 300
+// float 294 / 258, double 1396 / 257.
+inline bool fwgemm_one_thread_each(bool f64, bool k_contiguous_image, int m, int n, int k) {
+  const double tiles_worth = double((int64_t(m) + 63) / 64 * 64) * n / (128 * 128);
+  if (k_contiguous_image) return tiles_worth < (f64 ? 37 : 79);
+  if (f64) return tiles_worth < (k < 2048 ? 53 : 40) || (tiles_worth < 150 && tiles_worth * k < 20000);
+  return tiles_worth < (k < 2048 ? 128 : 64);
 }
 
 // ... and the double-precision tile: 64 x 128 by 256 threads while every one of them has a compute unit to itself, and
 // without the image (its lookups take the time) at any size; 128 x 128 by 512 threads otherwise.  Three squarings of n = 1024 / 1280 / 1408 /
 // 1536 / 1792: 797 / 963 / 1052 / 1718 / 1988 us on 64 x 128, 1174 / 1430 / 1558 / 1675 / 1940 on 128 x 128; one product
 // without the image 331 / 414 / 557 / 694 / 945 and 523 / 779 / 865 / 825 / 1153.
-inline bool fwgemm_f64_half_tile(bool k_contiguous_image, int64_t half_tiles) { return !k_contiguous_image || half_tiles <= 256; }
+// (Fewer than 64 rows, 30 x 30000 x 200: 160 and 143.)
+inline bool fwgemm_f64_half_tile(bool k_contiguous_image, int m, int64_t half_tiles) {
+  return m >= 64 && (!k_contiguous_image || half_tiles <= 256);
+}
 
 }  // namespace cuasr_amd

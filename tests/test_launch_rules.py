@@ -18,8 +18,13 @@ def test_fwgemm_takes_the_faster_kernel():
         (0, 1, 896, one), (0, 1, 1000, one), (0, 1, 1024, one), (0, 1, 1100, one), (0, 1, 1152, tile), (0, 1, 2100, tile),
         (1, 0, 800, one), (1, 0, 900, one), (1, 0, 1000, half), (1, 0, 1280, half), (1, 0, 1792, half),
         (1, 1, 700, one), (1, 1, 768, one), (1, 1, 800, half), (1, 1, 1024, half), (1, 1, 1408, half), (1, 1, 1536, tile), (1, 1, 2048, tile)]
-    got = _ask(["fwgemm %d %d %d %d" % (f64, image, n, n) for f64, image, n, _ in cases])
+    got = _ask(["fwgemm %d %d %d %d %d" % (f64, image, n, n, n) for f64, image, n, _ in cases])
     assert got == [kernel for *_, kernel in cases]
+    cases = [  # f64, m, n, k, kernel; without the image: long and short k, few rows and few columns
+        (0, 1100, 1100, 4000, tile), (0, 1100, 1100, 64, one), (0, 1, 100000, 300, tile), (0, 100000, 1, 300, one), (0, 30, 30000, 200, one),
+        (1, 1100, 1100, 4000, half), (1, 1100, 1100, 64, one), (1, 1, 100000, 300, tile), (1, 100000, 1, 300, one), (1, 30, 30000, 200, tile), (1, 200, 3000, 2500, half), (1, 64, 20000, 500, half), (1, 1500, 1500, 100, one)]
+    got = _ask(["fwgemm %d 0 %d %d %d" % c[:4] for c in cases])
+    assert got == [c[4] for c in cases]
 
 
 def test_staged_tiles_take_the_faster_size():
