@@ -28,6 +28,8 @@
 namespace cuasr_amd {
 namespace {
 
+constexpr int FW_BLOCK = 128;  // vertices per block step of the blocked Floyd-Warshall
+
 struct FwArgs {
   int m, n, k;
   const void *A; int64_t lda;
@@ -40,15 +42,13 @@ struct FwArgs {
   const void *At; int64_t ldat;
   int k_base;                               // recorded parents are k_base + k
   int skip_r0, skip_r1, skip_c0, skip_c1;   // outputs in these rows or these columns are left alone
-  // one-thread-per-element and row-by-four-columns kernels only: every output they compute is also stored transposed,
-  // out_t[col + row * ld_out_t] (the k-contiguous image a later product's lookups read)
-  void *out_t; int64_t ld_out_t;
   // tile kernel, blocked Floyd-Warshall only: the diagonal block that starts at (ahead0, ahead0) and has
   // ahead_bb (> 0) rows is the next block step's and has had this step's update already: the launch's
   // first workgroup closes its distances (fw_close_dist) while the others do the product, which leaves that
-  // block alone.  hist: 3 x FW_BLOCK x FW_BLOCK elements that take what fw_parents_block needs afterwards.
+  // block alone.  hist: 3 x FW_BLOCK x FW_BLOCK elements that take what fw_parents needs afterwards.
   int ahead0, ahead_bb;
   void *hist;
+  void *closed, *closed_t;   // ... and the closed block and its transpose, for that step's panels (FwPanels)
 };
 
 // cond ? a : b with a hidden from the optimiser: `x < y ? x : y` on floating point is
@@ -104,7 +104,6 @@ template <typename T> __device__ __forceinline__ void fwgemm_naive_block(const F
   }
   *d = curr;
   *pp = p;
-  if (g.out_t) static_cast<T *>(g.out_t)[col + int64_t(row) * g.ld_out_t] = curr;
 }
 
 template <typename T>
@@ -120,122 +119,296 @@ template <typename T> struct uvec4_of;
 template <> struct uvec4_of<float> { typedef float type __attribute__((ext_vector_type(4), aligned(4))); };
 template <> struct uvec4_of<double> { typedef double type __attribute__((ext_vector_type(4), aligned(8))); };
 
-// One thread per output row and four columns, for products too small for the tile kernel but on the
-// critical path (the block row and the block column of a blocked Floyd-Warshall step): a workgroup of 256
-// threads covers 64 rows x 16 columns.  Same order-free form as the tile kernel: per chunk of 16 k a plain
-// min-plus (a 3-input minimum per two products), and "chunk minimum < running minimum" (strict) moves the
-// running minimum.  A chunk in which any of the wave's 64 rows improved is resolved on the spot, from the
-// operands still in registers: the first k whose product equals the chunk minimum (the same single addition
-// of the same operands, so equality is exact) is the parent, and that product, sign of zero included, the
-// distance.  (Looking the chunk up after the loop, as the tile kernel does, costs a gather of 16 cache lines
-// per lane and column here: 27 us for the two panels at n = 4096.)  A's 16 values of a chunk serve four
-// columns.  The one-thread-per-element scan spends four instructions per term, two of which read a mask, and reads each A
-// value once per output column: 29 us.
-template <typename T> __device__ __forceinline__ void fwgemm_rowcols_block(const FwArgs &g, int bx, int by) {
-  constexpr int CK = 16, NC = 4;
-  const int row_of_lane = bx * 64 + (threadIdx.x & 63);
-  const int col0 = __builtin_amdgcn_readfirstlane(by * 16 + (threadIdx.x >> 6) * NC);
-  if (col0 >= g.n) return;  // (the whole wave)
-  // every lane stays to the end, because every lane fetches one of the chunk's B values for the wave: rows
-  // beyond the matrix or in the skipped range are computed on a clamped row and never stored
-  const bool row_live = row_of_lane < g.m && !(row_of_lane >= g.skip_r0 && row_of_lane < g.skip_r1);
-  const int row = row_of_lane < g.m ? row_of_lane : g.m - 1;
-  const T inf = std::numeric_limits<T>::infinity();
-  const int64_t lda = g.lda;
-  // columns beyond the matrix or in the skipped range: computed on a clamped column, never stored
-  int64_t out[NC];
-  bool live[NC];
-  T curr[NC];
-  int32_t par[NC];
+// The products a block step of the blocked Floyd-Warshall makes on its critical path -- block row, block column, the
+// predecessors of the diagonal block and the next diagonal block, each too small for the tile kernel.  A workgroup of 512
+// threads keeps one operand whole in LDS (FW_BLOCK lines x FW_BLOCK k, fetched with all its loads in flight) and 4 NC lines of
+// the other; a lane takes one line of the first and NC of the second.  Same order-free form as the tile kernel: per chunk of
+// 16 k a plain min-plus (a 3-input minimum per two products), "chunk minimum < running minimum" (strict) moves the running
+// minimum and records the chunk, and the recorded chunk is looked up once at the end: the first k whose product equals
+// the minimum (the same single addition of the same operands, so equality is exact) is the parent, and that product, sign
+// of zero included, the distance.
+// What bounds it is one launch, one round trip to memory and the instructions' own way from memory, which a kernel of a
+// few microseconds pays for in full: straight-line code (eight chunks unrolled, each with a lookup of its own, operands in
+// registers) took 14.9 us for both panels at n = 2000, as long as a kernel with one round trip per chunk; this 10.2.
+template <typename T> struct FwLineLds {
+  static constexpr int CK = 16, LINES = 16, STRIDE = FW_BLOCK + 4;
+  alignas(4 * sizeof(T)) T whole[FW_BLOCK][FW_BLOCK];   // [k][line]
+  alignas(4 * sizeof(T)) T other[LINES][STRIDE];        // [line][k], +infinity from the last k to the end of its chunk
+};
+constexpr int FW_LINE_THREADS = 512;
+
+// whole[k][line] = src[line + k * ld], lines up to `lines` (clamped; the rest are not stored by anybody)
+template <typename T> __device__ __forceinline__ void fw_fetch_whole(FwLineLds<T> &sm, const T *src, int64_t ld, int lines) {
+  typedef typename vec4_of<T>::type V4;
+  typedef typename uvec4_of<T>::type U4;
+  constexpr int N = FW_BLOCK * FW_BLOCK / 4 / FW_LINE_THREADS;
+  const int tid = threadIdx.x, line = (tid & 31) * 4, k0 = tid >> 5;
+  V4 v[N];
+  if (lines == FW_BLOCK) {
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const int cc = col0 + c, cl = cc < g.n ? cc : g.n - 1;
-    live[c] = row_live && cc < g.n && !(cc >= g.skip_c0 && cc < g.skip_c1);
-    out[c] = cl;
-    curr[c] = static_cast<const T *>(g.dist)[row + int64_t(cl) * g.ldc];
-    par[c] = -1;
-  }
-  // one chunk of CK k-values; FULL: all of them exist (the ragged last chunk takes +infinity for the others,
-  // which neither improves anything nor equals a minimum that did)
-  // B's 4 x 16 values of a chunk: one load per lane (lane = column, k), handed round through a piece of LDS that
-  // belongs to the wave (no barrier: a wave's LDS accesses complete in order) and read back as broadcasts.
-  // Through scalar loads instead, every chunk and column waited for a scalar-cache miss, and every add read
-  // a scalar register, which costs it a second issue slot.
-  __shared__ alignas(4 * sizeof(T)) T bstage[4][2][NC * CK];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const T *blane = static_cast<const T *>(g.B) + int64_t(min(col0 + (lane >> 4), g.n - 1)) * g.ldb;
-  const T *ap = static_cast<const T *>(g.A) + row;
-  auto load = [&](T (&av)[CK], T &bl, int k0, auto full) {
-    constexpr bool FULL = decltype(full)::value;
-    bl = blane[FULL ? k0 + (lane & 15) : min(k0 + (lane & 15), g.k - 1)];
+    for (int u = 0; u < N; ++u) v[u] = *reinterpret_cast<const U4 *>(src + line + int64_t(k0 + u * (FW_LINE_THREADS / 32)) * ld);
+  } else {
+#pragma unroll 1
+    for (int u = 0; u < N; ++u) {
+      V4 x;
 #pragma unroll
-    for (int u = 0; u < CK; ++u) {
-      if constexpr (FULL) av[u] = *ap;
-      else av[u] = k0 + u < g.k ? *ap : inf;
-      if (FULL || k0 + u + 1 < g.k) ap += lda;
+      for (int e = 0; e < 4; ++e) x[e] = src[min(line + e, lines - 1) + int64_t(k0 + u * (FW_LINE_THREADS / 32)) * ld];
+      *reinterpret_cast<V4 *>(&sm.whole[k0 + u * (FW_LINE_THREADS / 32)][line]) = x;
     }
-  };
-  auto compute = [&](const T (&av)[CK], T bl, int k0, int buf) {
-    typedef typename vec4_of<T>::type V4;
-    bstage[wave][buf][lane] = bl;
-    wave_lds_order();
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u) *reinterpret_cast<V4 *>(&sm.whole[k0 + u * (FW_LINE_THREADS / 32)][line]) = v[u];
+}
+
+// lane's line `line` of the whole operand with lines first .. first + NC - 1 of the other, chunks of CK k
+template <typename T, int NC>
+__device__ __forceinline__ void fw_lines(const FwLineLds<T> &sm, int line, int first, int chunks, int k_base, T (&curr)[NC],
+                                         int32_t (&par)[NC]) {
+  typedef typename vec4_of<T>::type V4;
+  constexpr int CK = FwLineLds<T>::CK;
+  const T inf = std::numeric_limits<T>::infinity();
+  int chunk[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) chunk[c] = -1;
+#pragma unroll 1
+  for (int ch = 0; ch < chunks; ++ch) {   // (the next chunk's operands read beside this one's work: 5.0 us where this takes 4.5)
+    T a[CK];
+#pragma unroll
+    for (int u = 0; u < CK; ++u) a[u] = sm.whole[ch * CK + u][line];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      T bv[CK];
+      T best = inf;
 #pragma unroll
-      for (int q = 0; q < CK / 4; ++q) {
-        const V4 v = *reinterpret_cast<const V4 *>(&bstage[wave][buf][c * CK + q * 4]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) bv[q * 4 + e] = v[e];
+      for (int q = 0; q < CK; q += 4) {
+        const V4 v = *reinterpret_cast<const V4 *>(&sm.other[first + c][ch * CK + q]);
+        best = hw_min<T>(hw_min<T>(best, a[q] + v[0]), a[q + 1] + v[1]);
+        best = hw_min<T>(hw_min<T>(best, a[q + 2] + v[2]), a[q + 3] + v[3]);
       }
-      T prod[CK], best = inf;
-#pragma unroll
-      for (int u = 0; u < CK; ++u) prod[u] = av[u] + bv[u];
-#pragma unroll
-      for (int u = 0; u < CK; u += 2) best = hw_min<T>(hw_min<T>(best, prod[u]), prod[u + 1]);
       const bool lower = best < curr[c];
-      if (__builtin_amdgcn_ballot_w64(lower)) {  // the same for the whole wave
-        int first = 0;
-#pragma unroll
-        for (int u = CK - 1; u >= 0; --u) first = prod[u] == best ? u : first;
-        T value = best;
-        // a minimum of zero: the hardware's may carry the other sign than the first product that equals it
-        if (__builtin_amdgcn_ballot_w64(lower && best == T(0))) {
-#pragma unroll
-          for (int u = CK - 1; u >= 0; --u) value = pick(prod[u] == best, prod[u], value);
-        }
-        curr[c] = lower ? value : curr[c];
-        par[c] = lower ? g.k_base + k0 + first : par[c];
-      }
+      curr[c] = pick(lower, best, curr[c]);
+      chunk[c] = lower ? ch : chunk[c];
     }
-    wave_lds_order();
-  };
-  // the next chunk's A values are requested before this chunk is worked on: a wave has eight chunks and a
-  // compute unit sixteen such waves, too few to hide a memory round trip per chunk behind each other
-  const int nfull = g.k / CK;
-  T av[2][CK], bl[2];
-  if (nfull > 0) load(av[0], bl[0], 0, std::true_type{});
-  for (int ch = 0; ch < nfull; ch += 2) {
-    if (ch + 1 < nfull) load(av[1], bl[1], (ch + 1) * CK, std::true_type{});
-    compute(av[0], bl[0], ch * CK, 0);
-    if (ch + 1 < nfull) {
-      if (ch + 2 < nfull) load(av[0], bl[0], (ch + 2) * CK, std::true_type{});
-      compute(av[1], bl[1], (ch + 1) * CK, 1);
-    }
-  }
-  if (nfull * CK < g.k) {
-    load(av[0], bl[0], nfull * CK, std::false_type{});
-    compute(av[0], bl[0], nfull * CK, 0);
   }
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    if (!live[c]) continue;
-    if (par[c] >= 0) {
-      static_cast<T *>(g.dist)[row + out[c] * g.ldc] = curr[c];
-      g.parent[row + out[c] * g.ldp] = par[c];
+    par[c] = -1;
+    if (__builtin_amdgcn_ballot_w64(chunk[c] >= 0) == 0) continue;
+    const int k0 = max(chunk[c], 0) * CK;
+    const T want = curr[c];
+    T value = want;
+    int k = 0;
+#pragma unroll
+    for (int q = CK - 4; q >= 0; q -= 4) {
+      const V4 v = *reinterpret_cast<const V4 *>(&sm.other[first + c][k0 + q]);
+#pragma unroll
+      for (int e = 3; e >= 0; --e) {
+        const T prod = sm.whole[k0 + q + e][line] + v[e];
+        const bool hit = prod == want;
+        k = hit ? q + e : k;
+        value = pick(hit, prod, value);   // (a minimum of zero: the hardware's may carry the other sign)
+      }
     }
-    if (g.out_t) static_cast<T *>(g.out_t)[out[c] + int64_t(row) * g.ld_out_t] = curr[c];
+    if (chunk[c] >= 0) {
+      curr[c] = value;
+      par[c] = k_base + k0 + k;
+    }
   }
+}
+
+// Block row and block column of the step whose diagonal block starts at k0 and has bb rows, in place: a workgroup reads the
+// whole lines that it will write -- sixteen columns of the block row, or sixteen rows of the block column -- into LDS
+// before it stores any of them, and the closed diagonal block is written by nobody, so no copies of the panels are needed
+// (they were a launch of 5 us).
+struct FwPanels {
+  int n, k0, bb;
+  void *dist; int64_t ld;
+  int32_t *parent; int64_t ldp;
+  const void *closed, *closed_t;   // the closed diagonal block and its transpose, FW_BLOCK x FW_BLOCK, +infinity beyond bb
+  void *col_t;                     // takes the updated block column with k contiguous, leading dimension FW_BLOCK
+  // the block being closed: columns and rows as its steps read them and the block as it was (fw_close_dist)
+  const void *hist;
+};
+
+// columns c0 .. c0 + 15 of the block row <- (closed block) x (block row)
+template <typename T> __device__ __forceinline__ void fw_row_panel(const FwPanels &p, int c0, FwLineLds<T> &sm) {
+  typedef typename vec4_of<T>::type V4;
+  typedef typename uvec4_of<T>::type U4;
+  const T inf = std::numeric_limits<T>::infinity();
+  const int tid = threadIdx.x;
+  T *const row0 = static_cast<T *>(p.dist) + p.k0;
+  V4 v;
+  {
+    const T *src = row0 + int64_t(min(c0 + (tid >> 5), p.n - 1)) * p.ld;
+    const int kk = (tid & 31) * 4;
+    if (p.bb == FW_BLOCK) {
+      v = *reinterpret_cast<const U4 *>(src + kk);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const T x = src[min(kk + e, p.bb - 1)];
+        v[e] = kk + e < p.bb ? x : inf;
+      }
+    }
+  }
+  fw_fetch_whole<T>(sm, static_cast<const T *>(p.closed), FW_BLOCK, FW_BLOCK);
+  *reinterpret_cast<V4 *>(&sm.other[tid >> 5][(tid & 31) * 4]) = v;
+  __syncthreads();
+  const int i = tid & 127, first = __builtin_amdgcn_readfirstlane(tid >> 7) * 4;
+  T curr[4];
+  int32_t par[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) curr[c] = sm.other[first + c][i];
+  fw_lines<T, 4>(sm, i, first, (p.bb + 15) / 16, p.k0, curr, par);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int col = c0 + first + c;
+    if (i >= p.bb || col >= p.n || par[c] < 0) continue;
+    row0[i + int64_t(col) * p.ld] = curr[c];
+    p.parent[p.k0 + i + int64_t(col) * p.ldp] = par[c];
+  }
+}
+
+// other[r][k] = src[r + k * ld], sixteen lines of which the first `lines` exist, +infinity from k = bb on
+template <typename T> __device__ __forceinline__ typename vec4_of<T>::type fw_fetch_across(const T *src, int64_t ld, int lines, int bb) {
+  typedef typename vec4_of<T>::type V4;
+  typedef typename uvec4_of<T>::type U4;
+  const T inf = std::numeric_limits<T>::infinity();
+  const int k = threadIdx.x >> 2, r = (threadIdx.x & 3) * 4;
+  src += int64_t(min(k, bb - 1)) * ld;
+  V4 v;
+  if (lines >= FwLineLds<T>::LINES) {
+    v = *reinterpret_cast<const U4 *>(src + r);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = src[min(r + e, lines - 1)];
+  }
+  return k < bb ? v : V4{inf, inf, inf, inf};
+}
+template <typename T> __device__ __forceinline__ void fw_put_across(FwLineLds<T> &sm, typename vec4_of<T>::type v) {
+  const int k = threadIdx.x >> 2, r = (threadIdx.x & 3) * 4;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) sm.other[r + e][k] = v[e];
+}
+
+// rows r0 .. r0 + 15 of the block column <- (block column) x (closed block), as the transposed product
+template <typename T> __device__ __forceinline__ void fw_col_panel(const FwPanels &p, int r0, FwLineLds<T> &sm) {
+  typedef typename vec4_of<T>::type V4;
+  typedef typename uvec4_of<T>::type U4;
+  T *const col0 = static_cast<T *>(p.dist) + int64_t(p.k0) * p.ld;
+  const V4 v = fw_fetch_across<T>(col0 + r0, p.ld, p.n - r0, p.bb);
+  fw_fetch_whole<T>(sm, static_cast<const T *>(p.closed_t), FW_BLOCK, FW_BLOCK);
+  fw_put_across<T>(sm, v);
+  __syncthreads();
+  const int tid = threadIdx.x, j = tid & 127, first = __builtin_amdgcn_readfirstlane(tid >> 7) * 4;
+  T curr[4];
+  int32_t par[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) curr[c] = sm.other[first + c][j];
+  fw_lines<T, 4>(sm, j, first, (p.bb + 15) / 16, p.k0, curr, par);
+  // The results go out sixteen rows of a column at a time (64 bytes of floats), through LDS; a lane per column would store
+  // every element by itself.
+  int32_t *const par_lds = reinterpret_cast<int32_t *>(&sm.whole[0][0]);   // [16][STRIDE], once everybody has done with it
+  constexpr int STRIDE = FwLineLds<T>::STRIDE;
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    sm.other[first + c][j] = curr[c];
+    par_lds[(first + c) * STRIDE + j] = par[c];
+    if (j < p.bb && r0 + first + c < p.n) static_cast<T *>(p.col_t)[j + int64_t(r0 + first + c) * FW_BLOCK] = curr[c];
+  }
+  __syncthreads();
+  const int jj = tid >> 2, r = (tid & 3) * 4;
+  if (jj >= p.bb) return;
+  T *const d = col0 + r0 + r + int64_t(jj) * p.ld;
+  int32_t *const q = p.parent + r0 + r + int64_t(p.k0 + jj) * p.ldp;
+  typedef int32_t I4 __attribute__((ext_vector_type(4), aligned(4)));
+  V4 value;
+  I4 from;
+  bool all = r0 + r + 4 <= p.n;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    value[e] = sm.other[r + e][jj];
+    from[e] = par_lds[(r + e) * STRIDE + jj];
+    all = all && from[e] >= 0;
+  }
+  if (all) {
+    *reinterpret_cast<U4 *>(d) = value;
+    *reinterpret_cast<I4 *>(q) = from;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (r0 + r + e >= p.n || from[e] < 0) continue;
+      d[e] = value[e];
+      q[e] = from[e];
+    }
+  }
+}
+
+// The predecessors of columns c0 .. c0 + 15 of a diagonal block whose distances fw_close_dist has closed: the product of the
+// recorded columns with the recorded rows, started from the block as it was.  Only predecessors are written: the distances
+// are those already there.
+template <typename T> __device__ __forceinline__ void fw_parents(const FwPanels &p, int c0, FwLineLds<T> &sm) {
+  const T *hist_col = static_cast<const T *>(p.hist), *hist_row = hist_col + FW_BLOCK * FW_BLOCK, *init = hist_row + FW_BLOCK * FW_BLOCK;
+  const int tid = threadIdx.x, i = tid & 127, first = __builtin_amdgcn_readfirstlane(tid >> 7) * 4;
+  T curr[4];
+  int32_t par[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) curr[c] = init[i + (c0 + first + c) * FW_BLOCK];
+  const typename vec4_of<T>::type v = fw_fetch_across<T>(hist_row + c0, FW_BLOCK, FwLineLds<T>::LINES, p.bb);
+  fw_fetch_whole<T>(sm, hist_col, FW_BLOCK, FW_BLOCK);   // (rows of k beyond the last chunk hold anything and are not read)
+  fw_put_across<T>(sm, v);
+  __syncthreads();
+  fw_lines<T, 4>(sm, i, first, (p.bb + 15) / 16, p.k0, curr, par);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int col = c0 + first + c;
+    if (i < p.bb && col < p.bb && par[c] >= 0) p.parent[p.k0 + i + int64_t(p.k0 + col) * p.ldp] = par[c];
+  }
+}
+
+// One launch: the predecessors of the diagonal block (closed by fw_close_dist in a launch before), the block row and the block
+// column, which are independent of each other.
+template <typename T> __global__ void __launch_bounds__(FW_LINE_THREADS) fw_panels_kernel(FwPanels p) {
+  __shared__ FwLineLds<T> sm;
+  const int lines = FwLineLds<T>::LINES, own = (p.bb + lines - 1) / lines, panel = (p.n + lines - 1) / lines - own;
+  int b = blockIdx.x;
+  if (b < own) {
+    fw_parents<T>(p, b * lines, sm);
+    return;
+  }
+  b -= own;
+  const bool row = b < panel;
+  b = (row ? b : b - panel) * lines;
+  if (b >= p.k0) b += p.bb;   // (the diagonal block's own lines are left out; where it is ragged none come after it)
+  if (row) fw_row_panel<T>(p, b, sm);
+  else fw_col_panel<T>(p, b, sm);
+}
+// workgroups: each fetches 64 KB (float) or 128 KB before it computes anything, so that one to a compute unit is worth having
+// (n = 2000, 242 of them: 10 us; with sixteen more, which had nothing to do, two CUs had two and the launch took 13)
+inline unsigned fw_panel_groups(int n, int bb, bool panels) {
+  constexpr int lines = FwLineLds<float>::LINES;
+  const int own = (bb + lines - 1) / lines;
+  return own + (panels ? 2 * ((n + lines - 1) / lines - own) : 0);
+}
+
+// The next step's diagonal block (a0, abb rows) <- (its rows of the block column) x (its columns of the block row): a
+// workgroup takes four of its columns.
+template <typename T> __global__ void __launch_bounds__(FW_LINE_THREADS) fw_ahead_kernel(FwPanels p, int a0, int abb) {
+  __shared__ FwLineLds<T> sm;
+  const int tid = threadIdx.x, i = tid & 127, row = min(i, abb - 1), first = __builtin_amdgcn_readfirstlane(tid >> 7);
+  const int col = blockIdx.x * 4 + first, col_in = min(col, abb - 1);
+  T *const block = static_cast<T *>(p.dist) + a0 + int64_t(a0) * p.ld;
+  T curr[1] = {block[row + int64_t(col_in) * p.ld]};
+  int32_t par[1];
+  const T b = (static_cast<const T *>(p.dist) + p.k0 + int64_t(a0 + col_in) * p.ld)[i];
+  fw_fetch_whole<T>(sm, static_cast<const T *>(p.dist) + a0 + int64_t(p.k0) * p.ld, p.ld, abb);
+  sm.other[first][i] = b;
+  __syncthreads();
+  fw_lines<T, 1>(sm, i, first, FW_BLOCK / 16, p.k0, curr, par);
+  if (i >= abb || col >= abb || par[0] < 0) return;
+  block[i + int64_t(col) * p.ld] = curr[0];
+  p.parent[a0 + i + int64_t(a0 + col) * p.ldp] = par[0];
 }
 
 // The improved elements of a tile, queued in LDS as (code = row in the tile | column << ROW_BITS | chunk <<
@@ -247,9 +420,9 @@ template <typename T> __device__ __forceinline__ void fwgemm_rowcols_block(const
 // element where one lane per element would touch 64.  A group takes UN elements per turn and requests all their
 // operands before it looks at any: a turn costs one round trip to memory, and a tile has few turns.
 template <int G> __device__ __forceinline__ int group_min(int v) {
-  // minimum over the G (4 or 8) adjacent lanes of a group, by data-parallel moves inside the row of 16 lanes
+  // minimum over the G (2, 4 or 8) adjacent lanes of a group, by data-parallel moves inside the row of 16 lanes
   v = min(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, true));   // lanes 1 0 3 2 of each four
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, true));   // lanes 2 3 0 1 of each four
+  if constexpr (G >= 4) v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, true));   // lanes 2 3 0 1 of each four
   if constexpr (G == 8) v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, true));  // each eight mirrored
   return v;
 }
@@ -259,7 +432,7 @@ __device__ __forceinline__ void lookup_queue(const FwArgs &g, const uint32_t *q_
   typedef typename vec4_of<T>::type V4;
   typedef typename uvec4_of<T>::type U4;
   constexpr int G = CHUNK / 4, GROUPS = THREADS / G;
-  static_assert(G == 4 || G == 8, "lanes per element");
+  static_assert(G == 2 || G == 4 || G == 8, "lanes per element");
   const T *A = static_cast<const T *>(g.A), *B = static_cast<const T *>(g.B), *At = static_cast<const T *>(g.At);
   T *dist = static_cast<T *>(g.dist);
   const int sub = tid % G;
@@ -309,6 +482,11 @@ __device__ __forceinline__ void lookup_queue(const FwArgs &g, const uint32_t *q_
   }
 }
 
+// CHUNK: the k-values whose products the lookup of an improved element reads.  Sixteen (BK) cost three instructions per output
+// and chunk; eight cost twice that and halve the bytes a lookup reads and, with two lanes to an element instead of four,
+// the turns: a block step's product (k = 128, float, two waves per SIMD) at n = 2000 71 -> 57 us where nearly every element
+// improves, 42 either way where a tenth does.  With four waves per SIMD, and in double, the registers are not there: 3014 us a
+// job on sixteen, 4712 on eight at n = 3000; double, n = 2000, 1666 and 1891.
 // NT threads as 16 x TY; each owns TM x TN outputs in groups of four rows / columns that
 // lie 64 / 4 TY apart, so a workgroup covers (16 TM) x (TY TN).
 // GUARD = false: at least one tile in either direction and four k; any alignment.  A tile at a far edge starts
@@ -324,7 +502,7 @@ template <typename T, int NT, int TM, int TN, int BK> struct FwTileLds {
   alignas(4 * sizeof(T)) T as[2][BK][BM + PAD], bs[2][BK][BN + PAD];   // (accessed four elements at a time)
   int wave_count[NT / 64][TN];
 };
-template <typename T, int NT, int TM, int TN, int WPE, int BK, bool GUARD, bool HAS_AT>
+template <typename T, int NT, int TM, int TN, int WPE, int BK, int CHUNK, bool GUARD, bool HAS_AT>
 __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int block_x, const int block_y, FwTileLds<T, NT, TM, TN, BK> &sm) {
   typedef typename vec4_of<T>::type V4;
   typedef typename uvec4_of<T>::type U4;
@@ -470,16 +648,18 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
     // The minima run on through the chunk; an element that is lower after it than before it improved in it.  (Each
     // operand fragment serves a thread's whole 8 x 4 outputs: with blocks of 4 x 4, each with chunk minima of its own, the
     // loop was bound by LDS reads.)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int i = 0; i < TM; ++i) seen[i][j] = acc[i][j];
     Frag f[NF];
     if constexpr (NF == 2) load_frag(f[0], cur, 0);
 #pragma unroll
     for (int s = 0; s < BK / U; ++s) {
       if constexpr (NF == 1) load_frag(f[0], cur, U * s);
       else if (s + 1 < BK / U) load_frag(f[(s + 1) % NF], cur, U * (s + 1));
+      if (U * s % CHUNK == 0) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int i = 0; i < TM; ++i) seen[i][j] = acc[i][j];
+      }
       __builtin_amdgcn_sched_barrier(0);
       const Frag &x = f[s % NF];
 #pragma unroll
@@ -500,11 +680,13 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
           if constexpr (WPE > 2) __builtin_amdgcn_sched_barrier(0);
         }
       __builtin_amdgcn_sched_barrier(0);
+      if (U * (s + 1) % CHUNK == 0) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int i = 0; i < TM; ++i) record(i, j, acc[i][j] < seen[i][j], t * (BK / CHUNK) + U * s / CHUNK);
+      }
     }
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int i = 0; i < TM; ++i) record(i, j, acc[i][j] < seen[i][j], t);
     if (t + 1 < tiles) stage(cur ^ 1);
     __syncthreads();
   }
@@ -581,7 +763,7 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
           base += col_count[j];
         }
         __syncthreads();
-        lookup_queue<T, NT, BK, HAS_AT, 7, 7, (sizeof(T) == 8 || WPE > 2) ? 4 : 8>(g, q_code, q_want, total, tid, m0, n0);
+        lookup_queue<T, NT, CHUNK, HAS_AT, 7, 7, (sizeof(T) == 8 || WPE > 2) ? 4 : 8>(g, q_code, q_want, total, tid, m0, n0);
         __syncthreads();  // the queue is free again
       }
       j0 = j1;
@@ -599,7 +781,7 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
       if constexpr (GUARD) {
         if (r >= g.m || c >= g.n) continue;
       }
-      const int k0 = ch * BK;
+      const int k0 = ch * CHUNK;
       const T *ap = HAS_AT ? static_cast<const T *>(g.At) + k0 + int64_t(r) * g.ldat : A + r + int64_t(k0) * g.lda;
       const int64_t a_step = HAS_AT ? 1 : g.lda;
       const T *bp = B + k0 + int64_t(c) * g.ldb;
@@ -607,7 +789,7 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
       T value = want;
       int first = 0;
 #pragma unroll 4
-      for (int kk = BK - 1; kk >= 0; --kk) {
+      for (int kk = CHUNK - 1; kk >= 0; --kk) {
         bool in = true;
         if constexpr (GUARD) in = k0 + kk < g.k;
         const T prod = in ? ap[int64_t(kk) * a_step] + bp[kk] : inf;
@@ -620,8 +802,6 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
     }
   }
 }
-
-constexpr int FW_BLOCK = 128;  // vertices per block step of the blocked Floyd-Warshall
 
 // ---- closing a diagonal block in two parts: distances first, predecessors afterwards
 //
@@ -879,8 +1059,11 @@ __device__ __forceinline__ void fw_load_patch(T (&cur)[FwPatch<NT>::PN][FwPatch<
       }
   }
 }
+// closed, closed_t (if given): the whole patch, padding included, and its transpose, leading dimension FW_BLOCK
 template <typename T, int NT>
-__device__ __forceinline__ void fw_store_patch(const T (&cur)[FwPatch<NT>::PN][FwPatch<NT>::PM], T *d, int64_t ld, int bb) {
+__device__ __forceinline__ void fw_store_patch(const T (&cur)[FwPatch<NT>::PN][FwPatch<NT>::PM], T *d, int64_t ld, int bb, T *closed,
+                                               T *closed_t) {
+  typedef typename vec4_of<T>::type V4;
   constexpr int PM = FwPatch<NT>::PM, PN = FwPatch<NT>::PN, TI = FwPatch<NT>::TI;
   const int ti = threadIdx.x % TI, tj = threadIdx.x / TI;
 #pragma unroll
@@ -890,6 +1073,21 @@ __device__ __forceinline__ void fw_store_patch(const T (&cur)[FwPatch<NT>::PN][F
       const int i = PM * ti + a, j = PN * tj + b;
       if (i < bb && j < bb) d[i + int64_t(j) * ld] = cur[b][a];
     }
+  if (!closed) return;
+#pragma unroll
+  for (int b = 0; b < PN; ++b)
+#pragma unroll
+    for (int a = 0; a < PM; a += 4) {
+      const V4 v = {cur[b][a], cur[b][a + 1], cur[b][a + 2], cur[b][a + 3]};
+      *reinterpret_cast<V4 *>(&closed[PM * ti + a + (PN * tj + b) * FW_BLOCK]) = v;
+    }
+#pragma unroll
+  for (int a = 0; a < PM; ++a)
+#pragma unroll
+    for (int b = 0; b < PN; b += 4) {
+      const V4 v = {cur[b][a], cur[b + 1][a], cur[b + 2][a], cur[b + 3][a]};
+      *reinterpret_cast<V4 *>(&closed_t[PN * tj + b + (PM * ti + a) * FW_BLOCK]) = v;
+    }
 }
 
 // A block that holds a -0, by a function of its own that fetches the block again: for patches that leave no registers (as
@@ -897,15 +1095,17 @@ __device__ __forceinline__ void fw_store_patch(const T (&cur)[FwPatch<NT>::PN][F
 template <typename T, int NT>
 __device__ __attribute__((noinline)) void fw_close_dist_exact(__attribute__((address_space(1))) T *d, int64_t ld, int bb,
                                                               __attribute__((address_space(1))) T *hist,
+                                                              __attribute__((address_space(1))) T *closed,
+                                                              __attribute__((address_space(1))) T *closed_t,
                                                               __attribute__((address_space(3))) FwCloseLds<T> *sm) {
   T cur[FwPatch<NT>::PN][FwPatch<NT>::PM];
   fw_load_patch<T, NT>(cur, (const T *)d, ld, bb);
   fw_close_strips<T, NT, true>(cur, bb, (T *)hist, *(FwCloseLds<T> *)sm);
-  fw_store_patch<T, NT>(cur, (T *)d, ld, bb);
+  fw_store_patch<T, NT>(cur, (T *)d, ld, bb, (T *)closed, (T *)closed_t);
 }
 
 template <typename T, int NT>
-__device__ __forceinline__ void fw_close_dist(T *d, int64_t ld, int bb, T *hist, FwCloseLds<T> &sm) {
+__device__ __forceinline__ void fw_close_dist(T *d, int64_t ld, int bb, T *hist, T *closed, T *closed_t, FwCloseLds<T> &sm) {
   typedef typename vec4_of<T>::type V4;
   constexpr int PM = FwPatch<NT>::PM, PN = FwPatch<NT>::PN, TI = FwPatch<NT>::TI;
   const int ti = threadIdx.x % TI, tj = threadIdx.x / TI;
@@ -929,6 +1129,7 @@ __device__ __forceinline__ void fw_close_dist(T *d, int64_t ld, int bb, T *hist,
   if (__syncthreads_or(negative_zero)) {
     if constexpr (PM * PN * sizeof(T) > 256) {
       fw_close_dist_exact<T, NT>((__attribute__((address_space(1))) T *)d, ld, bb, (__attribute__((address_space(1))) T *)hist,
+                                 (__attribute__((address_space(1))) T *)closed, (__attribute__((address_space(1))) T *)closed_t,
                                  (__attribute__((address_space(3))) FwCloseLds<T> *)&sm);
       return;
     } else {
@@ -937,67 +1138,7 @@ __device__ __forceinline__ void fw_close_dist(T *d, int64_t ld, int bb, T *hist,
   } else {
     fw_close_strips<T, NT, false>(cur, bb, hist, sm);
   }
-  fw_store_patch<T, NT>(cur, d, ld, bb);
-}
-
-// The predecessors of a diagonal block whose distances fw_close_dist has closed: workgroup b of 64 (256 threads)
-// takes rows 64 (b & 1) .. + 63 and columns 4 (b >> 1) .. + 3, one element per thread, and runs the literal scan
-// over the recorded columns and rows.  Only predecessors are written: the distances are those already there.
-template <typename T>
-__device__ __forceinline__ void fw_parents_block(const T *hist, int32_t *parent, int64_t ldp, int bb, int k_base, int b) {
-  const int row = (b & 1) * 64 + (threadIdx.x & 63);
-  const int col = __builtin_amdgcn_readfirstlane((b >> 1) * 4 + (threadIdx.x >> 6));
-  if (row >= bb || col >= bb) return;
-  const T *hist_row = hist + FW_BLOCK * FW_BLOCK;
-  const T *hc = hist + row, *hr = hist_row + col;
-  T curr = hist[2 * FW_BLOCK * FW_BLOCK + row + col * FW_BLOCK];
-  int32_t p = -1;
-  auto scan = [&](const T prod, int k) {
-    const bool lower = prod < curr;
-    curr = pick(lower, prod, curr);
-    p = lower ? k : p;
-  };
-  int k = 0;
-  for (; k + 16 <= bb; k += 16) {  // sixteen k at a time, their operands requested together
-    T cv[16], rv[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      cv[u] = hc[(k + u) * FW_BLOCK];
-      rv[u] = hr[(k + u) * FW_BLOCK];
-    }
-#pragma unroll
-    for (int u = 0; u < 16; ++u) scan(cv[u] + rv[u], k + u);
-  }
-  for (; k < bb; ++k) scan(hc[k * FW_BLOCK] + hr[k * FW_BLOCK], k);
-  if (p >= 0) parent[row + int64_t(col) * ldp] = k_base + p;
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) fw_parents_kernel(const T *hist, int32_t *parent, int64_t ldp, int bb, int k_base) {
-  fw_parents_block<T>(hist, parent, ldp, bb, k_base, blockIdx.x);
-}
-constexpr int FW_PARENT_BLOCKS = (FW_BLOCK / 64) * (FW_BLOCK / 4);
-
-// two independent products in one launch (the block row and the block column of a blocked
-// Floyd-Warshall step, each too small to fill the chip): after the first FW_PARENT_BLOCKS workgroups, which
-// find the predecessors of the diagonal block at k_base (closed by fw_close_dist in a launch before), the next
-// blocks0 workgroups work on g0, the others on g1
-template <typename T>
-__global__ void __launch_bounds__(256) fwgemm_pair_kernel(FwArgs g0, FwArgs g1, int blocks0, const T *hist, int32_t *hist_parent,
-                                                          int64_t ldp, int hist_bb, int k_base) {
-  int b = blockIdx.x;
-  if (b < FW_PARENT_BLOCKS) {
-    fw_parents_block<T>(hist, hist_parent, ldp, hist_bb, k_base, b);
-    return;
-  }
-  b -= FW_PARENT_BLOCKS;
-  if (b < blocks0) {
-    const int gx = (g0.m + 63) / 64;
-    fwgemm_rowcols_block<T>(g0, b % gx, b / gx);
-  } else {
-    const int gx = (g1.m + 63) / 64;
-    fwgemm_rowcols_block<T>(g1, (b - blocks0) % gx, (b - blocks0) / gx);
-  }
+  fw_store_patch<T, NT>(cur, d, ld, bb, closed, closed_t);
 }
 
 // The tile kernel.  Grid (tiles along m, tiles along n); with g.ahead_bb > 0 the grid has one more row,
@@ -1006,7 +1147,7 @@ __global__ void __launch_bounds__(256) fwgemm_pair_kernel(FwArgs g0, FwArgs g1, 
 // 128 dependent steps take about as long as the whole product and nothing else of the next block step can
 // start before them; here they cost one of the launch's 512 places.  Only where whole tiles make up a
 // diagonal block (all shapes the host launches, of either element type).
-template <typename T, int NT, int TM, int TN, int WPE, int BK, bool GUARD, bool HAS_AT>
+template <typename T, int NT, int TM, int TN, int WPE, int BK, int CHUNK, bool GUARD, bool HAS_AT>
 __global__ void __launch_bounds__(NT, WPE) fwgemm_tile_kernel(FwArgs g) {
   typedef FwTileLds<T, NT, TM, TN, BK> TileLds;
   constexpr int BM = TileLds::BM, BN = TileLds::BN;
@@ -1030,7 +1171,7 @@ __global__ void __launch_bounds__(NT, WPE) fwgemm_tile_kernel(FwArgs g) {
         const int closer = g.skip_r1 > g.skip_r0 ? g.skip_r0 / BM : 0;
         if (bx == closer)
           fw_close_dist<T, NT>(static_cast<T *>(g.dist) + g.ahead0 + int64_t(g.ahead0) * g.ldc, g.ldc, g.ahead_bb,
-                               static_cast<T *>(g.hist), sm.close);
+                               static_cast<T *>(g.hist), static_cast<T *>(g.closed), static_cast<T *>(g.closed_t), sm.close);
         return;
       }
       by -= 1;
@@ -1038,7 +1179,7 @@ __global__ void __launch_bounds__(NT, WPE) fwgemm_tile_kernel(FwArgs g) {
       if (r0 >= 0 && r0 < FW_BLOCK && c0 >= 0 && c0 < FW_BLOCK) return;
     }
   }
-  fwgemm_tile_body<T, NT, TM, TN, WPE, BK, GUARD, HAS_AT>(g, bx, by, sm.tile);
+  fwgemm_tile_body<T, NT, TM, TN, WPE, BK, CHUNK, GUARD, HAS_AT>(g, bx, by, sm.tile);
 }
 
 // ---- the predecessor-tracking product on the hand-scheduled direct-to-LDS tile (direct_tile.h, direct_asm.h)
@@ -1222,13 +1363,13 @@ bool fwgemm_direct_ok(const FwArgs &g) {
   if (g.m <= 0 || g.n <= 0 || g.k < 2 * FWD_CHUNK || g.m % 128 || g.n % 256 || g.k % FWD_CHUNK || g.k / FWD_CHUNK >= 0xffff) return false;
   if (!g.At || !al(g.A) || !al(g.B) || !al(g.dist) || !al(g.At)) return false;
   if (g.lda % 4 || g.ldb % 4 || g.ldc % 4 || g.ldat % 4) return false;
-  if (g.skip_r1 > g.skip_r0 || g.skip_c1 > g.skip_c0 || g.ahead_bb > 0 || g.out_t) return false;
+  if (g.skip_r1 > g.skip_r0 || g.skip_c1 > g.skip_c0 || g.ahead_bb > 0) return false;
   // 32-bit byte offsets inside a tile
   if (int64_t(g.ldb) * 256 * 4 >= (int64_t(1) << 31) || int64_t(g.lda) * 16 * 4 >= (int64_t(1) << 31)) return false;
   return int64_t(g.m / 128) * (g.n / 256) <= 0x7fffffff;
 }
 
-template <typename T, int NT, int TM, int TN, int WPE, int BK>
+template <typename T, int NT, int TM, int TN, int WPE, int BK, int STEP_CHUNK = BK>
 hipError_t launch_tile(const FwArgs &g, hipStream_t stream) {
   constexpr int BM = 16 * TM, BN = NT / 16 * TN;
   // (chunks of BK k-values are numbered in 15 bits)
@@ -1237,11 +1378,12 @@ hipError_t launch_tile(const FwArgs &g, hipStream_t stream) {
   dim3 grid((g.m + BM - 1) / BM, (g.n + BN - 1) / BN + (g.ahead_bb > 0 ? 1 : 0));
   // (GUARD form: fetches element by element, with registers to spare)
   if (g.At) {
-    if (whole) launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, WPE, BK, false, true>), grid, dim3(NT), 0, stream, g);
-    else launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, 2, BK, true, true>), grid, dim3(NT), 0, stream, g);
+    if (whole && STEP_CHUNK != BK && g.k <= FW_BLOCK) launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, WPE, BK, STEP_CHUNK, false, true>), grid, dim3(NT), 0, stream, g);
+    else if (whole) launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, WPE, BK, BK, false, true>), grid, dim3(NT), 0, stream, g);
+    else launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, 2, BK, BK, true, true>), grid, dim3(NT), 0, stream, g);
   } else {
-    if (whole) launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, WPE, BK, false, false>), grid, dim3(NT), 0, stream, g);
-    else launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, 2, BK, true, false>), grid, dim3(NT), 0, stream, g);
+    if (whole) launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, WPE, BK, BK, false, false>), grid, dim3(NT), 0, stream, g);
+    else launch_kernel((fwgemm_tile_kernel<T, NT, TM, TN, 2, BK, BK, true, false>), grid, dim3(NT), 0, stream, g);
   }
   return take_launch_status();
 }
@@ -1308,9 +1450,9 @@ __global__ void __launch_bounds__(256) snapshot_pair_kernel(const T *src0, T *w0
 // A diagonal block's distances closed by a launch of its own: a job's first block, and every block of a job too small for
 // the tile kernel.  Its predecessors follow with those of the other blocks.
 template <typename T>
-__global__ void __launch_bounds__(512) fw_close_kernel(T *d, int64_t ld, int bb, T *hist) {
+__global__ void __launch_bounds__(512) fw_close_kernel(T *d, int64_t ld, int bb, T *hist, T *closed, T *closed_t) {
   __shared__ FwCloseLds<T> sm;
-  fw_close_dist<T, 512>(d, ld, bb, hist, sm);
+  fw_close_dist<T, 512>(d, ld, bb, hist, closed, closed_t, sm);
 }
 
 template <typename T> hipError_t launch_naive(const FwArgs &g, hipStream_t stream) {
@@ -1348,7 +1490,7 @@ struct FwExtra {
   // blocked Floyd-Warshall: let the launch also close the diagonal block that starts at ahead0 (ahead_bb rows),
   // which the product then leaves alone.  Only the tile kernel can; *closed_ahead says whether this launch did.
   int ahead0 = 0, ahead_bb = 0;
-  void *hist = nullptr;
+  void *hist = nullptr, *closed = nullptr, *closed_t = nullptr;
   bool *closed_ahead = nullptr;
 };
 int fwgemm_run(int dtype, int m, int n, int k, const void *A, int64_t lda, const void *B, int64_t ldb, void *dist,
@@ -1356,7 +1498,7 @@ int fwgemm_run(int dtype, int m, int n, int k, const void *A, int64_t lda, const
   const int st = check(dtype, m, n, k, A, lda, B, ldb, dist, ldc, parent, ldp, kernel);
   if (st != CUASR_AMD_SUCCESS || m == 0 || n == 0 || k == 0) return st;
   FwArgs g{m, n, k, A, lda, B, ldb, dist, ldc, parent, ldp, x.At, x.ldat, x.k_base,
-           x.skip_r0, x.skip_r1, x.skip_c0, x.skip_c1, nullptr, 0, 0, 0, nullptr};
+           x.skip_r0, x.skip_r1, x.skip_c0, x.skip_c1, 0, 0, nullptr, nullptr, nullptr};
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool naive = kernel == CUASR_AMD_KERNEL_NAIVE ||
                      (kernel == CUASR_AMD_KERNEL_AUTO && fwgemm_one_thread_each(dtype == CUASR_AMD_F64, x.At != nullptr, m, n, k));
@@ -1364,6 +1506,8 @@ int fwgemm_run(int dtype, int m, int n, int k, const void *A, int64_t lda, const
     g.ahead0 = x.ahead0;
     g.ahead_bb = x.ahead_bb;
     g.hist = x.hist;
+    g.closed = x.closed;
+    g.closed_t = x.closed_t;
   }
   if (x.closed_ahead) *x.closed_ahead = g.ahead_bb > 0;
   hipError_t e;
@@ -1381,7 +1525,7 @@ int fwgemm_run(int dtype, int m, int n, int k, const void *A, int64_t lda, const
   const bool one_each = (tm - skip_m) * (tn - skip_n) <= 256;
   const bool half_tile = skip_m + skip_n == 0 && fwgemm_f64_half_tile(g.At != nullptr, g.m, (int64_t(g.m) + 63) / 64 * tn);
   if (dtype == CUASR_AMD_F32) {
-    e = naive ? launch_naive<float>(g, s) : one_each ? launch_tile<float, 512, 8, 4, 2, 16>(g, s) : launch_tile<float, 512, 8, 4, 4, 16>(g, s);
+    e = naive ? launch_naive<float>(g, s) : one_each ? launch_tile<float, 512, 8, 4, 2, 16, 8>(g, s) : launch_tile<float, 512, 8, 4, 4, 16>(g, s);
   }
   else {
     e = naive ? launch_naive<double>(g, s) : one_each && !half_tile ? launch_tile<double, 512, 8, 4, 2, 16>(g, s) : launch_tile<double, 256, 4, 8, 2, 16>(g, s);
@@ -1459,31 +1603,50 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
   const size_t es = f64 ? 8 : 4;
   hipStream_t s = static_cast<hipStream_t>(stream);
   char *D = static_cast<char *>(dist);
-  char *R = static_cast<char *>(workspace);             // block row,    FW_BLOCK x n,  leading dimension FW_BLOCK
-  char *C = R + es * FW_BLOCK * size_t(nn);             // block column, n x FW_BLOCK,  leading dimension nn
+  char *R = static_cast<char *>(workspace);             // FW_BLOCK x nn elements each: R, C, Ct
+  char *C = R + es * FW_BLOCK * size_t(nn);
   char *Ct = C + es * FW_BLOCK * size_t(nn);            // updated block column with k contiguous, leading dimension FW_BLOCK
   char *H = Ct + es * FW_BLOCK * size_t(nn);            // columns, rows and first state of the diagonal block being closed
+  // Block row and block column share one launch that works in place and reads the closed diagonal block and its transpose
+  // from C and R; from n = 16257 on each of the two products fills the chip on the tiled kernel, from copies of the panels in R
+  // (leading dimension FW_BLOCK) and C (leading dimension nn).
+  const bool paired = panels == CUASR_AMD_PANELS_AUTO ? (int64_t(n) + 127) / 128 < 128 : panels == CUASR_AMD_PANELS_PAIRED;
+  char *closed_copy = paired && n > FW_BLOCK ? C : nullptr, *closed_copy_t = paired && n > FW_BLOCK ? R : nullptr;
   // With tiles a step's launch also closes the next block, after a launch that updates it; without, a closure alone on
-  // the chip takes half a step.  f32, n = 1000 (64 tiles): 635 us a job with tiles, 595 without; from 81 tiles on the
-  // tiles win (f64 from 49: n = 1001 984 against 1130).
-  const bool naive = n <= (f64 ? 768 : 1024);
+  // the chip takes most of a step.  us a job with tiles / without: f32 n = 800 430 / 389, 896 460 / 439, 960 482 / 495,
+  // 1024 500 / 549; f64 700 689 / 638, 768 719 / 706 (n = 1001 984 / 1130 when the panels were copied first).
+  const bool naive = n <= (f64 ? 768 : 928);
   // this step's diagonal block had its distances closed during the step before, beside that step's big product
   // (its predecessors are always still to be found, from what the closure recorded in H)
   bool closed = false;
   for (int k0 = 0; k0 < n; k0 += FW_BLOCK) {
     const int bb = n - k0 < FW_BLOCK ? n - k0 : FW_BLOCK;
     char *Dkk = D + es * (size_t(k0) + size_t(k0) * size_t(ld));
-    int32_t *Pkk = parent + size_t(k0) + size_t(k0) * size_t(ldp);
     // 1. the diagonal block, closed by one workgroup
     if (!closed) {
-      if (f64) launch_kernel(fw_close_kernel<double>, dim3(1), dim3(512), 0, s, reinterpret_cast<double *>(Dkk), ld, bb, reinterpret_cast<double *>(H));
-      else launch_kernel(fw_close_kernel<float>, dim3(1), dim3(512), 0, s, reinterpret_cast<float *>(Dkk), ld, bb, reinterpret_cast<float *>(H));
+      if (f64) launch_kernel(fw_close_kernel<double>, dim3(1), dim3(512), 0, s, reinterpret_cast<double *>(Dkk), ld, bb, reinterpret_cast<double *>(H),
+                             reinterpret_cast<double *>(closed_copy), reinterpret_cast<double *>(closed_copy_t));
+      else launch_kernel(fw_close_kernel<float>, dim3(1), dim3(512), 0, s, reinterpret_cast<float *>(Dkk), ld, bb, reinterpret_cast<float *>(H),
+                         reinterpret_cast<float *>(closed_copy), reinterpret_cast<float *>(closed_copy_t));
       if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
     }
-    // 2. snapshots of block row and block column (the products below read these, so that no
-    //    workgroup sees another's updates)
     char *Drow = D + es * size_t(k0), *Dcol = D + es * size_t(k0) * size_t(ld);
-    {
+    hipError_t e = hipSuccess;
+    // 2. block row <- (closed diagonal block) x (block row); block column <- (block column) x (closed
+    //    diagonal block).  Neither touches the diagonal block itself (it is closed), so the two are
+    //    independent.  The column product also writes the updated column's k-contiguous image for step 3 (the rows
+    //    of the diagonal block, which it skips, are not read there).
+    FwExtra x;
+    x.k_base = k0;
+    int r;
+    const FwPanels panel{n, k0, bb, dist, ld, parent, ldp, closed_copy, closed_copy_t, Ct, H};
+    if (paired) {
+      const dim3 grid(fw_panel_groups(n, bb, true));
+      if (f64) launch_kernel(fw_panels_kernel<double>, grid, dim3(FW_LINE_THREADS), 0, s, panel);
+      else launch_kernel(fw_panels_kernel<float>, grid, dim3(FW_LINE_THREADS), 0, s, panel);
+      if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
+    } else {
+      // copies of block row and block column (the products read these, so that no workgroup sees another's updates)
       const int sb0 = ((bb + 63) / 64) * ((n + 63) / 64), sb1 = ((n + 63) / 64) * ((bb + 63) / 64);
       if (f64)
         launch_kernel(snapshot_pair_kernel<double>, dim3(sb0 + sb1), dim3(256), 0, s, reinterpret_cast<const double *>(Drow),
@@ -1494,36 +1657,8 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
                            reinterpret_cast<float *>(R), int64_t(FW_BLOCK), bb, n, reinterpret_cast<const float *>(Dcol),
                            reinterpret_cast<float *>(C), nn, n, bb, ld, sb0);
       if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
-    }
-    hipError_t e = hipSuccess;
-    // 3. block row <- (closed diagonal block) x (block row); block column <- (block column) x (closed
-    //    diagonal block).  Neither touches the diagonal block itself (it is closed), so the two are
-    //    independent, and while each is too small to fill the chip they share one launch.
-    FwExtra x;
-    x.k_base = k0;
-    int r;
-    // below 128 tiles per panel product the two share one launch of the one-thread-per-element kernel;
-    // from n = 16257 on each fills the chip on the tiled kernel
-    const bool paired = panels == CUASR_AMD_PANELS_AUTO ? (int64_t(n) + 127) / 128 < 128 : panels == CUASR_AMD_PANELS_PAIRED;
-    if (paired) {
-      const FwArgs g0{bb, n, bb, R + es * size_t(k0) * FW_BLOCK, FW_BLOCK, R, FW_BLOCK, Drow, ld, parent + k0, ldp,
-                      nullptr, 0, k0, 0, 0, k0, k0 + bb, nullptr, 0, 0, 0};
-      // (the column product also writes the updated column's k-contiguous image for step 4; the rows
-      // of the diagonal block, which it skips, are not read there)
-      const FwArgs g1{n, bb, bb, C, nn, C + es * size_t(k0), nn, Dcol, ld, parent + size_t(k0) * size_t(ldp), ldp,
-                      nullptr, 0, k0, k0, k0 + bb, 0, 0, Ct, FW_BLOCK, 0, 0};
-      const int blocks0 = ((bb + 63) / 64) * ((n + 15) / 16), blocks1 = ((n + 63) / 64) * ((bb + 15) / 16);
-      const dim3 grid(FW_PARENT_BLOCKS + blocks0 + blocks1);
-      if (f64)
-        launch_kernel(fwgemm_pair_kernel<double>, grid, dim3(256), 0, s, g0, g1, blocks0,
-                      reinterpret_cast<const double *>(H), Pkk, ldp, bb, k0);
-      else
-        launch_kernel(fwgemm_pair_kernel<float>, grid, dim3(256), 0, s, g0, g1, blocks0,
-                      reinterpret_cast<const float *>(H), Pkk, ldp, bb, k0);
-      if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
-    } else {
-      if (f64) launch_kernel(fw_parents_kernel<double>, dim3(FW_PARENT_BLOCKS), dim3(256), 0, s, reinterpret_cast<const double *>(H), Pkk, ldp, bb, k0);
-      else launch_kernel(fw_parents_kernel<float>, dim3(FW_PARENT_BLOCKS), dim3(256), 0, s, reinterpret_cast<const float *>(H), Pkk, ldp, bb, k0);
+      if (f64) launch_kernel(fw_panels_kernel<double>, dim3(fw_panel_groups(n, bb, false)), dim3(FW_LINE_THREADS), 0, s, panel);
+      else launch_kernel(fw_panels_kernel<float>, dim3(fw_panel_groups(n, bb, false)), dim3(FW_LINE_THREADS), 0, s, panel);
       if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
       FwExtra xr = x, xc = x;
       xr.skip_c0 = xc.skip_r0 = k0;
@@ -1537,7 +1672,7 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
       e = f64 ? snapshot<double>(Dcol, ld, nullptr, 0, Ct, FW_BLOCK, n, bb, s) : snapshot<float>(Dcol, ld, nullptr, 0, Ct, FW_BLOCK, n, bb, s);
       if (e != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
     }
-    // 4. everything outside block row and block column <- (block column) x (block row), read in place
+    // 3. everything outside block row and block column <- (block column) x (block row), read in place
     //    (those panels are not written in this step); the column's k-contiguous image serves the lookups.
     //    The next step's diagonal block gets its update first, so that the product's launch can close it
     //    at the same time (fwgemm_tile_kernel).
@@ -1546,6 +1681,8 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
       x.ahead0 = k0 + bb;
       x.ahead_bb = n - x.ahead0 < FW_BLOCK ? n - x.ahead0 : FW_BLOCK;
       x.hist = H;
+      x.closed = closed_copy;
+      x.closed_t = closed_copy_t;
       x.closed_ahead = &closed;
     }
     x.At = Ct;
@@ -1553,15 +1690,12 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
     x.skip_r0 = x.skip_c0 = k0;
     x.skip_r1 = x.skip_c1 = k0 + bb;
     if (x.ahead_bb > 0 && !naive) {
-      // this step's update of that block, by a launch of its own (64 workgroups, a few microseconds): the
+      // this step's update of that block, by a launch of its own (32 workgroups, a few microseconds): the
       // closure can then start with the big product instead of after one of its tiles
-      const int a0 = x.ahead0, abb = x.ahead_bb;
-      FwExtra xa;
-      xa.k_base = k0;
-      r = fwgemm_run(dtype, abb, abb, bb, Dcol + es * size_t(a0), ld, Drow + es * size_t(a0) * size_t(ld), ld,
-                     D + es * (size_t(a0) + size_t(a0) * size_t(ld)), ld, parent + size_t(a0) + size_t(a0) * size_t(ldp), ldp,
-                     xa, CUASR_AMD_KERNEL_AUTO, stream);
-      if (r != CUASR_AMD_SUCCESS) return r;
+      const dim3 grid((x.ahead_bb + 3) / 4);
+      if (f64) launch_kernel(fw_ahead_kernel<double>, grid, dim3(FW_LINE_THREADS), 0, s, panel, x.ahead0, x.ahead_bb);
+      else launch_kernel(fw_ahead_kernel<float>, grid, dim3(FW_LINE_THREADS), 0, s, panel, x.ahead0, x.ahead_bb);
+      if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
     } else {
       x.ahead_bb = 0;
     }

@@ -277,6 +277,31 @@ def test_apsp_blocked_keeps_the_sign_of_a_zero(oracle, n, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+# a last block of one vertex, of a chunk of sixteen and one less or more; the smallest n whose blocks are closed beside tiles
+@pytest.mark.parametrize("n,pad", [(129, 0), (143, 1), (144, 3), (145, 0), (271, 2), (929, 1), (1038, 5)])
+def test_apsp_blocked_panels_of_ragged_blocks(oracle, n, pad, dtype):
+    """Panels in place, sixteen lines to a workgroup: dense weights whose sums round, odd leading dimensions of both
+    matrices, nothing written past them; dist and parent equal the oracle's bit for bit."""
+    import torch
+    rng = np.random.default_rng(n)
+    W = np.where(rng.random((n, n)) < 0.4, rng.uniform(1, 100, (n, n)), np.inf).astype(dtype)
+    np.fill_diagonal(W, 0)
+    host = np.full((n + pad, n), -5.0, dtype=dtype, order="F")
+    host[:n] = W
+    dD = to_device(host)
+    dP = torch.full((n, n + pad + 1), -1, dtype=torch.int32, device="cuda").t()
+    ws = torch.full((cuasr_amd.apsp_blocked_workspace_bytes(n, "f32" if dtype == np.float32 else "f64"),), 0xff, dtype=torch.uint8,
+                    device="cuda")   # (NaN patterns)
+    cuasr_amd.apsp_blocked(dD[:n], dP[:n], ws)
+    got, parent = dD.cpu().numpy(), dP.cpu().numpy()
+    assert (got[n:] == -5.0).all() and (parent[n:] == -1).all()
+    want_d, want_p = np.asfortranarray(W), np.full((n, n), -1, np.int32, order="F")
+    oracle.apsp_blocked(want_d, want_p, 128)
+    assert_same_bits(np.ascontiguousarray(got[:n]), np.ascontiguousarray(want_d), "dist")
+    assert np.array_equal(parent[:n], want_p)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n,pad", [(100, 0), (384, 0), (513, 1), (700, 4), (1475, 1), (2193, 3)])
 def test_apsp_blocked_with_tiled_panels(oracle, n, pad, dtype):
     """The way a block step updates its block row and column from n = 16257 on (two launches of the tiled
