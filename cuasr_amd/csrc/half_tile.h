@@ -20,8 +20,9 @@
 // 16-byte vector of A (its 8 rows; the instruction's half-word selects broadcast one of them) and two
 // of B, and issues 64 packed adds + 32 three-input packed minima for 128 terms.
 // Outputs too small to give the 256 compute units two such tiles each take smaller ones of the same kernel, guarded
-// form only: 64 x 128 (4 rows and one column group per thread); below that 32 x 128 and 16 x 128 with every k-tile
-// shared out between the four waves (min, max, or), or 32 x 128 with 2 rows per thread (plus, whose order counts).
+// form only: 64 x 128 with every k-tile shared out between two pairs of waves (min, max, or: 8 rows and one column
+// group per thread) or whole in every thread (plus, whose order counts: 4 rows); below that 32 x 128 and 16 x 128 with
+// every k-tile shared out between the four waves, or 32 x 128 with 2 rows per thread (plus).
 //
 // int8 operands (CUASR_AMD_I8: int8 A and B, int32 everything else) ride on the same kernel for min-plus,
 // max-plus, min-max and max-min: every int8 value, and every sum of two, is a binary16 value, so the terms and
@@ -237,14 +238,19 @@ static __device__ __attribute__((noinline)) half_t last_zero_product(const half_
 }
 
 // TR rows and NG groups of 8 columns per thread.  KS = 1: the 256 threads are 16 x 16, the tile 16 TR x 128 NG.
-// KS = 4 (adds that do not care about order, and about repetition of the value every part starts from -- min, max,
+// KS = 4, and 2 in the same way (adds that do not care about order, and about repetition of the value every part starts from -- min, max,
 // or, and xor, which starts from zero): a wave is 16 x 4 threads and covers a
 // tile of 4 TR x 128 NG by itself, each of the four waves takes a quarter of every k-tile, and the four partial
 // accumulators meet in LDS before the epilogue.  A small output then still gives every SIMD a wave, and the wave
 // the full tile's work per LDS read.
+// KS = 2 is the 64 x 128 tile: two pairs of waves, each with 8 x 8 outputs per lane over half of every k-tile.  What
+// bounds that tile is the wait for LDS and for the panels of the next k-tile at two waves per SIMD, not issue: an LDS
+// read feeds twice the terms it feeds at 4 x 8, and loads two k-tiles ahead (AHEAD = 2) outlast a memory latency.
+// min-plus 2000^3, column-major: 273 us with whole k-tiles per thread, 268 with KS = 2, 258 with AHEAD = 2 as well;
+// 2048^3 249 -> 233 us.  Four parts of 16 x 8 per lane: 286, AHEAD = 2 265 (64 KB of partials, 179 - 230 registers).
 template <int ADD, int MUL, bool A_KC, bool B_KC, bool GUARD, int TR = 8, int NG = 2, typename TI = half_t, int KS = 1, int AHEAD = 1>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void half_tile_kernel(Problem p) {
-  static_assert(KS == 1 || (KS == 4 && ADD != kPlus && TR % KS == 0), "k is shared out between waves only for order-free adds");
+  static_assert(KS == 1 || ((KS == 2 || KS == 4) && ADD != kPlus && TR % KS == 0), "k is shared out between waves only for order-free adds");
   constexpr int TY = 16 / KS, BM = TY * TR, BN = 128 * NG;
   constexpr int KW = BK / KS;        // k per tile and part
   constexpr int IR = TR / KS;        // rows of its accumulators that a thread takes through the epilogue
@@ -254,6 +260,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   constexpr bool I16 = int16_lanes<ADD, MUL, TI>::value;
   typedef typename out_of<TI>::type TO;
   typedef typename vec8<TO>::type out8;
+  typedef TO loose_out8 __attribute__((ext_vector_type(8), aligned(sizeof(TO))));   // the same at any element boundary
   typedef typename frag_of<TR>::type rows_t;
   typedef Smem<BM, BN> panels_t;
   typedef h2 partials_t[KS][TR * 4 * NG][THREADS / KS];   // [part][accumulator][lane]
@@ -386,6 +393,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
       const int col = n0 + g * 128 + tx * 8;
+      // KS = 2: eight outputs that all exist go as one vector at any element boundary (2048^3 238 -> 233 us; the other
+      // guarded tiles got slower by up to 7 % together with such loads, and stay element by element)
+      const bool whole = KS == 2 && row < p.m && col <= p.n - 8;
       out8 v;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -409,6 +419,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
       if (ws) {
         if constexpr (!GUARD) {
           *reinterpret_cast<out8 *>(ws + (long long)row * p.n + col) = v;
+        } else if (whole) {
+          *reinterpret_cast<loose_out8 *>(ws + (long long)row * p.n + col) = v;
         } else {
 #pragma unroll
           for (int x = 0; x < 8; ++x)
@@ -422,6 +434,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
       if (e.source_needed) {
         if constexpr (!GUARD) {
           c = *reinterpret_cast<const out8 *>(C + (long long)row * p.ldc + col);
+        } else if (whole) {
+          c = *reinterpret_cast<const loose_out8 *>(C + (long long)row * p.ldc + col);
         } else {
 #pragma unroll
           for (int x = 0; x < 8; ++x)
@@ -436,6 +450,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
       }
       if constexpr (!GUARD) {
         *reinterpret_cast<out8 *>(D + (long long)row * p.ldd + col) = out;
+      } else if (whole) {
+        *reinterpret_cast<loose_out8 *>(D + (long long)row * p.ldd + col) = out;
       } else {
 #pragma unroll
         for (int x = 0; x < 8; ++x)
@@ -491,7 +507,11 @@ template <int ADD, int MUL, typename TI = half_t> static hipError_t launch(const
   };
   // (or-and: the full tile's term is half an instruction; the smaller tiles are bound by what surrounds the terms)
   const bool bits = masked<ADD, MUL>::value || MUL == kBitAnd;
-  const long long full = bits ? cost(128, 256, 95, 128) : cost(128, 256, 63, 83), mid = bits ? cost(64, 128, 50, 76) : cost(64, 128, 50, 68);
+  // 64 x 128: 68 with whole k-tiles per thread, 72 shared out between two pairs of waves (2000^3 min-plus 62, 2048^3 74;
+  // 3000 x 2900 x 500 takes it now instead of 32 x 128: 173 -> 157 us; at 74 it would take 1500 x 1500 x 4000 from the
+  // 32 x 128 tile too: 468 -> 508 us).  Products of binary16 keep 68: their lookups of zeros, not the loop, set the time
+  const int mid_paired = bits ? 76 : ADD == kPlus || (MUL == kMultiplies && !std::is_same<TI, int8_t>::value) ? 68 : 72;
+  const long long full = bits ? cost(128, 256, 95, 128) : cost(128, 256, 63, 83), mid = cost(64, 128, 50, mid_paired);
   if constexpr (ADD == kPlus) {
     // the sum's order is the reference's: every k-tile whole in one thread
     const long long small = cost(32, 128, 36, 55);
@@ -509,7 +529,7 @@ template <int ADD, int MUL, typename TI = half_t> static hipError_t launch(const
       if (exact<TI>(p, a_kc, b_kc)) return launch_tile<ADD, MUL, false, 8, 2, TI>(p, a_kc, b_kc, s);
       return launch_tile<ADD, MUL, true, 8, 2, TI>(p, a_kc, b_kc, s);
     }
-    if (mid <= sliced && mid <= narrow) return launch_tile<ADD, MUL, true, 4, 1, TI>(p, a_kc, b_kc, s);
+    if (mid <= sliced && mid <= narrow) return launch_tile<ADD, MUL, true, 8, 1, TI, 2, 2>(p, a_kc, b_kc, s);
     if (sliced <= narrow) return launch_tile<ADD, MUL, true, 8, 1, TI, 4, 2>(p, a_kc, b_kc, s);
     return launch_tile<ADD, MUL, true, 4, 1, TI, 4, 2>(p, a_kc, b_kc, s);
   }

@@ -70,11 +70,11 @@ def test_packed_tile(oracle, lib, sr, layouts):
 
 @pytest.mark.parametrize("layouts", LAYOUTS)
 def test_every_tile_size(oracle, lib, layouts):
-    """The kernel comes in three tile sizes, picked by how many workgroups the output gives the chip: the full
+    """The kernel comes in several tile sizes, picked by how many workgroups the output gives the chip: the full
     tile unguarded (whole tiles of aligned operands) and guarded, the 64 x 128 tile, the 32 x 128 tile."""
     check(oracle, "minimum", "plus", 4096, 4096, 64, layouts, "valu")              # 512 full tiles, unguarded
     check(oracle, "maximum", "minimum", 4000, 4100, 70, layouts, "valu", False)    # full tiles, ragged: guarded
-    check(oracle, "minimum", "plus", 2048, 2048, 96, layouts, "valu")              # 64 x 128 tiles
+    check(oracle, "minimum", "plus", 2048, 2048, 96, layouts, "valu")              # 64 x 128 tiles, k shared out between two pairs of waves
     check(oracle, "plus", "multiplies", 1000, 2000, 50, layouts, "valu")           # 64 x 128 tiles, ragged
     check(oracle, "maximum", "plus", 1536, 1536, 64, layouts, "valu")              # 32 x 128 tiles, k shared out between the waves
     check(oracle, "maximum", "plus", 1024, 1024, 64, layouts, "valu")              # 16 x 128 tiles, likewise
@@ -92,6 +92,17 @@ def test_k_shared_out_between_waves(oracle, lib, sr, layouts):
     check(oracle, *sr, 1530, 1300, 77, layouts, "valu")                             # 32 x 128 tiles
     check(oracle, *sr, 1530, 1300, 32, layouts, "valu", beta_one=False)
     check(oracle, *sr, 300, 260, 500, layouts, "valu", splitk=5)
+
+
+@pytest.mark.parametrize("sr", [x for x in TILE_PAIRS if x[0] != "plus"])
+@pytest.mark.parametrize("layouts", ["ccc", "rcr", "crr", "rrc"])
+def test_k_shared_out_between_two_pairs_of_waves(oracle, lib, sr, layouts):
+    """The 64 x 128 tile of the order-free adds: two halves of every k-tile, two k-tiles in flight.  k inside the
+    first and the second half of the only tile, one, two and three tiles, a ragged third; rows and columns one short
+    of, at and one past a tile's or a vector's end (outputs go out as vectors at any element boundary); slices."""
+    for m, n, k in [(1985, 2001, 9), (2000, 1999, 17), (1991, 2047, 32), (2047, 2049, 33), (1984, 2048, 64), (2001, 1993, 77), (2048, 2000, 96)]:
+        check(oracle, *sr, m, n, k, layouts, "valu", beta_one=bool(m & 1))
+    check(oracle, *sr, 1009, 1003, 203, layouts, "valu", splitk=4)
 
 
 def test_selected_family(lib):

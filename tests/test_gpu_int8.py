@@ -90,6 +90,14 @@ def test_tropical_pairs_on_the_packed_tile(oracle, lib, sr, layouts):
     check(oracle, *sr, 4000, 4100, 70, layouts, "valu", alpha=-100, beta=100)  # full tiles, guarded
 
 
+@pytest.mark.parametrize("sr", [("minimum", "plus"), ("maximum", "multiplies"), ("bit_xor", "bit_and")])
+@pytest.mark.parametrize("layouts", ["ccc", "rcr", "crr", "rrc"])
+def test_k_shared_out_between_two_pairs_of_waves(oracle, lib, sr, layouts):
+    """64 x 128 tiles at extents that are no multiple of a tile or a vector, k ending in either half of a k-tile."""
+    for m, n, k in [(1985, 2001, 9), (1991, 2047, 17), (2047, 2049, 32), (2001, 1993, 77)]:
+        check(oracle, *sr, m, n, k, layouts, "valu", alpha=7, beta=-3)
+
+
 @pytest.mark.parametrize("layouts", ["ccc", "rcr", "crr", "rrc"])
 def test_boolean_closure_on_masks(oracle, lib, layouts):
     """or-and on int8 operands: sparse (most entries zero), so that the answer is not all ones; every tile size;
