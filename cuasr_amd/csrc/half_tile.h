@@ -31,6 +31,7 @@
 // twice the rate integers get (three-input integer minima and byte-selecting adds issue at half rate).
 // min-times, max-times and the bitwise pairs on int8 operands use the kernel with int16 lanes (int16_lanes below).
 #pragma once
+#include "launch_rules.h"
 #include "semiring.h"
 
 namespace cuasr_amd {
@@ -246,8 +247,12 @@ static __device__ __attribute__((noinline)) half_t last_zero_product(const half_
 // KS = 2 is the 64 x 128 tile: two pairs of waves, each with 8 x 8 outputs per lane over half of every k-tile.  What
 // bounds that tile is the wait for LDS and for the panels of the next k-tile at two waves per SIMD, not issue: an LDS
 // read feeds twice the terms it feeds at 4 x 8, and loads two k-tiles ahead (AHEAD = 2) outlast a memory latency.
-// min-plus 2000^3, column-major: 273 us with whole k-tiles per thread, 268 with KS = 2, 258 with AHEAD = 2 as well;
-// 2048^3 249 -> 233 us.  Four parts of 16 x 8 per lane: 286, AHEAD = 2 265 (64 KB of partials, 179 - 230 registers).
+// min-plus 2000^3, column-major: 273 us with whole k-tiles per thread, 268 with KS = 2, 257 with AHEAD = 2 as well, 254
+// with halves exchanged 16 bytes at a time; 2048^3 249 -> 233 us.  Four parts of 16 x 8 per lane: 286, AHEAD = 2 265 (64 KB of
+// partials, 179 - 230 registers).  Short k, us with whole k-tiles per thread / here (by halves of a whole k-tile and every
+// accumulator through LDS): min-plus 2000 x 1648 x 80 16.6 / 17.0 (19.2), 3000 x 3000 x 76 45.3 / 34.3 (37.8), 2000 x 2000 x 90
+// 19.0 / 18.6 (19.5) and with a source 22.0 / 19.6 (20.4).  Two or three k-tiles without a source are where whole k-tiles are still
+// up to 4 % faster, at ten of 750 shapes; on average of those the two are even.
 template <int ADD, int MUL, bool A_KC, bool B_KC, bool GUARD, int TR = 8, int NG = 2, typename TI = half_t, int KS = 1, int AHEAD = 1>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void half_tile_kernel(Problem p) {
   static_assert(KS == 1 || ((KS == 2 || KS == 4) && ADD != kPlus && TR % KS == 0), "k is shared out between waves only for order-free adds");
@@ -264,7 +269,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
   typedef typename frag_of<TR>::type rows_t;
   typedef Smem<BM, BN> panels_t;
   typedef h2 partials_t[KS][TR * 4 * NG][THREADS / KS];   // [part][accumulator][lane]
-  constexpr size_t lds_bytes = KS > 1 && sizeof(partials_t) > sizeof(panels_t) ? sizeof(partials_t) : sizeof(panels_t);
+  constexpr size_t lds_bytes = KS > 2 && sizeof(partials_t) > sizeof(panels_t) ? sizeof(partials_t) : sizeof(panels_t);
+  static_assert(KS != 2 || sizeof(panels_t) >= size_t(16) * IR * NG * THREADS, "the parts' mail");
   __shared__ __attribute__((aligned(16))) unsigned char lds[lds_bytes];   // the panels, and after the last k-tile the partials
   panels_t &sm = *reinterpret_cast<panels_t *>(lds);
   select_batch<TO, TI>(p);
@@ -332,18 +338,34 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
               two_terms<ADD, MUL, I16>(acc[i][4 * g + j], both(a0[i]), pair_of(b0[g], j), both(a1[i]), pair_of(b1[g], j));
       }
     } else {
-      for (int kk = kf; kk < min(kf + KW, ke - k0); ++kk) {  // the ragged last k-tile
-        const rows_t a0 = *reinterpret_cast<const rows_t *>(&pa[kk][ty * TR]);
-        h8 b0[NG];
+      // the ragged last k-tile, a term at a time.  KS = 2: half of what there is of it to each part, operands of two k
+      // read together (by halves of a whole k-tile the second part has nothing to do beside the first one's sixteen: see the
+      // short k above)
+      const int rest = ke - k0;
+      int kk = KS == 2 ? ragged_share(rest, KS, part) : kf;
+      const int last = KS == 2 ? ragged_share(rest, KS, part + 1) : min(kf + KW, rest);
+      auto terms = [&](auto count) {
+        constexpr int N = count.value;
+        rows_t a[N];
+        h8 b[N][NG];
 #pragma unroll
-        for (int g = 0; g < NG; ++g) b0[g] = *reinterpret_cast<const h8 *>(&pb[kk][g * 128 + tx * 8]);
+        for (int u = 0; u < N; ++u) {
+          a[u] = *reinterpret_cast<const rows_t *>(&pa[kk + u][ty * TR]);
 #pragma unroll
-        for (int i = 0; i < TR; ++i)
+          for (int g = 0; g < NG; ++g) b[u][g] = *reinterpret_cast<const h8 *>(&pb[kk + u][g * 128 + tx * 8]);
+        }
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
+        for (int u = 0; u < N; ++u)
 #pragma unroll
-            for (int g = 0; g < NG; ++g) one_term<ADD, MUL, I16>(acc[i][4 * g + j], both(a0[i]), pair_of(b0[g], j));
-      }
+          for (int i = 0; i < TR; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+              for (int g = 0; g < NG; ++g) one_term<ADD, MUL, I16>(acc[i][4 * g + j], both(a[u][i]), pair_of(b[u][g], j));
+      };
+      if constexpr (KS == 2)
+        for (; kk + 1 < last; kk += 2) terms(std::integral_constant<int, 2>());
+      for (; kk < last; ++kk) terms(std::integral_constant<int, 1>());
     }
     if (t + 1 < tiles_k) {
       sa[next].store(sm.a[s ^ 1]);
@@ -363,8 +385,32 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     for (int i = 0; i < TR; ++i)
 #pragma unroll
       for (int j = 0; j < 4 * NG; ++j) fin[i][j] = acc[i][j];
+  } else if constexpr (KS == 2) {
+    // each part sends the other one the rows that the other one finishes, 16 bytes at a time, and keeps its own
+    h8(*const mail)[IR * NG][THREADS / KS] = reinterpret_cast<h8(*)[IR * NG][THREADS / KS]>(lds);   // (every wave is past the last k-tile's barrier)
+    const int lane = threadIdx.x % (THREADS / KS);
+    const bool second = __builtin_amdgcn_readfirstlane(part);
+    auto rows_of = [&](bool upper, auto &&f) {
+#pragma unroll
+      for (int i = 0; i < IR; ++i)
+#pragma unroll
+        for (int g = 0; g < NG; ++g) f(i, g, upper ? &acc[IR + i][4 * g] : &acc[i][4 * g]);
+    };
+    auto send = [&](int i, int g, const h2 *from) {
+      mail[part][i * NG + g][lane] = h8{from[0][0], from[0][1], from[1][0], from[1][1], from[2][0], from[2][1], from[3][0], from[3][1]};
+    };
+    if (second) rows_of(false, send);
+    else rows_of(true, send);
+    __syncthreads();
+    auto meet = [&](int i, int g, const h2 *own) {
+      const h8 v = mail[part ^ 1][i * NG + g][lane];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) fin[i][4 * g + j] = fold<ADD, MUL, I16>(own[j], pair_of(v, j));
+    };
+    if (second) rows_of(true, meet);
+    else rows_of(false, meet);
   } else {
-    partials_t &red = *reinterpret_cast<partials_t *>(lds);   // (every wave is past the last k-tile's barrier)
+    partials_t &red = *reinterpret_cast<partials_t *>(lds);   // (likewise)
     const int lane = threadIdx.x % (THREADS / KS);
 #pragma unroll
     for (int i = 0; i < TR; ++i)

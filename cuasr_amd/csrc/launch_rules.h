@@ -1,4 +1,5 @@
-// Rules that choose between two kernels by sizes alone: plain C++, so that they can be tested without a GPU.
+// Rules that choose between two kernels by sizes alone, and how work is shared out: plain C++, so that they can be tested
+// without a GPU.
 #pragma once
 
 #include <cstdint>
@@ -35,6 +36,12 @@ inline bool fwgemm_one_thread_each(bool f64, bool k_contiguous_image, int m, int
 // (Fewer than 64 rows, 30 x 30000 x 200: 160 and 143.)
 inline bool fwgemm_f64_half_tile(bool k_contiguous_image, int m, int64_t half_tiles) {
   return m >= 64 && (!k_contiguous_image || half_tiles <= 256);
+}
+
+// Where part `part` of `parts` begins in a k-tile that holds `rest` k-values only; part + 1's beginning is its end.
+constexpr int ragged_share(int rest, int parts, int part) {
+  const int begin = part * ((rest + parts - 1) / parts);
+  return begin < rest ? begin : rest;
 }
 
 }  // namespace cuasr_amd

@@ -105,6 +105,15 @@ def test_k_shared_out_between_two_pairs_of_waves(oracle, lib, sr, layouts):
     check(oracle, *sr, 1009, 1003, 203, layouts, "valu", splitk=4)
 
 
+@pytest.mark.parametrize("sr", [("minimum", "plus"), ("maximum", "multiplies"), ("logical_or", "logical_and")])
+@pytest.mark.parametrize("layouts", ["ccc", "rcr"])
+def test_two_parts_of_a_ragged_k_tile(oracle, lib, sr, layouts):
+    """The last k-tile of the 64 x 128 tile goes to its two parts by halves: one k (the second part has none), an odd number
+    and an even one, one short of a whole tile; as the only tile and after one or two whole ones."""
+    for k in (1, 2, 7, 31, 33, 43, 44, 63, 80):
+        check(oracle, *sr, 1999, 2001, k, layouts, "valu", beta_one=bool(k & 1))
+
+
 def test_selected_family(lib):
     import cuasr_amd
     dA = to_device(np.zeros((128, 64), np.float16))

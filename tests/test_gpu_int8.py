@@ -98,6 +98,13 @@ def test_k_shared_out_between_two_pairs_of_waves(oracle, lib, sr, layouts):
         check(oracle, *sr, m, n, k, layouts, "valu", alpha=7, beta=-3)
 
 
+@pytest.mark.parametrize("sr", [("minimum", "plus"), ("maximum", "multiplies"), ("bit_xor", "bit_and"), ("logical_or", "logical_and")])
+def test_two_parts_of_a_ragged_k_tile(oracle, lib, sr):
+    """As for binary16: one k, an odd number, an even one, after no and after two whole k-tiles."""
+    for k in (1, 7, 31, 80):
+        check(oracle, *sr, 1999, 2001, k, "crr", "valu")
+
+
 @pytest.mark.parametrize("layouts", ["ccc", "rcr", "crr", "rrc"])
 def test_boolean_closure_on_masks(oracle, lib, layouts):
     """or-and on int8 operands: sparse (most entries zero), so that the answer is not all ones; every tile size;

@@ -35,3 +35,13 @@ def test_staged_tiles_take_the_faster_size():
         (64, 64, 200, 128, 128, 0), (180, 200, 64, 128, 128, 0), (100, 100, 240, 128, 128, 1)]           # a batch of small products
     got = _ask(["staged %d %d %d %d %d" % c[:5] for c in cases])
     assert got == [c[5] for c in cases]
+
+
+def test_a_ragged_k_tile_is_shared_out_evenly():
+    """Every k-value of the last k-tile belongs to one part, and no part has more than its share rounded up."""
+    parts = 2
+    for rest in range(1, 32):
+        begin = _ask([f"share {rest} {parts} {part}" for part in range(parts + 1)])
+        assert begin[0] == 0 and begin[-1] == rest
+        sizes = [end - first for first, end in zip(begin, begin[1:])]
+        assert min(sizes) >= 0 and max(sizes) == (rest + parts - 1) // parts
