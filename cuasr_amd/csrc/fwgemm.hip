@@ -137,28 +137,56 @@ template <typename T> struct FwLineLds {
 };
 constexpr int FW_LINE_THREADS = 512;
 
-// whole[k][line] = src[line + k * ld], lines up to `lines` (clamped; the rest are not stored by anybody)
-template <typename T> __device__ __forceinline__ void fw_fetch_whole(FwLineLds<T> &sm, const T *src, int64_t ld, int lines) {
+// whole[k][line] = src[line + k * ld] for the first `lines` lines and `ks` k; +infinity from k = ks on, any value in lines
+// beyond (nobody stores those)
+template <typename T> __device__ __forceinline__ void fw_fetch_whole(FwLineLds<T> &sm, const T *src, int64_t ld, int lines, int ks) {
   typedef typename vec4_of<T>::type V4;
   typedef typename uvec4_of<T>::type U4;
-  constexpr int N = FW_BLOCK * FW_BLOCK / 4 / FW_LINE_THREADS;
+  const T inf = std::numeric_limits<T>::infinity();
+  constexpr int N = FW_BLOCK * FW_BLOCK / 4 / FW_LINE_THREADS, STEP = FW_LINE_THREADS / 32;
   const int tid = threadIdx.x, line = (tid & 31) * 4, k0 = tid >> 5;
   V4 v[N];
-  if (lines == FW_BLOCK) {
+  if (lines == FW_BLOCK && ks == FW_BLOCK) {
 #pragma unroll
-    for (int u = 0; u < N; ++u) v[u] = *reinterpret_cast<const U4 *>(src + line + int64_t(k0 + u * (FW_LINE_THREADS / 32)) * ld);
+    for (int u = 0; u < N; ++u) v[u] = *reinterpret_cast<const U4 *>(src + line + int64_t(k0 + u * STEP) * ld);
   } else {
-#pragma unroll 1
-    for (int u = 0; u < N; ++u) {
-      V4 x;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = src[min(line + e, lines - 1) + int64_t(k0 + u * (FW_LINE_THREADS / 32)) * ld];
-      *reinterpret_cast<V4 *>(&sm.whole[k0 + u * (FW_LINE_THREADS / 32)][line]) = x;
-    }
-    return;
+    for (int u = 0; u < N; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const T x = src[min(line + e, lines - 1) + int64_t(min(k0 + u * STEP, ks - 1)) * ld];
+        v[u][e] = k0 + u * STEP < ks ? x : inf;
+      }
   }
 #pragma unroll
-  for (int u = 0; u < N; ++u) *reinterpret_cast<V4 *>(&sm.whole[k0 + u * (FW_LINE_THREADS / 32)][line]) = v[u];
+  for (int u = 0; u < N; ++u) *reinterpret_cast<V4 *>(&sm.whole[k0 + u * STEP][line]) = v[u];
+}
+// whole[k][line] = src[k + line * ld], likewise: two neighbouring lanes take eight k of one line, so that a line of memory
+// is asked for in 32 or 64 bytes at once and the stores of an instruction meet two to a bank
+template <typename T> __device__ __forceinline__ void fw_fetch_turned(FwLineLds<T> &sm, const T *src, int64_t ld, int lines, int ks) {
+  typedef typename vec4_of<T>::type V4;
+  typedef typename uvec4_of<T>::type U4;
+  const T inf = std::numeric_limits<T>::infinity();
+  constexpr int N = FW_BLOCK * FW_BLOCK / 4 / FW_LINE_THREADS;
+  const int tid = threadIdx.x, line = (tid >> 1) & 127, k0 = (tid & 1) * 4 + (tid >> 8) * 8;
+  V4 v[N];
+  if (lines == FW_BLOCK && ks == FW_BLOCK) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) v[u] = *reinterpret_cast<const U4 *>(src + k0 + u * 16 + int64_t(line) * ld);
+  } else {
+    src += int64_t(min(line, lines - 1)) * ld;
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const T x = src[min(k0 + u * 16 + e, ks - 1)];
+        v[u][e] = k0 + u * 16 + e < ks ? x : inf;
+      }
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sm.whole[k0 + u * 16 + e][line] = v[u][e];
 }
 
 // lane's line `line` of the whole operand with lines first .. first + NC - 1 of the other, chunks of CK k
@@ -224,14 +252,14 @@ struct FwPanels {
   int n, k0, bb;
   void *dist; int64_t ld;
   int32_t *parent; int64_t ldp;
-  const void *closed, *closed_t;   // the closed diagonal block and its transpose, FW_BLOCK x FW_BLOCK, +infinity beyond bb
+  const void *closed, *closed_t;   // COPIES: the closed diagonal block and its transpose, FW_BLOCK x FW_BLOCK, +infinity beyond bb
   void *col_t;                     // takes the updated block column with k contiguous, leading dimension FW_BLOCK
   // the block being closed: columns and rows as its steps read them and the block as it was (fw_close_dist)
   const void *hist;
 };
 
 // columns c0 .. c0 + 15 of the block row <- (closed block) x (block row)
-template <typename T> __device__ __forceinline__ void fw_row_panel(const FwPanels &p, int c0, FwLineLds<T> &sm) {
+template <typename T, bool COPIES> __device__ __forceinline__ void fw_row_panel(const FwPanels &p, int c0, FwLineLds<T> &sm) {
   typedef typename vec4_of<T>::type V4;
   typedef typename uvec4_of<T>::type U4;
   const T inf = std::numeric_limits<T>::infinity();
@@ -251,7 +279,8 @@ template <typename T> __device__ __forceinline__ void fw_row_panel(const FwPanel
       }
     }
   }
-  fw_fetch_whole<T>(sm, static_cast<const T *>(p.closed), FW_BLOCK, FW_BLOCK);
+  if constexpr (COPIES) fw_fetch_whole<T>(sm, static_cast<const T *>(p.closed), FW_BLOCK, FW_BLOCK, FW_BLOCK);
+  else fw_fetch_whole<T>(sm, row0 + int64_t(p.k0) * p.ld, p.ld, p.bb, p.bb);
   *reinterpret_cast<V4 *>(&sm.other[tid >> 5][(tid & 31) * 4]) = v;
   __syncthreads();
   const int i = tid & 127, first = __builtin_amdgcn_readfirstlane(tid >> 7) * 4;
@@ -292,12 +321,13 @@ template <typename T> __device__ __forceinline__ void fw_put_across(FwLineLds<T>
 }
 
 // rows r0 .. r0 + 15 of the block column <- (block column) x (closed block), as the transposed product
-template <typename T> __device__ __forceinline__ void fw_col_panel(const FwPanels &p, int r0, FwLineLds<T> &sm) {
+template <typename T, bool COPIES> __device__ __forceinline__ void fw_col_panel(const FwPanels &p, int r0, FwLineLds<T> &sm) {
   typedef typename vec4_of<T>::type V4;
   typedef typename uvec4_of<T>::type U4;
   T *const col0 = static_cast<T *>(p.dist) + int64_t(p.k0) * p.ld;
   const V4 v = fw_fetch_across<T>(col0 + r0, p.ld, p.n - r0, p.bb);
-  fw_fetch_whole<T>(sm, static_cast<const T *>(p.closed_t), FW_BLOCK, FW_BLOCK);
+  if constexpr (COPIES) fw_fetch_whole<T>(sm, static_cast<const T *>(p.closed_t), FW_BLOCK, FW_BLOCK, FW_BLOCK);
+  else fw_fetch_turned<T>(sm, col0 + p.k0, p.ld, p.bb, p.bb);
   fw_put_across<T>(sm, v);
   __syncthreads();
   const int tid = threadIdx.x, j = tid & 127, first = __builtin_amdgcn_readfirstlane(tid >> 7) * 4;
@@ -356,7 +386,7 @@ template <typename T> __device__ __forceinline__ void fw_parents(const FwPanels 
 #pragma unroll
   for (int c = 0; c < 4; ++c) curr[c] = init[i + (c0 + first + c) * FW_BLOCK];
   const typename vec4_of<T>::type v = fw_fetch_across<T>(hist_row + c0, FW_BLOCK, FwLineLds<T>::LINES, p.bb);
-  fw_fetch_whole<T>(sm, hist_col, FW_BLOCK, FW_BLOCK);   // (rows of k beyond the last chunk hold anything and are not read)
+  fw_fetch_whole<T>(sm, hist_col, FW_BLOCK, FW_BLOCK, FW_BLOCK);   // (rows of k beyond the last chunk hold anything and are not read)
   fw_put_across<T>(sm, v);
   __syncthreads();
   fw_lines<T, 4>(sm, i, first, (p.bb + 15) / 16, p.k0, curr, par);
@@ -369,7 +399,7 @@ template <typename T> __device__ __forceinline__ void fw_parents(const FwPanels 
 
 // One launch: the predecessors of the diagonal block (closed by fw_close_dist in a launch before), the block row and the block
 // column, which are independent of each other.
-template <typename T> __global__ void __launch_bounds__(FW_LINE_THREADS) fw_panels_kernel(FwPanels p) {
+template <typename T, bool COPIES> __global__ void __launch_bounds__(FW_LINE_THREADS) fw_panels_kernel(FwPanels p) {
   __shared__ FwLineLds<T> sm;
   const int lines = FwLineLds<T>::LINES, own = (p.bb + lines - 1) / lines, panel = (p.n + lines - 1) / lines - own;
   int b = blockIdx.x;
@@ -381,8 +411,8 @@ template <typename T> __global__ void __launch_bounds__(FW_LINE_THREADS) fw_pane
   const bool row = b < panel;
   b = (row ? b : b - panel) * lines;
   if (b >= p.k0) b += p.bb;   // (the diagonal block's own lines are left out; where it is ragged none come after it)
-  if (row) fw_row_panel<T>(p, b, sm);
-  else fw_col_panel<T>(p, b, sm);
+  if (row) fw_row_panel<T, COPIES>(p, b, sm);
+  else fw_col_panel<T, COPIES>(p, b, sm);
 }
 // workgroups: each fetches 64 KB (float) or 128 KB before it computes anything, so that one to a compute unit is worth having
 // (n = 2000, 242 of them: 10 us; with sixteen more, which had nothing to do, two CUs had two and the launch took 13)
@@ -402,7 +432,7 @@ template <typename T> __global__ void __launch_bounds__(FW_LINE_THREADS) fw_ahea
   T curr[1] = {block[row + int64_t(col_in) * p.ld]};
   int32_t par[1];
   const T b = (static_cast<const T *>(p.dist) + p.k0 + int64_t(a0 + col_in) * p.ld)[i];
-  fw_fetch_whole<T>(sm, static_cast<const T *>(p.dist) + a0 + int64_t(p.k0) * p.ld, p.ld, abb);
+  fw_fetch_whole<T>(sm, static_cast<const T *>(p.dist) + a0 + int64_t(p.k0) * p.ld, p.ld, abb, FW_BLOCK);
   sm.other[first][i] = b;
   __syncthreads();
   fw_lines<T, 1>(sm, i, first, FW_BLOCK / 16, p.k0, curr, par);
@@ -1607,15 +1637,20 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
   char *C = R + es * FW_BLOCK * size_t(nn);
   char *Ct = C + es * FW_BLOCK * size_t(nn);            // updated block column with k contiguous, leading dimension FW_BLOCK
   char *H = Ct + es * FW_BLOCK * size_t(nn);            // columns, rows and first state of the diagonal block being closed
-  // Block row and block column share one launch that works in place and reads the closed diagonal block and its transpose
-  // from C and R; from n = 16257 on each of the two products fills the chip on the tiled kernel, from copies of the panels in R
+  // Block row and block column share one launch that works in place (beside tiles it reads the closed diagonal block and its
+  // transpose from C and R); from n = 16257 on each of the two products fills the chip on the tiled kernel, from copies of the panels in R
   // (leading dimension FW_BLOCK) and C (leading dimension nn).
   const bool paired = panels == CUASR_AMD_PANELS_AUTO ? (int64_t(n) + 127) / 128 < 128 : panels == CUASR_AMD_PANELS_PAIRED;
-  char *closed_copy = paired && n > FW_BLOCK ? C : nullptr, *closed_copy_t = paired && n > FW_BLOCK ? R : nullptr;
   // With tiles a step's launch also closes the next block, after a launch that updates it; without, a closure alone on
-  // the chip takes most of a step.  us a job with tiles / without: f32 n = 800 430 / 389, 896 460 / 439, 960 482 / 495,
-  // 1024 500 / 549; f64 700 689 / 638, 768 719 / 706 (n = 1001 984 / 1130 when the panels were copied first).
+  // the chip takes most of a step.  us a job with tiles at density 0.02 and 0.5 / without: f32 n = 768 400, 380 / 352, 850 463, 439 /
+  // 423, 928 477, 454 / 472, 1000 527, 487 / 560; f64 640 625, 601 / 518, 768 728, 687 / 683, 832 802, 752 / 764, 850 825, 775 / 815,
+  // 1024 921, 860 / 1102.
   const bool naive = n <= (f64 ? 768 : 928);
+  // Where the closure hides beside a product it leaves the panels a copy of its block and of the transpose.  Alone on the chip
+  // its stores are on the critical path (57.6 us a closure of doubles without them, 63.1 with; 31.6 and 34.0 of floats) and
+  // the panels read the block from the matrix: f64 n = 130 / 464 / 768 119 / 382 / 709 us a job with copies, 113 / 368 / 683 from
+  // the matrix, f32 72 / 205 / 363 and 69 / 201 / 352.  With tiles, from the matrix: f32 n = 1000 487 -> 494, 2000 1006 -> 1018.
+  char *closed_copy = paired && !naive ? C : nullptr, *closed_copy_t = paired && !naive ? R : nullptr;
   // this step's diagonal block had its distances closed during the step before, beside that step's big product
   // (its predecessors are always still to be found, from what the closure recorded in H)
   bool closed = false;
@@ -1642,8 +1677,13 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
     const FwPanels panel{n, k0, bb, dist, ld, parent, ldp, closed_copy, closed_copy_t, Ct, H};
     if (paired) {
       const dim3 grid(fw_panel_groups(n, bb, true));
-      if (f64) launch_kernel(fw_panels_kernel<double>, grid, dim3(FW_LINE_THREADS), 0, s, panel);
-      else launch_kernel(fw_panels_kernel<float>, grid, dim3(FW_LINE_THREADS), 0, s, panel);
+      if (naive) {
+        if (f64) launch_kernel((fw_panels_kernel<double, false>), grid, dim3(FW_LINE_THREADS), 0, s, panel);
+        else launch_kernel((fw_panels_kernel<float, false>), grid, dim3(FW_LINE_THREADS), 0, s, panel);
+      } else {
+        if (f64) launch_kernel((fw_panels_kernel<double, true>), grid, dim3(FW_LINE_THREADS), 0, s, panel);
+        else launch_kernel((fw_panels_kernel<float, true>), grid, dim3(FW_LINE_THREADS), 0, s, panel);
+      }
       if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
     } else {
       // copies of block row and block column (the products read these, so that no workgroup sees another's updates)
@@ -1657,8 +1697,8 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
                            reinterpret_cast<float *>(R), int64_t(FW_BLOCK), bb, n, reinterpret_cast<const float *>(Dcol),
                            reinterpret_cast<float *>(C), nn, n, bb, ld, sb0);
       if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
-      if (f64) launch_kernel(fw_panels_kernel<double>, dim3(fw_panel_groups(n, bb, false)), dim3(FW_LINE_THREADS), 0, s, panel);
-      else launch_kernel(fw_panels_kernel<float>, dim3(fw_panel_groups(n, bb, false)), dim3(FW_LINE_THREADS), 0, s, panel);
+      if (f64) launch_kernel((fw_panels_kernel<double, false>), dim3(fw_panel_groups(n, bb, false)), dim3(FW_LINE_THREADS), 0, s, panel);
+      else launch_kernel((fw_panels_kernel<float, false>), dim3(fw_panel_groups(n, bb, false)), dim3(FW_LINE_THREADS), 0, s, panel);
       if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
       FwExtra xr = x, xc = x;
       xr.skip_c0 = xc.skip_r0 = k0;

@@ -277,8 +277,9 @@ def test_apsp_blocked_keeps_the_sign_of_a_zero(oracle, n, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-# a last block of one vertex, of a chunk of sixteen and one less or more; the smallest n whose blocks are closed beside tiles
-@pytest.mark.parametrize("n,pad", [(129, 0), (143, 1), (144, 3), (145, 0), (271, 2), (929, 1), (1038, 5)])
+# a last block of one vertex, of a chunk of sixteen and one less or more; one short of whole, whole, and one block alone; the
+# smallest n whose blocks are closed beside tiles
+@pytest.mark.parametrize("n,pad", [(100, 1), (129, 0), (143, 1), (144, 3), (145, 0), (255, 1), (256, 3), (271, 2), (929, 1), (1038, 5)])
 def test_apsp_blocked_panels_of_ragged_blocks(oracle, n, pad, dtype):
     """Panels in place, sixteen lines to a workgroup: dense weights whose sums round, odd leading dimensions of both
     matrices, nothing written past them; dist and parent equal the oracle's bit for bit."""
