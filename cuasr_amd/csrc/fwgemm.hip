@@ -1638,9 +1638,11 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
   char *Ct = C + es * FW_BLOCK * size_t(nn);            // updated block column with k contiguous, leading dimension FW_BLOCK
   char *H = Ct + es * FW_BLOCK * size_t(nn);            // columns, rows and first state of the diagonal block being closed
   // Block row and block column share one launch that works in place (beside tiles it reads the closed diagonal block and its
-  // transpose from C and R); from n = 16257 on each of the two products fills the chip on the tiled kernel, from copies of the panels in R
-  // (leading dimension FW_BLOCK) and C (leading dimension nn).
-  const bool paired = panels == CUASR_AMD_PANELS_AUTO ? (int64_t(n) + 127) / 128 < 128 : panels == CUASR_AMD_PANELS_PAIRED;
+  // transpose from C and R).  The other form, two launches of the tiled kernel on copies of the panels in R (leading dimension
+  // FW_BLOCK) and C (leading dimension nn), is slower at every size, also where each of its products fills the chip; ms a job in
+  // one launch / tiled: f32 n = 8192 31 / 37, 16384 218 / 227, 20000 395 / 406, 30000 1238 / 1256, f64 8192 59 / 69, 16384 421 / 436,
+  // 18000 555 / 570.
+  const bool paired = panels != CUASR_AMD_PANELS_TILED;
   // With tiles a step's launch also closes the next block, after a launch that updates it; without, a closure alone on
   // the chip takes most of a step.  us a job with tiles at density 0.02 and 0.5 / without: f32 n = 768 400, 380 / 352, 850 463, 439 /
   // 423, 928 477, 454 / 472, 1000 527, 487 / 560; f64 640 625, 601 / 518, 768 728, 687 / 683, 832 802, 752 / 764, 850 825, 775 / 815,

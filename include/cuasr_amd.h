@@ -307,10 +307,11 @@ int cuasr_amd_apsp_blocked(int dtype, int n, void *dist, int64_t ld, int32_t *pa
                            int64_t ldp, void *workspace, void *stream);
 
 /* The same with the choice of how a block step updates its block row and block column made by the
- * caller: CUASR_AMD_PANELS_AUTO (what cuasr_amd_apsp_blocked does: PAIRED below n = 16257, TILED from
- * there on, where each panel product fills the chip on its own), CUASR_AMD_PANELS_PAIRED (both products
- * in one launch of the one-thread-per-element kernel) or CUASR_AMD_PANELS_TILED (two launches of the
- * tiled kernel and a transposing copy of the updated block column).  Results do not depend on it.
+ * caller: CUASR_AMD_PANELS_AUTO (what cuasr_amd_apsp_blocked does: PAIRED, the faster one at every size),
+ * CUASR_AMD_PANELS_PAIRED (both products, and the predecessors of the diagonal block, in one launch that
+ * updates the panels in place, sixteen lines to a workgroup) or CUASR_AMD_PANELS_TILED (copies of both
+ * panels, a launch for those predecessors, two launches of the tiled kernel and a transposing copy of the
+ * updated block column).  Results do not depend on it.
  * CUASR_AMD_ERROR_INVALID_PROBLEM for any other value. */
 #define CUASR_AMD_PANELS_AUTO 0
 #define CUASR_AMD_PANELS_PAIRED 1

@@ -305,9 +305,9 @@ def test_apsp_blocked_panels_of_ragged_blocks(oracle, n, pad, dtype):
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n,pad", [(100, 0), (384, 0), (513, 1), (700, 4), (1475, 1), (2193, 3)])
 def test_apsp_blocked_with_tiled_panels(oracle, n, pad, dtype):
-    """The way a block step updates its block row and column from n = 16257 on (two launches of the tiled
-    kernel with the diagonal block skipped, then a transposing copy of the column), forced at sizes the
-    oracle can run: dist and parent bit-identical to the oracle and to the paired form."""
+    """The other way a block step can update its block row and column (copies, two launches of the tiled kernel
+    with the diagonal block skipped, a transposing copy of the column): dist and parent bit-identical to the
+    oracle and to the paired form."""
     import torch
     rng = np.random.default_rng(177 + n)
     W = np.where(rng.random((n, n)) < max(0.02, 3.0 / n), rng.random((n, n)) * 9 + 0.5, np.inf).astype(dtype)   # sums round
