@@ -540,43 +540,20 @@ template <int ADD, int MUL, typename TI = half_t> static hipError_t launch(const
   // one direction of each operand is contiguous (the C ABI produces nothing else)
   if ((p.sa_m != 1 && p.sa_k != 1) || (p.sb_n != 1 && p.sb_k != 1)) return hipErrorNotSupported;
   const bool a_kc = p.sa_m != 1, b_kc = p.sb_n != 1;
-  // Which tile.  A compute unit holds at most two of these workgroups (two waves per SIMD) and works two off
-  // faster than one, but not twice as fast (a packed instruction occupies the vector ALU for four cycles: one
-  // wave per SIMD keeps it busy most of the time); smaller tiles do less work per LDS read and per barrier.
-  // `alone` / `paired`: the chip's rate in TOPS with one / two workgroups of that tile on every compute unit
-  // (min-plus, measured from 512^3 to 4096^3).  The time is about that of the rounds of 512 workgroups at the
-  // paired rate plus a last round at whichever rate its size gives; the tile with the smallest wins.
-  auto cost = [&](int bm, int bn, long long alone, long long paired) {
-    const long long groups = (long long)((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn) * (p.workspace ? p.slices : 1) * p.batch;
-    const long long rest = groups % 512, area = (long long)bm * bn;
-    return groups / 512 * (512 * area / paired) + (rest > 256 ? 512 * area / paired : rest > 0 ? 256 * area / alone : 0);
-  };
-  // (or-and: the full tile's term is half an instruction; the smaller tiles are bound by what surrounds the terms)
-  const bool bits = masked<ADD, MUL>::value || MUL == kBitAnd;
-  // 64 x 128: 68 with whole k-tiles per thread, 72 shared out between two pairs of waves (2000^3 min-plus 62, 2048^3 74;
-  // 3000 x 2900 x 500 takes it now instead of 32 x 128: 173 -> 157 us; at 74 it would take 1500 x 1500 x 4000 from the
-  // 32 x 128 tile too: 468 -> 508 us).  Products of binary16 keep 68: their lookups of zeros, not the loop, set the time
-  const int mid_paired = bits ? 76 : ADD == kPlus || (MUL == kMultiplies && !std::is_same<TI, int8_t>::value) ? 68 : 72;
-  const long long full = bits ? cost(128, 256, 95, 128) : cost(128, 256, 63, 83), mid = cost(64, 128, 50, mid_paired);
+  constexpr bool bits = masked<ADD, MUL>::value || MUL == kBitAnd;
+  constexpr bool zeros = MUL == kMultiplies && !std::is_same<TI, int8_t>::value;
+  const int rows = half_tile_rows(ADD == kPlus, bits, zeros, p.m, p.n, (long long)(p.workspace ? p.slices : 1) * p.batch);
+  if (rows == 128) {
+    if (exact<TI>(p, a_kc, b_kc)) return launch_tile<ADD, MUL, false, 8, 2, TI>(p, a_kc, b_kc, s);
+    return launch_tile<ADD, MUL, true, 8, 2, TI>(p, a_kc, b_kc, s);
+  }
   if constexpr (ADD == kPlus) {
     // the sum's order is the reference's: every k-tile whole in one thread
-    const long long small = cost(32, 128, 36, 55);
-    if (full <= mid && full <= small) {
-      if (exact<TI>(p, a_kc, b_kc)) return launch_tile<ADD, MUL, false, 8, 2, TI>(p, a_kc, b_kc, s);
-      return launch_tile<ADD, MUL, true, 8, 2, TI>(p, a_kc, b_kc, s);
-    }
-    if (mid <= small) return launch_tile<ADD, MUL, true, 4, 1, TI>(p, a_kc, b_kc, s);
+    if (rows == 64) return launch_tile<ADD, MUL, true, 4, 1, TI>(p, a_kc, b_kc, s);
     return launch_tile<ADD, MUL, true, 2, 1, TI>(p, a_kc, b_kc, s);
   } else {
-    // min, max, or: the small tiles share every k-tile out between the four waves (1024^3 min-plus: 47 - 49 TOPS
-    // against 33 - 37 with whole k-tiles per thread; 512^3: 13 - 14 against 8)
-    const long long sliced = cost(32, 128, 43, 62), narrow = cost(16, 128, 35, 48);
-    if (full <= mid && full <= sliced && full <= narrow) {
-      if (exact<TI>(p, a_kc, b_kc)) return launch_tile<ADD, MUL, false, 8, 2, TI>(p, a_kc, b_kc, s);
-      return launch_tile<ADD, MUL, true, 8, 2, TI>(p, a_kc, b_kc, s);
-    }
-    if (mid <= sliced && mid <= narrow) return launch_tile<ADD, MUL, true, 8, 1, TI, 2, 2>(p, a_kc, b_kc, s);
-    if (sliced <= narrow) return launch_tile<ADD, MUL, true, 8, 1, TI, 4, 2>(p, a_kc, b_kc, s);
+    if (rows == 64) return launch_tile<ADD, MUL, true, 8, 1, TI, 2, 2>(p, a_kc, b_kc, s);
+    if (rows == 32) return launch_tile<ADD, MUL, true, 8, 1, TI, 4, 2>(p, a_kc, b_kc, s);
     return launch_tile<ADD, MUL, true, 4, 1, TI, 4, 2>(p, a_kc, b_kc, s);
   }
 }

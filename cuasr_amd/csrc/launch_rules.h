@@ -38,6 +38,42 @@ inline bool fwgemm_f64_half_tile(bool k_contiguous_image, int m, int64_t half_ti
   return m >= 64 && (!k_contiguous_image || half_tiles <= 256);
 }
 
+// The binary16 tile (half_tile.h), by its rows: 128 x 256, 64 x 128, 32 x 128 and, for adds that do not care about order,
+// 16 x 128.  ordered: plus.  bits: or-and on masks and the bitwise pairs.  zeros: min- and max-times on binary16.
+// A compute unit holds at most two of these workgroups (two waves per SIMD) and works two off faster than one, but not
+// twice as fast (a packed instruction occupies the vector ALU for four cycles: one wave per SIMD keeps it busy most of the
+// time); smaller tiles do less work per LDS read and per barrier.  `alone` / `paired`: the chip's rate in TOPS with one / two
+// workgroups of that tile on every compute unit (min-plus, measured from 512^3 to 4096^3).  The time is about that of the
+// rounds of 512 workgroups at the paired rate plus a last round at whichever rate its size gives; the tile with the
+// smallest wins.
+// 64 x 128 of the order-free adds is the exception: it reaches 60 alone and 74 paired, but a last round of 257 to 340
+// workgroups takes it as long as one of 512, so at those rates it would be taken too often (1216 x 2048 x 2048, 304 workgroups,
+// 247 us where 32 x 128 takes 227; 1500 x 1500 x 4000 508 and 468).  50 and 72 choose the faster one, or one within 2 %, at 13 sizes of
+// 190 to 800 workgroups, binary16 min-plus and max-min, k = 512 and 2048 (1792^2, 392: 232 and 266; 2048 x 2176, 544: 338 and 327;
+// 2304^2, 648: 341 and 389; 2560^2, 800: 440 and 448); on int8 32 x 128 is kept at 1500 x 1500 x 2048, 321 us where this takes 307.
+// 72 instead of 68, what whole k-tiles per thread reach, moves a quarter of this tile's sizes to it: of 1131 drawn ones
+// (64 .. 4096 each way, binary16 and int8) none was slower by more than 0.4 %, on average they were 1.17 (binary16) and 1.23
+// times as fast.  Products of binary16 keep 68: their lookups of zeros, not the loop, set the time.
+inline int half_tile_rows(bool ordered, bool bits, bool zeros, int m, int n, long long products) {
+  auto cost = [&](int bm, int bn, long long alone, long long paired) {
+    const long long groups = (m + bm - 1LL) / bm * ((n + bn - 1LL) / bn) * products;
+    const long long rest = groups % 512, area = (long long)bm * bn;
+    return groups / 512 * (512 * area / paired) + (rest > 256 ? 512 * area / paired : rest > 0 ? 256 * area / alone : 0);
+  };
+  // (or-and: the full tile's term is half an instruction; the smaller tiles are bound by what surrounds the terms)
+  const long long full = bits ? cost(128, 256, 95, 128) : cost(128, 256, 63, 83);
+  const long long mid = cost(64, 128, 50, bits ? 76 : ordered || zeros ? 68 : 72);
+  if (ordered) {
+    const long long small = cost(32, 128, 36, 55);
+    return full <= mid && full <= small ? 128 : mid <= small ? 64 : 32;
+  }
+  // the small tiles share every k-tile out between the four waves (1024^3 min-plus: 47 - 49 TOPS against 33 - 37 with whole
+  // k-tiles per thread; 512^3: 13 - 14 against 8)
+  const long long sliced = cost(32, 128, 43, 62), narrow = cost(16, 128, 35, 48);
+  if (full <= mid && full <= sliced && full <= narrow) return 128;
+  return mid <= sliced && mid <= narrow ? 64 : sliced <= narrow ? 32 : 16;
+}
+
 // Where part `part` of `parts` begins in a k-tile that holds `rest` k-values only; part + 1's beginning is its end.
 constexpr int ragged_share(int rest, int parts, int part) {
   const int begin = part * ((rest + parts - 1) / parts);

@@ -1,6 +1,7 @@
 // Answers, for lines of sizes on standard input, what csrc/launch_rules.h chooses: host code only (g++).
 //   fwgemm <f64> <image> <m> <n> <k>       1: one thread per element, 2: tiles of 128 x 128, 3: of 64 x 128
 //   staged <m> <n> <batch> <full m> <full n>   1: the full-size tile in two groups, 0: not (quarter-size: 64 x 64)
+//   half <ordered> <bits> <zeros> <m> <n> <products>   rows of the binary16 tile
 //   share <rest> <parts> <part>            where the part of a ragged k-tile begins
 #include <cstdio>
 #include <cstring>
@@ -16,6 +17,11 @@ int main() {
       if (std::scanf("%d %d %d %d %d", &f64, &image, &m, &n, &k) != 5) return 2;
       const long long half_tiles = (long long)((m + 63) / 64) * ((n + 127) / 128);
       answer = cuasr_amd::fwgemm_one_thread_each(f64, image, m, n, k) ? 1 : f64 && cuasr_amd::fwgemm_f64_half_tile(image, m, half_tiles) ? 3 : 2;
+    } else if (!std::strcmp(what, "half")) {
+      int ordered, bits, zeros, m, n;
+      long long products;
+      if (std::scanf("%d %d %d %d %d %lld", &ordered, &bits, &zeros, &m, &n, &products) != 6) return 2;
+      answer = cuasr_amd::half_tile_rows(ordered, bits, zeros, m, n, products);
     } else if (!std::strcmp(what, "share")) {
       int rest, parts, part;
       if (std::scanf("%d %d %d", &rest, &parts, &part) != 3) return 2;

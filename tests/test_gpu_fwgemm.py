@@ -248,7 +248,8 @@ def test_apsp_blocked_floyd_warshall(oracle, n, pad, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("n", [113, 529, 1475, 2193])   # closed alone; beside tiles with a compute unit each; two workgroups on one
+# one block and five, closed alone; beside tiles with a compute unit each; beside tiles of which two workgroups share one
+@pytest.mark.parametrize("n", [113, 529, 1475, 2193])
 def test_apsp_blocked_keeps_the_sign_of_a_zero(oracle, n, dtype):
     """Edges of weight +0 and -0: a sum of two -0 is -0, and the strict comparison keeps whichever zero was
     there first, where a hardware minimum would prefer -0.  The diagonal blocks that hold a -0 are closed by
@@ -278,8 +279,8 @@ def test_apsp_blocked_keeps_the_sign_of_a_zero(oracle, n, dtype):
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 # a last block of one vertex, of a chunk of sixteen and one less or more; one short of whole, whole, and one block alone; the
-# smallest n whose blocks are closed beside tiles
-@pytest.mark.parametrize("n,pad", [(100, 1), (129, 0), (143, 1), (144, 3), (145, 0), (255, 1), (256, 3), (271, 2), (929, 1), (1038, 5)])
+# smallest n whose blocks are closed beside tiles (double 769, float 929); a last block of one vertex beside tiles in both types
+@pytest.mark.parametrize("n,pad", [(100, 1), (129, 0), (143, 1), (144, 3), (145, 0), (255, 1), (256, 3), (271, 2), (769, 0), (929, 1), (1025, 2), (1038, 5)])
 def test_apsp_blocked_panels_of_ragged_blocks(oracle, n, pad, dtype):
     """Panels in place, sixteen lines to a workgroup: dense weights whose sums round, odd leading dimensions of both
     matrices, nothing written past them; dist and parent equal the oracle's bit for bit."""

@@ -12,6 +12,25 @@ TILE_PAIRS = [("minimum", "plus"), ("maximum", "plus"), ("minimum", "maximum"), 
               ("minimum", "multiplies"), ("maximum", "multiplies"), ("logical_or", "logical_and")]
 OTHER_PAIRS = [("plus", "maximum"), ("logical_or", "plus")]     # (pairs no tile serves: the naive kernel)
 LAYOUTS = ["ccc", "rrr", "crc", "rcr", "rcc", "crr", "ccr", "rrc"]
+# Sizes by the rows of the tile that the size rule gives them (test_launch_rules.py asks the rule).
+# rows, pair, m, n, k, beta_one
+EVERY_TILE = [
+    (128, "minimum", "plus", 4096, 4096, 64, True),         # 512 full tiles, unguarded
+    (128, "maximum", "minimum", 4095, 4095, 70, False),     # full tiles, ragged: guarded
+    (64, "maximum", "minimum", 4000, 4100, 70, False),      # four rounds of 64 x 128 tiles and a little
+    (64, "minimum", "plus", 2048, 2048, 96, True),          # 64 x 128 tiles, k shared out between two pairs of waves
+    (64, "plus", "multiplies", 1000, 2050, 50, True),       # 64 x 128 tiles, whole k-tiles per thread, ragged
+    (64, "plus", "multiplies", 2048, 2048, 64, False),      # ... and whole tiles
+    (32, "plus", "multiplies", 1000, 2000, 50, True),
+    (32, "maximum", "plus", 1536, 1536, 64, True),          # 32 x 128 tiles, k shared out between the waves
+    (16, "maximum", "plus", 1024, 1024, 64, True),          # 16 x 128 tiles, likewise
+    (32, "plus", "multiplies", 1024, 1024, 64, True),       # 32 x 128 tiles, whole k-tiles per thread
+]
+# m, n, k: 64 x 128 tiles for every order-free pair
+TWO_PAIRS = [(1985, 2001, 9), (2000, 1999, 17), (1991, 2047, 32), (2047, 2047, 33), (2048, 1921, 33), (1984, 2048, 64), (2001, 1993, 77),
+             (2048, 2000, 96)]
+TWO_PAIRS_SLICED = (1009, 1003, 203, 4)   # m, n, k, slices
+RAGGED_K = (1999, 2001)                   # m, n
 
 
 def operands(add, mult, m, n, k, la, lb, lc, seed=1):
@@ -72,13 +91,8 @@ def test_packed_tile(oracle, lib, sr, layouts):
 def test_every_tile_size(oracle, lib, layouts):
     """The kernel comes in several tile sizes, picked by how many workgroups the output gives the chip: the full
     tile unguarded (whole tiles of aligned operands) and guarded, the 64 x 128 tile, the 32 x 128 tile."""
-    check(oracle, "minimum", "plus", 4096, 4096, 64, layouts, "valu")              # 512 full tiles, unguarded
-    check(oracle, "maximum", "minimum", 4000, 4100, 70, layouts, "valu", False)    # full tiles, ragged: guarded
-    check(oracle, "minimum", "plus", 2048, 2048, 96, layouts, "valu")              # 64 x 128 tiles, k shared out between two pairs of waves
-    check(oracle, "plus", "multiplies", 1000, 2000, 50, layouts, "valu")           # 64 x 128 tiles, ragged
-    check(oracle, "maximum", "plus", 1536, 1536, 64, layouts, "valu")              # 32 x 128 tiles, k shared out between the waves
-    check(oracle, "maximum", "plus", 1024, 1024, 64, layouts, "valu")              # 16 x 128 tiles, likewise
-    check(oracle, "plus", "multiplies", 1024, 1024, 64, layouts, "valu")           # 32 x 128 tiles, whole k-tiles per thread
+    for _, add, mult, m, n, k, beta_one in EVERY_TILE:
+        check(oracle, add, mult, m, n, k, layouts, "valu", beta_one)
 
 
 @pytest.mark.parametrize("sr", [x for x in TILE_PAIRS if x[0] != "plus"])
@@ -89,7 +103,7 @@ def test_k_shared_out_between_waves(oracle, lib, sr, layouts):
     shorter than a quarter; extents that are no multiple of anything; and the split-K forms on top."""
     for k in (3, 9, 17, 31, 32, 45, 64, 250):
         check(oracle, *sr, 520, 390, k, layouts, "valu", beta_one=bool(k & 1))       # 16 x 128 tiles
-    check(oracle, *sr, 1530, 1300, 77, layouts, "valu")                             # 32 x 128 tiles
+    check(oracle, *sr, 1530, 1300, 77, layouts, "valu")                             # 32 x 128 tiles (or-and: 64 x 128)
     check(oracle, *sr, 1530, 1300, 32, layouts, "valu", beta_one=False)
     check(oracle, *sr, 300, 260, 500, layouts, "valu", splitk=5)
 
@@ -100,9 +114,10 @@ def test_k_shared_out_between_two_pairs_of_waves(oracle, lib, sr, layouts):
     """The 64 x 128 tile of the order-free adds: two halves of every k-tile, two k-tiles in flight.  k inside the
     first and the second half of the only tile, one, two and three tiles, a ragged third; rows and columns one short
     of, at and one past a tile's or a vector's end (outputs go out as vectors at any element boundary); slices."""
-    for m, n, k in [(1985, 2001, 9), (2000, 1999, 17), (1991, 2047, 32), (2047, 2049, 33), (1984, 2048, 64), (2001, 1993, 77), (2048, 2000, 96)]:
+    for m, n, k in TWO_PAIRS:
         check(oracle, *sr, m, n, k, layouts, "valu", beta_one=bool(m & 1))
-    check(oracle, *sr, 1009, 1003, 203, layouts, "valu", splitk=4)
+    m, n, k, slices = TWO_PAIRS_SLICED
+    check(oracle, *sr, m, n, k, layouts, "valu", splitk=slices)
 
 
 @pytest.mark.parametrize("sr", [("minimum", "plus"), ("maximum", "multiplies"), ("logical_or", "logical_and")])
@@ -111,7 +126,7 @@ def test_two_parts_of_a_ragged_k_tile(oracle, lib, sr, layouts):
     """The last k-tile of the 64 x 128 tile goes to its two parts by halves: one k (the second part has none), an odd number
     and an even one, one short of a whole tile; as the only tile and after one or two whole ones."""
     for k in (1, 2, 7, 31, 33, 43, 44, 63, 80):
-        check(oracle, *sr, 1999, 2001, k, layouts, "valu", beta_one=bool(k & 1))
+        check(oracle, *sr, *RAGGED_K, k, layouts, "valu", beta_one=bool(k & 1))
 
 
 def test_selected_family(lib):
@@ -141,7 +156,7 @@ def test_every_pair(oracle, lib, sr, kernel):
 def test_boolean_closure_on_masks(oracle, lib, layouts):
     """or-and (functional.h:212, :252): the tile works on 16-bit masks; sparse operands so that the answer is
     not all ones, every tile size, an identity that is not zero, alpha / beta that are zero or not."""
-    check(oracle, "logical_or", "logical_and", 1024, 1024, 64, layouts, "valu")      # 32 x 128 tiles
+    check(oracle, "logical_or", "logical_and", 1024, 1024, 64, layouts, "valu")      # 16 x 128 tiles
     check(oracle, "logical_or", "logical_and", 2048, 2048, 40, layouts, "valu")      # 64 x 128 tiles
     check(oracle, "logical_or", "logical_and", 4096, 4096, 32, layouts, "valu")      # full tiles, unguarded
     check(oracle, "logical_or", "logical_and", 4000, 4100, 37, layouts, "valu", beta_one=False)

@@ -145,7 +145,8 @@ def test_or_and_large_outputs_on_packed_masks(oracle, lib, dtype, layouts):
     npd = NPD[dtype]
     la, lb, lc = [{"c": "col", "r": "row"}[x] for x in layouts]
     for (m, n, k), ident, alpha, beta in (((4096, 3072, 64), 0, 1, 1), ((4000, 4100, 37), 0, 1, 0), ((4000, 4100, 37), 0, 0, 1),
-                                          ((3968, 3328, 33), 2.5, 1, 1), ((2048, 2048, 40), 0, 1, 0)):   # (the last: on masks for f64 only)
+                                          ((3968, 3328, 33), 2.5, 1, 1), ((2048, 2048, 40), 0, 1, 0),
+                                          ((1999, 2001, 37), 0, 1, 1)):   # (the last two: on masks for f64 only, in 64 x 128 tiles)
         A, B = sparse(31, m, k, npd, order_of(la), 0.06), sparse(32, k, n, npd, order_of(lb), 0.06)
         C = sparse(33, m, n, npd, order_of(lc), 0.3)
         if dtype in ("f32", "f64"):

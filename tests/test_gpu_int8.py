@@ -9,6 +9,10 @@ from helpers import assert_same_bits, order_of, to_device
 pytestmark = pytest.mark.gpu
 
 LAYOUTS = ["ccc", "rrr", "crc", "rcr", "rcc", "crr", "ccr", "rrc"]
+# Sizes by the rows of the packed tile that the size rule gives them (test_launch_rules.py asks the rule).
+FULL_GUARDED = (4095, 4095)                                                                     # 128 rows
+TWO_PAIRS = [(1985, 2001, 9), (1991, 2047, 17), (2047, 2047, 32), (2048, 1921, 32), (2001, 1993, 77)]   # 64 rows
+RAGGED_K = (1999, 2001)                                                                         # 64 rows
 
 
 def operands(m, n, k, la, lb, lc, seed=1):
@@ -87,14 +91,15 @@ def test_tropical_pairs_on_the_packed_tile(oracle, lib, sr, layouts):
     check(oracle, *sr, 1, 1, 1, layouts, "valu")
     check(oracle, *sr, 2048, 2048, 96, layouts, "valu", alpha=7, beta=-3)    # 64 x 128 tiles
     check(oracle, *sr, 4096, 4096, 64, layouts, "valu")                      # full tiles, unguarded
-    check(oracle, *sr, 4000, 4100, 70, layouts, "valu", alpha=-100, beta=100)  # full tiles, guarded
+    check(oracle, *sr, 4000, 4100, 70, layouts, "valu", alpha=-100, beta=100)  # 64 x 128 tiles, four rounds (bitwise: full, guarded)
+    check(oracle, *sr, *FULL_GUARDED, 70, layouts, "valu", alpha=-100, beta=100)  # full tiles, guarded
 
 
 @pytest.mark.parametrize("sr", [("minimum", "plus"), ("maximum", "multiplies"), ("bit_xor", "bit_and")])
 @pytest.mark.parametrize("layouts", ["ccc", "rcr", "crr", "rrc"])
 def test_k_shared_out_between_two_pairs_of_waves(oracle, lib, sr, layouts):
     """64 x 128 tiles at extents that are no multiple of a tile or a vector, k ending in either half of a k-tile."""
-    for m, n, k in [(1985, 2001, 9), (1991, 2047, 17), (2047, 2049, 32), (2001, 1993, 77)]:
+    for m, n, k in TWO_PAIRS:
         check(oracle, *sr, m, n, k, layouts, "valu", alpha=7, beta=-3)
 
 
@@ -102,7 +107,7 @@ def test_k_shared_out_between_two_pairs_of_waves(oracle, lib, sr, layouts):
 def test_two_parts_of_a_ragged_k_tile(oracle, lib, sr):
     """As for binary16: one k, an odd number, an even one, after no and after two whole k-tiles."""
     for k in (1, 7, 31, 80):
-        check(oracle, *sr, 1999, 2001, k, "crr", "valu")
+        check(oracle, *sr, *RAGGED_K, k, "crr", "valu")
 
 
 @pytest.mark.parametrize("layouts", ["ccc", "rcr", "crr", "rrc"])

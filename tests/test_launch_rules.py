@@ -45,3 +45,30 @@ def test_a_ragged_k_tile_is_shared_out_evenly():
         assert begin[0] == 0 and begin[-1] == rest
         sizes = [end - first for first, end in zip(begin, begin[1:])]
         assert min(sizes) >= 0 and max(sizes) == (rest + parts - 1) // parts
+
+
+def _half(add, mult, m, n, products=1, int8=False):
+    bits = mult in ("logical_and", "bit_and")
+    return f"half {int(add == 'plus')} {int(bits)} {int(mult == 'multiplies' and not int8)} {m} {n} {products}"
+
+
+def test_binary16_tile_sizes():
+    """The tile that the tests of each tile's edges say they run, and 64 x 128 against 32 x 128 on both sides of the line at sizes
+    where both were timed."""
+    import test_gpu_half as half
+    import test_gpu_int8 as int8
+    asked = [(_half(add, mult, m, n), rows) for rows, add, mult, m, n, *_ in half.EVERY_TILE]
+    for add, mult in half.TILE_PAIRS:
+        if add == "plus":
+            continue
+        asked += [(_half(add, mult, m, n), 64) for m, n, _ in half.TWO_PAIRS]
+        m, n, _, slices = half.TWO_PAIRS_SLICED
+        asked += [(_half(add, mult, m, n, slices), 64), (_half(add, mult, *half.RAGGED_K), 64)]
+    for add, mult in [("minimum", "plus"), ("maximum", "multiplies"), ("bit_xor", "bit_and"), ("logical_or", "logical_and")]:
+        asked += [(_half(add, mult, m, n, int8=True), 64) for m, n, _ in int8.TWO_PAIRS]
+        asked += [(_half(add, mult, *int8.RAGGED_K, int8=True), 64), (_half(add, mult, *int8.FULL_GUARDED, int8=True), 128)]
+    asked += [(_half("logical_or", "logical_and", 1999, 2001), 64), (_half("logical_or", "logical_and", 2048, 2048), 64)]   # double
+    asked += [(_half("minimum", "plus", m, n), rows) for m, n, rows in
+              [(960, 2048, 32), (1216, 2048, 32), (1500, 1500, 32), (1664, 1664, 32), (1792, 1792, 64), (2048, 2176, 32), (2304, 2304, 64),
+               (2560, 2560, 64), (3000, 2900, 64)]]
+    assert _ask([question for question, _ in asked]) == [rows for _, rows in asked]
