@@ -337,13 +337,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
             for (int g = 0; g < NG; ++g)
               two_terms<ADD, MUL, I16>(acc[i][4 * g + j], both(a0[i]), pair_of(b0[g], j), both(a1[i]), pair_of(b1[g], j));
       }
-    } else {
-      // the ragged last k-tile, a term at a time.  KS = 2: half of what there is of it to each part, operands of two k
-      // read together (by halves of a whole k-tile the second part has nothing to do beside the first one's sixteen: see the
-      // short k above)
-      const int rest = ke - k0;
-      int kk = KS == 2 ? ragged_share(rest, KS, part) : kf;
-      const int last = KS == 2 ? ragged_share(rest, KS, part + 1) : min(kf + KW, rest);
+    } else if constexpr (KS == 2) {
+      // the ragged last k-tile, a term at a time: half of what there is of it to each part, operands of two k read together
+      // (by halves of a whole k-tile the second part has nothing to do beside the first one's sixteen: see the short k above)
+      const int rest = ke - k0, last = ragged_share(rest, KS, part + 1);
+      int kk = ragged_share(rest, KS, part);
       auto terms = [&](auto count) {
         constexpr int N = count.value;
         rows_t a[N];
@@ -363,9 +361,21 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
               for (int g = 0; g < NG; ++g) one_term<ADD, MUL, I16>(acc[i][4 * g + j], both(a[u][i]), pair_of(b[u][g], j));
       };
-      if constexpr (KS == 2)
-        for (; kk + 1 < last; kk += 2) terms(std::integral_constant<int, 2>());
-      for (; kk < last; ++kk) terms(std::integral_constant<int, 1>());
+      for (; kk + 1 < last; kk += 2) terms(std::integral_constant<int, 2>());
+      if (kk < last) terms(std::integral_constant<int, 1>());
+    } else {
+      for (int kk = kf; kk < min(kf + KW, ke - k0); ++kk) {  // the ragged last k-tile
+        const rows_t a0 = *reinterpret_cast<const rows_t *>(&pa[kk][ty * TR]);
+        h8 b0[NG];
+#pragma unroll
+        for (int g = 0; g < NG; ++g) b0[g] = *reinterpret_cast<const h8 *>(&pb[kk][g * 128 + tx * 8]);
+#pragma unroll
+        for (int i = 0; i < TR; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int g = 0; g < NG; ++g) one_term<ADD, MUL, I16>(acc[i][4 * g + j], both(a0[i]), pair_of(b0[g], j));
+      }
     }
     if (t + 1 < tiles_k) {
       sa[next].store(sm.a[s ^ 1]);
