@@ -1646,22 +1646,26 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
   char *C = R + es * FW_BLOCK * size_t(nn);
   char *Ct = C + es * FW_BLOCK * size_t(nn);            // updated block column with k contiguous, leading dimension FW_BLOCK
   char *H = Ct + es * FW_BLOCK * size_t(nn);            // columns, rows and first state of the diagonal block being closed
-  // Block row and block column share one launch that works in place (beside tiles it reads the closed diagonal block and its
+  // Block row and block column share one launch that works in place (with copies it reads the closed diagonal block and its
   // transpose from C and R).  The other form, two launches of the tiled kernel on copies of the panels in R (leading dimension
   // FW_BLOCK) and C (leading dimension nn), is slower at every size, also where each of its products fills the chip; ms a job in
   // one launch / tiled: f32 n = 8192 31 / 37, 16384 218 / 227, 20000 395 / 406, 30000 1238 / 1256, f64 8192 59 / 69, 16384 421 / 436,
   // 18000 555 / 570.
   const bool paired = panels != CUASR_AMD_PANELS_TILED;
   // With tiles a step's launch also closes the next block, after a launch that updates it; without, a closure alone on
-  // the chip takes most of a step.  us a job with tiles at density 0.02 and 0.5 / without: f32 n = 768 400, 380 / 352, 850 463, 439 /
+  // the chip takes most of a step.  us a job with tiles at density 0.02, 0.5 / without: f32 n = 768 400, 380 / 352, 850 463, 439 /
   // 423, 928 477, 454 / 472, 1000 527, 487 / 560; f64 640 625, 601 / 518, 768 728, 687 / 683, 832 802, 752 / 764, 850 825, 775 / 815,
   // 1024 921, 860 / 1102.
   const bool naive = n <= (f64 ? 768 : 928);
   // Where the closure hides beside a product it leaves the panels a copy of its block and of the transpose.  Alone on the chip
   // its stores are on the critical path (57.6 us a closure of doubles without them, 63.1 with; 31.6 and 34.0 of floats) and
   // the panels read the block from the matrix: f64 n = 130 / 464 / 768 119 / 382 / 709 us a job with copies, 113 / 368 / 683 from
-  // the matrix, f32 72 / 205 / 363 and 69 / 201 / 352.  With tiles, from the matrix: f32 n = 1000 487 -> 494, 2000 1006 -> 1018.
-  char *closed_copy = paired && !naive ? C : nullptr, *closed_copy_t = paired && !naive ? R : nullptr;
+  // the matrix, f32 72 / 205 / 363 and 69 / 201 / 352.  With tiles, from the matrix: f32 n = 1000 487 -> 494, 2000 1006 -> 1018,
+  // f64 1300 1210 -> 1219, 2800 3974 -> 3991.  But doubles with 18 to 20 blocks have 578 to 722 tiles (64 x 128) on 512 places, and
+  // the launch ends not long after the closure: from the matrix 2177 2858 -> 2807, 2304 2751 -> 2679, 2560 3238 -> 3218 (2450 3349 ->
+  // 3357 and, at half the edges, 3150 -> 3134).
+  const bool copies = paired && !naive && !(f64 && n > 17 * FW_BLOCK && n <= 20 * FW_BLOCK);
+  char *closed_copy = copies ? C : nullptr, *closed_copy_t = copies ? R : nullptr;
   // this step's diagonal block had its distances closed during the step before, beside that step's big product
   // (its predecessors are always still to be found, from what the closure recorded in H)
   bool closed = false;
@@ -1688,12 +1692,12 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
     const FwPanels panel{n, k0, bb, dist, ld, parent, ldp, closed_copy, closed_copy_t, Ct, H};
     if (paired) {
       const dim3 grid(fw_panel_groups(n, bb, true));
-      if (naive) {
-        if (f64) launch_kernel((fw_panels_kernel<double, false>), grid, dim3(FW_LINE_THREADS), 0, s, panel);
-        else launch_kernel((fw_panels_kernel<float, false>), grid, dim3(FW_LINE_THREADS), 0, s, panel);
-      } else {
+      if (copies) {
         if (f64) launch_kernel((fw_panels_kernel<double, true>), grid, dim3(FW_LINE_THREADS), 0, s, panel);
         else launch_kernel((fw_panels_kernel<float, true>), grid, dim3(FW_LINE_THREADS), 0, s, panel);
+      } else {
+        if (f64) launch_kernel((fw_panels_kernel<double, false>), grid, dim3(FW_LINE_THREADS), 0, s, panel);
+        else launch_kernel((fw_panels_kernel<float, false>), grid, dim3(FW_LINE_THREADS), 0, s, panel);
       }
       if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
     } else {
