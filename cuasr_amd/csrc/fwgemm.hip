@@ -137,56 +137,121 @@ template <typename T> struct FwLineLds {
 };
 constexpr int FW_LINE_THREADS = 512;
 
-// whole[k][line] = src[line + k * ld] for the first `lines` lines and `ks` k; +infinity from k = ks on, any value in lines
-// beyond (nobody stores those)
-template <typename T> __device__ __forceinline__ void fw_fetch_whole(FwLineLds<T> &sm, const T *src, int64_t ld, int lines, int ks) {
+// whole[k][line] = src[line + k * ld], lines up to `lines` (clamped; the rest are not stored by anybody)
+template <typename T> __device__ __forceinline__ void fw_fetch_whole(FwLineLds<T> &sm, const T *src, int64_t ld, int lines) {
+  typedef typename vec4_of<T>::type V4;
+  typedef typename uvec4_of<T>::type U4;
+  constexpr int N = FW_BLOCK * FW_BLOCK / 4 / FW_LINE_THREADS;
+  const int tid = threadIdx.x, line = (tid & 31) * 4, k0 = tid >> 5;
+  V4 v[N];
+  if (lines == FW_BLOCK) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) v[u] = *reinterpret_cast<const U4 *>(src + line + int64_t(k0 + u * (FW_LINE_THREADS / 32)) * ld);
+  } else {
+#pragma unroll 1
+    for (int u = 0; u < N; ++u) {
+      V4 x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = src[min(line + e, lines - 1) + int64_t(k0 + u * (FW_LINE_THREADS / 32)) * ld];
+      *reinterpret_cast<V4 *>(&sm.whole[k0 + u * (FW_LINE_THREADS / 32)][line]) = x;
+    }
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u) *reinterpret_cast<V4 *>(&sm.whole[k0 + u * (FW_LINE_THREADS / 32)][line]) = v[u];
+}
+
+// v[over], v[over + 1], ..., the last element in the place of those past the end
+template <typename V4> __device__ __forceinline__ V4 fw_from(const V4 v, int over) {
+  V4 r = v;
+#pragma unroll
+  for (int e = 0; e < 3; ++e)
+#pragma unroll
+    for (int o = 1; o <= 3 - e; ++o) r[e] = (o == 3 - e ? over >= o : over == o) ? v[e + o] : r[e];
+  return r;
+}
+// A closed block of bb rows where it lies: whole[k][line] = src[line + k * ld], +infinity from k = bb to the end of its chunk,
+// any value in lines beyond (nobody stores those).  Ragged blocks are fetched as vectors too, the one across the edge from
+// where it ends there (element by element, n = 240 in floats took 107.7 us a job, now 103.6).
+// (Of its own beside fw_fetch_whole: with both in one function a step beside tiles took 0.6 us longer.)
+template <typename T> __device__ __forceinline__ void fw_fetch_block(FwLineLds<T> &sm, const T *src, int64_t ld, int bb) {
   typedef typename vec4_of<T>::type V4;
   typedef typename uvec4_of<T>::type U4;
   const T inf = std::numeric_limits<T>::infinity();
   constexpr int N = FW_BLOCK * FW_BLOCK / 4 / FW_LINE_THREADS, STEP = FW_LINE_THREADS / 32;
+  static_assert(STEP == FwLineLds<T>::CK, "a chunk at a time");
   const int tid = threadIdx.x, line = (tid & 31) * 4, k0 = tid >> 5;
   V4 v[N];
-  if (lines == FW_BLOCK && ks == FW_BLOCK) {
+  if (bb == FW_BLOCK) {
 #pragma unroll
     for (int u = 0; u < N; ++u) v[u] = *reinterpret_cast<const U4 *>(src + line + int64_t(k0 + u * STEP) * ld);
   } else {
+    const int over = max(line + 4 - bb, 0);
 #pragma unroll
-    for (int u = 0; u < N; ++u)
+    for (int u = 0; u < N; ++u) {
+      if (u * STEP >= bb) break;
+      const int k = k0 + u * STEP;
+      const T *from = src + int64_t(min(k, bb - 1)) * ld;
+      if (bb >= 4) {
+        v[u] = *reinterpret_cast<const U4 *>(from + line - over);
+      } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const T x = src[min(line + e, lines - 1) + int64_t(min(k0 + u * STEP, ks - 1)) * ld];
-        v[u][e] = k0 + u * STEP < ks ? x : inf;
+        for (int e = 0; e < 4; ++e) v[u][e] = from[min(line + e, bb - 1)];
       }
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      if (u * STEP >= bb) break;
+      if (bb >= 4) v[u] = fw_from(v[u], over);
+      if (k0 + u * STEP >= bb) v[u] = V4{inf, inf, inf, inf};
+    }
   }
 #pragma unroll
-  for (int u = 0; u < N; ++u) *reinterpret_cast<V4 *>(&sm.whole[k0 + u * STEP][line]) = v[u];
+  for (int u = 0; u < N; ++u) {
+    if (u * STEP >= bb) break;
+    *reinterpret_cast<V4 *>(&sm.whole[k0 + u * STEP][line]) = v[u];
+  }
 }
 // whole[k][line] = src[k + line * ld], likewise: two neighbouring lanes take eight k of one line, so that a line of memory
 // is asked for in 32 or 64 bytes at once and the stores of an instruction meet two to a bank
-template <typename T> __device__ __forceinline__ void fw_fetch_turned(FwLineLds<T> &sm, const T *src, int64_t ld, int lines, int ks) {
+template <typename T> __device__ __forceinline__ void fw_fetch_turned(FwLineLds<T> &sm, const T *src, int64_t ld, int bb) {
   typedef typename vec4_of<T>::type V4;
   typedef typename uvec4_of<T>::type U4;
   const T inf = std::numeric_limits<T>::infinity();
-  constexpr int N = FW_BLOCK * FW_BLOCK / 4 / FW_LINE_THREADS;
+  constexpr int N = FW_BLOCK * FW_BLOCK / 4 / FW_LINE_THREADS, STEP = FwLineLds<T>::CK;
   const int tid = threadIdx.x, line = (tid >> 1) & 127, k0 = (tid & 1) * 4 + (tid >> 8) * 8;
+  src += int64_t(min(line, bb - 1)) * ld;
   V4 v[N];
-  if (lines == FW_BLOCK && ks == FW_BLOCK) {
+  if (bb == FW_BLOCK) {
 #pragma unroll
-    for (int u = 0; u < N; ++u) v[u] = *reinterpret_cast<const U4 *>(src + k0 + u * 16 + int64_t(line) * ld);
+    for (int u = 0; u < N; ++u) v[u] = *reinterpret_cast<const U4 *>(src + k0 + u * STEP);
   } else {
-    src += int64_t(min(line, lines - 1)) * ld;
 #pragma unroll
-    for (int u = 0; u < N; ++u)
+    for (int u = 0; u < N; ++u) {
+      if (u * STEP >= bb) break;
+      const int k = k0 + u * STEP;
+      if (bb >= 4) {
+        v[u] = *reinterpret_cast<const U4 *>(src + min(k, bb - 4));
+      } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const T x = src[min(k0 + u * 16 + e, ks - 1)];
-        v[u][e] = k0 + u * 16 + e < ks ? x : inf;
+        for (int e = 0; e < 4; ++e) v[u][e] = src[min(k + e, bb - 1)];
       }
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      if (u * STEP >= bb) break;
+      const int k = k0 + u * STEP;
+      if (bb >= 4) v[u] = fw_from(v[u], k - min(k, bb - 4));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[u][e] = k + e < bb ? v[u][e] : inf;
+    }
   }
 #pragma unroll
-  for (int u = 0; u < N; ++u)
+  for (int u = 0; u < N; ++u) {
+    if (u * STEP >= bb) break;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) sm.whole[k0 + u * 16 + e][line] = v[u][e];
+    for (int e = 0; e < 4; ++e) sm.whole[k0 + u * STEP + e][line] = v[u][e];
+  }
 }
 
 // lane's line `line` of the whole operand with lines first .. first + NC - 1 of the other, chunks of CK k
@@ -279,8 +344,8 @@ template <typename T, bool COPIES> __device__ __forceinline__ void fw_row_panel(
       }
     }
   }
-  if constexpr (COPIES) fw_fetch_whole<T>(sm, static_cast<const T *>(p.closed), FW_BLOCK, FW_BLOCK, FW_BLOCK);
-  else fw_fetch_whole<T>(sm, row0 + int64_t(p.k0) * p.ld, p.ld, p.bb, p.bb);
+  if constexpr (COPIES) fw_fetch_whole<T>(sm, static_cast<const T *>(p.closed), FW_BLOCK, FW_BLOCK);
+  else fw_fetch_block<T>(sm, row0 + int64_t(p.k0) * p.ld, p.ld, p.bb);
   *reinterpret_cast<V4 *>(&sm.other[tid >> 5][(tid & 31) * 4]) = v;
   __syncthreads();
   const int i = tid & 127, first = __builtin_amdgcn_readfirstlane(tid >> 7) * 4;
@@ -326,8 +391,8 @@ template <typename T, bool COPIES> __device__ __forceinline__ void fw_col_panel(
   typedef typename uvec4_of<T>::type U4;
   T *const col0 = static_cast<T *>(p.dist) + int64_t(p.k0) * p.ld;
   const V4 v = fw_fetch_across<T>(col0 + r0, p.ld, p.n - r0, p.bb);
-  if constexpr (COPIES) fw_fetch_whole<T>(sm, static_cast<const T *>(p.closed_t), FW_BLOCK, FW_BLOCK, FW_BLOCK);
-  else fw_fetch_turned<T>(sm, col0 + p.k0, p.ld, p.bb, p.bb);
+  if constexpr (COPIES) fw_fetch_whole<T>(sm, static_cast<const T *>(p.closed_t), FW_BLOCK, FW_BLOCK);
+  else fw_fetch_turned<T>(sm, col0 + p.k0, p.ld, p.bb);
   fw_put_across<T>(sm, v);
   __syncthreads();
   const int tid = threadIdx.x, j = tid & 127, first = __builtin_amdgcn_readfirstlane(tid >> 7) * 4;
@@ -386,7 +451,7 @@ template <typename T> __device__ __forceinline__ void fw_parents(const FwPanels 
 #pragma unroll
   for (int c = 0; c < 4; ++c) curr[c] = init[i + (c0 + first + c) * FW_BLOCK];
   const typename vec4_of<T>::type v = fw_fetch_across<T>(hist_row + c0, FW_BLOCK, FwLineLds<T>::LINES, p.bb);
-  fw_fetch_whole<T>(sm, hist_col, FW_BLOCK, FW_BLOCK, FW_BLOCK);   // (rows of k beyond the last chunk hold anything and are not read)
+  fw_fetch_whole<T>(sm, hist_col, FW_BLOCK, FW_BLOCK);   // (rows of k beyond the last chunk hold anything and are not read)
   fw_put_across<T>(sm, v);
   __syncthreads();
   fw_lines<T, 4>(sm, i, first, (p.bb + 15) / 16, p.k0, curr, par);
@@ -432,7 +497,7 @@ template <typename T> __global__ void __launch_bounds__(FW_LINE_THREADS) fw_ahea
   T curr[1] = {block[row + int64_t(col_in) * p.ld]};
   int32_t par[1];
   const T b = (static_cast<const T *>(p.dist) + p.k0 + int64_t(a0 + col_in) * p.ld)[i];
-  fw_fetch_whole<T>(sm, static_cast<const T *>(p.dist) + a0 + int64_t(p.k0) * p.ld, p.ld, abb, FW_BLOCK);
+  fw_fetch_whole<T>(sm, static_cast<const T *>(p.dist) + a0 + int64_t(p.k0) * p.ld, p.ld, abb);
   sm.other[first][i] = b;
   __syncthreads();
   fw_lines<T, 1>(sm, i, first, FW_BLOCK / 16, p.k0, curr, par);
@@ -847,8 +912,8 @@ __device__ __forceinline__ void fwgemm_tile_body(const FwArgs &g, const int bloc
 // predecessors are those of one min-plus product with predecessor tracking (fwgemm's own semantics, strict
 // comparison, k ascending) of a matrix whose column k is "column k before step k" with one whose row k is
 // "row k before step k", started from the block as it was before the closure.  Nothing of that product is on the
-// critical path: nothing that follows reads a diagonal block's predecessors, and the product is spread over 64
-// workgroups of a later launch.
+// critical path: nothing that follows reads a diagonal block's predecessors, and the product is at most eight
+// workgroups of a later launch (fw_parents, sixteen columns each).
 //
 // What stays on the critical path is fw_close_dist: the 128 dependent steps for the distances alone, by one workgroup.
 // They are taken in strips of sixteen.  The steps of a strip read nothing but its sixteen rows and its sixteen columns,

@@ -278,10 +278,11 @@ def test_apsp_blocked_keeps_the_sign_of_a_zero(oracle, n, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-# a last block of one vertex, of a chunk of sixteen and one less or more; one short of whole, whole, and one block alone; the
-# smallest n whose blocks are closed beside tiles (double 769, float 929); a last block of one vertex beside tiles in both types
-# beside tiles, the panels reading the closed block from the matrix (double)
-@pytest.mark.parametrize("n,pad", [(100, 1), (129, 0), (143, 1), (144, 3), (145, 0), (255, 1), (256, 3), (271, 2), (769, 0), (929, 1), (1025, 2), (1038, 5), (2182, 1)])
+# a last block of one vertex, of less than a vector, of one and a vector, of a chunk of sixteen and one less or more; one short
+# of whole, whole, and one block alone; the smallest n whose blocks are closed beside tiles (double 769, float 929); a last block
+# of one vertex beside tiles in both types; beside tiles, the panels reading the closed block from the matrix (double)
+@pytest.mark.parametrize("n,pad", [(3, 1), (100, 1), (129, 0), (130, 0), (131, 2), (133, 1), (143, 1), (144, 3), (145, 0), (255, 1), (256, 3),
+                                   (271, 2), (769, 0), (929, 1), (1025, 2), (1038, 5), (2182, 1)])
 def test_apsp_blocked_panels_of_ragged_blocks(oracle, n, pad, dtype):
     """Panels in place, sixteen lines to a workgroup: dense weights whose sums round, odd leading dimensions of both
     matrices, nothing written past them; dist and parent equal the oracle's bit for bit."""
