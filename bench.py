@@ -582,7 +582,7 @@ def extra_configs(np, torch, cuasr_amd, inputs, oracle, base_args):
     cuasr_amd.apsp_blocked(gd, gp, gws)
     torch.cuda.synchronize()
     exact = bool(np.ascontiguousarray(gd.cpu().numpy()).tobytes() == np.ascontiguousarray(hd).tobytes() and (gp.cpu().numpy() == hp).all())
-    out.append(entry(wl, ms, steps, "fw_close + fwgemm_pair + fwgemm_tile (closing the next diagonal block)",
+    out.append(entry(wl, ms, steps, "fw_close + fw_panels + fw_ahead + fwgemm_tile (closing the next diagonal block)",
                      bit_exact=exact, checked=f"dist and parent of the same job at n = {nc}"))
     return out
 

@@ -267,7 +267,8 @@ static int pick_family(const cuasr_amd_srgemm_desc *d, long long batch = 1) {
   if (streamk_preferred(d, batch)) return kStreamK;
   // min-plus / max-plus and, nearer to a full round, bit operations, which would otherwise share their tiles out
   // (generalised to every pair, type and share of the round, the rule lost as often as it won; xor-and on words at
-  // 2560^3, 200 tiles: 63 against 66 TOPS on the staged tile)
+  // 2560^3, 200 tiles, where the staged tile has no ragged edge: 63 against 66 TOPS on it; at 2500^3, where it has one, the
+  // rule is the slower choice: 459 - 523 us by layout on plain direct tiles, 534 - 553 on the staged ones)
   if (batch == 1 && d->split_k_slices == 1 && streamk_usable(d) && one_tile_each(d, c)) return kDirect;
   if (direct_usable(d) && ((fills && !((both_kc || masked || slow_direct) && have_valu)) || !have_valu)) return kDirect;
   if (have_valu) return kValu;
