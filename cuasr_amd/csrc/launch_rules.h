@@ -15,6 +15,112 @@ inline bool two_group_full_tile(long long full, long long quarter, int area_rati
   return full >= 192 && full <= 256 && quarter > 256LL * (area_ratio - 1);
 }
 
+// The block of 32 x 32 (small_tile.h), against the 64 x 64 staged tile with its k range shared out over 1024 threads, which is
+// the better one from about 176 workgroups on
+// (min-plus f32, 60 % of the chip's compute units: 832^3, 169 of them, 30.3 against 26.8 us here; 896^3, 196, 31.5
+// against 36.5), for 8-byte elements from 128 (640^3, 100: 47.9 against 34.3 us; 768^3, 144: 56.8 against 56.1; 832^3:
+// 60.8 against 62.5; this kernel's double figures are 6 - 10 % lower since, 512^3 17.6 -> 15.7).
+inline bool small_blocks_preferred(bool f64, int m, int n, long long products) {
+  const long long groups64 = (m + 63LL) / 64 * ((n + 63LL) / 64) * products;
+  if (groups64 <= (f64 ? 128 : 176)) return true;
+  // ... and where 64 x 64 tiles would cover 1.6 times as much as 32 x 32 blocks, which is more than their better rate is
+  // worth on 4-byte elements (1000 products of 32^3: 10.5 us there, 6.8 here; 100 of 80^3, 1.78 times: 13.0 and 9.6;
+  // 64 of 100^3, the same cover: 11.2 and 11.4)
+  const long long groups32 = (m + 31LL) / 32 * ((n + 31LL) / 32) * products;
+  return !f64 && groups32 * 10 <= groups64 * 25;
+}
+
+// The staged family's full-size tile (128 x 128, 8-byte elements 128 x 64), against the quarter-size one of 64 x 64.
+// The chip holds 1024 full-size workgroups at a time (four per compute unit),
+// and a launch runs in rounds of that many.  The full-size tile is a few per
+// cent faster than the quarter-size one when its workgroups fill whole rounds
+// (4096^2: exactly one), and much slower when a round is mostly empty (fewer
+// than 1024 workgroups: split-K of a small output, matrices below ~3000^2) or
+// the last round is (5120^2: 1.56 rounds).  The quarter-size tile -- four times
+// as many, shorter workgroups -- balances in all those cases, so the full-size
+// one is used only when at least 95 % of its rounds are filled ...
+inline bool quarter_tile_preferred(long long full, long long full_area, long long quarter) {
+  // ... and those tiles do not reach much further past the edges than the quarter-size ones: a batch of 1000 products of
+  // 64 x 64 filled 1000 full-size tiles to a quarter (37.8 us; 18.2 on the quarter-size ones).  An eighth more is less than
+  // their rate is worth (940 x 16384 x 500, a fifteenth more, both operands k-contiguous: 246 us, 261 on the smaller ones)
+  const long long rounds = (full + 1023) / 1024;
+  return full * full_area * 8 > quarter * 4096 * 9 || full * 100 < rounds * 1024 * 95;
+}
+
+// Tiles of one launch on the vector ALU, and about how long they take.  Of `blocks` of them the fullest of the 256 compute
+// units gets n = ceil(blocks / 256); the launch then takes about
+//   fixed + n (per_k k / 1000 + each)   us, with `lone` in the place of per_k where n = 1 (half the waves).
+// Fitted to min-plus on 290 float and 270 double products (64 .. 4096 each way, squares from 200, four layouts); the
+// deviation is 3 - 8 % (root mean square).
+struct TileTime {
+  double fixed, lone, per_k, each;
+};
+inline double tile_us(const TileTime &t, long long blocks, double k) {
+  const double n = double((blocks + 255) / 256);
+  return t.fixed + (n > 1 ? n * t.per_k : t.lone) * k / 1000 + n * t.each;
+}
+
+// The blocks of small_tile.h, rows x columns of an output, for adds that may count a term twice.
+struct BlockShape {
+  int rows, cols;
+};
+struct BlockTime {
+  BlockShape shape;
+  TileTime time;
+};
+constexpr BlockTime block_times_4[] = {{{32, 32}, {2.9, 10.6, 9.1, 1.23}}, {{48, 32}, {2.8, 13.8, 12.1, 1.42}}, {{64, 32}, {3.06, 16.3, 15.3, 1.58}},
+                                       {{48, 48}, {3.4, 18.8, 17.4, 2.08}}, {{64, 48}, {3.1, 25.1, 23.0, 2.05}}, {{64, 64}, {3.5, 29.7, 28.7, 2.27}}};
+constexpr BlockTime block_times_8[] = {{{32, 32}, {2.75, 25.0, 20.0, 1.7}}, {{40, 32}, {2.63, 27.6, 21.8, 1.73}}, {{48, 32}, {2.6, 31.2, 25.2, 1.92}},
+                                       {{48, 48}, {0.8, 42.5, 42.1, 4.85}}};
+// ... and the staged family's: 64 x 64 with k shared by four, two and one group of threads, the full-size tile
+// (float 128 x 128, double 128 x 64) with one and two
+constexpr TileTime quarter4_4{5.7, 30.9, 30.9, 0.2}, quarter2_4{3.8, 31.3, 31.3, 1.3}, quarter1_4{1.4, 86, 33.6, 2.5}, full1_4{-1.5, 199, 112, 9.7}, full2_4{1.0, 105, 109, 10.3};
+constexpr TileTime quarter4_8{6.1, 65.9, 65.9, 0}, quarter2_8{5.9, 65.5, 65.5, 1.2}, quarter1_8{5.6, 76.7, 70.3, 0.6}, full1_8{2.3, 177, 143.5, 3.1}, full2_8{-0.1, 136, 138, 6.7};
+
+// The fastest of the blocks by those times, or {0, 0} where the staged family's tile (which of them, the launch decides) or
+// the block of 32 x 32 that it would take is faster.  k: one product's or slice's; products: of a batch, or slices.
+// What it is about is how evenly an output divides over the compute units: 1533^3 is 576 tiles of 64 x 64, three on some
+// units and two on most (148 us), 768 blocks of 64 x 48, three on all (118); double 600 x 500 x 700 304 blocks of
+// 32 x 32 (33.5 us), 240 of 40 x 32 (22); 1053^3 73 us on 64 x 64, 45 on 48 x 48.
+inline BlockShape block_shape(bool f64, int m, int n, double k, long long products, double staged_us) {
+  const BlockTime *times = f64 ? block_times_8 : block_times_4;
+  const int count = f64 ? int(sizeof(block_times_8) / sizeof(BlockTime)) : int(sizeof(block_times_4) / sizeof(BlockTime));
+  BlockShape best{0, 0};
+  double best_us = staged_us;
+  for (int i = 0; i < count; ++i) {
+    const BlockShape s = times[i].shape;
+    if (m < s.rows || n < s.cols) continue;
+    const long long blocks = ((long long)m + s.rows - 1) / s.rows * (((long long)n + s.cols - 1) / s.cols) * products;
+    // (the waves of a block take whole chunks of 64 bytes: short k is worth a chunk for each of them)
+    const double us = tile_us(times[i].time, blocks, f64 || s.rows * s.cols >= 64 * 48 ? (k > 64 ? k : 64) : (k > 128 ? k : 128));
+    // (smaller blocks read their operands more often: beyond ten rounds they have to be worth a tenth to come out ahead)
+    if (us < best_us && us < staged_us * (blocks > 10 * 256 ? 0.9 : f64 ? 0.95 : 0.96)) {
+      best_us = us;
+      best = s;
+    }
+  }
+  return best;
+}
+
+// ... as a launch asks it.  two_groups: the full-size tile may share its k between two groups of threads; whole_vectors: nothing
+// reaches past an edge in a vector (the staged tiles' ragged last k-tile costs: 959^3 45 us, 960^3 39).
+inline BlockShape vector_block(bool f64, bool whole_vectors, bool two_groups, int m, int n, double k, long long products) {
+  // (a block of 32 x 32 for every compute unit or fewer: nothing to even out, and a call of 6 us that the host sets the pace of)
+  if ((m + 31LL) / 32 * ((n + 31LL) / 32) * products <= 256) return BlockShape{0, 0};
+  const long long full = (m + 127LL) / 128 * ((n + (f64 ? 63LL : 127LL)) / (f64 ? 64 : 128)) * products;
+  const long long quarter = (m + 63LL) / 64 * ((n + 63LL) / 64) * products, area = f64 ? 8192 : 16384;
+  double us;
+  if (small_blocks_preferred(f64, m, n, products)) {
+    us = tile_us(f64 ? block_times_8[0].time : block_times_4[0].time, (m + 31LL) / 32 * ((n + 31LL) / 32) * products, k);
+    whole_vectors = true;
+  } else if (two_groups && two_group_full_tile(full, quarter, int(area / 4096))) us = tile_us(f64 ? full2_8 : full2_4, full, k);
+  else if (!quarter_tile_preferred(full, area, quarter)) us = tile_us(f64 ? full1_8 : full1_4, full, k);
+  else if (quarter <= 256 && k >= 128) us = tile_us(f64 ? quarter4_8 : quarter4_4, quarter, k);
+  else if (quarter <= 1024 && k >= 128) us = tile_us(f64 ? quarter2_8 : quarter2_4, quarter, k);
+  else us = tile_us(f64 ? quarter1_8 : quarter1_4, quarter, k);
+  return block_shape(f64, m, n, k, products, whole_vectors ? us : us * 1.05);
+}
+
 // fwgemm: one thread per element, or tiles of 128 x 128.  The first takes time by columns of 64 outputs, and more than its share
 // once A's columns leave the L2 (long k); the second by the tiles on the fullest compute unit (one, here) and, without a
 // k-contiguous image of A at hand, by lookups that gather 16 cache lines per improved element, whatever k.  us on square problems, one thread per element / tiles.  Without the image: float 1000^3 165 / 310, 1152^3

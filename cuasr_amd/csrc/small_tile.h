@@ -1,127 +1,189 @@
-// Vector-ALU SRGEMM kernel for outputs too small to give the 64 x 64 staged tile a workgroup per compute unit.
+// Vector-ALU SRGEMM kernel for outputs that the staged tiles do not share out well between the compute units: too small to give the
+// 64 x 64 tile a workgroup per unit, or of a size that leaves the last round of tiles mostly empty.
 //
-// One WAVE owns a 32 x 32 block of the output (8 x 8 lanes of 4 x 4) and a share of k; the W waves of a workgroup
+// One WAVE owns a block of the output (8 x 8 lanes of RM x RN: 32 x 32 up to 64 x 64) and a share of k; the W waves of a workgroup
 // work on the same block, wave w on the k-chunks w, w + W, ...  A wave stages its own chunk of A and B through its
 // own piece of LDS, so the main loop has no barrier: a wave's LDS accesses complete in order, and its next chunk
-// waits in registers while it computes.  After the loop the W accumulators of every output meet in LDS and each
-// thread folds and finishes 1024 / (64 W) outputs of a row-contiguous run.
+// waits in registers while it computes.  After the loop the W accumulators of every output meet in LDS, up to four of a lane's
+// rows at a time, and each thread folds and finishes 1 / (64 W) of the outputs, in row-contiguous runs.
 //
 // Why: an output of 256 x 256 is 16 blocks of 64 x 64, which left 240 of 256 compute units idle; 32 x 32 blocks
-// spread it over 64 of them, with four to sixteen waves each by the length of k (launch_small).
+// spread it over 64 of them, with four to sixteen waves each by the length of k (launch_small).  Larger outputs take the block
+// that divides most evenly (launch_rules.h, block_shape): 1533^3 148 -> 115 us on 64 x 48, double 600 x 500 x 700 33.4 -> 22.6 on 40 x 32.
+//
+// What bounds the loop: in float the way of the fragments from LDS (128 bytes a cycle for 16 waves: 72 % of what a block of
+// 64 x 64 spends on its additions and minima, 85 % of 48 x 48, more than all of 32 x 32) and the clock on dense data: 57, 66 and 68
+// TOPS on 32 x 32, 48 x 48 and 64 x 64 at long k; in double the issue of 8-byte instructions.
 #pragma once
 
 namespace cuasr_amd {
 
-// KC: k per chunk.
-template <typename T, int ADD, int MUL, int KC, int W> struct SmallTile {
+// adds that take a term any number of times
+template <int ADD> struct may_count_twice
+    : std::integral_constant<bool, ADD == kMinimum || ADD == kMaximum || ADD == kLogicalOr || ADD == kLogicalAnd || ADD == kBitOr || ADD == kBitAnd> {};
+
+// KC: k per chunk.  A lane holds RM x RN outputs, a wave's block has 8 RM x 8 RN of them.
+template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> struct SmallTile {
   using Ops = ValuTile<T, ADD, MUL, 4, 4, 32, true, false>;   // its operators, masks and zero-sign lookup
   using S = typename Ops::S;
   static constexpr int VW = 16 / sizeof(T);
-  static constexpr int R = 4, BLOCK = 8 * R;       // outputs per lane and per wave along either direction
-  // rows of 36 floats (40 doubles) more than a multiple of 32: the four k-groups that neighbouring lanes of a
-  // k-contiguous load write lie 16 (doubles: 32) banks apart, so the transposing stores do not collide
-  static constexpr int PAD = sizeof(S) == 8 ? 8 : 4;
+  static constexpr int BM = 8 * RM, BN = 8 * RN;
+  // per SIMD (36 doubles and their fragments leave registers for two, which LDS has room for)
+  static constexpr int WAVES = RM * RN * sizeof(T) > 256 ? 2 : 4;
+  // only blocks of 32 x 32 take outputs narrower than a block
+  static constexpr bool NARROW = RM == 4 && RN == 4;
+  // The k-groups that neighbouring lanes of a k-contiguous load write lie 16 banks apart where there are four of them
+  // and 32 where there are two (8-byte elements: 32, two to an instruction's half), so the transposing stores do not collide.
+  static constexpr int pad(int b) { return sizeof(S) == 8 ? (b % 16 == 8 ? 0 : 8) : KC / VW == 2 ? 8 : 4; }
   static constexpr int ASTRIDE = 64 + 8;           // accumulator e of all lanes; the fold reads e = 0..3 of 8 lanes at once
-  static constexpr int OUTS = 1024 / (64 * W);     // outputs per thread of a folded 32 x 32 block
   typedef T gvec_t __attribute__((ext_vector_type(VW), aligned(sizeof(T))));
   static constexpr int SV = 16 / sizeof(S);
   typedef S s4_t __attribute__((ext_vector_type(SV)));
 
-  struct alignas(16) Panels { S a[KC][BLOCK + PAD], b[KC][BLOCK + PAD]; };
+  struct alignas(16) Panels { S a[KC][BM + pad(BM)], b[KC][BN + pad(BN)]; };
   union Smem {
     Panels p[W];
-    S acc[W][16 * ASTRIDE];
+    S acc[W][4 * RN * ASTRIDE];
   };
 
-  static constexpr int PER = BLOCK * KC / 64;      // elements of a chunk per lane and operand
-  static constexpr int XV = BLOCK / VW, KV = KC / VW, DK = 64 / XV, DX = 64 / KV;   // DK of k (DX of x): what one load of the wave covers
+  // Lane l's elements along a side of R: groups of four, then what is left of R, each group 8 lanes wide.
+  template <int R> static __host__ __device__ constexpr int place(int l, int i) {
+    return i / 4 < R / 4 ? i / 4 * 32 + l * 4 + i % 4 : R / 4 * 32 + l * (R % 4) + i % 4;
+  }
 
-  // One operand's chunk, BLOCK x KC, into registers.  VEC: the block lies inside the matrix (the caller moved its origin
-  // back where it would not) and the chunk is whole, so 16-byte loads at element alignment.  A matrix narrower than a block
-  // still takes them along k, from clamped rows.  Otherwise element by element with clamped indices (what lands past an edge
-  // is never stored, k past the end never used).
-  static __device__ __forceinline__ void load(T (&r)[PER], const T *base, long long s_x, long long s_k, int x_end, int k0, int k_end, bool xc,
-                                              bool vec, int lane) {
-    if (vec && (xc || x_end >= BLOCK)) {
-      const int xx = xc ? lane % XV * VW : lane / KV, kk = xc ? lane / XV : lane % KV * VW;
-      const T *src = base + (long long)xx * s_x + (long long)(k0 + kk) * s_k;
-      const long long next = xc ? DK * s_k : DX * s_x;
+  // One operand's chunk, B x KC.
+  template <int B> struct Side {
+    static constexpr int XV = B / VW, KV = KC / VW, COUNT = B * KC / VW, VECS = (COUNT + 63) / 64, PER = VECS * VW;
+    // The element a lane's vector p starts at.  (The last vectors are asked for twice where 64 lanes do not share them out evenly.)
+    static __device__ __forceinline__ void at(int p, bool xc, int lane, int &xx, int &kk) {
+      int v = lane + 64 * p;
+      if constexpr (COUNT % 64 != 0) v = min(v, COUNT - 1);
+      xx = xc ? v % XV * VW : v / KV;
+      kk = xc ? v / XV : v % KV * VW;
+    }
+    struct Places {
+      const T *src[VECS];
+      __device__ __forceinline__ void init(const T *base, long long s_x, long long s_k, int k0, bool xc, int lane) {
 #pragma unroll
-      for (int p = 0; p < PER / VW; ++p) {
-        const gvec_t t = *reinterpret_cast<const gvec_t *>(src + p * next);
-#pragma unroll
-        for (int e = 0; e < VW; ++e) r[p * VW + e] = t[e];
+        for (int p = 0; p < VECS; ++p) {
+          int xx, kk;
+          at(p, xc, lane, xx, kk);
+          src[p] = base + (long long)xx * s_x + (long long)(k0 + kk) * s_k;
+        }
       }
-    } else if (vec) {
-      int l = lane;   // (as below)
-      asm volatile("" : "+v"(l));
+      __device__ __forceinline__ void move(long long by) {
 #pragma unroll
-      for (int p = 0; p < PER / VW; ++p) {
-        const gvec_t t = *reinterpret_cast<const gvec_t *>(base + (long long)min(l / KV + p * DX, x_end - 1) * s_x + (k0 + l % KV * VW));
-#pragma unroll
-        for (int e = 0; e < VW; ++e) r[p * VW + e] = t[e];
+        for (int p = 0; p < VECS; ++p) src[p] += by;
       }
-    } else {
-      // (worked out again each time: kept from chunk to chunk, these addresses take the main loop's registers)
-      int l = lane;
-      asm volatile("" : "+v"(l));
+      __device__ __forceinline__ void load(T (&r)[PER]) const {
 #pragma unroll
-      for (int p = 0; p < PER; ++p) {
-        const int el = l + 64 * p;
-        const int xx = min(xc ? el % BLOCK : el / KC, x_end - 1), kk = min(k0 + (xc ? el / BLOCK : el % KC), k_end - 1);
-        r[p] = base[(long long)xx * s_x + (long long)kk * s_k];
+        for (int p = 0; p < VECS; ++p) {
+          const gvec_t t = *reinterpret_cast<const gvec_t *>(src[p]);
+#pragma unroll
+          for (int e = 0; e < VW; ++e) r[p * VW + e] = t[e];
+        }
+      }
+    };
+    static __device__ __forceinline__ int element(int p, int lane) {
+      return B * KC % 64 ? min(lane + 64 * p, B * KC - 1) : lane + 64 * p;
+    }
+    // Into registers (blocks of 32 x 32).  VEC: the block lies inside the matrix (the caller moved its origin
+    // back where it would not) and the chunk is whole, so 16-byte loads at element alignment.  A matrix narrower than a block
+    // still takes them along k, from clamped rows.  Otherwise element by element with clamped indices (what lands past an edge
+    // is never stored, k past the end never used).
+    static __device__ __forceinline__ void load(T (&r)[PER], const T *base, long long s_x, long long s_k, int x_end, int k0, int k_end, bool xc,
+                                                bool vec, int lane) {
+      if (vec && (xc || x_end >= B)) {
+        int xx, kk;
+        at(0, xc, lane, xx, kk);
+        const T *src = base + (long long)xx * s_x + (long long)(k0 + kk) * s_k;
+        const long long next = xc ? 64 / XV * s_k : 64 / KV * s_x;
+#pragma unroll
+        for (int p = 0; p < VECS; ++p) {
+          const gvec_t t = *reinterpret_cast<const gvec_t *>(src + p * next);
+#pragma unroll
+          for (int e = 0; e < VW; ++e) r[p * VW + e] = t[e];
+        }
+      } else if (vec) {
+        int l = lane;   // (as below)
+        asm volatile("" : "+v"(l));
+#pragma unroll
+        for (int p = 0; p < VECS; ++p) {
+          int xx, kk;
+          at(p, false, l, xx, kk);
+          const gvec_t t = *reinterpret_cast<const gvec_t *>(base + (long long)min(xx, x_end - 1) * s_x + (k0 + kk));
+#pragma unroll
+          for (int e = 0; e < VW; ++e) r[p * VW + e] = t[e];
+        }
+      } else {
+        // (worked out again each time: kept from chunk to chunk, these addresses take the main loop's registers)
+        int l = lane;
+        asm volatile("" : "+v"(l));
+#pragma unroll
+        for (int p = 0; p < PER; ++p) {
+          const int el = element(p, l);
+          const int xx = min(xc ? el % B : el / KC, x_end - 1), kk = min(k0 + (xc ? el / B : el % KC), k_end - 1);
+          r[p] = base[(long long)xx * s_x + (long long)kk * s_k];
+        }
       }
     }
-  }
-  static __device__ __forceinline__ void store(const T (&r)[PER], S (*dst)[BLOCK + PAD], bool xc, bool vec, int lane) {
-    if (vec) {
-      if (xc) {
+    static __device__ __forceinline__ void store(const T (&r)[PER], S (*dst)[B + pad(B)], bool xc, bool vec, int lane) {
+      if (vec) {
 #pragma unroll
-        for (int p = 0; p < PER / VW; ++p) {
-          typedef S svec_t __attribute__((ext_vector_type(VW)));
-          svec_t t;
+        for (int p = 0; p < VECS; ++p) {
+          int xx, kk;
+          at(p, xc, lane, xx, kk);
+          if (xc) {
+            typedef S svec_t __attribute__((ext_vector_type(VW)));
+            svec_t t;
 #pragma unroll
-          for (int e = 0; e < VW; ++e) t[e] = Ops::staged(r[p * VW + e]);
-          *reinterpret_cast<svec_t *>(&dst[lane / XV + p * DK][lane % XV * VW]) = t;
+            for (int e = 0; e < VW; ++e) t[e] = Ops::staged(r[p * VW + e]);
+            *reinterpret_cast<svec_t *>(&dst[kk][xx]) = t;
+          } else {
+#pragma unroll
+            for (int e = 0; e < VW; ++e) dst[kk + e][xx] = Ops::staged(r[p * VW + e]);
+          }
         }
       } else {
 #pragma unroll
-        for (int p = 0; p < PER / VW; ++p)
-#pragma unroll
-          for (int e = 0; e < VW; ++e) dst[lane % KV * VW + e][lane / KV + p * DX] = Ops::staged(r[p * VW + e]);
-      }
-    } else {
-#pragma unroll
-      for (int p = 0; p < PER; ++p) {
-        const int el = lane + 64 * p;
-        dst[xc ? el / BLOCK : el % KC][xc ? el % BLOCK : el / KC] = Ops::staged(r[p]);
+        for (int p = 0; p < PER; ++p) {
+          const int el = element(p, lane);
+          dst[xc ? el / B : el % KC][xc ? el % B : el / KC] = Ops::staged(r[p]);
+        }
       }
     }
-  }
+  };
 
-  template <int U> struct Frag { S a[U][R], b[U][R]; };
+  template <int U> struct Frag { S a[U][RM], b[U][RN]; };
+  template <int R> static __device__ __forceinline__ void line(S (&f)[R], const S *row, int l) {
+#pragma unroll
+    for (int i = 0; i < R / 4 * 4; i += SV) {
+      const s4_t t = *reinterpret_cast<const s4_t *>(row + place<R>(l, i));
+#pragma unroll
+      for (int e = 0; e < SV; ++e) f[i + e] = t[e];
+    }
+    if constexpr (R % 4 == 2) {
+      typedef S s2_t __attribute__((ext_vector_type(2)));
+      const s2_t t = *reinterpret_cast<const s2_t *>(row + place<R>(l, R - 2));
+      f[R - 2] = t[0];
+      f[R - 1] = t[1];
+    } else {
+#pragma unroll
+      for (int i = R / 4 * 4; i < R; ++i) f[i] = row[place<R>(l, i)];
+    }
+  }
   template <int U> static __device__ __forceinline__ void fragment(Frag<U> &f, const Panels &pn, int kk, int ly, int lx) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-#pragma unroll
-      for (int h = 0; h < R / SV; ++h) {
-        const s4_t t = *reinterpret_cast<const s4_t *>(&pn.a[kk + u][ly * R + h * SV]);
-#pragma unroll
-        for (int e = 0; e < SV; ++e) f.a[u][h * SV + e] = t[e];
-      }
-#pragma unroll
-      for (int h = 0; h < R / SV; ++h) {
-        const s4_t t = *reinterpret_cast<const s4_t *>(&pn.b[kk + u][lx * R + h * SV]);
-#pragma unroll
-        for (int e = 0; e < SV; ++e) f.b[u][h * SV + e] = t[e];
-      }
+      line<RM>(f.a[u], pn.a[kk + u], ly);
+      line<RN>(f.b[u], pn.b[kk + u], lx);
     }
   }
-  template <int U> static __device__ __forceinline__ void compute(S (&acc)[R][R], const Frag<U> &f) {
+  template <int U> static __device__ __forceinline__ void compute(S (&acc)[RM][RN], const Frag<U> &f) {
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
+    for (int i = 0; i < RM; ++i) {
 #pragma unroll
-      for (int j = 0; j < R; ++j) {
+      for (int j = 0; j < RN; ++j) {
         if constexpr (U == 2 && !(Ops::MASKED || Ops::ZERO_SIGN || Ops::FUSED)) {
           const T t0 = Op<MUL>::apply(f.a[0][i], f.b[0][j]), t1 = Op<MUL>::apply(f.a[1][i], f.b[1][j]);
           acc[i][j] = fold<ADD, MUL>(t1, fold<ADD, MUL>(t0, acc[i][j]));   // one three-input minimum
@@ -130,18 +192,19 @@ template <typename T, int ADD, int MUL, int KC, int W> struct SmallTile {
           for (int u = 0; u < U; ++u) acc[i][j] = Ops::term(acc[i][j], f.a[u][i], f.b[u][j]);
         }
       }
+      if constexpr (RM * RN > 16) __builtin_amdgcn_sched_barrier(0);
     }
   }
 
   static __device__ __forceinline__ void run(const Problem &p, const Operands &ops, Smem &sm) {
     constexpr int U = sizeof(S) == 8 ? 1 : 2;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lx = lane & 7, ly = lane >> 3;
-    const int tiles_m = (p.m + BLOCK - 1) / BLOCK, tiles_n = (p.n + BLOCK - 1) / BLOCK;
+    const int tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN;
     int bm, bn;
     Ops::tile_coords(blockIdx.x, tiles_m, tiles_n, bm, bn);
-    const int first_m = bm * BLOCK, first_n = bn * BLOCK;       // the first row and column this workgroup stores
+    const int first_m = bm * BM, first_n = bn * BN;       // the first row and column this workgroup stores
     // blocks at the far edges start earlier instead of reaching past the matrix: what they compute twice is not stored
-    const int m0 = p.m >= BLOCK ? min(first_m, p.m - BLOCK) : first_m, n0 = p.n >= BLOCK ? min(first_n, p.n - BLOCK) : first_n;
+    const int m0 = !NARROW || p.m >= BM ? min(first_m, p.m - BM) : first_m, n0 = !NARROW || p.n >= BN ? min(first_n, p.n - BN) : first_n;
     int kb = 0, ke = p.k;
     if (p.workspace) {
       const int parts = p.k_sub > 1 ? p.k_sub : 1, slice = blockIdx.y / parts, part = blockIdx.y % parts;
@@ -160,43 +223,96 @@ template <typename T, int ADD, int MUL, int KC, int W> struct SmallTile {
     e.source_needed = false;
     if (!partial) e = resolve_scalars<T>(p, MUL);
     const T *C = reinterpret_cast<const T *>(ops.C);
-    const int oc = threadIdx.x & 31, orow0 = threadIdx.x >> 5;   // this thread's outputs of the block: column oc, rows orow0 + 2 W o
-    T src[OUTS];
-    if (e.source_needed) {   // it arrives under the product
+    // this thread's outputs of the block, in the order they are folded: a group of the lanes' rows at a time (32 of the
+    // block's, or what is left), row by row
+    constexpr int GROUPS = (RM + 3) / 4;
+    constexpr int OUTS = (32 * BN + 64 * W - 1) / (64 * W);
+    auto output = [&](int o, int &orow, int &oc) {
+      if constexpr (64 * W % BN == 0) {
+        orow = int(threadIdx.x) / BN + 64 * W / BN * o;
+        oc = int(threadIdx.x) % BN;
+      } else {
+        const int x = int(threadIdx.x) + 64 * W * o;
+        orow = x / BN;
+        oc = x % BN;
+      }
+    };
+    T src[GROUPS][OUTS];
+    auto fetch_source = [&] {
 #pragma unroll
-      for (int o = 0; o < OUTS; ++o)
-        src[o] = C[(long long)min(m0 + orow0 + 2 * W * o, p.m - 1) * p.ldc + min(n0 + oc, p.n - 1)];
-    }
+      for (int g = 0; g < GROUPS; ++g) {
+        const int count = (g < RM / 4 ? 32 : 8 * (RM % 4)) * BN;
+#pragma unroll
+        for (int o = 0; o < OUTS; ++o) {
+          if (64 * W * o >= count) continue;
+          int orow, oc;
+          output(o, orow, oc);
+          src[g][o] = C[(long long)min(m0 + 32 * g + orow, p.m - 1) * p.ldc + min(n0 + oc, p.n - 1)];
+        }
+      }
+    };
+    if (NARROW && e.source_needed) fetch_source();   // it arrives under the product
 
-    S acc[R][R];
+    S acc[RM][RN];
     const S init = Ops::start(p, wave == 0 && p.k_sub <= 1);
 #pragma unroll
-    for (int i = 0; i < R; ++i)
+    for (int i = 0; i < RM; ++i)
 #pragma unroll
-      for (int j = 0; j < R; ++j) acc[i][j] = init;
+      for (int j = 0; j < RN; ++j) acc[i][j] = init;
     // an output narrower than a block gives up the vectors along its narrow side, and no others (or-and, 1 x 65536 x 256: 42.7
     // us with every operand element by element, 23.5 now; 10 x 60000 x 200: 38.6 and 24.5)
-    const bool vec_a = p.m >= BLOCK || !a_xc, vec_b = p.n >= BLOCK || !b_xc;
+    const bool vec_a = !NARROW || p.m >= BM || !a_xc, vec_b = !NARROW || p.n >= BN || !b_xc;
     Panels &pn = sm.p[wave];
-    T ra[PER], rb[PER];
+    T ra[Side<BM>::PER], rb[Side<BN>::PER];
     int k0 = kb + wave * KC;
+    if constexpr (!NARROW) {
+      // every chunk is whole: a ragged last one goes back over k that has been counted (there is a chunk or more)
+      static_assert(may_count_twice<ADD>::value, "k of two chunks is counted twice");
+      typename Side<BM>::Places pa;
+      typename Side<BN>::Places pb;
+      pa.init(A, p.sa_m, p.sa_k, min(k0, ke - KC), a_xc, lane);
+      pb.init(B, p.sb_n, p.sb_k, min(k0, ke - KC), b_xc, lane);
+      pa.load(ra);
+      pb.load(rb);
+      for (; k0 < ke; k0 += W * KC) {
+        Side<BM>::store(ra, pn.a, a_xc, true, lane);
+        Side<BN>::store(rb, pn.b, b_xc, true, lane);
+        wave_lds_order();
+        if (k0 + W * KC < ke) {
+          const int on = min(k0 + W * KC, ke - KC) - k0;
+          pa.move((long long)on * p.sa_k);
+          pb.move((long long)on * p.sb_k);
+          pa.load(ra);
+          pb.load(rb);
+        }
+        // (one set of fragments: a second one's registers are the accumulators', and four waves hide the reads)
+#pragma unroll
+        for (int s = 0; s < KC / U; ++s) {
+          Frag<U> f;
+          fragment<U>(f, pn, U * s, ly, lx);
+          __builtin_amdgcn_sched_barrier(0);
+          compute<U>(acc, f);
+        }
+        wave_lds_order();
+      }
+    } else {
     if (k0 < ke) {
       const bool whole = k0 + KC <= ke;
-      load(ra, A, p.sa_m, p.sa_k, p.m - m0, k0, ke, a_xc, vec_a && whole, lane);
-      load(rb, B, p.sb_n, p.sb_k, p.n - n0, k0, ke, b_xc, vec_b && whole, lane);
+      Side<BM>::load(ra, A, p.sa_m, p.sa_k, p.m - m0, k0, ke, a_xc, vec_a && whole, lane);
+      Side<BN>::load(rb, B, p.sb_n, p.sb_k, p.n - n0, k0, ke, b_xc, vec_b && whole, lane);
     }
     for (; k0 < ke; k0 += W * KC) {
       const bool whole = k0 + KC <= ke;
-      store(ra, pn.a, a_xc, vec_a && whole, lane);
-      store(rb, pn.b, b_xc, vec_b && whole, lane);
+      Side<BM>::store(ra, pn.a, a_xc, vec_a && whole, lane);
+      Side<BN>::store(rb, pn.b, b_xc, vec_b && whole, lane);
       wave_lds_order();   // other lanes read what a lane has stored
       const int kn = k0 + W * KC;
       if (kn < ke) {
         const bool whole_next = kn + KC <= ke;
-        load(ra, A, p.sa_m, p.sa_k, p.m - m0, kn, ke, a_xc, vec_a && whole_next, lane);
-        load(rb, B, p.sb_n, p.sb_k, p.n - n0, kn, ke, b_xc, vec_b && whole_next, lane);
+        Side<BM>::load(ra, A, p.sa_m, p.sa_k, p.m - m0, kn, ke, a_xc, vec_a && whole_next, lane);
+        Side<BN>::load(rb, B, p.sb_n, p.sb_k, p.n - n0, kn, ke, b_xc, vec_b && whole_next, lane);
       }
-      if (k0 + KC <= ke) {
+      if (whole) {
         Frag<U> f[2];
         fragment<U>(f[0], pn, 0, ly, lx);
 #pragma unroll
@@ -215,79 +331,83 @@ template <typename T, int ADD, int MUL, int KC, int W> struct SmallTile {
       }
       wave_lds_order();   // ... before the next chunk takes its place
     }
+    }
+    if (!NARROW && e.source_needed) fetch_source();   // (it arrives under the fold: the product has no registers for it)
     T *out = reinterpret_cast<T *>(ops.D);
     long long ld_out = p.ldd;
     if (partial) {
       out = reinterpret_cast<T *>(p.workspace) + (long long)(p.k_sub > 1 ? blockIdx.y / p.k_sub : blockIdx.y) * p.m * p.n;
       ld_out = p.n;
     }
-    __syncthreads();   // the panels are dead: their space takes the accumulators
 #pragma unroll
-    for (int i = 0; i < R; ++i)
+    for (int g = 0; g < GROUPS; ++g) {
+      const int rows = g < RM / 4 ? 4 : RM % 4, count = 8 * rows * BN;   // rows of a lane in this group; outputs of the block
+      __syncthreads();   // the panels, or the group before, are dead: their space takes the accumulators
 #pragma unroll
-      for (int j = 0; j < R; ++j) sm.acc[wave][(i * R + j) * ASTRIDE + lane] = acc[i][j];
-    __syncthreads();
+      for (int i = 0; i < rows; ++i)
 #pragma unroll
-    for (int o = 0; o < OUTS; ++o) {
-      const int orow = orow0 + 2 * W * o, row = m0 + orow, col = n0 + oc;
-      const int at = ((orow & 3) * 4 + (oc & 3)) * ASTRIDE + (orow >> 2) * 8 + (oc >> 2);
-      S s = sm.acc[0][at];
+        for (int j = 0; j < RN; ++j) sm.acc[wave][(i * RN + j) * ASTRIDE + lane] = acc[4 * g + i][j];
+      __syncthreads();
 #pragma unroll
-      for (int w = 1; w < W; ++w) {
-        if constexpr (Ops::MASKED) s |= sm.acc[w][at];
-        else s = Op<ADD>::apply(s, sm.acc[w][at]);
-      }
-      if (row < first_m || row >= p.m || col < first_n || col >= p.n) continue;
-      T v;
-      if constexpr (Ops::MASKED) v = s ? T(1) : T(0);
-      else v = s;
-      if constexpr (Ops::ZERO_SIGN) {
-        if (v == T(0) && ke > kb)
-          v = Ops::last_zero_product(A + (long long)(row - m0) * p.sa_m + (long long)kb * p.sa_k, p.sa_k,
-                                     B + (long long)(col - n0) * p.sb_n + (long long)kb * p.sb_k, p.sb_k, ke - kb, v);
-      }
-      T *dst = out + (long long)row * ld_out + col;
-      if constexpr (Ops::SUB_SLICES) {
-        if (partial && p.k_sub > 1) {
-          native_fold<ADD>(dst, v);
-          continue;
+      for (int o = 0; o < OUTS; ++o) {
+        if (64 * W * o >= count) continue;
+        int orow, oc;
+        output(o, orow, oc);
+        if (count % (64 * W) && orow >= 8 * rows) continue;
+        const int row = m0 + 32 * g + orow, col = n0 + oc;
+        const bool last = RN % 4 && oc >= RN / 4 * 32;   // the columns that are left beside the groups of four
+        const int left = RN % 4 ? RN % 4 : 1;
+        const int ol = last ? (oc - RN / 4 * 32) / left : oc % 32 / 4, j = last ? RN / 4 * 4 + (oc - RN / 4 * 32) % left : oc / 32 * 4 + oc % 4;
+        const int at = (orow % rows * RN + j) * ASTRIDE + orow / rows * 8 + ol;
+        S s = sm.acc[0][at];
+#pragma unroll
+        for (int w = 1; w < W; ++w) {
+          if constexpr (Ops::MASKED) s |= sm.acc[w][at];
+          else s = Op<ADD>::apply(s, sm.acc[w][at]);
         }
+        if (row < first_m || row >= p.m || col < first_n || col >= p.n) continue;
+        T v;
+        if constexpr (Ops::MASKED) v = s ? T(1) : T(0);
+        else v = s;
+        if constexpr (Ops::ZERO_SIGN) {
+          if (v == T(0) && ke > kb)
+            v = Ops::last_zero_product(A + (long long)(row - m0) * p.sa_m + (long long)kb * p.sa_k, p.sa_k,
+                                       B + (long long)(col - n0) * p.sb_n + (long long)kb * p.sb_k, p.sb_k, ke - kb, v);
+        }
+        T *dst = out + (long long)row * ld_out + col;
+        if constexpr (Ops::SUB_SLICES) {
+          if (partial && p.k_sub > 1) {
+            native_fold<ADD>(dst, v);
+            continue;
+          }
+        }
+        if (!partial) {
+          v = Op<MUL>::apply(e.alpha, v);
+          if (e.source_needed) v = fold_epilogue<ADD, MUL>(v, Op<MUL>::apply(e.beta, src[g][o]));
+        }
+        *dst = v;
       }
-      if (!partial) {
-        v = Op<MUL>::apply(e.alpha, v);
-        if (e.source_needed) v = fold_epilogue<ADD, MUL>(v, Op<MUL>::apply(e.beta, src[o]));
-      }
-      *dst = v;
     }
   }
 };
 
-template <typename T, int ADD, int MUL, int KC, int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void small_srgemm_kernel(const Problem p) {
-  using Tile = SmallTile<T, ADD, MUL, KC, W>;
+template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(SmallTile<T, ADD, MUL, RM, RN, KC, W>::WAVES))) void small_srgemm_kernel(const Problem p) {
+  using Tile = SmallTile<T, ADD, MUL, RM, RN, KC, W>;
   __shared__ typename Tile::Smem sm;
   Tile::run(p, batch_operands<T>(p), sm);
 }
 
-// The 64 x 64 staged tile with its k range shared out over 1024 threads is the better one from about 176 workgroups on
-// (min-plus f32, 60 % of the chip's compute units: 832^3, 169 of them, 30.3 against 26.8 us here; 896^3, 196, 31.5
-// against 36.5), for 8-byte elements from 128 (640^3, 100: 47.9 against 34.3 us; 768^3, 144: 56.8 against 56.1; 832^3:
-// 60.8 against 62.5; this kernel's double figures are 6 - 10 % lower since, 512^3 17.6 -> 15.7).  Integer plus-times stays there at every size (its multiply-adds spill here: 512^3 30.9 against 48 us).
+// Integer plus-times stays on the staged tile at every size (its multiply-adds spill here: 512^3 30.9 against 48 us).
 template <typename T, int ADD> static bool small_preferred(const Problem &p) {
-  if (ADD == kPlus || p.k < 1) return false;
-  const long long groups64 = (long long)((p.m + 63) / 64) * ((p.n + 63) / 64) * slice_groups(p) * p.batch;
-  if (groups64 <= (sizeof(T) == 8 ? 128 : 176)) return true;
-  // ... and where 64 x 64 tiles would cover 1.6 times as much as 32 x 32 blocks, which is more than their better rate is
-  // worth on 4-byte elements (1000 products of 32^3: 10.5 us there, 6.8 here; 100 of 80^3, 1.78 times: 13.0 and 9.6;
-  // 64 of 100^3, the same cover: 11.2 and 11.4)
-  const long long groups32 = (long long)((p.m + 31) / 32) * ((p.n + 31) / 32) * slice_groups(p) * p.batch;
-  return sizeof(T) == 4 && groups32 * 10 <= groups64 * 25;
+  return ADD != kPlus && p.k >= 1 && small_blocks_preferred(sizeof(T) == 8, p.m, p.n, (long long)slice_groups(p) * p.batch);
 }
-template <typename T, int ADD, int MUL, int KC, int W> static hipError_t launch_small_as(const Problem &p, hipStream_t s) {
-  const long long tiles = (long long)((p.m + 31) / 32) * ((p.n + 31) / 32);
+template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> static hipError_t launch_small_as(const Problem &p, hipStream_t s) {
+  using Tile = SmallTile<T, ADD, MUL, RM, RN, KC, W>;
+  const long long tiles = (long long)((p.m + Tile::BM - 1) / Tile::BM) * ((p.n + Tile::BN - 1) / Tile::BN);
   if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
   const dim3 grid((unsigned)tiles, slice_groups(p), p.batch);
-  launch_kernel((small_srgemm_kernel<T, ADD, MUL, KC, W>), grid, dim3(64 * W), 0, s, p);
+  launch_kernel((small_srgemm_kernel<T, ADD, MUL, RM, RN, KC, W>), grid, dim3(64 * W), 0, s, p);
   return take_launch_status();
 }
 
@@ -303,9 +423,36 @@ template <typename T, int ADD, int MUL> static hipError_t launch_small(const Pro
   // 2048: 21.8 us against 24.1 with eight; 512^3, two chunks each: 10.3 against 9.6), eight want two (900 x 900 x 200,
   // 841 blocks: 16.5 us against 14.6 with four; 832^3, 676 blocks of 52 chunks: 26.8 against 29.5).
   const int w = groups <= 256 && chunks >= 64 ? 16 : (groups <= 512 && chunks >= 8) || chunks >= 32 ? 8 : 4;
-  if (w == 16) return launch_small_as<T, ADD, MUL, KC, 16>(p, s);
-  if (w == 8) return launch_small_as<T, ADD, MUL, KC, 8>(p, s);
-  return launch_small_as<T, ADD, MUL, KC, 4>(p, s);
+  if (w == 16) return launch_small_as<T, ADD, MUL, 4, 4, KC, 16>(p, s);
+  if (w == 8) return launch_small_as<T, ADD, MUL, 4, 4, KC, 8>(p, s);
+  return launch_small_as<T, ADD, MUL, 4, 4, KC, 4>(p, s);
+}
+
+// The larger blocks (block_shape): eight waves each, so that two workgroups share a compute unit.
+template <typename T, int ADD, int MUL> static hipError_t launch_block(const Problem &p, BlockShape b, hipStream_t s) {
+  constexpr int KC = 64 / sizeof(T);
+  if constexpr (sizeof(T) == 8) {
+    if (b.rows == 40) {
+      // (one block per compute unit and k for all: sixteen waves, 600 x 500 x 700 21.6 us against 23.6)
+      const long long groups = (long long)((p.m + 39) / 40) * ((p.n + 31) / 32) * slice_groups(p) * p.batch;
+      if (groups <= 256 && (p.workspace ? p.k_per_slice : p.k) >= 512) return launch_small_as<T, ADD, MUL, 5, 4, KC, 16>(p, s);
+      return launch_small_as<T, ADD, MUL, 5, 4, KC, 8>(p, s);
+    }
+    if (b.cols == 32) return launch_small_as<T, ADD, MUL, 6, 4, KC, 8>(p, s);
+    return launch_small_as<T, ADD, MUL, 6, 6, KC, 8>(p, s);
+  } else {
+    if (b.rows == 48) return b.cols == 32 ? launch_small_as<T, ADD, MUL, 6, 4, KC, 8>(p, s) : launch_small_as<T, ADD, MUL, 6, 6, KC, 8>(p, s);
+    if (b.cols == 32) return launch_small_as<T, ADD, MUL, 8, 4, KC, 8>(p, s);
+    // (chunks of half as many k: their way through the registers has none to spare)
+    return b.cols == 48 ? launch_small_as<T, ADD, MUL, 8, 6, KC / 2, 8>(p, s) : launch_small_as<T, ADD, MUL, 8, 8, KC / 2, 8>(p, s);
+  }
+}
+// The blocks larger than 32 x 32 take whole chunks of k only and go back over k that has been counted for the last one.
+template <typename T, int ADD> static bool blocks_possible(const Problem &p) {
+  constexpr int KC = 64 / sizeof(T);
+  if (!may_count_twice<ADD>::value || sizeof(T) < 4 || p.k_sub > 1 || !vector_possible<T>(p)) return false;
+  // (a slice that is empty or shorter than a chunk has none to go back over)
+  return p.workspace ? (p.slices - 1LL) * p.k_per_slice + KC <= p.k : p.k >= KC;
 }
 
 }  // namespace cuasr_amd

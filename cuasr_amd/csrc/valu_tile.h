@@ -728,47 +728,37 @@ static hipError_t launch_valu(const Problem &p, hipStream_t s) {
   return take_launch_status();
 }
 
-// The chip holds 1024 full-size workgroups at a time (four per compute unit),
-// and a launch runs in rounds of that many.  The full-size tile is a few per
-// cent faster than the quarter-size one when its workgroups fill whole rounds
-// (4096^2: exactly one), and much slower when a round is mostly empty (fewer
-// than 1024 workgroups: split-K of a small output, matrices below ~3000^2) or
-// the last round is (5120^2: 1.56 rounds).  The quarter-size tile -- four times
-// as many, shorter workgroups -- balances in all those cases, so the full-size
-// one is used only when at least 95 % of its rounds are filled.
-#ifndef CUASR_AMD_FULL_TILE_FILL_PERCENT
-#define CUASR_AMD_FULL_TILE_FILL_PERCENT 95
-#endif
-
+// Full-size tile (16 TM x 16 TN), quarter-size tile or the blocks of small_tile.h: launch_rules.h
 template <typename T, int ADD, int MUL, int TM, int TN, int BK, int TM_SMALL, int TN_SMALL, int BK_SMALL = BK>
 static hipError_t launch_valu_sized(const Problem &p, hipStream_t s) {
   constexpr int BM = 16 * TM, BN = 16 * TN;
+  static_assert(BM == 128 && BN == (sizeof(T) == 8 ? 64 : 128) && TM_SMALL == 4 && TN_SMALL == 4, "the tiles that the rules are about");
+  const long long products = (long long)slice_groups(p) * p.batch;
+  const long long k_range = p.workspace ? p.k_per_slice / (p.k_sub > 1 ? p.k_sub : 1) : p.k;
+  const long long full = (long long)((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN) * products;
+  const long long quarter = (long long)((p.m + 63) / 64) * ((p.n + 63) / 64) * products;
+  // (two groups: not with one instruction per term, or-and 1984^3 203 us against 209 on the full-size tile, xor-and 1950^3 200
+  // against 213)
+  constexpr bool TWO_GROUPS = order_free<T, ADD>::value && ADD != kLogicalOr && ADD != kBitXor && ADD != kBitOr && ADD != kBitAnd;
+  const bool two_groups = TWO_GROUPS && k_range >= 8LL * BK && vector_possible<T>(p) && p.m > 0 && p.n > 0;
+  // (masks are left out: their term is one instruction and the panels' way to LDS longer; the times do not hold for them)
+  if constexpr (order_free<T, ADD>::value && may_count_twice<ADD>::value && !ValuTile<T, ADD, MUL, 4, 4, 32, true, false>::MASKED) {
+    if (blocks_possible<T, ADD>(p)) {
+      const BlockShape b = vector_block(sizeof(T) == 8, vector_exact<T>(p), two_groups, p.m, p.n, double(k_range), products);
+      if (b.rows == 32) return launch_small<T, ADD, MUL>(p, s);
+      if (b.rows) return launch_block<T, ADD, MUL>(p, b, s);
+    }
+  }
   if constexpr (order_free<T, ADD>::value) {
     if (small_preferred<T, ADD>(p)) return launch_small<T, ADD, MUL>(p, s);
   }
-  const long long groups = (long long)((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN) * slice_groups(p) * p.batch;
-  const long long rounds = (groups + 1023) / 1024;
-  // ... and those tiles do not reach much further past the edges than the quarter-size ones: a batch of 1000 products of
-  // 64 x 64 filled 1000 full-size tiles to a quarter (37.8 us; 18.2 on the quarter-size ones).  An eighth more is less than
-  // their rate is worth (940 x 16384 x 500, a fifteenth more, both operands k-contiguous: 246 us, 261 on the smaller ones)
-  constexpr int SM = 16 * TM_SMALL, SN = 16 * TN_SMALL;
-  const long long groups_small = (long long)((p.m + SM - 1) / SM) * ((p.n + SN - 1) / SN) * slice_groups(p) * p.batch;
-  const bool covers_more = groups * BM * BN * 8 > groups_small * SM * SN * 9;
-  if constexpr (order_free<T, ADD>::value) {
-    // 192 .. 256 full-size workgroups (2048^2: exactly 256) are one per compute unit for most of the
-    // chip: two groups per workgroup give every SIMD its two waves, and the full-size tile then runs
-    // at the rate it has on large problems, which the quarter-size tile does not reach.  With one instruction per term it
-    // does (or-and 1984^3 203 us against 209 on the full-size tile, xor-and 1950^3 200 against 213).
-    if constexpr (ADD != kLogicalOr && ADD != kBitXor && ADD != kBitOr && ADD != kBitAnd) {
-      const long long k_range = p.workspace ? p.k_per_slice / (p.k_sub > 1 ? p.k_sub : 1) : p.k;
-      if (two_group_full_tile(groups, groups_small, BM * BN / (SM * SN)) && k_range >= 8LL * BK && vector_possible<T>(p) && p.m > 0 && p.n > 0) {
-        launch_ksplit<T, ADD, MUL, TM, TN, BK, 2>(p, dim3((unsigned)(groups / slice_groups(p) / p.batch), slice_groups(p), p.batch), s);
-        return take_launch_status();
-      }
+  if constexpr (TWO_GROUPS) {
+    if (two_groups && two_group_full_tile(full, quarter, BM * BN / 4096)) {
+      launch_ksplit<T, ADD, MUL, TM, TN, BK, 2>(p, dim3((unsigned)(full / products), slice_groups(p), p.batch), s);
+      return take_launch_status();
     }
   }
-  if (covers_more || groups * 100 < rounds * 1024 * (long long)(CUASR_AMD_FULL_TILE_FILL_PERCENT))
-    return launch_valu<T, ADD, MUL, TM_SMALL, TN_SMALL, BK_SMALL, true>(p, s);
+  if (quarter_tile_preferred(full, BM * BN, quarter)) return launch_valu<T, ADD, MUL, TM_SMALL, TN_SMALL, BK_SMALL, true>(p, s);
   return launch_valu<T, ADD, MUL, TM, TN, BK>(p, s);
 }
 

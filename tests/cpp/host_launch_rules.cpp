@@ -2,6 +2,7 @@
 //   fwgemm <f64> <image> <m> <n> <k>       1: one thread per element, 2: tiles of 128 x 128, 3: of 64 x 128
 //   staged <m> <n> <batch> <full m> <full n>   1: the full-size tile in two groups, 0: not (quarter-size: 64 x 64)
 //   half <ordered> <bits> <zeros> <m> <n> <products>   rows of the binary16 tile
+//   block <f64> <whole vectors> <m> <n> <k> <products>   100 rows + columns of the block, 0: the staged family's tile or 32 x 32
 //   share <rest> <parts> <part>            where the part of a ragged k-tile begins
 #include <cstdio>
 #include <cstring>
@@ -22,6 +23,12 @@ int main() {
       long long products;
       if (std::scanf("%d %d %d %d %d %lld", &ordered, &bits, &zeros, &m, &n, &products) != 6) return 2;
       answer = cuasr_amd::half_tile_rows(ordered, bits, zeros, m, n, products);
+    } else if (!std::strcmp(what, "block")) {
+      int f64, whole, m, n, k;
+      long long products;
+      if (std::scanf("%d %d %d %d %d %lld", &f64, &whole, &m, &n, &k, &products) != 6) return 2;
+      const cuasr_amd::BlockShape b = cuasr_amd::vector_block(f64, whole, k >= (f64 ? 128 : 256), m, n, k, products);
+      answer = b.rows * 100 + b.cols;
     } else if (!std::strcmp(what, "share")) {
       int rest, parts, part;
       if (std::scanf("%d %d %d", &rest, &parts, &part) != 3) return 2;

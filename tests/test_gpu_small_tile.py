@@ -105,3 +105,76 @@ def test_outputs_narrower_than_a_block(oracle, lib, pair, shape):
         cuasr_amd.srgemm(add, mult, *wide, to_device(C), dD, one, one, ident, one, dtype=dt, kernel="valu")
         torch.cuda.synchronize()
         assert_same_bits(to_host(dD, dt), want, f"{pair} {shape} {order}")
+
+
+# (block, double, m, n, k), row-major C: one chunk of k, a chunk and one, one more than the waves' first chunks, whole blocks and
+# not, in either direction (test_launch_rules.py asks the rule for the block)
+BLOCKS = [(4832, 0, 294, 822, 70), (4832, 0, 294, 822, 257), (6432, 0, 541, 679, 100), (6448, 0, 1475, 321, 17), (6448, 0, 832, 624, 70), (6464, 0, 400, 1800, 101),
+          (6464, 0, 833, 865, 70), (4848, 0, 836, 581, 129), (4848, 0, 768, 768, 160), (4032, 1, 386, 615, 16), (4032, 1, 600, 500, 515),
+          (4032, 1, 640, 480, 70), (4832, 1, 361, 801, 33), (4848, 1, 585, 776, 33), (4848, 1, 768, 768, 40)]
+# (block, double, products, m, n, k)
+BLOCK_BATCHES = [(6432, 0, 7, 885, 46, 100), (6448, 0, 7, 99, 587, 30), (4032, 1, 7, 583, 40, 16), (4848, 1, 7, 624, 71, 33)]
+# (block, double, slices, m, n, k of a slice): the last slice shorter than the others
+BLOCK_SLICES = [(4848, 0, 8, 136, 480, 144), (4032, 1, 8, 160, 220, 272)]
+
+
+@pytest.mark.parametrize("case", BLOCKS, ids=lambda c: "x".join(map(str, c)))
+def test_larger_blocks(oracle, lib, case):
+    """Blocks of more than 32 x 32: every chunk of k is whole and the last one goes back over k that has been counted; blocks at
+    the far edges start earlier; outputs in groups of the lanes' rows."""
+    import torch
+    import cuasr_amd
+    from cuasr_amd import inputs
+    _, f64, m, n, k = case
+    dt = "f64" if f64 else "f32"
+    pairs = [("minimum", "plus"), ("maximum", "minimum"), ("minimum", "multiplies")]
+    pairs = [(a, b, dt) for a, b in pairs] + ([] if f64 else [("maximum", "plus", "i32"), ("bit_or", "bit_and", "u32")])
+    for add, mult, dt in pairs:
+        ident, one = cuasr_amd.op_identity(add, dt, True), cuasr_amd.op_identity(mult, dt, True)
+        for i, order in enumerate(("FFC", "CCC", "CFF")):
+            shape = (n, m, k) if order[2] == "F" else (m, n, k)   # (a column-major output is the transposed problem)
+            A, B, C = _case(inputs, dt, *shape, order, 231 + i)
+            want = oracle.srgemm(add, mult, A, B, C, one, one, ident)
+            dC = to_device(C)
+            dD = dC if i == 1 else to_device(np.zeros_like(C))     # in place, too
+            cuasr_amd.srgemm(add, mult, to_device(A), to_device(B), dC, dD, one, one, ident, one, dtype=dt, kernel="valu")
+            torch.cuda.synchronize()
+            assert_same_bits(to_host(dD, dt), want, f"{add} {mult} {dt} {shape} {order}")
+
+
+@pytest.mark.parametrize("case", BLOCK_BATCHES, ids=lambda c: "x".join(map(str, c)))
+def test_larger_blocks_in_batches(oracle, lib, case):
+    import torch
+    import cuasr_amd
+    from cuasr_amd import inputs
+    _, f64, products, m, n, k = case
+    dt = "f64" if f64 else "f32"
+    for add, mult in (("minimum", "plus"), ("maximum", "multiplies")):
+        ident, one = cuasr_amd.op_identity(add, dt, True), cuasr_amd.op_identity(mult, dt, True)
+        ops = [_case(inputs, dt, m, n, k, "CCC", 3000 + 7 * i) for i in range(products)]
+        up = lambda j: torch.stack([to_device(np.ascontiguousarray(o[j])) for o in ops])
+        dA, dB, dC = up(0), up(1), up(2)
+        dD = torch.zeros_like(dC)
+        cuasr_amd.srgemm_batched(add, mult, dA, dB, dC, dD, one, one, ident, one, dtype=dt, kernel="valu")
+        torch.cuda.synchronize()
+        for i in range(products):
+            assert_same_bits(to_host(dD[i], dt), oracle.srgemm(add, mult, *ops[i], one, one, ident), f"{add} {mult} {case} product {i}")
+
+
+@pytest.mark.parametrize("case", BLOCK_SLICES, ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("short", [0, 100])
+def test_larger_blocks_in_slices(oracle, lib, case, short):
+    import torch
+    import cuasr_amd
+    from cuasr_amd import inputs
+    _, f64, slices, m, n, per = case
+    dt, k = "f64" if f64 else "f32", slices * per - short
+    ident, one = cuasr_amd.op_identity("minimum", dt, True), cuasr_amd.op_identity("plus", dt, True)
+    A, B, C = _case(inputs, dt, m, n, k, "CFC", 79)
+    want = oracle.srgemm("minimum", "plus", A, B, C, one, one, ident)
+    work = torch.empty(cuasr_amd.splitk_workspace_bytes(m, n, slices, dt), dtype=torch.uint8, device="cuda")
+    dD = to_device(np.zeros_like(C))
+    cuasr_amd.srgemm_splitk("minimum", "plus", to_device(A), to_device(B), to_device(C), dD, slices, work, one, one, ident, one, dtype=dt,
+                            kernel="valu")
+    torch.cuda.synchronize()
+    assert_same_bits(to_host(dD, dt), want, f"{case} {short}")

@@ -72,3 +72,18 @@ def test_binary16_tile_sizes():
               [(960, 2048, 32), (1216, 2048, 32), (1500, 1500, 32), (1664, 1664, 32), (1792, 1792, 64), (2048, 2176, 32), (2304, 2304, 64),
                (2560, 2560, 64), (3000, 2900, 64)]]
     assert _ask([question for question, _ in asked]) == [rows for _, rows in asked]
+
+
+def test_vector_blocks():
+    """The block that the tests of each block's edges say they run; and at sizes where all were timed, the fastest or one within
+    a few per cent of it (0: the staged family's tile, or 32 x 32)."""
+    import test_gpu_small_tile as small
+    asked = [(f"block {f64} 0 {m} {n} {k} 1", block) for block, f64, m, n, k in small.BLOCKS]
+    asked += [(f"block {f64} 0 {m} {n} {k} {products}", block) for block, f64, products, m, n, k in small.BLOCK_BATCHES]
+    asked += [(f"block {f64} 0 {m} {n} {k} {slices}", block) for block, f64, slices, m, n, k in small.BLOCK_SLICES]
+    asked += [(f"block 0 {int(n % 4 == 0)} {n} {n} {n} 1", block) for n, block in
+              [(256, 0), (500, 0), (577, 4832), (620, 6432), (736, 4848), (768, 4848), (1024, 0), (1053, 4848), (1152, 6448), (1533, 6448),
+               (2048, 0), (2200, 6464), (2547, 6432)]]
+    asked += [(f"block 1 {int(n % 2 == 0)} {n} {n} {n} 1", block) for n, block in
+              [(300, 0), (480, 0), (518, 4032), (560, 4032), (600, 4832), (758, 4848), (800, 4032), (1008, 0), (1100, 4032), (1408, 0)]]
+    assert _ask([question for question, _ in asked]) == [block for _, block in asked]
