@@ -333,6 +333,7 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> struct Sm
     }
     }
     if (!NARROW && e.source_needed) fetch_source();   // (it arrives under the fold: the product has no registers for it)
+    int zeros = 0;   // ZERO_SIGN: 1 where the block's zeros are all +0, -1 where they are not known to be
     T *out = reinterpret_cast<T *>(ops.D);
     long long ld_out = p.ldd;
     if (partial) {
@@ -348,13 +349,13 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> struct Sm
 #pragma unroll
         for (int j = 0; j < RN; ++j) sm.acc[wave][(i * RN + j) * ASTRIDE + lane] = acc[4 * g + i][j];
       __syncthreads();
-#pragma unroll
-      for (int o = 0; o < OUTS; ++o) {
-        if (64 * W * o >= count) continue;
+      // output o: false where it is not this workgroup's to store
+      auto folded = [&](int o, T &v, int &row, int &col) {
+        if (64 * W * o >= count) return false;
         int orow, oc;
         output(o, orow, oc);
-        if (count % (64 * W) && orow >= 8 * rows) continue;
-        const int row = m0 + 32 * g + orow, col = n0 + oc;
+        if (count % (64 * W) && orow >= 8 * rows) return false;
+        row = m0 + 32 * g + orow, col = n0 + oc;
         const bool last = RN % 4 && oc >= RN / 4 * 32;   // the columns that are left beside the groups of four
         const int left = RN % 4 ? RN % 4 : 1;
         const int ol = last ? (oc - RN / 4 * 32) / left : oc % 32 / 4, j = last ? RN / 4 * 4 + (oc - RN / 4 * 32) % left : oc / 32 * 4 + oc % 4;
@@ -365,20 +366,17 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> struct Sm
           if constexpr (Ops::MASKED) s |= sm.acc[w][at];
           else s = Op<ADD>::apply(s, sm.acc[w][at]);
         }
-        if (row < first_m || row >= p.m || col < first_n || col >= p.n) continue;
-        T v;
+        if (row < first_m || row >= p.m || col < first_n || col >= p.n) return false;
         if constexpr (Ops::MASKED) v = s ? T(1) : T(0);
         else v = s;
-        if constexpr (Ops::ZERO_SIGN) {
-          if (v == T(0) && ke > kb)
-            v = Ops::last_zero_product(A + (long long)(row - m0) * p.sa_m + (long long)kb * p.sa_k, p.sa_k,
-                                       B + (long long)(col - n0) * p.sb_n + (long long)kb * p.sb_k, p.sb_k, ke - kb, v);
-        }
+        return true;
+      };
+      auto finish = [&](int o, T v, int row, int col) {
         T *dst = out + (long long)row * ld_out + col;
         if constexpr (Ops::SUB_SLICES) {
           if (partial && p.k_sub > 1) {
             native_fold<ADD>(dst, v);
-            continue;
+            return;
           }
         }
         if (!partial) {
@@ -386,6 +384,41 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> struct Sm
           if (e.source_needed) v = fold_epilogue<ADD, MUL>(v, Op<MUL>::apply(e.beta, src[g][o]));
         }
         *dst = v;
+      };
+      if constexpr (Ops::ZERO_SIGN) {
+        const T *Ab = A + (long long)kb * p.sa_k, *Bb = B + (long long)kb * p.sb_k;
+        T v[OUTS];
+        int row[OUTS], col[OUTS];
+        unsigned mine = 0, open = 0;
+        static_assert(OUTS <= 32, "a bit per output");
+#pragma unroll
+        for (int o = 0; o < OUTS; ++o) {
+          if (!folded(o, v[o], row[o], col[o])) continue;
+          mine |= 1u << o;
+          if (v[o] == T(0) && ke > kb) {
+            const auto z = Ops::zero_result(Ab + (long long)(row[o] - m0) * p.sa_m, p.sa_k, Bb + (long long)(col[o] - n0) * p.sb_n, p.sb_k, ke - kb, v[o]);
+            v[o] = z.value;
+            open |= (unsigned)z.open << o;
+          }
+        }
+        if (__syncthreads_or(open != 0)) {
+          if (zeros == 0) zeros = Ops::zeros_are_positive(p, Ab, Bb, min(BM, p.m - m0), min(BN, p.n - n0), ke - kb) ? 1 : -1;
+#pragma unroll
+          for (int o = 0; o < OUTS; ++o) {
+            if (!(open >> o & 1)) continue;
+            v[o] = zeros > 0 ? T(0) : Ops::last_zero_product(Ab + (long long)(row[o] - m0) * p.sa_m, p.sa_k, Bb + (long long)(col[o] - n0) * p.sb_n, p.sb_k, ke - kb - 8, v[o]);
+          }
+        }
+#pragma unroll
+        for (int o = 0; o < OUTS; ++o)
+          if (mine >> o & 1) finish(o, v[o], row[o], col[o]);
+      } else {
+#pragma unroll
+        for (int o = 0; o < OUTS; ++o) {
+          T v;
+          int row, col;
+          if (folded(o, v, row, col)) finish(o, v, row, col);
+        }
       }
     }
   }

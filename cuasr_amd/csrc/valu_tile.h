@@ -75,16 +75,84 @@ struct ValuTile {
     else if constexpr (ZERO_SIGN) return Op<ADD>::apply(acc, Op<MUL>::apply(a, b));
     else return cuasr_amd::term<ADD, MUL>(acc, a, b);
   }
-  // ZERO_SIGN: the last product of the k range that is zero (acc itself when there is none: an
-  // empty range, or a zero identity).  Not inlined: it runs for the few accumulators that ended
-  // at zero, after the main loop.
+  // ZERO_SIGN: the last product of the k range that is zero, if it is among the last eight (kcount: what is left of the
+  // range).  Eight at a time: one by one, every product waited for memory.
+  static __device__ __forceinline__ bool zero_among_last(const T *a_row, long long sa_k, const T *b_col, long long sb_k, int kcount, T &v) {
+    T prod[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int kk = max(kcount - 1 - j, 0);
+      prod[j] = a_row[(long long)kk * sa_k] * b_col[(long long)kk * sb_k];
+    }
+    bool found = false;
+#pragma unroll
+    for (int j = 7; j >= 0; --j) {
+      if (prod[j] == T(0)) {
+        v = prod[j];
+        found = true;
+      }
+    }
+    return found;
+  }
+  // ... or wherever it is (acc itself when there is none: a zero identity).  Neither is inlined where it is used: they run
+  // for the few accumulators that ended at zero, after the main loop.
   static __device__ __attribute__((noinline)) T last_zero_product(const T *a_row, long long sa_k, const T *b_col,
                                                                  long long sb_k, int kcount, T acc) {
-    for (int kk = kcount - 1; kk >= 0; --kk) {
-      const T prod = a_row[(long long)kk * sa_k] * b_col[(long long)kk * sb_k];
-      if (prod == T(0)) return prod;
-    }
+    for (int left = kcount; left > 0; left -= 8)
+      if (zero_among_last(a_row, sa_k, b_col, sb_k, left, acc)) break;
     return acc;
+  }
+  // A zero result with its sign as the last products alone say it; open where it has to be looked for further back.
+  struct ZeroResult {
+    T value;
+    int open;
+  };
+  static __device__ __attribute__((noinline)) ZeroResult zero_result(const T *a_row, long long sa_k, const T *b_col, long long sb_k, int kcount, T acc) {
+    const bool found = zero_among_last(a_row, sa_k, b_col, sb_k, kcount, acc);
+    return ZeroResult{acc, !found && kcount > 8};
+  }
+
+  // ZERO_SIGN: where nothing in the two panels has its sign bit set, as reliabilities and capacities have not, every
+  // zero is +0 and none has to be looked for.  A zero in A makes a whole row of zeros, and looking for them took as long as the
+  // longest chain of them: min-times 672 x 2816 x 2211 with one zero in A 2950 us, 187 with the panels read, in about 10 us by all
+  // threads of the workgroups that have zeros whose sign the last eight products do not say.  Reading them before looking at those eight
+  // cost where every seventh row is zero, 300^3 10 -> 13.5 us.  ks: k of the panel; xs: its rows (columns of B).
+  static __device__ __attribute__((noinline)) bool has_sign(const T *base, long long s_x, long long s_k, int xs, int ks, bool xc) {
+    auto bits = [](T x) {
+      if constexpr (sizeof(T) == 8) return int(__builtin_bit_cast(long long, x) >> 32);
+      else return __builtin_bit_cast(int, x);
+    };
+    const int len = xc ? xs : ks, lines = xc ? ks : xs, first = threadIdx.x >> 5, step = blockDim.x >> 5;
+    const long long ld = xc ? s_k : s_x;
+    int any = 0;
+    if (len < VW) {
+      for (int l = threadIdx.x; l < lines; l += blockDim.x)
+        for (int e = 0; e < len; ++e) any |= bits(base[l * ld + e]);
+    } else {
+      // (the last vector of a line goes back to where it ends with the line)
+      auto vector = [&](int l, int f) {
+        const gvec_t t = *reinterpret_cast<const gvec_t *>(base + l * ld + min(f, len - VW));
+#pragma unroll
+        for (int e = 0; e < VW; ++e) any |= bits(t[e]);
+      };
+      if (xc) {
+        for (int f = (threadIdx.x & 31) * VW; f < len; f += 32 * VW) {
+#pragma unroll 8
+          for (int l = first; l < lines; l += step) vector(l, f);
+        }
+      } else {
+        for (int l = first; l < lines; l += step) {
+#pragma unroll 8
+          for (int f = (threadIdx.x & 31) * VW; f < len; f += 32 * VW) vector(l, f);
+        }
+      }
+    }
+    return any < 0;
+  }
+  // ... asked by the whole workgroup
+  static __device__ __forceinline__ bool zeros_are_positive(const Problem &p, const T *A, const T *B, int rows, int cols, int ks) {
+    const bool sign = has_sign(A, p.sa_m, p.sa_k, rows, ks, p.sa_m == 1) || has_sign(B, p.sb_n, p.sb_k, cols, ks, p.sb_n == 1);
+    return !__syncthreads_or(sign || __builtin_signbit(scalar_as<T>(p.add_identity)));
   }
 
   struct Smem {
@@ -523,6 +591,32 @@ struct ValuTile {
         return;
       }
     }
+    if constexpr (ZERO_SIGN) {
+      const T *Ab = A + (long long)kb * p.sa_k, *Bb = B + (long long)kb * p.sb_k;
+      auto row = [&](int q) { return Ab + (long long)min(row_of(q), p.m - 1) * p.sa_m; };
+      auto column = [&](int j) { return Bb + (long long)min(n0 + tx * VW + (j / VW) * 16 * VW + (j % VW), p.n - 1) * p.sb_n; };
+      unsigned long long open = 0;
+      static_assert(NR * TN <= 64, "a bit per output");
+      if (ke > kb) {
+#pragma unroll
+        for (int q = 0; q < NR; ++q)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            if (acc[q][j] == T(0)) {
+              const ZeroResult z = zero_result(row(q), p.sa_k, column(j), p.sb_k, ke - kb, acc[q][j]);
+              acc[q][j] = z.value;
+              open |= (unsigned long long)z.open << (q * TN + j);
+            }
+      }
+      if (__syncthreads_or(open != 0)) {
+        const bool positive = zeros_are_positive(p, Ab + (long long)m0 * p.sa_m, Bb + (long long)n0 * p.sb_n, min(BM, p.m - m0), min(BN, p.n - n0), ke - kb);
+#pragma unroll
+        for (int q = 0; q < NR; ++q)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            if (open >> (q * TN + j) & 1) acc[q][j] = positive ? T(0) : last_zero_product(row(q), p.sa_k, column(j), p.sb_k, ke - kb - 8, acc[q][j]);
+      }
+    }
     const T *C = reinterpret_cast<const T *>(o.C);
     // All of the thread's source elements are requested together, at clamped indices (the main loop's fragments are
     // dead, so there are registers for them): D may be C, so the compiler keeps every load behind the store before it,
@@ -561,12 +655,6 @@ struct ValuTile {
             v[c] = acc[q][g * VW + c] ? T(1) : T(0);
           } else {
             v[c] = acc[q][g * VW + c];
-            if constexpr (ZERO_SIGN) {
-              if (v[c] == T(0) && ke > kb)
-                v[c] = last_zero_product(A + (long long)row * p.sa_m + (long long)kb * p.sa_k, p.sa_k,
-                                         B + (long long)min(col + c, p.n - 1) * p.sb_n + (long long)kb * p.sb_k, p.sb_k,
-                                         ke - kb, v[c]);
-            }
           }
         }
         if (!partial) {

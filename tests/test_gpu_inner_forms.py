@@ -220,3 +220,30 @@ def test_bit_operations_with_a_direct_tile_per_compute_unit(oracle, lib, shape, 
         cuasr_amd.srgemm("bit_xor", "bit_and", dA, dB, dC, dD, ones, ones, 0, ones, dtype="u32")
         torch.cuda.synchronize()
         assert_same_bits(to_host(dD, "u32"), want, f"{shape} {order}")
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f64"])
+@pytest.mark.parametrize("add", ["minimum", "maximum"])
+@pytest.mark.parametrize("shape", [(3, 2, 9), (5, 40, 300), (33, 31, 1), (130, 70, 45), (300, 257, 129), (1000, 901, 66)])
+def test_zeros_of_products_without_signs(oracle, lib, dtype, add, shape):
+    """Panels without a sign bit give +0 without a lookup; one -0 at either end of either operand, or an identity of -0,
+    and the zeros are looked up.  Rows of zeros make zero results for both adds."""
+    npd = NPD[dtype]
+    m, n, k = shape
+    rng = np.random.default_rng(m + n + k)
+    C = np.full((m, n), 9.0 if add == "minimum" else -1.0, npd)
+    for layouts in ("ccc", "rrr", "rcr", "crc"):
+        la, lb, lc = (order_of({"c": "col", "r": "row"}[x]) for x in layouts)
+        for case in ("none", "A first", "A last", "B first", "B last", "identity"):
+            A, B = 0.1 + rng.random((m, k)), 0.1 + rng.random((k, n))
+            A[:: 3], B[:, 1:: 5] = 0.0, 0.0
+            if case[0] in "AB":
+                x = A if case[0] == "A" else B
+                x[(0, 0) if case[2:] == "first" else (-1, -1)] = -0.0
+            ident = -0.0 if case == "identity" else INF if add == "minimum" else -INF
+            A, B, Co = np.asarray(A.astype(npd), order=la), np.asarray(B.astype(npd), order=lb), np.asarray(C, order=lc)
+            want = oracle.srgemm(add, "multiplies", A, B, Co, 1, 1, ident)
+            assert (want == 0).any()
+            for kernel in ("auto", "valu"):
+                got = launch(add, "multiplies", dtype, A, B, Co, 1, 1, ident, 1, kernel)
+                assert_same_bits(got, want, f"{add} {dtype} {shape} {layouts} {kernel} {case}")
