@@ -10,7 +10,7 @@
 // indices are clamped lane by lane, and only the last chunk of a k range that is not whole chunks looks at its end
 // (k past it is multiplied as zero).  The next chunk is requested before a chunk's eight matrix instructions (512
 // cycles; 2 x 2 blocks: 2048) are issued.  The KG partial sums meet in LDS, each wave finishing a KG-th of the block's
-// rows.  512^3 41.5 -> 6.7 us (float), 55.4 -> 9.6 (double); 1024^3 80.6 -> 24 - 28 by layout and 110 -> 42 - 45 (operands in cache; 30.7 and up on new ones); 64 x 4096 x 4096 308 ->
+// rows.  512^3 41.5 -> 6.7 us (float), 55.4 -> 9.6 (double); 1024^3 80.6 -> 24 - 28 by layout and 110 -> 42 - 45 (operands in cache; on new ones 27 - 29 and 46 - 50); 64 x 4096 x 4096 308 ->
 // 34 and 421 -> 48 (the vector-ALU tiles before it); 2048 products of 100^3, each a launch of its own before, 25 ms -> 0.16.
 // Bound: most likely the operands' way from L2 (1024^3 moves 134 MB in 64 x 64 tiles, 4.4 - 5.6 TB/s); no counter has been read.
 #include "mfma_common.h"
@@ -67,8 +67,12 @@ template <> struct Form<double> {
   static __device__ __forceinline__ int out_col(int lane, int e) { return 16 * ((e >> 2) & 1) + (lane & 15); }
 };
 
-// RB: 32 x 32 blocks per wave along either direction
-template <typename T, int RB, int WM, int WN, int KG>
+// RB: 32 x 32 blocks per wave along either direction.
+// DEPTH: 1, the next chunk is requested before a chunk is multiplied; more: as many chunks in flight.  One chunk ahead is 2048
+// cycles of a float wave of 2 x 2 blocks, less than operands take that are in no cache yet; four in flight, for which one wave per
+// SIMD has registers (256): 1024^3 on new operands 31.6 - 35.4 -> 27.2 - 29.3 us (three layouts; six 29.9 - 31.5).  Double has
+// none for a third chunk (181 spills, 81 - 100 us).
+template <typename T, int RB, int WM, int WN, int KG, int DEPTH>
 __global__ __launch_bounds__(64 * WM * WN * KG) void mfma_small_kernel(const Problem p) {
   using F = Form<T>;
   constexpr int WT = 32 * RB, BM = WT * WM, BN = WT * WN, OUTS = 16 / KG;
@@ -138,17 +142,43 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void mfma_small_kernel(const Pro
   };
   const int whole = max(ke - kb, 0) / F::KC;                  // whole chunks of the range
   int chunks = whole > kg ? (whole - kg + KG - 1) / KG : 0;   // ... of which this wave's
-  Chunk c0, c1;
-  if (chunks > 0) fetch(c0);
-  for (; chunks >= 2; chunks -= 2) {
-    fetch(c1);
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(c0);
-    if (chunks > 2) fetch(c0);
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(c1);
+  constexpr int SLOTS = DEPTH > 1 ? DEPTH : 2;
+  Chunk c[SLOTS];
+  if constexpr (DEPTH == 1) {
+    if (chunks > 0) fetch(c[0]);
+    for (; chunks >= 2; chunks -= 2) {
+      fetch(c[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(c[0]);
+      if (chunks > 2) fetch(c[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(c[1]);
+    }
+    if (chunks == 1) multiply(c[0]);
+  } else {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+      if (d < chunks) fetch(c[d]);
+    int t = 0;   // chunks multiplied; t .. t + DEPTH - 1 are in flight
+    for (; t + 2 * DEPTH <= chunks; t += DEPTH) {   // (nothing conditional in here: the waits count the loads)
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+        multiply(c[d]);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(c[d]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      if (t + d < chunks) multiply(c[d]);
+      if (t + DEPTH + d < chunks) fetch(c[d]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+      if (t + DEPTH + d < chunks) multiply(c[d]);
   }
-  if (chunks == 1) multiply(c0);
   if (whole % KG == kg && kb + whole * F::KC < ke) {
     // the rest of the k range, less than a chunk: what is past its end counts as zero in both operands
     const int left = ke - (kb + whole * F::KC);
@@ -158,10 +188,10 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void mfma_small_kernel(const Pro
       for (int i = 0; i < F::PER; ++i) {
         const int kk = F::k_of(lane, i), back = min(kk, left - 1) - F::k_of(lane, 0);   // (pointers stand at k_of(lane, 0))
         const T va = pa[x][back * p.sa_k], vb = pb[x][back * p.sb_k];
-        c0.a[x / F::ROWS][x % F::ROWS][i] = kk < left ? va : T(0);
-        c0.b[x / F::ROWS][x % F::ROWS][i] = kk < left ? vb : T(0);
+        c[0].a[x / F::ROWS][x % F::ROWS][i] = kk < left ? va : T(0);
+        c[0].b[x / F::ROWS][x % F::ROWS][i] = kk < left ? vb : T(0);
       }
-    multiply(c0);
+    multiply(c[0]);
   }
 
   // ---- epilogue: this wave finishes accumulators kg * OUTS ... of every lane of each of its blocks
@@ -219,11 +249,11 @@ __global__ __launch_bounds__(64 * WM * WN * KG) void mfma_small_kernel(const Pro
     }
 }
 
-template <typename T, int RB, int WM, int WN, int KG> static hipError_t launch_as(const Problem &p, hipStream_t s) {
+template <typename T, int RB, int WM, int WN, int KG, int DEPTH = 1> static hipError_t launch_as(const Problem &p, hipStream_t s) {
   constexpr int BM = 32 * RB * WM, BN = 32 * RB * WN;
   const long long tiles = (long long)((p.m + BM - 1) / BM) * ((p.n + BN - 1) / BN);
   if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
-  launch_kernel((mfma_small_kernel<T, RB, WM, WN, KG>), dim3((unsigned)tiles, p.workspace ? p.slices : 1, p.batch), dim3(64 * WM * WN * KG), 0, s, p);
+  launch_kernel((mfma_small_kernel<T, RB, WM, WN, KG, DEPTH>), dim3((unsigned)tiles, p.workspace ? p.slices : 1, p.batch), dim3(64 * WM * WN * KG), 0, s, p);
   return take_launch_status();
 }
 
@@ -251,12 +281,17 @@ template <typename T> static Shape shape_for(const Problem &p) {
 
 template <typename T> static hipError_t launch(const Problem &p, hipStream_t s) {
   if (p.m == 0 || p.n == 0) return hipSuccess;
+  constexpr bool f64 = sizeof(T) == 8;
+  // (float, single blocks: two chunks in flight where both operands are k-contiguous, four 16-byte loads a chunk: 512^3 7.7 -> 7.0 us,
+  // 128 x 96 x 1360 13.1 -> 11.9, 1200^3 66 -> 56.  Elsewhere a chunk is more loads of single elements and the plain loop is a few per
+  // cent faster: 624 x 1184 x 299 11.5 / 12.1; double 1984 x 432 x 286 18.7 / 20.3.)
+  const bool vectors = !f64 && p.sa_k == 1 && p.sb_k == 1;
   switch (shape_for<T>(p)) {
-    case kWide: return launch_as<T, 2, 1, 1, sizeof(T)>(p, s);
+    case kWide: return launch_as<T, 2, 1, 1, sizeof(T), f64 ? 1 : 4>(p, s);
     case kSideBySide: return launch_as<T, 1, 2, 2, 1>(p, s);
-    case kBlock16: return launch_as<T, 1, 1, 1, 16>(p, s);
-    case kBlock8: return launch_as<T, 1, 1, 1, 8>(p, s);
-    default: return launch_as<T, 1, 1, 1, 4>(p, s);
+    case kBlock16: return vectors ? launch_as<T, 1, 1, 1, 16, f64 ? 1 : 2>(p, s) : launch_as<T, 1, 1, 1, 16>(p, s);
+    case kBlock8: return vectors ? launch_as<T, 1, 1, 1, 8, f64 ? 1 : 2>(p, s) : launch_as<T, 1, 1, 1, 8>(p, s);
+    default: return vectors ? launch_as<T, 1, 1, 1, 4, f64 ? 1 : 2>(p, s) : launch_as<T, 1, 1, 1, 4>(p, s);
   }
 }
 

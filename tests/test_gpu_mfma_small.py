@@ -84,3 +84,22 @@ def test_sums_of_numbers_that_round(lib, dtype, shape):
         torch.cuda.synchronize()
         diff = np.abs(dD.cpu().numpy().astype(wide) - want).astype(np.float64)
         assert (diff <= bound).all(), (shape, order, float((diff / bound).max()))
+
+
+@pytest.mark.parametrize("shape", [(1000, 840), (50, 40)])
+def test_chunks_in_flight(lib, shape):
+    """Float: none to eleven chunks of 16 k for a wave of four (2 x 2 blocks each, 1000 x 840; one block, 50 x 40), whole and
+    ragged, so that a range ends at every place of the ring of chunks under way."""
+    import torch
+    import cuasr_amd
+    m, n = shape
+    rng = np.random.default_rng(3)
+    for k in [512 + 16 * i for i in range(13)] + [519, 545, 575, 700] if m == 1000 else [16 * i for i in range(1, 45)] + [5, 33, 97, 350]:
+        A, B = rng.integers(-4, 5, (m, k)).astype(np.float32), rng.integers(-4, 5, (k, n)).astype(np.float32)
+        want = A @ B   # (small integers: exact)
+        for order in ("CF", "FC"):
+            dA, dB = (torch.from_numpy(np.ascontiguousarray(x if o == "C" else x.T)).cuda() for x, o in zip((A, B), order))
+            dA, dB = dA if order[0] == "C" else dA.t(), dB if order[1] == "C" else dB.t()
+            D = torch.zeros(m, n, device="cuda")
+            cuasr_amd.srgemm("plus", "multiplies", dA, dB, D, D, 1.0, 0.0, 0.0, 1.0)
+            assert np.array_equal(D.cpu().numpy(), want), (shape, k, order)
