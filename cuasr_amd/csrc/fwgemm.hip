@@ -1559,6 +1559,82 @@ __global__ void __launch_bounds__(512) fw_close_kernel(T *d, int64_t ld, int bb,
   fw_close_dist<T, 512>(d, ld, bb, hist, closed, closed_t, sm);
 }
 
+// A block step's product, everything outside block row and block column (and the next diagonal block, which has had its
+// update), while the first workgroup closes that next diagonal block.  A workgroup keeps 128 rows of the block column in LDS
+// and takes its share of the matrix's columns, sixteen at a time, the next sixteen on their way meanwhile; improved elements
+// are looked up in LDS, where the tile kernel gathers them from memory.
+// What bounds it: the closure, 33 us of floats and 62 of doubles, up to about n = 1600 (a step is panels 9, update 5, closure;
+// with one thread per element after the closure, or the closure beside tiles on all of a compute unit's registers, us a job at
+// density 0.1, before / now: f32 n = 704 328 / 292, 1050 566 / 446, 1408 690 / 580; f64 768 685 / 542, 1152 1028 / 835, 1600 1387 / 1182);
+// then the products' chains of minima, 27 TOPS, at two workgroups per compute unit: n = 2100, where 256 tiles and a closure are two
+// rounds, 1704 / 1038, 3000 3130 / 2530.  (Two rows to a lane, for half the reads of LDS per term: 951 -> 1030 at n = 2000.)
+// 128 registers for floats: two workgroups to a compute unit, at five spilled registers of the closure's, which does not show.
+template <typename T> __global__ void __launch_bounds__(FW_LINE_THREADS, sizeof(T) == 4 ? 4 : 2) fw_step_kernel(FwPanels p, int a0, int abb) {
+  __shared__ union {
+    FwLineLds<T> lines;
+    FwCloseLds<T> close;
+  } sm;
+  typedef typename vec4_of<T>::type V4;
+  typedef typename uvec4_of<T>::type U4;
+  T *const dist = static_cast<T *>(p.dist);
+  if (abb > 0 && blockIdx.x == 0) {
+    fw_close_dist<T, FW_LINE_THREADS>(dist + a0 + int64_t(a0) * p.ld, p.ld, abb, const_cast<T *>(static_cast<const T *>(p.hist)), nullptr, nullptr, sm.close);
+    return;
+  }
+  constexpr int LINES = FwLineLds<T>::LINES;
+  const int rows = (p.n + FW_BLOCK - 1) / FW_BLOCK - 1, columns = (p.n + LINES - 1) / LINES - FW_BLOCK / LINES;   // groups of either
+  const int b = blockIdx.x - (abb > 0), parts = (gridDim.x - (abb > 0)) / rows;
+  int r0 = b % rows * FW_BLOCK;
+  if (r0 >= p.k0) r0 += FW_BLOCK;
+  // (the last rows are taken from where 128 of them end with the matrix; the rows that are another workgroup's are not stored)
+  const int tid = threadIdx.x, i = tid & 127, first = __builtin_amdgcn_readfirstlane(tid >> 7) * 4, base = min(r0, p.n - FW_BLOCK), row = base + i;
+  V4 v;
+  T next[4];
+  auto column = [&](int g) { return g * LINES + (g * LINES >= p.k0 ? FW_BLOCK : 0); };
+  auto request = [&](int c0) {
+    v = *reinterpret_cast<const U4 *>(dist + p.k0 + (tid & 31) * 4 + int64_t(min(c0 + (tid >> 5), p.n - 1)) * p.ld);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) next[c] = dist[row + int64_t(min(c0 + first + c, p.n - 1)) * p.ld];
+  };
+  int g = b / rows;
+  request(column(g));
+  fw_fetch_whole<T>(sm.lines, dist + base + int64_t(p.k0) * p.ld, p.ld, FW_BLOCK);
+#pragma unroll 1
+  for (;;) {
+    *reinterpret_cast<V4 *>(&sm.lines.other[tid >> 5][(tid & 31) * 4]) = v;
+    T curr[4];
+    int32_t par[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) curr[c] = next[c];
+    __syncthreads();
+    const int c0 = column(g);
+    g += parts;
+    if (g < columns) request(column(g));
+    if (!(abb > 0 && r0 == a0 && c0 >= a0 && c0 < a0 + FW_BLOCK)) {
+      fw_lines<T, 4>(sm.lines, i, first, FW_BLOCK / FwLineLds<T>::CK, p.k0, curr, par);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int col = c0 + first + c;
+        if (row < r0 || col >= p.n || par[c] < 0) continue;
+        dist[row + int64_t(col) * p.ld] = curr[c];
+        p.parent[row + int64_t(col) * p.ldp] = par[c];
+      }
+    }
+    if (g >= columns) break;
+    __syncthreads();   // these columns have been read
+  }
+}
+// Workgroups: as many shares of the columns per 128 rows as leave every workgroup a place, in shares that differ by no more than
+// sixteen columns.  One to a compute unit while the closure takes longer than all of them (f32 n = 1408 580 us a job, 587 with
+// two; 1900 905, 915), two from there on (2300 1470 with one, 1319 with two); doubles have the LDS for one.
+inline unsigned fw_step_groups(bool f64, int n, int abb) {
+  constexpr int lines = FwLineLds<float>::LINES;
+  const int rows = (n + FW_BLOCK - 1) / FW_BLOCK - 1, columns = (n + lines - 1) / lines - FW_BLOCK / lines;
+  if (rows == 0) return 0;
+  const int places = f64 || n <= 1920 ? 255 : 510, shares = max(min(places / rows, columns), 1), each = (columns + shares - 1) / shares;
+  return unsigned(rows * ((columns + each - 1) / each) + (abb > 0));
+}
+
 template <typename T> hipError_t launch_naive(const FwArgs &g, hipStream_t stream) {
   dim3 grid((g.m + 63) / 64, (g.n + 3) / 4);
   launch_kernel(fwgemm_naive_kernel<T>, grid, dim3(256), 0, stream, g);
@@ -1717,19 +1793,17 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
   // one launch / tiled: f32 n = 8192 31 / 37, 16384 218 / 227, 20000 395 / 406, 30000 1238 / 1256, f64 8192 59 / 69, 16384 421 / 436,
   // 18000 555 / 570.
   const bool paired = panels != CUASR_AMD_PANELS_TILED;
-  // With tiles a step's launch also closes the next block, after a launch that updates it; without, a closure alone on
-  // the chip takes most of a step.  us a job with tiles at density 0.02, 0.5 / without: f32 n = 768 400, 380 / 352, 850 463, 439 /
-  // 423, 928 477, 454 / 472, 1000 527, 487 / 560; f64 640 625, 601 / 518, 768 728, 687 / 683, 832 802, 752 / 764, 850 825, 775 / 815,
-  // 1024 921, 860 / 1102.
-  const bool naive = n <= (f64 ? 768 : 928);
-  // Where the closure hides beside a product it leaves the panels a copy of its block and of the transpose.  Alone on the chip
-  // its stores are on the critical path (57.6 us a closure of doubles without them, 63.1 with; 31.6 and 34.0 of floats) and
-  // the panels read the block from the matrix: f64 n = 130 / 464 / 768 119 / 382 / 709 us a job with copies, 113 / 368 / 683 from
-  // the matrix, f32 72 / 205 / 363 and 69 / 201 / 352.  With tiles, from the matrix: f32 n = 1000 487 -> 494, 2000 1006 -> 1018,
+  // The product and the closure of the next block (after a launch that updates that) are one launch, of fw_step_kernel or of
+  // the tile kernel: fw_step_in_lines.  Panels by tiles leave the closure a launch of its own where one thread per element is
+  // faster than tiles, as does the last product of a graph that does not end with a whole block.
+  const bool lines = paired && fw_step_in_lines(f64, n), naive = n <= (f64 ? 768 : 928);
+  // Where the closure hides beside a product it leaves the panels a copy of its block and of the transpose.  Where it is on the
+  // critical path its stores would be too (57.6 us a closure of doubles without them, 63.1 with; 31.6 and 34.0 of floats) and
+  // the panels read the block from the matrix.  With tiles, from the matrix: f32 n = 1000 487 -> 494, 2000 1006 -> 1018,
   // f64 1300 1210 -> 1219, 2800 3974 -> 3991.  But doubles with 18 to 20 blocks have 578 to 722 tiles (64 x 128) on 512 places, and
-  // the launch ends not long after the closure: from the matrix 2177 2858 -> 2807, 2304 2751 -> 2679, 2560 3238 -> 3218 (2450 3349 ->
+  // the launch ends not long after the closure: from the matrix 2560 3238 -> 3218 (2450 3349 ->
   // 3357 and, at half the edges, 3150 -> 3134).
-  const bool copies = paired && !naive && !(f64 && n > 17 * FW_BLOCK && n <= 20 * FW_BLOCK);
+  const bool copies = paired && !lines && !naive && !(f64 && n > 17 * FW_BLOCK && n <= 20 * FW_BLOCK);
   char *closed_copy = copies ? C : nullptr, *closed_copy_t = copies ? R : nullptr;
   // this step's diagonal block had its distances closed during the step before, beside that step's big product
   // (its predecessors are always still to be found, from what the closure recorded in H)
@@ -1809,7 +1883,7 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
     x.ldat = FW_BLOCK;
     x.skip_r0 = x.skip_c0 = k0;
     x.skip_r1 = x.skip_c1 = k0 + bb;
-    if (x.ahead_bb > 0 && !naive) {
+    if (x.ahead_bb > 0 && (lines || !naive)) {
       // this step's update of that block, by a launch of its own (32 workgroups, a few microseconds): the
       // closure can then start with the big product instead of after one of its tiles
       const dim3 grid((x.ahead_bb + 3) / 4);
@@ -1818,6 +1892,16 @@ extern "C" int cuasr_amd_apsp_blocked_panels(int dtype, int n, void *dist, int64
       if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
     } else {
       x.ahead_bb = 0;
+    }
+    if (lines && bb == FW_BLOCK) {
+      const dim3 grid(fw_step_groups(f64, n, x.ahead_bb));
+      if (grid.x > 0) {
+        if (f64) launch_kernel(fw_step_kernel<double>, grid, dim3(FW_LINE_THREADS), 0, s, panel, x.ahead0, x.ahead_bb);
+        else launch_kernel(fw_step_kernel<float>, grid, dim3(FW_LINE_THREADS), 0, s, panel, x.ahead0, x.ahead_bb);
+        if (take_launch_status() != hipSuccess) return CUASR_AMD_ERROR_INTERNAL;
+      }
+      closed = x.ahead_bb > 0;
+      continue;
     }
     r = fwgemm_run(dtype, n, n, bb, Dcol, ld, Drow, ld, dist, ld, parent, ldp, x, naive ? CUASR_AMD_KERNEL_NAIVE : CUASR_AMD_KERNEL_VALU, stream);
     if (r != CUASR_AMD_SUCCESS) return r;

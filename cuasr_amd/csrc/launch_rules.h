@@ -144,6 +144,14 @@ inline bool fwgemm_f64_half_tile(bool k_contiguous_image, int m, int64_t half_ti
   return m >= 64 && (!k_contiguous_image || half_tiles <= 256);
 }
 
+// A block step of Floyd-Warshall: 128 rows x 16 columns at a time with the block column in LDS (fw_step_kernel), or tiles of
+// 128 x 128 (doubles 64 x 128 where they are more than the compute units).  Tiles are faster per term and bound by
+// their lookups; up to 256 of them run beside a closure at half the registers' worth of waves, and the 257th workgroup is a second
+// round.  us a job, tiles at density 0.02, 0.5 / lines (0.5): f32 n = 1900 997, 928 / 905; 2000 1005, 942 / 944; 2100 1704, 1567 / 1028;
+// 3000 3130, 2825 / 2510; 3600 4415, 3998 / 3921; 3800 4784, 4385 / 4362; 4096 5021, 4490 / 5110; f64 n = 1850 1664, 1566 / 1397; 2000 1725, 1619 / 1640;
+// 2048 1799, 1684 / 1837; 2100 2951, 2676 / 2084; 2304 2842, 2653 / 2616; 2400 3132, 2873 / 2894; 3000 4864, 4465 / 5035.
+inline bool fw_step_in_lines(bool f64, int n) { return f64 ? n <= 1920 || (n > 2048 && n <= 2304) : n <= 3712; }
+
 // The binary16 tile (half_tile.h), by its rows: 128 x 256, 64 x 128, 32 x 128 and, for adds that do not care about order,
 // 16 x 128.  ordered: plus.  bits: or-and on masks and the bitwise pairs.  zeros: min- and max-times on binary16.
 // A compute unit holds at most two of these workgroups (two waves per SIMD) and works two off faster than one, but not

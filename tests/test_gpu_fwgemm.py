@@ -306,6 +306,32 @@ def test_apsp_blocked_panels_of_ragged_blocks(oracle, n, pad, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+# one group of rows, whole and ragged, and of columns; the sizes at which the product's form or the share of a workgroup changes (float
+# 1920, double 1920, 2048 and 2304)
+@pytest.mark.parametrize("n,pad", [(256, 0), (257, 1), (272, 2), (300, 0), (384, 4), (1537, 3), (1920, 0), (1921, 1), (2049, 1), (2304, 0), (2305, 2)])
+def test_apsp_blocked_products_beside_the_closure(oracle, n, pad, dtype):
+    """Block steps in 128 rows x 16 columns: most pairs improve at every step's rate, weights round, odd leading dimensions,
+    nothing written past the matrices; dist and parent equal the oracle's bit for bit."""
+    import torch
+    rng = np.random.default_rng(3 * n)
+    W = np.where(rng.random((n, n)) < (0.4 if n < 1000 else 0.03), rng.uniform(1, 100, (n, n)), np.inf).astype(dtype)
+    np.fill_diagonal(W, 0)
+    host = np.full((n + pad, n), -5.0, dtype=dtype, order="F")
+    host[:n] = W
+    dD = to_device(host)
+    dP = torch.full((n, n + pad), -1, dtype=torch.int32, device="cuda").t()
+    ws = torch.full((cuasr_amd.apsp_blocked_workspace_bytes(n, "f32" if dtype == np.float32 else "f64"),), 0xff, dtype=torch.uint8,
+                    device="cuda")   # (NaN patterns)
+    cuasr_amd.apsp_blocked(dD[:n], dP[:n], ws)
+    got, parent = dD.cpu().numpy(), dP.cpu().numpy()
+    assert (got[n:] == -5.0).all() and (parent[n:] == -1).all()
+    want_d, want_p = np.asfortranarray(W), np.full((n, n), -1, np.int32, order="F")
+    oracle.apsp_blocked(want_d, want_p, 128)
+    assert_same_bits(np.ascontiguousarray(got[:n]), np.ascontiguousarray(want_d), "dist")
+    assert np.array_equal(parent[:n], want_p)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n,pad", [(100, 0), (384, 0), (513, 1), (700, 4), (1475, 1), (2193, 3)])
 def test_apsp_blocked_with_tiled_panels(oracle, n, pad, dtype):
     """The other way a block step can update its block row and column (copies, two launches of the tiled kernel
