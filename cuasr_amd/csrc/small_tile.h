@@ -128,21 +128,24 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> struct Sm
       }
     }
     static __device__ __forceinline__ void store(const T (&r)[PER], S (*dst)[B + pad(B)], bool xc, bool vec, int lane) {
-      if (vec) {
+      if (vec && xc) {
 #pragma unroll
         for (int p = 0; p < VECS; ++p) {
           int xx, kk;
-          at(p, xc, lane, xx, kk);
-          if (xc) {
-            typedef S svec_t __attribute__((ext_vector_type(VW)));
-            svec_t t;
+          at(p, true, lane, xx, kk);
+          typedef S svec_t __attribute__((ext_vector_type(VW)));
+          svec_t t;
 #pragma unroll
-            for (int e = 0; e < VW; ++e) t[e] = Ops::staged(r[p * VW + e]);
-            *reinterpret_cast<svec_t *>(&dst[kk][xx]) = t;
-          } else {
+          for (int e = 0; e < VW; ++e) t[e] = Ops::staged(r[p * VW + e]);
+          *reinterpret_cast<svec_t *>(&dst[kk][xx]) = t;
+        }
+      } else if (vec) {
 #pragma unroll
-            for (int e = 0; e < VW; ++e) dst[kk + e][xx] = Ops::staged(r[p * VW + e]);
-          }
+        for (int p = 0; p < VECS; ++p) {
+          int xx, kk;
+          at(p, false, lane, xx, kk);
+#pragma unroll
+          for (int e = 0; e < VW; ++e) dst[kk + e][xx] = Ops::staged(r[p * VW + e]);
         }
       } else {
 #pragma unroll
