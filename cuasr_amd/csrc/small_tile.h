@@ -30,8 +30,8 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> struct Sm
   static constexpr int BM = 8 * RM, BN = 8 * RN;
   // per SIMD (36 doubles and their fragments leave registers for two, which LDS has room for)
   static constexpr int WAVES = RM * RN * sizeof(T) > 256 ? 2 : 4;
-  // only blocks of 32 x 32 take outputs narrower than a block
-  static constexpr bool NARROW = RM == 4 && RN == 4;
+  // only blocks of 32 x 32 take outputs narrower than a block; they, and adds that count every term, take a ragged last chunk
+  static constexpr bool NARROW = (RM == 4 && RN == 4) || !may_count_twice<ADD>::value;
   // The k-groups that neighbouring lanes of a k-contiguous load write lie 16 banks apart where there are four of them
   // and 32 where there are two (8-byte elements: 32, two to an instruction's half), so the transposing stores do not collide.
   static constexpr int pad(int b) { return sizeof(S) == 8 ? (b % 16 == 8 ? 0 : 8) : KC / VW == 2 ? 8 : 4; }
@@ -270,7 +270,6 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> struct Sm
     int k0 = kb + wave * KC;
     if constexpr (!NARROW) {
       // every chunk is whole: a ragged last one goes back over k that has been counted (there is a chunk or more)
-      static_assert(may_count_twice<ADD>::value, "k of two chunks is counted twice");
       typename Side<BM>::Places pa;
       typename Side<BN>::Places pb;
       pa.init(A, p.sa_m, p.sa_k, min(k0, ke - KC), a_xc, lane);
@@ -464,6 +463,16 @@ template <typename T, int ADD, int MUL> static hipError_t launch_small(const Pro
   return launch_small_as<T, ADD, MUL, 4, 4, KC, 4>(p, s);
 }
 
+// The smaller blocks (lone_block), sixteen waves each; 32 x 16 by eight where those have two chunks each at most (or-and counts as 4-byte
+// elements do): float 272 x 560 x 80 4.7 / 4.2 us, double 84 x 881 x 96 4.5 / 4.2, but 629 x 112 x 2400 16.2 / 18.3.
+template <typename T, int ADD, int MUL> static hipError_t launch_lone_block(const Problem &p, BlockShape b, hipStream_t s) {
+  constexpr int KC = 64 / sizeof(T);
+  if (b.cols == 32) return launch_small_as<T, ADD, MUL, 2, 4, KC, 16>(p, s);
+  if (b.rows == 16) return launch_small_as<T, ADD, MUL, 2, 2, KC, 16>(p, s);
+  if ((p.workspace ? p.k_per_slice : p.k) <= 16 * KC) return launch_small_as<T, ADD, MUL, 4, 2, KC, 8>(p, s);
+  return launch_small_as<T, ADD, MUL, 4, 2, KC, 16>(p, s);
+}
+
 // The larger blocks (block_shape): eight waves each, so that two workgroups share a compute unit.
 template <typename T, int ADD, int MUL> static hipError_t launch_block(const Problem &p, BlockShape b, hipStream_t s) {
   constexpr int KC = 64 / sizeof(T);
@@ -483,10 +492,11 @@ template <typename T, int ADD, int MUL> static hipError_t launch_block(const Pro
     return b.cols == 48 ? launch_small_as<T, ADD, MUL, 8, 6, KC / 2, 8>(p, s) : launch_small_as<T, ADD, MUL, 8, 8, KC / 2, 8>(p, s);
   }
 }
-// The blocks larger than 32 x 32 take whole chunks of k only and go back over k that has been counted for the last one.
+// The blocks other than 32 x 32 take whole chunks of k only and go back over k that has been counted for the last one, where
+// the add allows it.
 template <typename T, int ADD> static bool blocks_possible(const Problem &p) {
   constexpr int KC = 64 / sizeof(T);
-  if (!may_count_twice<ADD>::value || sizeof(T) < 4 || p.k_sub > 1 || !vector_possible<T>(p)) return false;
+  if (sizeof(T) < 4 || p.k_sub > 1 || !vector_possible<T>(p)) return false;
   // (a slice that is empty or shorter than a chunk has none to go back over)
   return p.workspace ? (p.slices - 1LL) * p.k_per_slice + KC <= p.k : p.k >= KC;
 }

@@ -829,12 +829,18 @@ static hipError_t launch_valu_sized(const Problem &p, hipStream_t s) {
   // against 213)
   constexpr bool TWO_GROUPS = order_free<T, ADD>::value && ADD != kLogicalOr && ADD != kBitXor && ADD != kBitOr && ADD != kBitAnd;
   const bool two_groups = TWO_GROUPS && k_range >= 8LL * BK && vector_possible<T>(p) && p.m > 0 && p.n > 0;
-  // (masks are left out: their term is one instruction and the panels' way to LDS longer; the times do not hold for them)
-  if constexpr (order_free<T, ADD>::value && may_count_twice<ADD>::value && !ValuTile<T, ADD, MUL, 4, 4, 32, true, false>::MASKED) {
+  // (masks and bits are left out of the larger blocks: their term is one instruction and the panels' way to LDS longer; the times do
+  // not hold for them.  Integer sums spill in blocks.)
+  constexpr bool BLOCKS = may_count_twice<ADD>::value && !ValuTile<T, ADD, MUL, 4, 4, 32, true, false>::MASKED;
+  if constexpr (order_free<T, ADD>::value && ADD != kPlus) {
     if (blocks_possible<T, ADD>(p)) {
-      const BlockShape b = vector_block(sizeof(T) == 8, vector_exact<T>(p), two_groups, p.m, p.n, double(k_range), products);
-      if (b.rows == 32) return launch_small<T, ADD, MUL>(p, s);
-      if (b.rows) return launch_block<T, ADD, MUL>(p, b, s);
+      const BlockShape lone = lone_block(sizeof(T) == 8, p.m, p.n, double(k_range), products);
+      if (lone.rows) return launch_lone_block<T, ADD, MUL>(p, lone, s);
+      if constexpr (BLOCKS) {
+        const BlockShape b = vector_block(sizeof(T) == 8, vector_exact<T>(p), two_groups, p.m, p.n, double(k_range), products);
+        if (b.rows == 32 && b.cols == 32) return launch_small<T, ADD, MUL>(p, s);
+        if (b.rows) return launch_block<T, ADD, MUL>(p, b, s);
+      }
     }
   }
   if constexpr (order_free<T, ADD>::value) {

@@ -3,6 +3,8 @@
 //   staged <m> <n> <batch> <full m> <full n>   1: the full-size tile in two groups, 0: not (quarter-size: 64 x 64)
 //   half <ordered> <bits> <zeros> <m> <n> <products>   rows of the binary16 tile
 //   block <f64> <whole vectors> <m> <n> <k> <products>   100 rows + columns of the block, 0: the staged family's tile or 32 x 32
+//   lone <f64> <m> <n> <k> <products>      the same of the blocks that get a compute unit each, 0: none
+//   lines <f64> <n>                        1: a block step of Floyd-Warshall keeps the block column in LDS, 0: tiles
 //   share <rest> <parts> <part>            where the part of a ragged k-tile begins
 #include <cstdio>
 #include <cstring>
@@ -29,6 +31,16 @@ int main() {
       if (std::scanf("%d %d %d %d %d %lld", &f64, &whole, &m, &n, &k, &products) != 6) return 2;
       const cuasr_amd::BlockShape b = cuasr_amd::vector_block(f64, whole, k >= (f64 ? 128 : 256), m, n, k, products);
       answer = b.rows * 100 + b.cols;
+    } else if (!std::strcmp(what, "lone")) {
+      int f64, m, n, k;
+      long long products;
+      if (std::scanf("%d %d %d %d %lld", &f64, &m, &n, &k, &products) != 5) return 2;
+      const cuasr_amd::BlockShape b = cuasr_amd::lone_block(f64, m, n, k, products);
+      answer = b.rows * 100 + b.cols;
+    } else if (!std::strcmp(what, "lines")) {
+      int f64, n;
+      if (std::scanf("%d %d", &f64, &n) != 2) return 2;
+      answer = cuasr_amd::fw_step_in_lines(f64, n);
     } else if (!std::strcmp(what, "share")) {
       int rest, parts, part;
       if (std::scanf("%d %d %d", &rest, &parts, &part) != 3) return 2;

@@ -178,3 +178,61 @@ def test_larger_blocks_in_slices(oracle, lib, case, short):
                             kernel="valu")
     torch.cuda.synchronize()
     assert_same_bits(to_host(dD, dt), want, f"{case} {short}")
+
+
+# (block, double, products, m, n, k), row-major C: the smallest of each, whole and ragged, 256 of them, one chunk of k and a ragged one,
+# fewer chunks than waves and more; 32 x 16 by eight waves and by sixteen (test_launch_rules.py asks the rule for the block)
+LONE = [(1616, 0, 1, 16, 16, 16), (1616, 0, 1, 17, 31, 17), (1616, 0, 1, 250, 255, 33), (1616, 0, 1, 256, 256, 515), (1616, 1, 1, 16, 18, 8),
+        (1616, 1, 1, 33, 47, 9), (1616, 1, 1, 240, 270, 300), (3216, 0, 1, 629, 112, 300), (3216, 0, 1, 500, 250, 256), (3216, 0, 1, 275, 559, 81),
+        (3216, 1, 1, 300, 400, 129), (3216, 1, 1, 1024, 93, 100), (1632, 0, 1, 109, 1027, 130), (1632, 1, 1, 110, 1028, 21), (1616, 0, 9, 33, 63, 50),
+        (3216, 1, 5, 129, 130, 41), (1632, 0, 6, 17, 599, 140)]
+
+
+@pytest.mark.parametrize("case", LONE, ids=lambda c: "x".join(map(str, c)))
+def test_blocks_of_a_compute_unit_each(oracle, lib, case):
+    """Blocks of 16 x 16, 32 x 16 and 16 x 32: chunks that go back over counted k (minima, masks), ragged chunks (exclusive or), blocks at
+    the far edges that start earlier, C in place; products of a batch."""
+    import torch
+    import cuasr_amd
+    from cuasr_amd import inputs
+    _, f64, products, m, n, k = case
+    pairs = [("minimum", "plus"), ("maximum", "minimum"), ("maximum", "multiplies"), ("logical_or", "logical_and")]
+    pairs = [(a, b, "f64" if f64 else "f32") for a, b in pairs] + ([] if f64 else [("minimum", "plus", "i32"), ("bit_xor", "bit_and", "u32")])
+    for add, mult, dt in pairs:
+        ident, one = cuasr_amd.op_identity(add, dt, True), cuasr_amd.op_identity(mult, dt, True)
+        if products > 1:
+            ops = [_case(inputs, dt, m, n, k, "CCC", 5000 + 7 * i) for i in range(products)]
+            dA, dB, dC = (torch.stack([to_device(np.ascontiguousarray(o[j])) for o in ops]) for j in range(3))
+            cuasr_amd.srgemm_batched(add, mult, dA, dB, dC, dC, one, one, ident, one, dtype=dt, kernel="valu")
+            torch.cuda.synchronize()
+            for i in range(products):
+                assert_same_bits(to_host(dC[i], dt), oracle.srgemm(add, mult, *ops[i], one, one, ident), f"{add} {mult} {dt} product {i}")
+            continue
+        for i, order in enumerate(("FFC", "CCC", "CFF", "FCC")):
+            shape = (n, m, k) if order[2] == "F" else (m, n, k)   # (a column-major output is the transposed problem)
+            A, B, C = _case(inputs, dt, *shape, order, 331 + i)
+            want = oracle.srgemm(add, mult, A, B, C, one, one, ident)
+            dC = to_device(C)
+            dD = dC if i == 1 else to_device(np.zeros_like(C))
+            cuasr_amd.srgemm(add, mult, to_device(A), to_device(B), dC, dD, one, one, ident, one, dtype=dt, kernel="valu")
+            torch.cuda.synchronize()
+            assert_same_bits(to_host(dD, dt), want, f"{add} {mult} {dt} {shape} {order}")
+
+
+@pytest.mark.parametrize("dt", ["f32", "f64"])
+@pytest.mark.parametrize("short", [0, 30])
+def test_blocks_of_a_compute_unit_each_in_slices(oracle, lib, dt, short):
+    import torch
+    import cuasr_amd
+    from cuasr_amd import inputs
+    for m, n, slices, per in ((60, 70, 8, 144), (100, 130, 4, 96)):   # (16 x 16: 160 blocks; 252)
+        k = slices * per - short
+        for add, mult in (("minimum", "plus"), ("maximum", "minimum")):
+            ident, one = cuasr_amd.op_identity(add, dt, True), cuasr_amd.op_identity(mult, dt, True)
+            A, B, C = _case(inputs, dt, m, n, k, "CFC", 83)
+            want = oracle.srgemm(add, mult, A, B, C, one, one, ident)
+            work = torch.empty(cuasr_amd.splitk_workspace_bytes(m, n, slices, dt), dtype=torch.uint8, device="cuda")
+            dD = to_device(np.zeros_like(C))
+            cuasr_amd.srgemm_splitk(add, mult, to_device(A), to_device(B), to_device(C), dD, slices, work, one, one, ident, one, dtype=dt, kernel="valu")
+            torch.cuda.synchronize()
+            assert_same_bits(to_host(dD, dt), want, f"{m} {n} {add} {slices} {short}")

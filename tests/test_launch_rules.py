@@ -87,3 +87,22 @@ def test_vector_blocks():
     asked += [(f"block 1 {int(n % 2 == 0)} {n} {n} {n} 1", block) for n, block in
               [(300, 0), (480, 0), (518, 4032), (560, 4032), (600, 4832), (758, 4848), (800, 4032), (1008, 0), (1100, 4032), (1408, 0)]]
     assert _ask([question for question, _ in asked]) == [block for _, block in asked]
+
+
+def test_lone_blocks():
+    """The block that the tests of the smaller blocks say they run, both sides of the lines at sizes where both were timed, and
+    none for a side shorter than a block."""
+    import test_gpu_small_tile as small
+    asked = [(f"lone {f64} {m} {n} {k} {products}", block) for block, f64, products, m, n, k in small.LONE]
+    asked += [(f"lone 0 {m} {n} {k} 1", block) for m, n, k, block in
+              [(256, 256, 256, 1616), (112, 128, 1674, 1616), (812, 80, 1040, 1616), (629, 112, 2400, 3216), (885, 133, 3690, 3216),
+               (400, 323, 1088, 0), (311, 704, 90, 3216), (311, 704, 129, 0), (15, 64, 300, 0), (15, 16, 16, 0), (16, 16, 16, 1616)]]
+    asked += [(f"lone 1 {m} {n} {k} 1", block) for m, n, k, block in
+              [(96, 128, 2336, 1616), (1024, 93, 3328, 3216), (109, 1027, 2021, 1632), (582, 212, 3083, 0), (304, 736, 96, 0)]]
+    assert _ask([question for question, _ in asked]) == [block for _, block in asked]
+
+
+def test_steps_in_lines():
+    asked = [(f"lines {f64} {n}", n_lines) for f64, n, n_lines in
+             [(0, 129, 1), (0, 3712, 1), (0, 3713, 0), (1, 1920, 1), (1, 1921, 0), (1, 2048, 0), (1, 2049, 1), (1, 2304, 1), (1, 2305, 0)]]
+    assert _ask([question for question, _ in asked]) == [n_lines for _, n_lines in asked]
