@@ -1626,12 +1626,12 @@ template <typename T> __global__ void __launch_bounds__(FW_LINE_THREADS, sizeof(
 }
 // Workgroups: as many shares of the columns per 128 rows as leave every workgroup a place, in shares that differ by no more than
 // sixteen columns.  One to a compute unit while the closure takes longer than all of them (f32 n = 1408 580 us a job, 587 with
-// two; 1900 905, 915), two from there on (2300 1470 with one, 1319 with two); doubles have the LDS for one.
+// two; 1900 905, 915), two from there on (2000 949, 950; 2048 1050 with one, 965 with two); doubles have the LDS for one.
 inline unsigned fw_step_groups(bool f64, int n, int abb) {
   constexpr int lines = FwLineLds<float>::LINES;
   const int rows = (n + FW_BLOCK - 1) / FW_BLOCK - 1, columns = (n + lines - 1) / lines - FW_BLOCK / lines;
   if (rows == 0) return 0;
-  const int places = f64 || n <= 1920 ? 255 : 510, shares = max(min(places / rows, columns), 1), each = (columns + shares - 1) / shares;
+  const int places = f64 || n <= 1984 ? 255 : 510, shares = max(min(places / rows, columns), 1), each = (columns + shares - 1) / shares;
   return unsigned(rows * ((columns + each - 1) / each) + (abb > 0));
 }
 

@@ -102,19 +102,20 @@ inline BlockShape block_shape(bool f64, int m, int n, double k, long long produc
   return best;
 }
 
-// The blocks of outputs too small to give every compute unit one of 32 x 32: the largest of which each still gets one
-// at most, smallest first.  A block's time is nearly its waves' alone, so half the block is little more than half the time although it
+// The blocks of outputs too small to give every compute unit one of 32 x 32: the smallest of which each still gets one
+// at most.  A block's time is nearly its waves' alone, so half the block is little more than half the time although it
 // reads more of LDS per term.  Where there are more blocks than compute units that reverses.
 // us, min-plus on 32 x 32 / here: float 112 x 128 x 1674 (56 blocks of 16 x 16) 18.4 / 10.3, 812 x 80 x 1040 (255) 13.1 / 7.8, 629 x 112 x 2400 (280;
 // on 32 x 16, 140, 24.1 / 16.2), 885 x 133 x 3690 (252 of 32 x 16, 504 of 16 x 16) 35.9 / 24.5 and 37.4, 400 x 323 x 1088 (273 of 32 x 16) 13.2 / 14.9,
 // 64 x 112 x 94 7.4 / 3.1; double 96 x 128 x 2336 47.6 / 16.7, 1024 x 93 x 3328 69.3 / 39.6, 582 x 212 x 3083 (266 of 32 x 16) 65 / 67.
-// 4-byte elements and at most 128 of k: two blocks of 32 x 16 on a compute unit too, 311 x 704 x 90 (440) 7.2 / 4.5, 174 x 880 x 80 (330) 5.3 / 4.2.
+// Up to 480 of k, 256 in double, two blocks of 32 x 16 on a compute unit too where 32 x 32 leaves some idle: 311 x 704 x 90 (440) 7.2 / 4.5,
+// 496 x 314 x 284 (320) 8.4 / 6.3, but 720 x 192 x 512 8.3 / 8.5; double 271 x 736 x 143 (414) 7.4 / 6.6, but 1434 x 134 x 512 15.3 / 16.5.
 inline BlockShape lone_block(bool f64, int m, int n, double k, long long products) {
   auto blocks = [&](int rows, int cols) {
     return m < rows || n < cols ? 1LL << 40 : ((long long)m + rows - 1) / rows * (((long long)n + cols - 1) / cols) * products;
   };
   if (blocks(16, 16) <= 256) return BlockShape{16, 16};
-  if (blocks(32, 16) <= (f64 || k > 128 ? 256 : 512)) return BlockShape{32, 16};
+  if (blocks(32, 16) <= (k <= (f64 ? 256 : 480) && blocks(32, 32) <= 256 ? 512 : 256)) return BlockShape{32, 16};
   if (blocks(16, 32) <= 256) return BlockShape{16, 32};
   return BlockShape{0, 0};
 }

@@ -41,9 +41,12 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> struct Sm
   typedef S s4_t __attribute__((ext_vector_type(SV)));
 
   struct alignas(16) Panels { S a[KC][BM + pad(BM)], b[KC][BN + pad(BN)]; };
-  union Smem {
-    Panels p[W];
-    S acc[W][4 * RN * ASTRIDE];
+  struct Smem {
+    union {
+      Panels p[W];
+      S acc[W][4 * RN * ASTRIDE];
+    };
+    int has_zero[Ops::ZERO_SIGN ? W : 1];   // ZERO_SIGN: wave w has an accumulator that is zero
   };
 
   // Lane l's elements along a side of R: groups of four, then what is left of R, each group 8 lanes wide.
@@ -336,6 +339,18 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> struct Sm
     }
     if (!NARROW && e.source_needed) fetch_source();   // (it arrives under the fold: the product has no registers for it)
     int zeros = 0;   // ZERO_SIGN: 1 where the block's zeros are all +0, -1 where they are not known to be
+    bool any_zero = false;
+    if constexpr (Ops::ZERO_SIGN) {
+      // (a minimum that is zero is one of the waves': without any, the fold below passes no barrier for it, which two per
+      // cent of double 416 x 339 x 736 went to)
+      bool zero = false;
+#pragma unroll
+      for (int i = 0; i < RM; ++i)
+#pragma unroll
+        for (int j = 0; j < RN; ++j) zero |= acc[i][j] == T(0);
+      const bool wave_has = __builtin_amdgcn_ballot_w64(zero) != 0;
+      if (lane == 0) sm.has_zero[wave] = wave_has;
+    }
     T *out = reinterpret_cast<T *>(ops.D);
     long long ld_out = p.ldd;
     if (partial) {
@@ -351,6 +366,14 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> struct Sm
 #pragma unroll
         for (int j = 0; j < RN; ++j) sm.acc[wave][(i * RN + j) * ASTRIDE + lane] = acc[4 * g + i][j];
       __syncthreads();
+      if constexpr (Ops::ZERO_SIGN) {
+        if (g == 0) {
+          int any = 0;
+#pragma unroll
+          for (int w = 0; w < W; ++w) any |= sm.has_zero[w];
+          any_zero = __builtin_amdgcn_readfirstlane(any) != 0;
+        }
+      }
       // output o: false where it is not this workgroup's to store
       auto folded = [&](int o, T &v, int &row, int &col) {
         if (64 * W * o >= count) return false;
@@ -403,7 +426,7 @@ template <typename T, int ADD, int MUL, int RM, int RN, int KC, int W> struct Sm
             open |= (unsigned)z.open << o;
           }
         }
-        if (__syncthreads_or(open != 0)) {
+        if (any_zero && __syncthreads_or(open != 0)) {
           if (zeros == 0) zeros = Ops::zeros_are_positive(p, Ab, Bb, min(BM, p.m - m0), min(BN, p.n - n0), ke - kb) ? 1 : -1;
 #pragma unroll
           for (int o = 0; o < OUTS; ++o) {
@@ -463,13 +486,14 @@ template <typename T, int ADD, int MUL> static hipError_t launch_small(const Pro
   return launch_small_as<T, ADD, MUL, 4, 4, KC, 4>(p, s);
 }
 
-// The smaller blocks (lone_block), sixteen waves each; 32 x 16 by eight where those have two chunks each at most (or-and counts as 4-byte
-// elements do): float 272 x 560 x 80 4.7 / 4.2 us, double 84 x 881 x 96 4.5 / 4.2, but 629 x 112 x 2400 16.2 / 18.3.
+// The smaller blocks (lone_block), sixteen waves each; 32 x 16 by eight where those have two chunks each at most or two blocks share
+// a compute unit: float 272 x 560 x 80 4.7 / 4.2 us, double 84 x 881 x 96 4.5 / 4.2, but 629 x 112 x 2400 16.2 / 18.3.
 template <typename T, int ADD, int MUL> static hipError_t launch_lone_block(const Problem &p, BlockShape b, hipStream_t s) {
   constexpr int KC = 64 / sizeof(T);
   if (b.cols == 32) return launch_small_as<T, ADD, MUL, 2, 4, KC, 16>(p, s);
   if (b.rows == 16) return launch_small_as<T, ADD, MUL, 2, 2, KC, 16>(p, s);
-  if ((p.workspace ? p.k_per_slice : p.k) <= 16 * KC) return launch_small_as<T, ADD, MUL, 4, 2, KC, 8>(p, s);
+  const long long groups = (long long)((p.m + 31) / 32) * ((p.n + 15) / 16) * slice_groups(p) * p.batch;
+  if (groups > 256 || (p.workspace ? p.k_per_slice : p.k) <= 16 * KC) return launch_small_as<T, ADD, MUL, 4, 2, KC, 8>(p, s);
   return launch_small_as<T, ADD, MUL, 4, 2, KC, 16>(p, s);
 }
 

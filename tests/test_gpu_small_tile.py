@@ -183,8 +183,8 @@ def test_larger_blocks_in_slices(oracle, lib, case, short):
 # (block, double, products, m, n, k), row-major C: the smallest of each, whole and ragged, 256 of them, one chunk of k and a ragged one,
 # fewer chunks than waves and more; 32 x 16 by eight waves and by sixteen (test_launch_rules.py asks the rule for the block)
 LONE = [(1616, 0, 1, 16, 16, 16), (1616, 0, 1, 17, 31, 17), (1616, 0, 1, 250, 255, 33), (1616, 0, 1, 256, 256, 515), (1616, 1, 1, 16, 18, 8),
-        (1616, 1, 1, 33, 47, 9), (1616, 1, 1, 240, 270, 300), (3216, 0, 1, 629, 112, 300), (3216, 0, 1, 500, 250, 256), (3216, 0, 1, 275, 559, 81),
-        (3216, 1, 1, 300, 400, 129), (3216, 1, 1, 1024, 93, 100), (1632, 0, 1, 109, 1027, 130), (1632, 1, 1, 110, 1028, 21), (1616, 0, 9, 33, 63, 50),
+        (1616, 1, 1, 33, 47, 9), (1616, 1, 1, 240, 270, 300), (3216, 0, 1, 629, 112, 300), (3216, 0, 1, 500, 250, 256), (3216, 0, 1, 275, 559, 81), (3216, 0, 1, 350, 641, 479), (3216, 1, 1, 305, 737, 33),
+        (3216, 1, 1, 300, 400, 129), (3216, 1, 1, 1024, 93, 100), (1632, 0, 1, 109, 1027, 500), (1632, 1, 1, 110, 1028, 300), (1616, 0, 9, 33, 63, 50),
         (3216, 1, 5, 129, 130, 41), (1632, 0, 6, 17, 599, 140)]
 
 

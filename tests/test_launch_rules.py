@@ -96,9 +96,9 @@ def test_lone_blocks():
     asked = [(f"lone {f64} {m} {n} {k} {products}", block) for block, f64, products, m, n, k in small.LONE]
     asked += [(f"lone 0 {m} {n} {k} 1", block) for m, n, k, block in
               [(256, 256, 256, 1616), (112, 128, 1674, 1616), (812, 80, 1040, 1616), (629, 112, 2400, 3216), (885, 133, 3690, 3216),
-               (400, 323, 1088, 0), (311, 704, 90, 3216), (311, 704, 129, 0), (15, 64, 300, 0), (15, 16, 16, 0), (16, 16, 16, 1616)]]
+               (400, 323, 1088, 0), (311, 704, 90, 3216), (311, 704, 480, 3216), (311, 704, 481, 0), (294, 822, 70, 0), (15, 64, 300, 0), (15, 16, 16, 0), (16, 16, 16, 1616)]]
     asked += [(f"lone 1 {m} {n} {k} 1", block) for m, n, k, block in
-              [(96, 128, 2336, 1616), (1024, 93, 3328, 3216), (109, 1027, 2021, 1632), (582, 212, 3083, 0), (304, 736, 96, 0)]]
+              [(96, 128, 2336, 1616), (1024, 93, 3328, 3216), (109, 1027, 2021, 1632), (582, 212, 3083, 0), (304, 736, 256, 3216), (304, 736, 257, 0), (386, 615, 16, 0)]]
     assert _ask([question for question, _ in asked]) == [block for _, block in asked]
 
 
