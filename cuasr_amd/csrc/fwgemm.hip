@@ -1551,8 +1551,8 @@ __global__ void __launch_bounds__(256) snapshot_pair_kernel(const T *src0, T *w0
     if (c0 + 4 * u < cols) w[r + int64_t(c0 + 4 * u) * ldw] = v[u];
 }
 
-// A diagonal block's distances closed by a launch of its own: a job's first block, and every block of a job too small for
-// the tile kernel.  Its predecessors follow with those of the other blocks.
+// A diagonal block's distances closed by a launch of its own: a job's first block (with panels by tiles every block of a graph too
+// small for the tile kernel).  Its predecessors follow with those of the other blocks.
 template <typename T>
 __global__ void __launch_bounds__(512) fw_close_kernel(T *d, int64_t ld, int bb, T *hist, T *closed, T *closed_t) {
   __shared__ FwCloseLds<T> sm;
