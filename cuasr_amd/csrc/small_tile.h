@@ -1,14 +1,15 @@
 // Vector-ALU SRGEMM kernel for outputs that the staged tiles do not share out well between the compute units: too small to give the
 // 64 x 64 tile a workgroup per unit, or of a size that leaves the last round of tiles mostly empty.
 //
-// One WAVE owns a block of the output (8 x 8 lanes of RM x RN: 32 x 32 up to 64 x 64) and a share of k; the W waves of a workgroup
+// One WAVE owns a block of the output (8 x 8 lanes of RM x RN: 16 x 16 up to 64 x 64) and a share of k; the W waves of a workgroup
 // work on the same block, wave w on the k-chunks w, w + W, ...  A wave stages its own chunk of A and B through its
 // own piece of LDS, so the main loop has no barrier: a wave's LDS accesses complete in order, and its next chunk
 // waits in registers while it computes.  After the loop the W accumulators of every output meet in LDS, up to four of a lane's
 // rows at a time, and each thread folds and finishes 1 / (64 W) of the outputs, in row-contiguous runs.
 //
 // Why: an output of 256 x 256 is 16 blocks of 64 x 64, which left 240 of 256 compute units idle; 32 x 32 blocks
-// spread it over 64 of them, with four to sixteen waves each by the length of k (launch_small).  Larger outputs take the block
+// spread it over 64 of them, with four to sixteen waves each by the length of k (launch_small), blocks of 16 x 16 over all (lone_block,
+// launch_rules.h: 6.4 -> 5.6 us, where the host's call sets the pace; double 208^3 8.8 -> 5.6).  Larger outputs take the block
 // that divides most evenly (launch_rules.h, block_shape): 1533^3 148 -> 115 us on 64 x 48, double 600 x 500 x 700 33.4 -> 22.6 on 40 x 32.
 //
 // What bounds the loop: in float the way of the fragments from LDS (128 bytes a cycle for 16 waves: 72 % of what a block of
